@@ -65,6 +65,22 @@ mk_status Ctx::small(size_t nbytes, void** out) {
 }
 
 
+void* Ctx::gemm_ws() {
+  const FixedScratch& fx = fixed_scratch();
+  if (fx.base) return fx.gemm_ws;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();   // the null stream while another stream captures
+    return nullptr;
+  }
+  if (cap != hipStreamCaptureStatusNone) return nullptr;
+  for (int i = 0; i < ngemmws; ++i)
+    if (gemmws[i].stream == stream) return gemmws[i].buf.ptr;
+  if (ngemmws == MAX_GEMM_WS || gemmws[ngemmws].buf.alloc(GEMM_WS_BYTES) != MK_OK) return nullptr;
+  gemmws[ngemmws].stream = stream;
+  return gemmws[ngemmws++].buf.ptr;
+}
+
 FixedScratch& fixed_scratch() {
   static thread_local FixedScratch f;
   return f;
@@ -182,10 +198,11 @@ size_t view_bytes(int64_t rows, int64_t cols, char role, int prec) {
   return prec == MK_BF16X3 ? 2 * align256(n * 2) : align256(n * 4);
 }
 
-mk_status run_gemm(const ProbSpec* p, int np, int prec, GemmShape sh, hipStream_t st) {
-  if (prec == MK_FP64) return gemm_f64(p, np, sh, st);
-  if (prec == MK_BF16X3) return gemm_bf16x3(p, np, st);
-  return gemm_f32(p, np, st);
+mk_status run_gemm(Ctx* ctx, const ProbSpec* p, int np, int prec, GemmShape sh) {
+  void* ws = ctx->gemm_ws();
+  if (prec == MK_FP64) return gemm_f64(p, np, sh, ctx->stream, ws);
+  if (prec == MK_BF16X3) return gemm_bf16x3(p, np, ctx->stream, ws);
+  return gemm_f32(p, np, ctx->stream, ws);
 }
 
 }  // namespace mk
@@ -259,12 +276,12 @@ static mk_status tl_mps_run(Ctx* ctx, const double* v, const double* A, const do
   ProbSpec p1;
   p1.M = Dm; p1.N = d * Dc; p1.C = t; p1.ldc = Dm;
   p1.add(v, Dm, A, Dn, Dn);
-  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream));
+  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream, ctx->gemm_ws()));
   // y[a,c] = Ab[(m,h),a]^T t[(m,h),c]
   ProbSpec p2;
   p2.M = Da; p2.N = Dc; p2.C = y; p2.ldc = Da;
   p2.add(Ab, Dm * d, t, Dm * d, Dm * d);
-  return gemm_f64(&p2, 1, GemmShape{true, false}, ctx->stream);
+  return gemm_f64(&p2, 1, GemmShape{true, false}, ctx->stream, ctx->gemm_ws());
 }
 
 // y[a,b] = A[a,h,i] Ab[b,h,j] v[i,j]; t holds Da d Dj doubles
@@ -274,12 +291,12 @@ static mk_status tr_mps_run(Ctx* ctx, const double* v, const double* A, const do
   ProbSpec p1;
   p1.M = Da * d; p1.N = Dj; p1.C = t; p1.ldc = Da * d;
   p1.add(A, Da * d, v, Di, Di);
-  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream));
+  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream, ctx->gemm_ws()));
   // y[a,b] = t[a,(h,j)] Ab[b,(h,j)]^T
   ProbSpec p2;
   p2.M = Da; p2.N = Db; p2.C = y; p2.ldc = Da;
   p2.add(t, Da, Ab, Db, d * Dj);
-  return gemm_f64(&p2, 1, GemmShape{false, true}, ctx->stream);
+  return gemm_f64(&p2, 1, GemmShape{false, true}, ctx->stream, ctx->gemm_ws());
 }
 
 // y[a,b,c] = x[m,g,n] A[n,h,c] O[g,k,h,b] Ab[m,k,a]; t1 holds Dm wl d Dc and
@@ -291,13 +308,13 @@ static mk_status tl_mpo_run(Ctx* ctx, const double* x, const double* O, const do
   ProbSpec p1;
   p1.M = Dm * wl; p1.N = d * Dc; p1.C = t1; p1.ldc = Dm * wl;
   p1.add(x, Dm * wl, A, Dn, Dn);
-  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream));
+  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream, ctx->gemm_ws()));
   MK_TRY(k_tl_mid(t1, O, Dm, (int)wl, (int)d, (int)wr, Dc, t2, ctx->stream));
   // y[a,(b,c)] = Ab[(m,k),a]^T t2[(m,k),(b,c)]
   ProbSpec p2;
   p2.M = Da; p2.N = wr * Dc; p2.C = y; p2.ldc = Da;
   p2.add(Ab, Dm * d, t2, Dm * d, Dm * d);
-  return gemm_f64(&p2, 1, GemmShape{true, false}, ctx->stream);
+  return gemm_f64(&p2, 1, GemmShape{true, false}, ctx->stream, ctx->gemm_ws());
 }
 
 // y[a,b,c] = A[a,h,i] O[b,k,h,l] Ab[c,k,o] v[i,l,o]; t1 holds Da d wr Do and
@@ -309,13 +326,13 @@ static mk_status tr_mpo_run(Ctx* ctx, const double* v, const double* O, const do
   ProbSpec p1;
   p1.M = Da * d; p1.N = wr * Do; p1.C = t1; p1.ldc = Da * d;
   p1.add(A, Da * d, v, Di, Di);
-  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream));
+  MK_TRY(gemm_f64(&p1, 1, GemmShape{false, false}, ctx->stream, ctx->gemm_ws()));
   MK_TRY(k_tr_mid(t1, O, Da, (int)wl, (int)d, (int)wr, Do, t2, ctx->stream));
   // y[(a,b),c] = t2[(a,b),(k,o)] Ab[c,(k,o)]^T
   ProbSpec p2;
   p2.M = Da * wl; p2.N = Dc; p2.C = y; p2.ldc = Da * wl;
   p2.add(t2, Da * wl, Ab, Dc, d * Do);
-  return gemm_f64(&p2, 1, GemmShape{false, true}, ctx->stream);
+  return gemm_f64(&p2, 1, GemmShape{false, true}, ctx->stream, ctx->gemm_ws());
 }
 
 static size_t f64b(int64_t n) { return (size_t)n * 8; }
@@ -517,7 +534,7 @@ extern "C" mk_status mk_gemm(mk_ctx h, int transa, int transb, int64_t M, int64_
   p.M = M; p.N = N; p.C = C; p.ldc = ldc; p.alpha = alpha; p.beta = beta;
   if (precision == MK_FP64) {
     p.add(A, lda, B, ldb, K);
-    return gemm_f64(&p, 1, GemmShape{transa != 0, transb != 0}, ctx->stream);
+    return gemm_f64(&p, 1, GemmShape{transa != 0, transb != 0}, ctx->stream, ctx->gemm_ws());
   }
   // K-contiguous copies: stored A is M x K (convert with transposition) or,
   // transposed, K x M (plain); stored B is K x N (plain) or N x K (transposed)
@@ -528,5 +545,5 @@ extern "C" mk_status mk_gemm(mk_ctx h, int transa, int transb, int64_t M, int64_
   MK_TRY(convert_view(ctx, A, transa ? K : M, transa ? M : K, lda, transa ? 'B' : 'A', precision, &va, ma));
   MK_TRY(convert_view(ctx, B, transb ? N : K, transb ? K : N, ldb, transb ? 'A' : 'B', precision, &vb, mb));
   p.add(va.hi, va.kpad, vb.hi, vb.kpad, K, va.lo, vb.lo);
-  return run_gemm(&p, 1, precision, GemmShape{}, ctx->stream);
+  return run_gemm(ctx, &p, 1, precision, GemmShape{});
 }

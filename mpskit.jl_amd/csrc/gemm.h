@@ -39,10 +39,18 @@ struct GemmProb {
 };
 
 // Up to MAX_PROB problems passed by value as the kernel argument.
+//
+// Tiles past the first `full_tiles` are split along K: unit u >= full_tiles is
+// slice (u - full_tiles) / tail of tile full_tiles + (u - full_tiles) % tail
+// (tail = total_tiles - full_tiles), which leaves its partial sums in `ws`;
+// splitk_reduce adds the slices in order and writes C.
 struct GemmBatch {
   GemmProb p[MAX_PROB];
   int32_t nprob;
   int32_t total_tiles;
+  int32_t full_tiles;
+  int32_t ksplit;      // slices per tail tile (1: no tail)
+  void* ws;            // (total_tiles - full_tiles) * ksplit partial tiles
 };
 
 // Any number of problems in a device-resident array (problems sorted by
@@ -114,17 +122,33 @@ struct GemmShape {
   bool ta = false, tb = false;
 };
 
-// FP64 MFMA path (gemm_f64.hip).  Enqueues on `stream`.
-mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream);
+// Workspace of the K-split launches: a fixed GEMM_WS_BYTES region per context
+// (allocated with it, so a call under stream capture allocates nothing), or
+// per GPU for the allocation-free apply.  64 MiB hold the partial tiles of one
+// full round of workgroups (512 FP64 tiles of 128 x 128, or 256 fp32 ones of
+// 256 x 256), and no split makes more.
+constexpr size_t GEMM_WS_BYTES = (size_t)64 << 20;
+
+// FP64 MFMA path (gemm_f64.hip).  Enqueues on `stream`; `ws` (GEMM_WS_BYTES, or
+// null: no K split) must not be in use by other work than the stream's own.
+mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream, void* ws);
 
 // Mixed paths (gemm_mixed.hip).  Operands are pre-converted and K-contiguous:
 //   A(i,k) = A[i*lda + k], B(k,j) = B[j*ldb + k]  (bf16 hi/lo or fp32),
 // accumulation in fp32, output C is float64 column-major (alpha/beta in fp64).
-mk_status gemm_bf16x3(const ProbSpec* probs, int nprob, hipStream_t stream);
-mk_status gemm_f32(const ProbSpec* probs, int nprob, hipStream_t stream);
+mk_status gemm_bf16x3(const ProbSpec* probs, int nprob, hipStream_t stream, void* ws);
+mk_status gemm_f32(const ProbSpec* probs, int nprob, hipStream_t stream, void* ws);
 // Whether one M x N problem whose segments have the given K values runs on the
 // 256 x 256 kernel with packed operands (the only kernel that reads them).
 bool mixed_packed_ok(int64_t M, int64_t N, const int64_t* Ks, int nk);
+
+// How a launch of `tiles` output tiles of `nsteps` K steps each (the fewest of
+// its problems) is split: the first `full` tiles whole, the others `ksplit`
+// ways.
+struct SplitPlan {
+  int full = 0;
+  int ksplit = 1;
+};
 
 // Grouped (persistent) launches over a device descriptor array.  Tile kinds:
 //   FP64:  TK_64 (64x64), TK_128 (128x128)

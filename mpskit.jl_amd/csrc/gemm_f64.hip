@@ -4,6 +4,7 @@
 // of one problem, summing every segment of that problem into the same
 // accumulators before a single fused epilogue (alpha/beta and optional CB term).
 #include "gemm_dev.h"
+#include "gemm_plan.h"
 #include "prof.h"
 
 #include <algorithm>
@@ -119,7 +120,9 @@ void gemm_f64_kernel(Src src) {
   __shared__ double As[2][BK][LDA_S];
   __shared__ double Bs[2][BK][LDB_S];
 
-  for (int t = src_first(src); t < src.total_tiles; t += src_stride(src)) {
+  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
+  int t, slice, nslice;
+  src_unit(src, un, t, slice, nslice);
   const GemmProb& P = src_prob(src, t);
   int tm, tn;
   tile_coords(P, t - P.tile_start, tm, tn);
@@ -177,22 +180,23 @@ void gemm_f64_kernel(Src src) {
     else     store_fastdir<BN, LDB_S, BK>(Bs[buf], rb);
   };
 
-  int s = 0, k0 = 0;
-  if (nsteps > 0) {
-    load(0, 0);
+  int s, k0, step0, step1;
+  slice_range<BK>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  if (step1 > step0) {
+    load(s, k0);
     store(0);
   }
   __syncthreads();
   int buf = 0;
-  int kcur = nsteps > 0 ? P.seg[0].K : 0;
-  for (int step = 0; step < nsteps; ++step) {
+  int kcur = step1 > step0 ? P.seg[s].K : 0;
+  for (int step = step0; step < step1; ++step) {
     int ns = s, nk0 = k0 + BK;
     if (nk0 >= kcur) {
       ns = s + 1;
       nk0 = 0;
       kcur = ns < P.nseg ? P.seg[ns].K : 0;
     }
-    const bool has_next = step + 1 < nsteps;
+    const bool has_next = step + 1 < step1;
     if (has_next) load(ns, nk0);
 #pragma unroll
     for (int kk = 0; kk < BK / 4; ++kk) {
@@ -221,8 +225,11 @@ void gemm_f64_kernel(Src src) {
   // at block row lk + 4 r, column li; with the B fragment as first operand the
   // block is C^T, so the lane holds C[row li][col lk + 4 r]: the 16 lanes of a
   // quarter-wave store 16 consecutive rows (128 B) of one column.
-  epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lk, P.alpha, P.beta);
-  }  // tiles
+  if (slice < 0)
+    epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lk, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<double>(src, t, slice, BM * BN), wave, lane);
+  }  // units
 }
 
 // ---------------------------------------------------------------------------
@@ -267,7 +274,9 @@ void gemm_f64_buf_kernel(Src src) {
   const int li = lane & 15;
   const int lk = lane >> 4;
 
-  for (int t = src_first(src); t < src.total_tiles; t += src_stride(src)) {
+  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
+  int t, slice, nslice;
+  src_unit(src, un, t, slice, nslice);
   const GemmProb& P = src_prob(src, t);
   int tm, tn;
   tile_coords(P, t - P.tile_start, tm, tn);
@@ -363,23 +372,24 @@ void gemm_f64_buf_kernel(Src src) {
   };
   double fa[2][FM], fb[2][FN];
 
-  int s = 0, k0 = 0;
-  if (nsteps > 0) {
-    set_seg(0);
-    load(0);
+  int s, k0, step0, step1;
+  slice_range<BK>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  if (step1 > step0) {
+    set_seg(s);
+    load(k0);
     store(0);
   }
   __syncthreads();
-  if (ROT && nsteps > 0) read_frag(0, 0, fa[0], fb[0]);
+  if (ROT && step1 > step0) read_frag(0, 0, fa[0], fb[0]);
   int buf = 0;
-  for (int step = 0; step < nsteps; ++step) {
+  for (int step = step0; step < step1; ++step) {
     k0 += BK;
     while (k0 >= K && s + 1 < P.nseg) {
       ++s;
       k0 = 0;
       set_seg(s);
     }
-    const bool has_next = step + 1 < nsteps;
+    const bool has_next = step + 1 < step1;
     if (has_next) load(k0);
     if constexpr (!ROT) {
 #pragma unroll
@@ -422,8 +432,11 @@ void gemm_f64_buf_kernel(Src src) {
   }
 
   // epilogue: as in gemm_f64_kernel
-  epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, M, N, m0 + wm0, n0 + wn0, li, lk, P.alpha, P.beta);
-  }  // tiles
+  if (slice < 0)
+    epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, M, N, m0 + wm0, n0 + wn0, li, lk, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<double>(src, t, slice, BM * BN), wave, lane);
+  }  // units
 }
 
 // Host check of the branch-free kernel's conditions for one problem.
@@ -485,7 +498,7 @@ void launch4(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src&
 }
 
 template <int BM, int BN>
-mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t stream) {
+mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t stream, SplitPlan sp, void* ws) {
   GemmBatch b{};
   int total = 0;
   for (int i = 0; i < nprob; ++i) {
@@ -519,10 +532,16 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
   b.nprob = nprob;
   b.total_tiles = total;
   if (total == 0) return MK_OK;
+  b.full_tiles = sp.ksplit > 1 ? sp.full : total;
+  b.ksplit = sp.ksplit;
+  b.ws = ws;
+  const int tail = total - b.full_tiles;
+  MK_REQUIRE(tail == 0 || (ws != nullptr && (size_t)tail * sp.ksplit * BM * BN * 8 <= GEMM_WS_BYTES), MK_BAD_ARG,
+             "gemm_f64: %d tiles split %d ways exceed the workspace", tail, sp.ksplit);
   const int var = f64_variant();
   bool buf = var != F64_BRANCH && f64_bk() == 16;
   for (int i = 0; i < nprob && buf; ++i) buf = buf_ok_prob<BM, BN>(probs[i], sh);
-  dim3 grid(total), block(NT);
+  dim3 grid(b.full_tiles + tail * b.ksplit), block(NT);
   ProfScope prof("gemm_f64", stream);
   // the rotated schedule holds two fragment sets; with a K-contiguous A the
   // extra registers would spill, so those launches keep the plain schedule
@@ -531,6 +550,12 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
   else if (f64_bk() == 16) launch4<BM, BN, GemmBatch, 16>(sh, grid, block, stream, b);
   else launch4<BM, BN, GemmBatch, BK32>(sh, grid, block, stream, b);
   MK_CHECK_HIP(hipGetLastError());
+  if (tail > 0) {
+    constexpr int NBLK = BM * BN / 256;
+    hipLaunchKernelGGL((splitk_reduce_kernel<false, 2, BM / 32, BN / 32, 2, dx4>), dim3((unsigned)cdiv((int64_t)tail * NBLK, 4)),
+                       dim3(256), 0, stream, b);
+    MK_CHECK_HIP(hipGetLastError());
+  }
   return MK_OK;
 }
 
@@ -583,20 +608,24 @@ mk_status gemm_f64_group(const GemmGroup& g, int kind, GemmShape sh, int grid, h
   return launch_group<64, 64>(g, sh, grid, st);
 }
 
-mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream) {
+mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream, void* ws) {
   MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "gemm_f64: %d problems (max %d)", nprob, MAX_PROB);
-  int64_t tiles128 = 0;
   for (int i = 0; i < nprob; ++i) {
     MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "gemm_f64: too many segments");
     MK_REQUIRE(probs[i].M >= 0 && probs[i].N >= 0 && probs[i].M < (1ll << 31) && probs[i].N < (1ll << 31),
                MK_BAD_SHAPE, "gemm_f64: bad M/N");
     for (int s = 0; s < probs[i].nseg; ++s)
       MK_REQUIRE(probs[i].seg[s].K >= 0 && probs[i].seg[s].K < (1ll << 31), MK_BAD_SHAPE, "gemm_f64: bad K");
-    tiles128 += cdiv(probs[i].M, 128) * cdiv(probs[i].N, 128);
   }
-  // 128x128 tiles once they fill the 256 CUs, else 64x64 for more parallelism
-  if (tiles128 >= 256) return launch_cfg<128, 128>(probs, nprob, shape, stream);
-  return launch_cfg<64, 64>(probs, nprob, shape, stream);
+  // Measured on 1024 x 1024 x 8192 (us, 64 x 64 tiles: 1, 2, 3, 4 workgroups a
+  // CU 419, 331, 305, 298; 128 x 128: 1, 2 a CU 309, 279); one step is 64 (16)
+  // v_mfma_f64_16x16x4 of 64 cycles per wave.
+  static const TileModel m128{128, 128, 16, 1.74, {0.76, 0.87, 0.87, 0.87}, 2, 128 * 128 * 8};
+  static const TileModel m64{64, 64, 16, 0.436, {0.53, 0.70, 0.77, 0.79}, 4, 64 * 64 * 8};
+  const bool split = ws != nullptr && f64_bk() == 16;
+  const TileChoice c128 = plan_launch(m128, probs, nprob, split), c64 = plan_launch(m64, probs, nprob, split);
+  if (c128.us <= c64.us) return launch_cfg<128, 128>(probs, nprob, shape, stream, c128.split, ws);
+  return launch_cfg<64, 64>(probs, nprob, shape, stream, c64.split, ws);
 }
 
 }  // namespace mk

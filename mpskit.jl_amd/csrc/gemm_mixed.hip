@@ -19,6 +19,7 @@
 #include <cstring>
 
 #include "gemm_dev.h"
+#include "gemm_plan.h"
 #include "prof.h"
 
 namespace mk {
@@ -102,7 +103,9 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
   __shared__ __attribute__((aligned(16))) char As[2][NPART][BM * ROWP];
   __shared__ __attribute__((aligned(16))) char Bs[2][NPART][BN * ROWP];
 
-  for (int t = src_first(src); t < src.total_tiles; t += src_stride(src)) {
+  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
+  int t, slice, nslice;
+  src_unit(src, un, t, slice, nslice);
   const GemmProb& P = src_prob(src, t);
   int tm, tn;
   tile_coords(P, t - P.tile_start, tm, tn);
@@ -145,17 +148,18 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
     }
   };
 
-  int s = 0, k0 = 0;
-  if (nsteps > 0) {
-    load(0, 0);
+  int s, k0, step0, step1;
+  slice_range<KSTEP>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  if (step1 > step0) {
+    load(s, k0);
     store(0);
   }
   __syncthreads();
   int buf = 0;
-  for (int step = 0; step < nsteps; ++step) {
+  for (int step = step0; step < step1; ++step) {
     int ns = s, nk0 = k0 + KSTEP;
     if (nk0 >= P.seg[s].K) { ns = s + 1; nk0 = 0; }
-    const bool has_next = step + 1 < nsteps;
+    const bool has_next = step + 1 < step1;
     if (has_next) load(ns, nk0);
 
     ux4 fa[NPART][FM], fb[NPART][FN];
@@ -203,8 +207,11 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
     k0 = nk0;
   }
 
-  store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
-  }  // tiles
+  if (slice < 0)
+    store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<float>(src, t, slice, BM * BN), wave, lane);
+  }  // units
 }
 
 // ---------------------------------------------------------------------------
@@ -259,7 +266,9 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big_kernel(Src src) {
   __shared__ __attribute__((aligned(16))) char As[2][NPART][BIG * ROWB];
   __shared__ __attribute__((aligned(16))) char Bs[2][NPART][BIG * ROWB];
 
-  for (int t = src_first(src); t < src.total_tiles; t += src_stride(src)) {
+  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
+  int t, slice, nslice;
+  src_unit(src, un, t, slice, nslice);
   const GemmProb& P = src_prob(src, t);
   int tm, tn;
   tile_coords(P, t - P.tile_start, tm, tn);
@@ -302,19 +311,20 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big_kernel(Src src) {
     }
   };
 
-  int s = 0, k0 = 0;
-  if (nsteps > 0) {
-    load(0, 0);
+  int s, k0, step0, step1;
+  slice_range<KSTEP>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  if (step1 > step0) {
+    load(s, k0);
     store(0);
   }
   __syncthreads();
   int buf = 0;
   const int aoff = swz(wm0 + li, lg);   // same swizzle for every 16-row block
   const int boff = swz(wn0 + li, lg);
-  for (int step = 0; step < nsteps; ++step) {
+  for (int step = step0; step < step1; ++step) {
     int ns = s, nk0 = k0 + KSTEP;
     if (nk0 >= P.seg[s].K) { ns = s + 1; nk0 = 0; }
-    const bool has_next = step + 1 < nsteps;
+    const bool has_next = step + 1 < step1;
     if (has_next) load(ns, nk0);
 
     ux4 fb[NPART][FN];
@@ -358,8 +368,11 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big_kernel(Src src) {
     k0 = nk0;
   }
 
-  store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
-  }  // tiles
+  if (slice < 0)
+    store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<float>(src, t, slice, BIG * BIG), wave, lane);
+  }  // units
 }
 
 // Raw (stride 0) buffer resource over p with num_records = 2^31 - 1 bytes and
@@ -401,7 +414,9 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big2_kernel(Src src) {
   const int aoff = swz(wm0 + li, lg);
   const int boff = swz(wn0 + li, lg);
 
-  for (int t = src_first(src); t < src.total_tiles; t += src_stride(src)) {
+  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
+  int t, slice, nslice;
+  src_unit(src, un, t, slice, nslice);
   const GemmProb& P = src_prob(src, t);
   int tm, tn;
   tile_coords(P, t - P.tile_start, tm, tn);
@@ -475,22 +490,23 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big2_kernel(Src src) {
       }
   };
 
-  int s = 0, k0 = 0;
-  if (nsteps > 0) {
-    set_seg(0);
-    load(0);
+  int s, k0, step0, step1;
+  slice_range<KSTEP>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  if (step1 > step0) {
+    set_seg(s);
+    load(k0);
     store(0);
   }
   __syncthreads();
   int buf = 0;
-  for (int step = 0; step < nsteps; ++step) {
+  for (int step = step0; step < step1; ++step) {
     k0 += KSTEP;
     while (k0 >= kend && s + 1 < nseg) {
       ++s;
       k0 = 0;
       set_seg(s);
     }
-    const bool has_next = step + 1 < nsteps;
+    const bool has_next = step + 1 < step1;
     if (has_next) load(k0);
 
     ux4 fb[NPART][FN];
@@ -532,8 +548,11 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big2_kernel(Src src) {
     buf ^= 1;
   }
 
-  store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
-  }  // tiles
+  if (slice < 0)
+    store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<float>(src, t, slice, BIG * BIG), wave, lane);
+  }  // units
 }
 
 // ---------------------------------------------------------------------------
@@ -697,7 +716,7 @@ __global__ __launch_bounds__(PNT) void gemm_mixed_pipe_kernel(GemmBatch batch) {
 }
 
 template <int BM, int BN, int MODE, int VAR>
-mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream) {
+mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream, SplitPlan sp = {}, void* ws = nullptr) {
   constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
   GemmBatch b{};
   int total = 0;
@@ -738,16 +757,30 @@ mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream) {
   b.nprob = nprob;
   b.total_tiles = total;
   if (total == 0) return MK_OK;
+  b.full_tiles = sp.ksplit > 1 && VAR != V_PIPE ? sp.full : total;
+  b.ksplit = b.full_tiles < total ? sp.ksplit : 1;
+  b.ws = ws;
+  const int tail = total - b.full_tiles, units = b.full_tiles + tail * b.ksplit;
+  MK_REQUIRE(tail == 0 || (ws != nullptr && (size_t)tail * b.ksplit * BM * BN * 4 <= GEMM_WS_BYTES), MK_BAD_ARG,
+             "mixed gemm: %d tiles split %d ways exceed the workspace", tail, b.ksplit);
   ProfScope prof(MODE == M_BF16X3 ? "gemm_bf16x3" : "gemm_f32", stream);
   if constexpr (VAR == V_PIPE)
     hipLaunchKernelGGL((gemm_mixed_pipe_kernel<MODE>), dim3(total), dim3(PNT), 0, stream, b);
   else if constexpr (VAR == V_BIG)
-    hipLaunchKernelGGL((gemm_mixed_big_kernel<MODE, GemmBatch>), dim3(total), dim3(BNT), 0, stream, b);
+    hipLaunchKernelGGL((gemm_mixed_big_kernel<MODE, GemmBatch>), dim3(units), dim3(BNT), 0, stream, b);
   else if constexpr (VAR == V_BIG2)
-    hipLaunchKernelGGL((gemm_mixed_big2_kernel<MODE, GemmBatch>), dim3(total), dim3(BNT), 0, stream, b);
+    hipLaunchKernelGGL((gemm_mixed_big2_kernel<MODE, GemmBatch>), dim3(units), dim3(BNT), 0, stream, b);
   else
-    hipLaunchKernelGGL((gemm_mixed_kernel<BM, BN, MODE, GemmBatch>), dim3(total), dim3(NT), 0, stream, b);
+    hipLaunchKernelGGL((gemm_mixed_kernel<BM, BN, MODE, GemmBatch>), dim3(units), dim3(NT), 0, stream, b);
   MK_CHECK_HIP(hipGetLastError());
+  if (tail > 0) {
+    // waves of a tile: 2 x 2 of BM/2 x BN/2, or (256 x 256) 2 x 4 of 128 x 64
+    constexpr int WGN = VAR == V_TILE ? 2 : 4;
+    constexpr int NBLK = BM * BN / 256;
+    hipLaunchKernelGGL((splitk_reduce_kernel<true, 2, BM / 32, BN / 16 / WGN, WGN, fx4>),
+                       dim3((unsigned)cdiv((int64_t)tail * NBLK, 4)), dim3(256), 0, stream, b);
+    MK_CHECK_HIP(hipGetLastError());
+  }
   return MK_OK;
 }
 
@@ -762,13 +795,10 @@ bool rows256_fit(const ProbSpec* probs, int nprob) {
 }
 
 template <int MODE>
-mk_status dispatch(const ProbSpec* probs, int nprob, hipStream_t stream) {
+mk_status dispatch(const ProbSpec* probs, int nprob, hipStream_t stream, void* ws) {
   MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "mixed gemm: too many problems");
-  int64_t tiles128 = 0;
-  for (int i = 0; i < nprob; ++i) {
+  for (int i = 0; i < nprob; ++i)
     MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "mixed gemm: too many segments");
-    tiles128 += cdiv(probs[i].M, 128) * cdiv(probs[i].N, 128);
-  }
   constexpr int64_t EB = MODE == M_BF16X3 ? 2 : 4;
   int64_t tiles256 = 0, tilesp = 0;
   bool off32 = true;   // buffer offsets of the pipelined kernel are 32-bit
@@ -788,14 +818,32 @@ mk_status dispatch(const ProbSpec* probs, int nprob, hipStream_t stream) {
                "mixed gemm: packed operands are read by the 256 x 256 kernel only");
     return launch_mixed<256, 256, MODE, V_BIG2>(probs, nprob, stream);
   }
-  // large tiles once they alone fill the 256 CUs; 128x128 while they fill them; else 64x64
   if (var == V_PIPE && tilesp >= 256 && off32) return launch_mixed<PBM, PBN, MODE, V_PIPE>(probs, nprob, stream);
-  if (var == V_BIG2 && tiles256 >= 256 && rows256_fit<MODE>(probs, nprob))
-    return launch_mixed<256, 256, MODE, V_BIG2>(probs, nprob, stream);
-  if ((var == V_BIG || var == V_BIG2) && tiles256 >= 256)
-    return launch_mixed<256, 256, MODE, V_BIG>(probs, nprob, stream);
-  if (tiles128 >= 256) return launch_mixed<128, 128, MODE, V_TILE>(probs, nprob, stream);
-  return launch_mixed<64, 64, MODE, V_TILE>(probs, nprob, stream);
+  // Measured on 2048 x 2048 x 4096 and 1024 x 2048 x 2048.  The bf16 steps are
+  // short (48 MFMAs of 16 cycles a wave on a 128 x 128 tile), so one step of
+  // prefetch covers little of the load latency and the operand traffic of a
+  // small tile (32 KB a step through the CU's 64 B / cycle) is near its limit:
+  // large tiles cut along K win.  The fp32 steps are 2.7 times longer.
+  static const TileModel m64{64, 64, 64 / (int)EB, MODE == M_BF16X3 ? 0.095 : 0.22,
+                             MODE == M_BF16X3 ? TileModel::Eff{0.18, 0.24, 0.28, 0.30} : TileModel::Eff{0.40, 0.55, 0.60, 0.62},
+                             4, 64 * 64 * 4};
+  static const TileModel m128{128, 128, 64 / (int)EB, MODE == M_BF16X3 ? 0.38 : 0.87,
+                              MODE == M_BF16X3 ? TileModel::Eff{0.32, 0.45, 0.45, 0.45} : TileModel::Eff{0.63, 0.75, 0.75, 0.75},
+                              2, 128 * 128 * 4};
+  static const TileModel m256{256, 256, 64 / (int)EB, MODE == M_BF16X3 ? 1.5 : 3.5,
+                              MODE == M_BF16X3 ? TileModel::Eff{0.62, 0.62, 0.62, 0.62} : TileModel::Eff{0.82, 0.82, 0.82, 0.82},
+                              1, 256 * 256 * 4};
+  const TileChoice c64 = plan_launch(m64, probs, nprob, ws != nullptr);
+  const TileChoice c128 = plan_launch(m128, probs, nprob, ws != nullptr);
+  TileChoice c256 = plan_launch(m256, probs, nprob, ws != nullptr);
+  if (var == V_TILE) c256.us = 1e30;
+  if (c256.us <= c128.us && c256.us <= c64.us) {
+    if (var == V_BIG2 && rows256_fit<MODE>(probs, nprob))
+      return launch_mixed<256, 256, MODE, V_BIG2>(probs, nprob, stream, c256.split, ws);
+    return launch_mixed<256, 256, MODE, V_BIG>(probs, nprob, stream, c256.split, ws);
+  }
+  if (c128.us <= c64.us) return launch_mixed<128, 128, MODE, V_TILE>(probs, nprob, stream, c128.split, ws);
+  return launch_mixed<64, 64, MODE, V_TILE>(probs, nprob, stream, c64.split, ws);
 }
 
 template <int MODE>
@@ -846,11 +894,11 @@ bool mixed_packed_ok(int64_t M, int64_t N, const int64_t* Ks, int nk) {
   return true;
 }
 
-mk_status gemm_bf16x3(const ProbSpec* probs, int nprob, hipStream_t stream) {
-  return dispatch<M_BF16X3>(probs, nprob, stream);
+mk_status gemm_bf16x3(const ProbSpec* probs, int nprob, hipStream_t stream, void* ws) {
+  return dispatch<M_BF16X3>(probs, nprob, stream, ws);
 }
-mk_status gemm_f32(const ProbSpec* probs, int nprob, hipStream_t stream) {
-  return dispatch<M_F32>(probs, nprob, stream);
+mk_status gemm_f32(const ProbSpec* probs, int nprob, hipStream_t stream, void* ws) {
+  return dispatch<M_F32>(probs, nprob, stream, ws);
 }
 
 }  // namespace mk

@@ -187,7 +187,7 @@ mk_status GroupPlan::run(const void* const base[NBASE], hipStream_t st) const {
           ps[i].seg[s].B = absolute(ps[i].seg[s].B, base);
         }
       }
-      MK_TRY(gemm_f64(ps, np, sh, st));
+      MK_TRY(gemm_f64(ps, np, sh, st, nullptr));
     }
     return MK_OK;
   }

@@ -336,7 +336,7 @@ extern "C" mk_status mk_eigsolve(mk_op h, double* x, int krylovdim, int maxiter,
     ProbSpec ps;
     ps.M = n; ps.N = pn; ps.C = col(K); ps.ldc = n;
     ps.add(Q, n, sb.ptr, kk, kk);
-    MK_TRY(gemm_f64(&ps, 1, GemmShape{}, st));
+    MK_TRY(gemm_f64(&ps, 1, GemmShape{}, st, ctx->gemm_ws()));
     MK_CHECK_HIP(hipMemcpyAsync(col(0), col(K), (size_t)n * pn * 8, hipMemcpyDeviceToDevice, st));
     MK_TRY(dv.norm(col(0), n, nrm));
     MK_TRY(k_axpby(1.0 / nrm, col(0), 0.0, col(0), n, st));

@@ -15,11 +15,15 @@ constexpr int kMaxDevices = 64;
 // code `scratch` only names the array; its device address is resolved once per
 // device by noalloc_setup and only that address is handed to kernels.
 static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
+// The K-split workspace of the GEMMs, apart from it, so that an apply splits
+// (and rounds) as mk_apply does whatever its own scratch takes.
+static __device__ __align__(256) unsigned char gemm_scratch[mk::GEMM_WS_BYTES];
 
 namespace mk {
 namespace {
 std::mutex g_mu;
 void* g_ptr[kMaxDevices] = {};
+void* g_ws[kMaxDevices] = {};
 }  // namespace
 
 mk_status noalloc_setup(int device) {
@@ -33,6 +37,14 @@ mk_status noalloc_setup(int device) {
               hipGetErrorString(e));
     return MK_HIP_ERROR;
   }
+  void* ws = nullptr;
+  const hipError_t e2 = hipGetSymbolAddress(&ws, HIP_SYMBOL(gemm_scratch));
+  if (e2 != hipSuccess || ws == nullptr) {
+    set_error("noalloc: hipGetSymbolAddress of the GEMM workspace failed on device %d: %s", device,
+              hipGetErrorString(e2));
+    return MK_HIP_ERROR;
+  }
+  g_ws[device] = ws;
   g_ptr[device] = ptr;
   return MK_OK;
 }
@@ -49,12 +61,13 @@ extern "C" mk_status mk_apply_noalloc(mk_op h, const double* x, double* y, doubl
              "apply_noalloc: an operator with charge blocks builds its launch plan on first use (call mk_apply)");
   const int dev = op->ctx->device;
   MK_CHECK_HIP(hipSetDevice(dev));
-  void* ptr = nullptr;
+  void *ptr = nullptr, *ws = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_mu);
     ptr = (dev >= 0 && dev < kMaxDevices) ? g_ptr[dev] : nullptr;
+    ws = ptr ? g_ws[dev] : nullptr;
   }
   MK_REQUIRE(ptr != nullptr, MK_HIP_ERROR, "apply_noalloc: scratch array not set up on device %d", dev);
-  FixedScratchGuard guard(ptr, kNoallocBytes);
+  FixedScratchGuard guard(ptr, kNoallocBytes, ws);
   return op_apply(op, x, y, alpha, beta, precision);
 }

@@ -187,11 +187,11 @@ mk_status apply_lxr(Op* op, const LxR& blk, const double* x, double* y, double a
     ProbSpec p1;
     p1.M = Mx; p1.N = nk * Ny; p1.C = xR; p1.ldc = Mx;
     p1.add(x, Mx, blk.R.f64(), Ki, Ki);
-    MK_TRY(gemm_f64(&p1, 1, GemmShape{}, ctx->stream));
+    MK_TRY(gemm_f64(&p1, 1, GemmShape{}, ctx->stream, ctx->gemm_ws()));
     ProbSpec p2;
     p2.M = Mo; p2.N = Ny; p2.C = y; p2.ldc = Mo; p2.alpha = alpha; p2.beta = beta;
     p2.add(blk.L.f64(), Mo, xR, Mx * nk, Mx * nk);
-    return gemm_f64(&p2, 1, GemmShape{}, ctx->stream);
+    return gemm_f64(&p2, 1, GemmShape{}, ctx->stream, ctx->gemm_ws());
   }
   const bool bf = prec == MK_BF16X3;
   double* xR = nullptr;
@@ -205,13 +205,13 @@ mk_status apply_lxr(Op* op, const LxR& blk, const double* x, double* y, double a
   p1.M = Mx; p1.N = nk * Ny; p1.C = xR; p1.ldc = Mx;
   if (bf) p1.add(vx.hi, vx.kpad, blk.R.hi.ptr, blk.R.kpad, Ki, vx.lo, blk.R.lo.ptr);
   else p1.add(vx.hi, vx.kpad, blk.R.f32.ptr, blk.R.kpad, Ki);
-  MK_TRY(run_gemm(&p1, 1, prec, GemmShape{}, ctx->stream));
+  MK_TRY(run_gemm(ctx, &p1, 1, prec, GemmShape{}));
   MK_TRY(convert_view(ctx, xR, Mx * nk, Ny, Mx * nk, 'B', prec, &vxr, mxr));
   ProbSpec p2;
   p2.M = Mo; p2.N = Ny; p2.C = y; p2.ldc = Mo; p2.alpha = alpha; p2.beta = beta;
   if (bf) p2.add(blk.L.hi.ptr, blk.L.kpad, vxr.hi, vxr.kpad, Mx * nk, blk.L.lo.ptr, vxr.lo);
   else p2.add(blk.L.f32.ptr, blk.L.kpad, vxr.hi, vxr.kpad, Mx * nk);
-  return run_gemm(&p2, 1, prec, GemmShape{}, ctx->stream);
+  return run_gemm(ctx, &p2, 1, prec, GemmShape{});
 }
 
 // Operand pointers of one GEMM side for precision `prec`.
@@ -524,7 +524,7 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
       p.add(a.p, a.ld, b.p, b.ld, M, a.lo, b.lo);
       p.seg[p.nseg - 1].packA = p.seg[p.nseg - 1].packB = packed;
     }
-    MK_TRY(run_gemm(&p, 1, prec, nn, ctx->stream));
+    MK_TRY(run_gemm(ctx, &p, 1, prec, nn));
   }
   if (op->CA.present()) {
     // y[a,(b,c,e)] += x[a,(h,i,j)] CA[(h,i,j),(b,c,e)]
@@ -533,7 +533,7 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
     Side a = prec == MK_FP64 ? Side{x, nullptr, Dl} : view_side(xca);
     Side b = mat_side(op->CA, prec);
     p.add(a.p, a.ld, b.p, b.ld, d1 * N, a.lo, b.lo);
-    MK_TRY(run_gemm(&p, 1, prec, nn, ctx->stream));
+    MK_TRY(run_gemm(ctx, &p, 1, prec, nn));
   }
   if (!op->AB.empty()) {
     // y_e[(a,b),c] += sum_j AB_{e,j}[(a,b),(f,h)] x_j[(f,h),c]
@@ -551,7 +551,7 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
         p.add(a.p, a.ld, b.p, b.ld, M, a.lo, b.lo);
       }
     }
-    MK_TRY(run_gemm(ps, (int)d2, prec, nn, ctx->stream));
+    MK_TRY(run_gemm(ctx, ps, (int)d2, prec, nn));
   }
   if (op->gen.present()) MK_TRY(apply_lxr(op, op->gen, x, y, alpha, bs.next(), prec));
   if (bs.first) MK_TRY(k_axpby(0.0, y, beta, y, op->y_elems, ctx->stream));
@@ -578,7 +578,7 @@ mk_status apply_ac_jordan(Op* op, const double* x, double* y, double alpha, doub
     Side a = prec == MK_FP64 ? Side{x, nullptr, Dl} : view_side(xc);
     Side b = mat_side(op->Cp, prec);
     p.add(a.p, a.ld, b.p, b.ld, d * Dr, a.lo, b.lo);
-    MK_TRY(run_gemm(&p, 1, prec, nn, ctx->stream));
+    MK_TRY(run_gemm(ctx, &p, 1, prec, nn));
   }
   if (op->Bp.present()) {
     // y[(a,b),c] += B'[(a,b),(f,h)] x[(f,h),c]
@@ -587,7 +587,7 @@ mk_status apply_ac_jordan(Op* op, const double* x, double* y, double alpha, doub
     Side a = mat_side(op->Bp, prec);
     Side b = prec == MK_FP64 ? Side{x, nullptr, Dl * d} : view_side(xb);
     p.add(a.p, a.ld, b.p, b.ld, Dl * d, a.lo, b.lo);
-    MK_TRY(run_gemm(&p, 1, prec, nn, ctx->stream));
+    MK_TRY(run_gemm(ctx, &p, 1, prec, nn));
   }
   if (op->gen.present()) MK_TRY(apply_lxr(op, op->gen, x, y, alpha, bs.next(), prec));
   if (bs.first) MK_TRY(k_axpby(0.0, y, beta, y, op->y_elems, ctx->stream));
@@ -613,13 +613,13 @@ mk_status apply_transfer_left(Op* op, const double* x, double* y, double alpha, 
     ProbSpec p1;
     p1.M = M1; p1.N = N1; p1.C = t1; p1.ldc = M1;
     p1.add(x, M1, op->TA.f64(), Dn, Dn);
-    MK_TRY(gemm_f64(&p1, 1, GemmShape{}, st));
+    MK_TRY(gemm_f64(&p1, 1, GemmShape{}, st, ctx->gemm_ws()));
     if (op->tmpo) MK_TRY(k_tl_mid(t1, O, Dm, wl, d, wr, Dc, t2, st));
     else t2 = t1;
     ProbSpec p2;
     p2.M = Da; p2.N = N2; p2.C = y; p2.ldc = Da; p2.alpha = alpha; p2.beta = beta;
     p2.add(op->TB.f64(), K2, t2, K2, K2);
-    return gemm_f64(&p2, 1, GemmShape{true, false}, st);
+    return gemm_f64(&p2, 1, GemmShape{true, false}, st, ctx->gemm_ws());
   }
   const bool bf = prec == MK_BF16X3;
   double* t1 = nullptr;
@@ -633,7 +633,7 @@ mk_status apply_transfer_left(Op* op, const double* x, double* y, double alpha, 
   p1.M = M1; p1.N = N1; p1.C = t1; p1.ldc = M1;
   if (bf) p1.add(vx.hi, vx.kpad, op->TA.hi.ptr, op->TA.kpad, Dn, vx.lo, op->TA.lo.ptr);
   else p1.add(vx.hi, vx.kpad, op->TA.f32.ptr, op->TA.kpad, Dn);
-  MK_TRY(run_gemm(&p1, 1, prec, GemmShape{}, st));
+  MK_TRY(run_gemm(ctx, &p1, 1, prec, GemmShape{}));
   if (op->tmpo) {
     vt = view_layout(K2, N2, 'B', prec, mt);
     MK_TRY(k_tl_mid_mixed(t1, O, Dm, wl, d, wr, Dc, vt.kpad, bf ? 1 : 0, vt.hi, vt.lo, st));
@@ -644,7 +644,7 @@ mk_status apply_transfer_left(Op* op, const double* x, double* y, double alpha, 
   p2.M = Da; p2.N = N2; p2.C = y; p2.ldc = Da; p2.alpha = alpha; p2.beta = beta;
   if (bf) p2.add(op->TB.hi.ptr, op->TB.kpad, vt.hi, vt.kpad, K2, op->TB.lo.ptr, vt.lo);
   else p2.add(op->TB.f32.ptr, op->TB.kpad, vt.hi, vt.kpad, K2);
-  return run_gemm(&p2, 1, prec, GemmShape{}, st);
+  return run_gemm(ctx, &p2, 1, prec, GemmShape{});
 }
 
 // Right transfer y = alpha T v + beta y (transfer_right, transfer.jl:128-130
@@ -663,13 +663,13 @@ mk_status apply_transfer_right(Op* op, const double* v, double* y, double alpha,
     ProbSpec p1;
     p1.M = M1; p1.N = N1; p1.C = t1; p1.ldc = M1;
     p1.add(op->TA.f64(), M1, v, Di, Di);
-    MK_TRY(gemm_f64(&p1, 1, GemmShape{}, st));
+    MK_TRY(gemm_f64(&p1, 1, GemmShape{}, st, ctx->gemm_ws()));
     if (op->tmpo) MK_TRY(k_tr_mid(t1, O, Da, wl, d, wr, Do, t2, st));
     else t2 = t1;
     ProbSpec p2;
     p2.M = M2; p2.N = Dc; p2.C = y; p2.ldc = M2; p2.alpha = alpha; p2.beta = beta;
     p2.add(t2, M2, op->TB.f64(), Dc, K2);
-    return gemm_f64(&p2, 1, GemmShape{false, true}, st);
+    return gemm_f64(&p2, 1, GemmShape{false, true}, st, ctx->gemm_ws());
   }
   const bool bf = prec == MK_BF16X3;
   double* t1 = nullptr;
@@ -683,7 +683,7 @@ mk_status apply_transfer_right(Op* op, const double* v, double* y, double alpha,
   p1.M = M1; p1.N = N1; p1.C = t1; p1.ldc = M1;
   if (bf) p1.add(op->TA.hi.ptr, op->TA.kpad, vv.hi, vv.kpad, Di, op->TA.lo.ptr, vv.lo);
   else p1.add(op->TA.f32.ptr, op->TA.kpad, vv.hi, vv.kpad, Di);
-  MK_TRY(run_gemm(&p1, 1, prec, GemmShape{}, st));
+  MK_TRY(run_gemm(ctx, &p1, 1, prec, GemmShape{}));
   if (op->tmpo) {
     vt = view_layout(M2, K2, 'A', prec, mt);
     MK_TRY(k_tr_mid_mixed(t1, O, Da, wl, d, wr, Do, vt.kpad, bf ? 1 : 0, vt.hi, vt.lo, st));
@@ -694,7 +694,7 @@ mk_status apply_transfer_right(Op* op, const double* v, double* y, double alpha,
   p2.M = M2; p2.N = Dc; p2.C = y; p2.ldc = M2; p2.alpha = alpha; p2.beta = beta;
   if (bf) p2.add(vt.hi, vt.kpad, op->TB.hi.ptr, op->TB.kpad, K2, vt.lo, op->TB.lo.ptr);
   else p2.add(vt.hi, vt.kpad, op->TB.f32.ptr, op->TB.kpad, K2);
-  return run_gemm(&p2, 1, prec, GemmShape{}, st);
+  return run_gemm(ctx, &p2, 1, prec, GemmShape{});
 }
 
 }  // namespace

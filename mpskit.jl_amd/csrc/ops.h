@@ -35,8 +35,23 @@ struct Ctx {
   }
   DevBuf arena;      // stream-ordered scratch for applies / transfers
   DevBuf smallbuf;   // small stream-ordered scratch (reduction partials, scalars)
+  // K-split workspaces (GEMM_WS_BYTES each) of the streams this context has
+  // enqueued on, at most MAX_GEMM_WS; kept until the context goes
+  static constexpr int MAX_GEMM_WS = 4;
+  struct GemmWs {
+    hipStream_t stream = nullptr;
+    DevBuf buf;
+  };
+  GemmWs gemmws[MAX_GEMM_WS];
+  int ngemmws = 0;
   mk_status scratch(size_t nbytes, void** out);
   mk_status small(size_t nbytes, void** out);
+  // The K-split workspace of a GEMM about to be enqueued on `stream`, or null
+  // (the launch then splits nothing): each stream has its own, so callers that
+  // move one context between streams need not order them; a stream past the
+  // first MAX_GEMM_WS gets none, and neither does one under capture, whose
+  // graph may later run beside the stream's eager work.
+  void* gemm_ws();
 };
 
 mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regions);
@@ -48,11 +63,12 @@ mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regio
 struct FixedScratch {
   char* base = nullptr;
   size_t bytes = 0;
+  void* gemm_ws = nullptr;   // GEMM_WS_BYTES
 };
 FixedScratch& fixed_scratch();
 struct FixedScratchGuard {
-  explicit FixedScratchGuard(void* base, size_t bytes) {
-    fixed_scratch() = FixedScratch{static_cast<char*>(base), bytes};
+  FixedScratchGuard(void* base, size_t bytes, void* gemm_ws) {
+    fixed_scratch() = FixedScratch{static_cast<char*>(base), bytes, gemm_ws};
   }
   ~FixedScratchGuard() { fixed_scratch() = FixedScratch{}; }
   FixedScratchGuard(const FixedScratchGuard&) = delete;
@@ -101,7 +117,8 @@ mk_status convert_view(Ctx* ctx, const double* M, int64_t rows, int64_t cols, in
 // Where convert_view puts the converted (rows x cols) view in `mem`, without converting.
 MixedView view_layout(int64_t rows, int64_t cols, char role, int prec, void* mem);
 size_t view_bytes(int64_t rows, int64_t cols, char role, int prec);
-mk_status run_gemm(const ProbSpec* p, int np, int prec, GemmShape sh, hipStream_t st);
+// A GEMM in arithmetic `prec` on the context's stream, with its K-split workspace.
+mk_status run_gemm(Ctx* ctx, const ProbSpec* p, int np, int prec, GemmShape sh);
 
 enum OpKind { OP_C = 0, OP_AC_GEN = 1, OP_AC2_GEN = 2, OP_AC_JOR = 3, OP_AC2_JOR = 4, OP_TL = 5, OP_TR = 6 };
 

@@ -139,7 +139,7 @@ mk_status potrf_lower(double* A, int64_t n, int64_t lda, int* info_dev, double* 
     pp.add(A21, lda, Linv, NB, nb);
     GemmShape tb;
     tb.tb = true;   // B(k, j) = Linv[j + k NB] = L11^-1(j, k)
-    MK_TRY(gemm_f64(&pp, 1, tb, st));
+    MK_TRY(gemm_f64(&pp, 1, tb, st, nullptr));
     MK_CHECK_HIP(hipMemcpy2DAsync(A21, lda * sizeof(double), X, m * sizeof(double), m * sizeof(double), nb,
                                   hipMemcpyDeviceToDevice, st));
     // A22 -= X X^T (full square; the strict upper part is zeroed at the end)
@@ -150,7 +150,7 @@ mk_status potrf_lower(double* A, int64_t n, int64_t lda, int* info_dev, double* 
     p.alpha = -1.0;
     p.beta = 1.0;
     p.add(X, m, X, m, nb);
-    MK_TRY(gemm_f64(&p, 1, tb, st));   // B(k, j) = X[j + k m] = X(j, k)
+    MK_TRY(gemm_f64(&p, 1, tb, st, nullptr));   // B(k, j) = X[j + k m] = X(j, k)
   }
   hipLaunchKernelGGL(zero_upper_kernel, dim3((unsigned)std::min<int64_t>(cdiv(n * n, (int64_t)256), 4096)), dim3(256),
                      0, st, A, lda, n);

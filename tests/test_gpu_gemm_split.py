@@ -1,0 +1,88 @@
+"""GEMM launches whose tiles are cut along K (mk_gemm, all three arithmetics).
+
+Sizes whose tiles do not fill the GPU are split: all of them, or those of the
+last round.  Edges: one tile with a long K, K that is not a multiple of a step
+or of the slices, odd sizes and leading dimensions, a last round of few tiles,
+beta != 0 (C is read by the reduction only).  Against float64 torch.
+
+Tolerances: the partial sums of a slice and their sum have the same bound as
+one long sum, K u |A||B|; on Gaussian operands the relative 2-norm error stays
+below sqrt(K) u for u the unit roundoff of the accumulation (2^-53, 2^-24),
+plus for the mixed arithmetics the rounding of the operands (2^-24; 2^-16 for
+hi + lo bf16, whose lo * lo product is dropped).
+"""
+import math
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mk():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a ROCm device"
+    import mpskit_amd
+    mpskit_amd.load()
+    return mpskit_amd
+
+
+def bound(prec, K):
+    return {"fp64": 4 * math.sqrt(K) * 2.0 ** -53, "fp32": 4 * (math.sqrt(K) * 2.0 ** -24 + 2.0 ** -24),
+            "bf16x3": 4 * (math.sqrt(K) * 2.0 ** -24 + 2.0 ** -16)}[prec]
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 64, 4096), (1, 1, 5000), (130, 70, 4100), (129, 1, 1031), (777, 1001, 3001),
+                                   (1024, 1024, 2048), (640, 512, 8190), (2176, 2048, 1026), (5120, 2048, 520)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
+def test_split_gemm_matches_torch(mk, M, N, K, prec):
+    import torch
+    T = mk.tensors
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + 3 * N + 7 * K)
+    for ta, tb, alpha, beta in ((False, False, 1.0, 0.0), (True, False, -0.5, 2.0), (False, True, 2.0, -1.0),
+                                (True, True, 1.0, 1.0)):
+        A = T.randn((K, M) if ta else (M, K), g)
+        B = T.randn((N, K) if tb else (K, N), g)
+        C = T.randn((M, N), g)
+        ref = alpha * ((A.t() if ta else A) @ (B.t() if tb else B)) + beta * C
+        scale = float(torch.linalg.vector_norm(ref))
+        print("split gemm", M, N, K, prec, ta, tb, flush=True)
+        out = mk.gemm(A, B, C, alpha=alpha, beta=beta, transa=ta, transb=tb, precision=prec)
+        assert float(torch.linalg.vector_norm(out - ref)) <= bound(prec, K) * scale
+
+
+def test_split_gemm_repeats_bitwise(mk):
+    """The slices are added in a fixed order, and an unordered second stream has a workspace of its own."""
+    import torch
+    T = mk.tensors
+    A, B = T.randn((1000, 3000)), T.randn((3000, 500))
+    first = mk.gemm(A, B).clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    outs = []
+    for _ in range(3):
+        outs.append(mk.gemm(A, B))
+        with torch.cuda.stream(s):
+            outs.append(mk.gemm(A, B))
+    torch.cuda.synchronize()
+    for o in outs:
+        assert torch.equal(o, first)
+
+
+def test_split_gemm_not_split_under_capture(mk):
+    """A captured call takes no shared workspace; replays agree with the eager result."""
+    import torch
+    T = mk.tensors
+    A, B, C = T.randn((500, 3000)), T.randn((3000, 400)), T.empty((500, 400))
+    ref = mk.gemm(A, B).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        mk.gemm(A, B, C)
+    for _ in range(3):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(torch.linalg.vector_norm(C - ref)) <= bound("fp64", 3000) * float(torch.linalg.vector_norm(ref))
+        mk.gemm(A, B)
