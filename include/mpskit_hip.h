@@ -284,7 +284,10 @@ mk_status mk_apply(mk_op op, const double* x, double* y, double alpha, double be
  * operators need none), and operators with charge blocks return
  * MK_NOT_SUPPORTED.  All calls on one GPU share the array: calls that overlap
  * on one GPU (different streams or threads) race; calls ordered on one stream
- * do not.  Nothing in the array needs to start at zero. */
+ * do not.  Nothing in the array needs to start at zero.  A generic operator
+ * whose MPO bonds at the ends are wider than the one in the middle may go
+ * through the array in several column chunks; its result then equals
+ * mk_apply's to rounding. */
 #define MK_NOALLOC_SCRATCH_MB 160
 mk_status mk_apply_noalloc(mk_op op, const double* x, double* y, double alpha, double beta,
                            int precision);

@@ -123,6 +123,9 @@ int64_t pad8(int64_t k) {
   return p;
 }
 
+int64_t up8(int64_t k) { return (k + 7) / 8 * 8; }
+int64_t runs_k(int64_t K, int nrun) { return nrun == 1 ? K : nrun * up8(K / nrun); }
+
 // A float64 column-major operator matrix (rows x cols) used as GEMM operand
 // `role` ('A' = left factor, rows = M, cols = K;  'B' = right factor,
 // rows = K, cols = N).  Mixed copies are K-contiguous with padded rows.
@@ -130,15 +133,16 @@ mk_status OpMat::make_mixed(int precisions, hipStream_t st) {
   const bool kfast = (role == 'B');   // col-major B: K is the fast index
   const int64_t K = kfast ? rows : cols;
   const int64_t MN = kfast ? cols : rows;
-  kpad = pad8(K);
+  const int64_t run = K / nrun;
+  kpad = pad8(runs_k(K, nrun));
   if (precisions & MK_PREC_BF16X3) {
     MK_TRY(hi.alloc((size_t)MN * kpad * 2));
     MK_TRY(lo.alloc((size_t)MN * kpad * 2));
-    MK_TRY(k_split_bf16(f64(), rows, cols, rows, kfast ? 1 : 0, kpad, hi.ptr, lo.ptr, st));
+    MK_TRY(k_convert(f64(), MN, run, nrun, up8(run), rows, kfast ? 1 : 0, kpad, 1, hi.ptr, lo.ptr, st));
   }
   if (precisions & MK_PREC_FP32) {
     MK_TRY(f32.alloc((size_t)MN * kpad * 4));
-    MK_TRY(k_to_f32(f64(), rows, cols, rows, kfast ? 1 : 0, kpad, static_cast<float*>(f32.ptr), st));
+    MK_TRY(k_convert(f64(), MN, run, nrun, up8(run), rows, kfast ? 1 : 0, kpad, 0, f32.ptr, nullptr, st));
   }
   return MK_OK;
 }
@@ -166,12 +170,12 @@ mk_status OpMat::make_packed(int precisions, hipStream_t st) {
 // ---------------------------------------------------------------------------
 
 // A transient float64 view converted for a mixed apply (x, xR...).
-MixedView view_layout(int64_t rows, int64_t cols, char role, int prec, void* mem) {
+MixedView view_layout(int64_t rows, int64_t cols, char role, int prec, void* mem, int nrun) {
   const bool kfast = (role == 'B');
   const int64_t K = kfast ? rows : cols;
   const int64_t MN = kfast ? cols : rows;
   MixedView v;
-  v.kpad = pad8(K);
+  v.kpad = pad8(runs_k(K, nrun));
   const size_t n = (size_t)MN * v.kpad;
   char* p = static_cast<char*>(mem);
   v.hi = p;
@@ -180,21 +184,19 @@ MixedView view_layout(int64_t rows, int64_t cols, char role, int prec, void* mem
 }
 
 mk_status convert_view(Ctx* ctx, const double* M, int64_t rows, int64_t cols, int64_t ld, char role,
-                       int prec, MixedView* out, void* mem) {
+                       int prec, MixedView* out, void* mem, int nrun) {
   const bool kfast = (role == 'B');
-  *out = view_layout(rows, cols, role, prec, mem);
-  if (prec == MK_BF16X3)
-    MK_TRY(k_split_bf16(M, rows, cols, ld, kfast ? 1 : 0, out->kpad, out->hi, out->lo, ctx->stream));
-  else
-    MK_TRY(k_to_f32(M, rows, cols, ld, kfast ? 1 : 0, out->kpad, static_cast<float*>(out->hi), ctx->stream));
-  return MK_OK;
+  *out = view_layout(rows, cols, role, prec, mem, nrun);
+  const int64_t run = (kfast ? rows : cols) / nrun;
+  return k_convert(M, kfast ? cols : rows, run, nrun, up8(run), ld, kfast ? 1 : 0, out->kpad, prec == MK_BF16X3 ? 1 : 0,
+                   out->hi, out->lo, ctx->stream);
 }
 
-size_t view_bytes(int64_t rows, int64_t cols, char role, int prec) {
+size_t view_bytes(int64_t rows, int64_t cols, char role, int prec, int nrun) {
   const bool kfast = (role == 'B');
   const int64_t K = kfast ? rows : cols;
   const int64_t MN = kfast ? cols : rows;
-  const size_t n = (size_t)MN * pad8(K);
+  const size_t n = (size_t)MN * pad8(runs_k(K, nrun));
   return prec == MK_BF16X3 ? 2 * align256(n * 2) : align256(n * 4);
 }
 

@@ -59,7 +59,8 @@ inline TileChoice plan_tile(const TileModel& m, int64_t tiles, int64_t nsteps, b
     if (tail <= 0) continue;
     const double base = tile_rounds_us(m, full, (double)nsteps);
     for (int s = 2; s <= MAX_KSPLIT && nsteps / s >= MIN_SLICE_STEPS; ++s) {
-      if ((size_t)tail * s * m.part_bytes > GEMM_WS_BYTES) break;
+      // past one round of workgroups a finer cut gains nothing
+      if (tail * (s - 1) >= round || (size_t)tail * s * m.part_bytes > GEMM_WS_BYTES) break;
       // partial tiles written and read back at about 4.5 TB/s
       const double us = base + tile_rounds_us(m, tail * s, (double)cdiv(nsteps, s)) + 4.0 +
                         2.0 * (double)tail * s * m.part_bytes / 4.5e6;

@@ -42,6 +42,10 @@ mk_status k_swap23(const double* in, int64_t D0, int64_t D1, int64_t D2, double*
 mk_status k_env_channels(const double* src, int64_t Di, int w, int64_t Dc, const int* klist,
                          int nk, double* dst, hipStream_t st);
 
+// dst[a + Da*(f + Df*k)] = src[a + Da*(klist[k] + w*f)]     (channel subset, channels slowest)
+mk_status k_env_channels_last(const double* src, int64_t Da, int w, int64_t Df, const int* klist, int nk, double* dst,
+                              hipStream_t st);
+
 // transfer-left middle step: t2[m,k,b,c] = sum_{g,h} t1[m,g,h,c] O[g,k,h,b]
 mk_status k_tl_mid(const double* t1, const double* O, int64_t Dm, int wl, int d, int wr,
                    int64_t Dc, double* t2, hipStream_t st);
@@ -101,15 +105,22 @@ mk_status k_gemv(const double* V, int64_t ldv, int k, const double* s, double* x
 mk_status k_nonfinite(const double* x, int64_t n, int* flag, hipStream_t st);
 
 // ---- precision conversion --------------------------------------------------
-// Convert a column-major float64 matrix M (rows x cols, leading dim ld) into a
-// K-contiguous operand whose rows have length ldo (>= K, padding zeroed):
-//   trans == 1: K = rows, out[c*ldo + r] = M(r,c)   (no data transposition)
-//   trans == 0: K = cols, out[r*ldo + c] = M(r,c)   (LDS-tiled transposition)
-// bf16: hi = bf16(M), lo = bf16(M - hi).
-mk_status k_split_bf16(const double* M, int64_t rows, int64_t cols, int64_t ld, int trans,
-                       int64_t ldo, void* hi, void* lo, hipStream_t st);
-mk_status k_to_f32(const double* M, int64_t rows, int64_t cols, int64_t ld, int trans,
-                   int64_t ldo, float* out, hipStream_t st);
+// Convert a column-major float64 matrix (leading dim ld) into MN K-contiguous
+// rows of length ldo.  K is nrun runs of `run` elements, each padded with zeros
+// to runpad (a multiple of 8); the rest of a row is zero.
+//   trans == 1: K along the rows, MN columns (no data transposition)
+//   trans == 0: K along the columns, MN rows (LDS-tiled transposition)
+// split: bf16 hi = bf16(M), lo = bf16(M - hi); else fp32 in hi.
+mk_status k_convert(const double* M, int64_t MN, int64_t run, int nrun, int64_t runpad, int64_t ld, int trans,
+                    int64_t ldo, int split, void* hi, void* lo, hipStream_t st);
+
+// t2[f,g,b,c,e] = sum_{h,l,j} Wc[(g,b,e)][(h,l,j)] t1[f,h,l,c,j] for nc columns
+// c, Wc rows (g + wl (b + d1 e)) of gen_mid_nin(d1 wr d2) entries (0: too many
+// inputs).  prec FP64: t2 (t1 itself is allowed when wl == wr); else rows
+// (b + d1 (c + nc e)) of length ldo in hi / lo (bf16) or hi (fp32).
+int gen_mid_nin(int nin);
+mk_status k_gen_mid(const double* t1, const double* Wc, int64_t Df, int wl, int d1, int wr, int d2, int64_t nc,
+                    int prec, double* t2, int64_t ldo, void* hi, void* lo, hipStream_t st);
 
 // One pass over x (d1 = d2 = 2, M = 2 Dl and N = 2 Dr multiples of 8) for the
 // mixed-precision nearest-neighbour apply: y = alpha CB(x) + beta y and the

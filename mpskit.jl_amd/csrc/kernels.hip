@@ -167,6 +167,17 @@ __global__ void env_channels_kernel(const double* __restrict__ src, int64_t Di, 
   }
 }
 
+__global__ void env_channels_last_kernel(const double* __restrict__ src, int64_t Da, int w, int64_t Df,
+                                         const int* __restrict__ klist, int nk, double* __restrict__ dst) {
+  const int64_t n = Da * Df * nk;
+  GRID_STRIDE(idx, n) {
+    const int64_t a = idx % Da, q = idx / Da;
+    const int64_t f = q % Df;
+    const int k = (int)(q / Df);
+    dst[idx] = src[a + Da * (klist[k] + (int64_t)w * f)];
+  }
+}
+
 __global__ void tl_mid_kernel(const double* __restrict__ t1, const double* __restrict__ O,
                               int64_t Dm, int wl, int d, int wr, int64_t Dc, double* __restrict__ t2) {
   const int64_t n = Dm * d * wr * Dc;
@@ -582,65 +593,141 @@ __global__ void nonfinite_kernel(const double* __restrict__ x, int64_t n, int* f
 
 // ---- precision conversion ---------------------------------------------------
 
-// plain conversion (no transposition): out[c*ldo + r] = M[r + c*ld], zero for rows <= r < ldo
-__global__ void split_plain_kernel(const double* __restrict__ M, int64_t rows, int64_t cols, int64_t ld,
-                                   int64_t ldo, __hip_bfloat16* __restrict__ hi,
-                                   __hip_bfloat16* __restrict__ lo) {
-  const int64_t n = ldo * cols;
-  GRID_STRIDE(idx, n) {
-    const int64_t r = idx % ldo, c = idx / ldo;
-    __hip_bfloat16 h = __float2bfloat16(0.f), l = __float2bfloat16(0.f);
-    if (r < rows) split2(M[r + c * ld], h, l);
-    hi[idx] = h;
-    lo[idx] = l;
+// Eight consecutive elements of a converted row: bf16 hi and lo (SPLIT) or fp32.
+template <bool SPLIT>
+__device__ __forceinline__ void put8(const double (&v)[8], void* __restrict__ hi, void* __restrict__ lo, int64_t at) {
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(1))) u4 gu4;
+  if constexpr (SPLIT) {
+    u4 a, b;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      __hip_bfloat16 h0, l0, h1, l1;
+      split2(v[2 * q], h0, l0);
+      split2(v[2 * q + 1], h1, l1);
+      a[q] = (unsigned)__builtin_bit_cast(unsigned short, h0) | ((unsigned)__builtin_bit_cast(unsigned short, h1) << 16);
+      b[q] = (unsigned)__builtin_bit_cast(unsigned short, l0) | ((unsigned)__builtin_bit_cast(unsigned short, l1) << 16);
+    }
+    *(gu4*)((char*)hi + at * 2) = a;
+    *(gu4*)((char*)lo + at * 2) = b;
+  } else {
+    u4 a, b;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      a[q] = __float_as_uint((float)v[q]);
+      b[q] = __float_as_uint((float)v[4 + q]);
+    }
+    *(gu4*)((char*)hi + at * 4) = a;
+    *(gu4*)((char*)hi + at * 4 + 16) = b;
   }
 }
 
-// transposed conversion: out[r*ldo + c] = M[r + c*ld] (zero for cols <= c < ldo), 64x64 LDS tiles
-__global__ void split_trans_kernel(const double* __restrict__ M, int64_t rows, int64_t cols, int64_t ld,
-                                   int64_t ldo, __hip_bfloat16* __restrict__ hi,
-                                   __hip_bfloat16* __restrict__ lo) {
+// Conversions of a float64 matrix into K-contiguous rows of length ldo (a
+// multiple of 8).  K may come in `nrun` runs of `run` source elements, each
+// padded with zeros to `runpad` (a multiple of 8); what is left of the row is
+// zero.  Both are memory-bound: a thread converts 8 elements of a row and
+// writes them as 16-byte stores (2-byte stores, one element a thread, ran at
+// 1.4 TB/s on a 2048 x 1024 matrix).
+//
+// plain (K = rows): out[c * ldo + k] = M[r + c * ld]
+template <bool SPLIT>
+__global__ void conv_plain_kernel(const double* __restrict__ M, int64_t run, int nrun, int64_t runpad, int64_t cols,
+                                  int64_t ld, int64_t ldo, void* __restrict__ hi, void* __restrict__ lo) {
+  const int64_t nch = ldo / 8, n = nch * cols;
+  typedef const __attribute__((address_space(1))) double gd;
+  GRID_STRIDE(idx, n) {
+    const int64_t c = idx / nch, k = (idx - c * nch) * 8;
+    const int64_t q = k / runpad, o = k - q * runpad;
+    double v[8];
+    gd* p = (gd*)M + c * ld + q * run + o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (q < nrun && o + i < run) ? p[i] : 0.0;
+    put8<SPLIT>(v, hi, lo, c * ldo + k);
+  }
+}
+
+// transposed (K = cols): out[r * ldo + k] = M[r + c * ld], 64 x 64 LDS tiles
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void conv_trans_kernel(const double* __restrict__ M, int64_t rows, int64_t run,
+                                                         int nrun, int64_t runpad, int64_t ld, int64_t ldo,
+                                                         void* __restrict__ hi, void* __restrict__ lo) {
   __shared__ double tile[64][65];
-  const int64_t r0 = (int64_t)blockIdx.x * 64, c0 = (int64_t)blockIdx.y * 64;
+  const int64_t r0 = (int64_t)blockIdx.x * 64, k0 = (int64_t)blockIdx.y * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 4 rows of threads
+  typedef const __attribute__((address_space(1))) double gd;
+#pragma unroll 4
   for (int cc = ty; cc < 64; cc += 4) {
-    const int64_t r = r0 + tx, c = c0 + cc;
-    tile[cc][tx] = (r < rows && c < cols) ? M[r + c * ld] : 0.0;
+    const int64_t r = r0 + tx, k = k0 + cc;
+    const int64_t q = k / runpad, o = k - q * runpad;
+    tile[cc][tx] = (r < rows && q < nrun && o < run) ? ((gd*)M)[r + (q * run + o) * ld] : 0.0;
   }
   __syncthreads();
-  for (int rr = ty; rr < 64; rr += 4) {
-    const int64_t r = r0 + rr, c = c0 + tx;
-    if (r < rows && c < ldo) {
-      __hip_bfloat16 h, l;
-      split2(tile[tx][rr], h, l);
-      hi[r * ldo + c] = h;
-      lo[r * ldo + c] = l;
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int id = threadIdx.x + it * 256, rr = id >> 3, q8 = (id & 7) * 8;
+    const int64_t r = r0 + rr, k = k0 + q8;
+    if (r < rows && k < ldo) {
+      double v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = tile[q8 + i][rr];
+      put8<SPLIT>(v, hi, lo, r * ldo + k);
     }
   }
 }
 
-__global__ void f32_plain_kernel(const double* __restrict__ M, int64_t rows, int64_t cols, int64_t ld,
-                                 int64_t ldo, float* __restrict__ out) {
-  const int64_t n = ldo * cols;
+// The middle step of a generic operator's apply, between x GR and GL:
+//   t2[f,g,b,c,e] = sum_{h,l,j} Wc[(g,b,e)][(h,l,j)] t1[f,h,l,c,j]
+// One thread per (f, c) holds its NIN >= d1 wr d2 inputs in registers, so t1
+// is read once and t2 written once (memory-bound); Wc is uniform over the
+// threads and zero-padded to NIN columns.  Each thread writes only the places
+// it has read, so with wl == wr t2 may be t1 itself.  MODE 0: float64 t2; 1,
+// 2: the K-contiguous rows (b,c,e) of length ldo of the next product's right
+// factor, K = (f, g), as bf16 hi and lo or fp32, zero from K to the next
+// multiple of 8.
+template <int NIN, int MODE>
+__global__ __launch_bounds__(256) void gen_mid_kernel(const double* t1, const double* __restrict__ Wc, int64_t Df,
+                                                      int wl, int d1, int wr, int d2, int64_t nc, double* t2,
+                                                      int64_t ldo, void* __restrict__ hi, void* __restrict__ lo) {
+  const int nin1 = d1 * wr, nout1 = wl * d1;
+  const int64_t n = Df * nc, K = Df * wl, pad = (K + 7) / 8 * 8 - K;
   GRID_STRIDE(idx, n) {
-    const int64_t r = idx % ldo, c = idx / ldo;
-    out[idx] = r < rows ? (float)M[r + c * ld] : 0.f;
-  }
-}
-
-__global__ void f32_trans_kernel(const double* __restrict__ M, int64_t rows, int64_t cols, int64_t ld,
-                                 int64_t ldo, float* __restrict__ out) {
-  __shared__ double tile[64][65];
-  const int64_t r0 = (int64_t)blockIdx.x * 64, c0 = (int64_t)blockIdx.y * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int cc = ty; cc < 64; cc += 4) {
-    const int64_t r = r0 + tx, c = c0 + cc;
-    tile[cc][tx] = (r < rows && c < cols) ? M[r + c * ld] : 0.0;
-  }
-  __syncthreads();
-  for (int rr = ty; rr < 64; rr += 4) {
-    const int64_t r = r0 + rr, c = c0 + tx;
-    if (r < rows && c < ldo) out[r * ldo + c] = (float)tile[tx][rr];
+    const int64_t c = idx / Df, f = idx - c * Df;
+    double v[NIN];
+#pragma unroll
+    for (int i = 0; i < NIN; ++i) {
+      const int q = i % nin1, j = i / nin1;
+      v[i] = j < d2 ? t1[f + Df * (q + (int64_t)nin1 * (c + nc * j))] : 0.0;
+    }
+    for (int e = 0; e < d2; ++e)
+      for (int b = 0; b < d1; ++b) {
+        const int64_t row = b + d1 * (c + nc * e);
+        for (int g = 0; g < wl; ++g) {
+          const double* w = Wc + (int64_t)(g + wl * (b + d1 * e)) * NIN;
+          double s = 0.0;
+#pragma unroll
+          for (int i = 0; i < NIN; ++i) s += w[i] * v[i];
+          if constexpr (MODE == 0) {
+            t2[f + Df * (g + (int64_t)nout1 * (c + nc * e) + (int64_t)wl * b)] = s;
+          } else if constexpr (MODE == 1) {
+            __hip_bfloat16 h, l;
+            split2(s, h, l);
+            static_cast<__hip_bfloat16*>(hi)[row * ldo + f + Df * g] = h;
+            static_cast<__hip_bfloat16*>(lo)[row * ldo + f + Df * g] = l;
+          } else {
+            static_cast<float*>(hi)[row * ldo + f + Df * g] = (float)s;
+          }
+        }
+        if (MODE != 0) {
+          for (int64_t z = f; z < pad; z += Df) {
+            if constexpr (MODE == 1) {
+              static_cast<__hip_bfloat16*>(hi)[row * ldo + K + z] = __float2bfloat16(0.f);
+              static_cast<__hip_bfloat16*>(lo)[row * ldo + K + z] = __float2bfloat16(0.f);
+            } else {
+              static_cast<float*>(hi)[row * ldo + K + z] = 0.f;
+            }
+          }
+        }
+      }
   }
 }
 
@@ -800,6 +887,10 @@ mk_status k_env_channels(const double* src, int64_t Di, int w, int64_t Dc, const
                          double* dst, hipStream_t st) {
   LAUNCH_1D(env_channels_kernel, Di * nk * Dc, st, src, Di, w, Dc, klist, nk, dst);
 }
+mk_status k_env_channels_last(const double* src, int64_t Da, int w, int64_t Df, const int* klist, int nk, double* dst,
+                              hipStream_t st) {
+  LAUNCH_1D(env_channels_last_kernel, Da * Df * nk, st, src, Da, w, Df, klist, nk, dst);
+}
 mk_status k_tl_mid(const double* t1, const double* O, int64_t Dm, int wl, int d, int wr, int64_t Dc,
                    double* t2, hipStream_t st) {
   LAUNCH_1D(tl_mid_kernel, Dm * d * wr * Dc, st, t1, O, Dm, wl, d, wr, Dc, t2);
@@ -944,32 +1035,56 @@ mk_status k_nonfinite(const double* x, int64_t n, int* flag, hipStream_t st) {
   LAUNCH_1D(nonfinite_kernel, n, st, x, n, flag);
 }
 
-mk_status k_split_bf16(const double* M, int64_t rows, int64_t cols, int64_t ld, int trans, int64_t ldo,
-                       void* hi, void* lo, hipStream_t st) {
-  if (rows * cols == 0) return MK_OK;
-  auto* h = static_cast<__hip_bfloat16*>(hi);
-  auto* l = static_cast<__hip_bfloat16*>(lo);
+mk_status k_convert(const double* M, int64_t MN, int64_t run, int nrun, int64_t runpad, int64_t ld, int trans,
+                    int64_t ldo, int split, void* hi, void* lo, hipStream_t st) {
+  if (MN * run * nrun == 0) return MK_OK;
+  MK_REQUIRE(runpad % 8 == 0 && ldo % 8 == 0 && runpad >= run && runpad * nrun <= ldo, MK_BAD_ARG,
+             "convert: runs of %lld padded to %lld, rows of %lld", (long long)run, (long long)runpad, (long long)ldo);
   if (trans) {
-    hipLaunchKernelGGL(split_plain_kernel, grid1d(ldo * cols, 4), dim3(TPB), 0, st, M, rows, cols, ld, ldo, h, l);
+    const dim3 g = grid1d(ldo / 8 * MN, 1);
+    if (split)
+      hipLaunchKernelGGL((conv_plain_kernel<true>), g, dim3(TPB), 0, st, M, run, nrun, runpad, MN, ld, ldo, hi, lo);
+    else
+      hipLaunchKernelGGL((conv_plain_kernel<false>), g, dim3(TPB), 0, st, M, run, nrun, runpad, MN, ld, ldo, hi, lo);
   } else {
-    dim3 g((unsigned)cdiv(rows, 64), (unsigned)cdiv(ldo, 64));
-    hipLaunchKernelGGL(split_trans_kernel, g, dim3(TPB), 0, st, M, rows, cols, ld, ldo, h, l);
+    dim3 g((unsigned)cdiv(MN, 64), (unsigned)cdiv(ldo, 64));
+    if (split)
+      hipLaunchKernelGGL((conv_trans_kernel<true>), g, dim3(256), 0, st, M, MN, run, nrun, runpad, ld, ldo, hi, lo);
+    else
+      hipLaunchKernelGGL((conv_trans_kernel<false>), g, dim3(256), 0, st, M, MN, run, nrun, runpad, ld, ldo, hi, lo);
   }
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
 }
 
-mk_status k_to_f32(const double* M, int64_t rows, int64_t cols, int64_t ld, int trans, int64_t ldo,
-                   float* out, hipStream_t st) {
-  if (rows * cols == 0) return MK_OK;
-  if (trans) {
-    hipLaunchKernelGGL(f32_plain_kernel, grid1d(ldo * cols, 4), dim3(TPB), 0, st, M, rows, cols, ld, ldo, out);
-  } else {
-    dim3 g((unsigned)cdiv(rows, 64), (unsigned)cdiv(ldo, 64));
-    hipLaunchKernelGGL(f32_trans_kernel, g, dim3(TPB), 0, st, M, rows, cols, ld, ldo, out);
+int gen_mid_nin(int nin) { return nin <= 8 ? 8 : nin <= 16 ? 16 : nin <= 20 ? 20 : nin <= 32 ? 32 : 0; }
+
+template <int MODE>
+static mk_status launch_gen_mid(int nin, dim3 g, hipStream_t st, const double* t1, const double* Wc, int64_t Df, int wl,
+                                int d1, int wr, int d2, int64_t nc, double* t2, int64_t ldo, void* hi, void* lo) {
+#define GEN_MID(N) \
+  hipLaunchKernelGGL((gen_mid_kernel<N, MODE>), g, dim3(256), 0, st, t1, Wc, Df, wl, d1, wr, d2, nc, t2, ldo, hi, lo)
+  switch (gen_mid_nin(nin)) {
+    case 8: GEN_MID(8); break;
+    case 16: GEN_MID(16); break;
+    case 20: GEN_MID(20); break;
+    case 32: GEN_MID(32); break;
+    default: MK_REQUIRE(false, MK_BAD_ARG, "gen_mid: %d inputs", nin);
   }
+#undef GEN_MID
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
+}
+
+mk_status k_gen_mid(const double* t1, const double* Wc, int64_t Df, int wl, int d1, int wr, int d2, int64_t nc,
+                    int prec, double* t2, int64_t ldo, void* hi, void* lo, hipStream_t st) {
+  if (Df * nc == 0) return MK_OK;
+  MK_REQUIRE(prec == MK_FP64 || ldo >= Df * wl, MK_BAD_ARG, "gen_mid: rows of %lld", (long long)ldo);
+  const dim3 g = grid1d(Df * nc, 1);
+  const int nin = d1 * wr * d2;
+  if (prec == MK_FP64) return launch_gen_mid<0>(nin, g, st, t1, Wc, Df, wl, d1, wr, d2, nc, t2, ldo, hi, lo);
+  if (prec == MK_BF16X3) return launch_gen_mid<1>(nin, g, st, t1, Wc, Df, wl, d1, wr, d2, nc, t2, ldo, hi, lo);
+  return launch_gen_mid<2>(nin, g, st, t1, Wc, Df, wl, d1, wr, d2, nc, t2, ldo, hi, lo);
 }
 
 mk_status k_nn_prologue(const double* P, const double* x, int64_t Dl, int64_t Dr, double alpha, double beta,

@@ -17,6 +17,7 @@
 // into AB when AB exists, and CB folds into AB when only AB exists.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <vector>
 
@@ -118,7 +119,7 @@ mk_status make_all_mixed(Op* op) {
   hipStream_t st = op->ctx->stream;
   const int pm = op->precisions & (MK_PREC_BF16X3 | MK_PREC_FP32);
   if (!pm) return MK_OK;
-  OpMat* mats[] = {&op->gen.L, &op->gen.R, &op->IC, &op->BE, &op->CA, &op->Cp, &op->Bp, &op->TA, &op->TB};
+  OpMat* mats[] = {&op->gen.L, &op->gen.R, &op->xrl.L, &op->xrl.R, &op->IC, &op->BE, &op->CA, &op->Cp, &op->Bp, &op->TA, &op->TB};
   for (OpMat* m : mats)
     if (m->present()) MK_TRY(m->make_mixed(pm, st));
   for (OpMat& m : op->AB) MK_TRY(m.make_mixed(pm, st));
@@ -161,6 +162,70 @@ mk_status build_lxr(Op* op, LxR& blk, const double* GL, const Wh& W1, int64_t Da
   blk.Ny = Dc * d2;
   blk.Mo = Da * d1;
   return MK_OK;
+}
+
+// Flops one byte of the middle pass of Xrl is worth: the pass moves its bytes at
+// about 4.5 TB/s while the products run at 60 (FP64) to 250 (BF16x3) TFLOP/s, and
+// an operator serves all precisions.  At w = 5 and d = 2 the two-site form
+// changes at D = 160, the one-site form at D = 300; measured at the two-site
+// line either form takes the same time within 10%.
+constexpr double XRL_FLOPS_PER_BYTE = 40.0;
+
+// The channel form of sum_k W1[g,b,h,k] W2[k,e,j,l] (two sites) or W1[g,b,h,l]
+// (W2 null) between GL (Da x W1.wl x Df) and GR (Di x wr x Dc), over the channels
+// gs and ls, or no operator if the fused form (lxr_flops, nk channels) is the faster one.
+mk_status build_xrl(Op* op, double lxr_flops, int64_t nk, const double* GL, const Wh& W1, int64_t Da, int64_t Df,
+                    const std::vector<int>& gs, const double* GR, const Wh* W2, int64_t Di, int64_t Dc,
+                    const std::vector<int>& ls, bool* built) {
+  *built = false;
+  Xrl& x = op->xrl;
+  const int wl = (int)gs.size(), wr = (int)ls.size(), d1 = W1.d, d2 = W2 ? W2->d : 1, wr_all = W2 ? W2->wr : W1.wr;
+  const int nin = d1 * wr * d2, nout = wl * d1 * d2, ldw = gen_mid_nin(nin);
+  if (ldw == 0 || nout == 0) return MK_OK;
+  const double flops = 2.0 * d1 * d2 * Df * Dc * ((double)wr * Di + (double)wl * Da);
+  const double bytes = 8.0 * Df * Dc * (nin + nout);
+  if (flops + XRL_FLOPS_PER_BYTE * bytes >= lxr_flops) return MK_OK;
+  hipStream_t st = op->ctx->stream;
+  std::vector<double> wc((size_t)nout * ldw, 0.0);
+  for (int gi = 0; gi < wl; ++gi)
+    for (int b = 0; b < d1; ++b)
+      for (int e = 0; e < d2; ++e)
+        for (int h = 0; h < d1; ++h)
+          for (int li = 0; li < wr; ++li)
+            for (int j = 0; j < d2; ++j) {
+              double s = 0.0;
+              if (W2)
+                for (int k = 0; k < W1.wr; ++k) s += W1.at(gs[gi], b, h, k) * W2->at(k, e, j, ls[li]);
+              else
+                s = W1.at(gs[gi], b, h, ls[li]);
+              wc[(size_t)(gi + wl * (b + d1 * e)) * ldw + h + d1 * (li + wr * j)] = s;
+            }
+  // coefficients, then the two channel lists, in one upload (the operator keeps it)
+  const size_t nw = wc.size() * 8;
+  std::vector<char> host(nw + (size_t)(wl + wr) * sizeof(int));
+  memcpy(host.data(), wc.data(), nw);
+  memcpy(host.data() + nw, gs.data(), gs.size() * sizeof(int));
+  memcpy(host.data() + nw + gs.size() * sizeof(int), ls.data(), ls.size() * sizeof(int));
+  MK_TRY(upload(host.data(), host.size(), x.Wc, st));
+  const int* gd = reinterpret_cast<const int*>(static_cast<const char*>(x.Wc.ptr) + nw);
+  MK_TRY(x.R.alloc('B', Di, wr * Dc));
+  MK_TRY(k_env_channels(GR, Di, wr_all, Dc, gd + wl, wr, x.R.f64(), st));
+  MK_TRY(x.L.alloc('A', Da, Df * wl));
+  MK_TRY(k_env_channels_last(GL, Da, W1.wl, Df, gd, wl, x.L.f64(), st));
+  x.Da = Da; x.Df = Df; x.Di = Di; x.Dc = Dc;
+  x.wl = wl; x.d1 = d1; x.wr = wr; x.d2 = d2; x.nk = nk;
+  *built = true;
+  return MK_OK;
+}
+
+std::vector<int> all_channels(int64_t w) {
+  std::vector<int> v((size_t)w);
+  for (int k = 0; k < (int)w; ++k) v[k] = k;
+  return v;
+}
+
+double lxr_flops(int64_t Mx, int64_t Ki, int64_t nk, int64_t Ny, int64_t Mo) {
+  return 2.0 * Mx * Ki * nk * Ny + 2.0 * Mo * Mx * nk * Ny;
 }
 
 // ---------------------------------------------------------------------------
@@ -212,6 +277,89 @@ mk_status apply_lxr(Op* op, const LxR& blk, const double* x, double* y, double a
   if (bf) p2.add(blk.L.hi.ptr, blk.L.kpad, vxr.hi, vxr.kpad, Mx * nk, blk.L.lo.ptr, vxr.lo);
   else p2.add(blk.L.f32.ptr, blk.L.kpad, vxr.hi, vxr.kpad, Mx * nk);
   return run_gemm(ctx, &p2, 1, prec, GemmShape{});
+}
+
+// y = alpha (x R) W L + beta y (Xrl).  With the scratch of a caller that cannot
+// allocate the columns c go through in as many chunks as make the intermediates
+// fit; otherwise all at once.
+mk_status apply_xrl(Op* op, const Xrl& k, const double* x, double* y, double alpha, double beta, int prec) {
+  Ctx* ctx = op->ctx;
+  hipStream_t st = ctx->stream;
+  const bool bf = prec == MK_BF16X3, f64 = prec == MK_FP64;
+  const int64_t M1 = k.Df * k.d1, K2 = k.Df * k.wl;
+  const int d2 = k.d2;
+  const bool in_place = f64 && k.wl == k.wr;
+  const size_t vx = f64 ? 0 : align256(view_bytes(M1, k.Di, 'A', prec));
+  auto t1_bytes = [&](int64_t nc) { return (size_t)M1 * k.wr * nc * d2 * 8; };
+  auto t2_bytes = [&](int64_t nc) {
+    if (in_place) return (size_t)0;
+    return f64 ? (size_t)K2 * k.d1 * nc * d2 * 8 : view_bytes(K2, k.d1 * nc * d2, 'B', prec);
+  };
+  int64_t nc = k.Dc;
+  const FixedScratch& fx = fixed_scratch();
+  if (fx.base) {
+    // the limit of the allocation-free apply counts the fused form's scratch
+    const int64_t Mx = M1, Ki = k.Di * d2, Nx = k.nk * k.Dc * d2;
+    const size_t need = align256(Mx * Nx * 8) + (f64 ? 0 : align256(view_bytes(Mx, Ki, 'A', prec)) +
+                                                              align256(view_bytes(Mx * k.nk, k.Dc * d2, 'B', prec)));
+    MK_REQUIRE(need <= fx.bytes, MK_BAD_SHAPE, "this apply needs %zu bytes of scratch; the fixed scratch holds %zu", need,
+               fx.bytes);
+  }
+  if (fx.base)
+    while (nc > 1 && align256(t1_bytes(nc)) + align256(t2_bytes(nc)) + (int64_t)vx * d2 > (int64_t)fx.bytes)
+      nc = cdiv(nc, 2);
+  double *t1 = nullptr, *t2 = nullptr;
+  char* mx = nullptr;
+  MK_TRY(carve(ctx, {{t1_bytes(nc), (void**)&t1}, {t2_bytes(nc), (void**)&t2}, {vx * d2, (void**)&mx}}));
+  if (in_place) t2 = t1;
+  std::vector<MixedView> v((size_t)d2);
+  if (!f64)
+    for (int j = 0; j < d2; ++j)
+      MK_TRY(convert_view(ctx, x + j * M1 * k.Di, M1, k.Di, M1, 'A', prec, &v[j], mx + j * vx));
+  for (int64_t c0 = 0; c0 < k.Dc; c0 += nc) {
+    const int64_t n = std::min(nc, k.Dc - c0);
+    for (int j0 = 0; j0 < d2; j0 += MAX_PROB) {
+      ProbSpec p[MAX_PROB];
+      const int np = std::min(MAX_PROB, d2 - j0);
+      for (int q = 0; q < np; ++q) {
+        const int j = j0 + q;
+        p[q].M = M1; p[q].N = k.wr * n; p[q].C = t1 + j * M1 * k.wr * n; p[q].ldc = M1;
+        if (f64) {
+          p[q].add(x + j * M1 * k.Di, M1, k.R.f64() + k.Di * k.wr * c0, k.Di, k.Di);
+        } else {
+          const size_t o = (size_t)k.wr * c0 * k.R.kpad * (bf ? 2 : 4);
+          const char* r = static_cast<const char*>(bf ? k.R.hi.ptr : k.R.f32.ptr) + o;
+          p[q].add(v[j].hi, v[j].kpad, r, k.R.kpad, k.Di, v[j].lo, bf ? static_cast<const char*>(k.R.lo.ptr) + o : nullptr);
+        }
+      }
+      MK_TRY(run_gemm(ctx, p, np, prec, GemmShape{}));
+    }
+    MixedView w;
+    if (!f64) w = view_layout(K2, k.d1 * n * d2, 'B', prec, t2);
+    MK_TRY(k_gen_mid(t1, static_cast<const double*>(k.Wc.ptr), k.Df, k.wl, k.d1, k.wr, d2, n, prec, t2, w.kpad, w.hi,
+                     w.lo, st));
+    // every column at once is one product; a chunk is one per e
+    const int ne = n == k.Dc ? 1 : d2;
+    const int64_t cols = n == k.Dc ? k.d1 * n * d2 : k.d1 * n;
+    for (int e = 0; e < ne; ++e) {
+      ProbSpec p;
+      p.M = k.Da; p.N = cols; p.C = y + k.Da * k.d1 * (c0 + k.Dc * e); p.ldc = k.Da; p.alpha = alpha; p.beta = beta;
+      if (f64) {
+        p.add(k.L.f64(), k.Da, t2 + e * K2 * cols, K2, K2);
+      } else {
+        const size_t o = (size_t)e * cols * w.kpad * (bf ? 2 : 4);
+        p.add(bf ? k.L.hi.ptr : k.L.f32.ptr, k.L.kpad, static_cast<const char*>(w.hi) + o, w.kpad, K2,
+              bf ? k.L.lo.ptr : nullptr, bf ? static_cast<const char*>(w.lo) + o : nullptr);
+      }
+      MK_TRY(run_gemm(ctx, &p, 1, prec, GemmShape{}));
+    }
+  }
+  return MK_OK;
+}
+
+mk_status apply_gen(Op* op, const double* x, double* y, double alpha, double beta, int prec) {
+  if (op->xrl.present()) return apply_xrl(op, op->xrl, x, y, alpha, beta, prec);
+  return apply_lxr(op, op->gen, x, y, alpha, beta, prec);
 }
 
 // Operand pointers of one GEMM side for precision `prec`.
@@ -553,7 +701,7 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
     }
     MK_TRY(run_gemm(ctx, ps, (int)d2, prec, nn));
   }
-  if (op->gen.present()) MK_TRY(apply_lxr(op, op->gen, x, y, alpha, bs.next(), prec));
+  if (op->has_gen()) MK_TRY(apply_gen(op, x, y, alpha, bs.next(), prec));
   if (bs.first) MK_TRY(k_axpby(0.0, y, beta, y, op->y_elems, ctx->stream));
   return MK_OK;
 }
@@ -589,7 +737,7 @@ mk_status apply_ac_jordan(Op* op, const double* x, double* y, double alpha, doub
     p.add(a.p, a.ld, b.p, b.ld, Dl * d, a.lo, b.lo);
     MK_TRY(run_gemm(ctx, &p, 1, prec, nn));
   }
-  if (op->gen.present()) MK_TRY(apply_lxr(op, op->gen, x, y, alpha, bs.next(), prec));
+  if (op->has_gen()) MK_TRY(apply_gen(op, x, y, alpha, bs.next(), prec));
   if (bs.first) MK_TRY(k_axpby(0.0, y, beta, y, op->y_elems, ctx->stream));
   return MK_OK;
 }
@@ -709,7 +857,7 @@ mk_status op_apply(Op* op, const double* x, double* y, double alpha, double beta
     case OP_C:
     case OP_AC_GEN:
     case OP_AC2_GEN:
-      return apply_lxr(op, op->gen, x, y, alpha, beta, prec);
+      return apply_gen(op, x, y, alpha, beta, prec);
     case OP_AC2_JOR:
       return apply_ac2_jordan(op, x, y, alpha, beta, prec);
     case OP_AC_JOR:
@@ -748,7 +896,7 @@ extern "C" mk_status mk_op_set_charge_blocks(mk_op h, int nl, const int64_t* lof
                                              const int64_t* roff, const int* rq, const int* pq) {
   MK_REQUIRE(h != nullptr && loff && lq && roff && rq && pq, MK_BAD_ARG, "charge blocks: null argument");
   Op* op = reinterpret_cast<Op*>(h);
-  MK_REQUIRE(op->kind == OP_AC2_JOR && !op->CA.present() && op->AB.empty() && !op->gen.present(),
+  MK_REQUIRE(op->kind == OP_AC2_JOR && !op->CA.present() && op->AB.empty() && !op->has_gen(),
              MK_NOT_SUPPORTED, "charge blocks: only nearest-neighbour two-site Jordan operators");
   MK_REQUIRE(op->d1 == op->d2 && op->d1 + op->d2 <= MAX_SEG, MK_NOT_SUPPORTED,
              "charge blocks: equal physical spaces with d1 + d2 <= %d", MAX_SEG);
@@ -974,6 +1122,13 @@ extern "C" mk_status mk_prepare_ac_generic(mk_ctx h, const double* GL, const dou
   Wh Wm;
   Wm.wl = (int)wl; Wm.d = (int)d; Wm.wr = (int)wr;
   OP_TRY(fetch(W, (size_t)wl * d * d * wr, Wm.v));
+  op->x_elems = Df * d * Di;
+  op->y_elems = Da * d * Dc;
+  op->flops = lxr_flops(Df * d, Di, wr, Dc, Da * d);
+  bool channel_form = false;
+  OP_TRY(build_xrl(op, op->flops, wr, GL, Wm, Da, Df, all_channels(wl), GR, nullptr, Di, Dc, all_channels(wr),
+                   &channel_form));
+  if (channel_form) return finish(op, out);
   LxR& g = op->gen;
   DevBuf wd, kd;
   std::vector<int> kl(wr);
@@ -988,9 +1143,6 @@ extern "C" mk_status mk_prepare_ac_generic(mk_ctx h, const double* GL, const dou
   if (e != hipSuccess) { drop(op); set_error("prepare_ac: copy failed"); return MK_HIP_ERROR; }
   if (hipStreamSynchronize(st) != hipSuccess) { drop(op); set_error("prepare_ac: sync failed"); return MK_HIP_ERROR; }
   g.Mx = Df * d; g.Ki = Di; g.nk = wr; g.Ny = Dc; g.Mo = Da * d;
-  op->x_elems = Df * d * Di;
-  op->y_elems = Da * d * Dc;
-  op->flops = g.flops();
   return finish(op, out);
 }
 
@@ -1009,12 +1161,13 @@ extern "C" mk_status mk_prepare_ac2_generic(mk_ctx h, const double* GL, const do
   B.wl = (int)wm; B.d = (int)d2; B.wr = (int)wr;
   OP_TRY(fetch(W1, (size_t)wl * d1 * d1 * wm, A.v));
   OP_TRY(fetch(W2, (size_t)wm * d2 * d2 * wr, B.v));
-  std::vector<int> kl(wm);
-  for (int k = 0; k < wm; ++k) kl[k] = k;
-  OP_TRY(build_lxr(op, op->gen, GL, A, Da, Df, -1, GR, B, Di, Dc, -1, kl));
   op->x_elems = Df * d1 * Di * d2;
   op->y_elems = Da * d1 * Dc * d2;
-  op->flops = op->gen.flops();
+  op->flops = lxr_flops(Df * d1, Di * d2, wm, Dc * d2, Da * d1);
+  bool channel_form = false;
+  OP_TRY(build_xrl(op, op->flops, wm, GL, A, Da, Df, all_channels(wl), GR, &B, Di, Dc, all_channels(wr), &channel_form));
+  if (!channel_form)
+    OP_TRY(build_lxr(op, op->gen, GL, A, Da, Df, -1, GR, B, Di, Dc, -1, all_channels(wm)));
   return finish(op, out);
 }
 
@@ -1145,8 +1298,18 @@ extern "C" mk_status mk_prepare_ac2_jordan(mk_ctx h, const double* GL, const dou
       for (int g : midL) for (int k : mids) keepL[g][k] = true;
       auto keepR = mask_none((int)wm, (int)wr);
       for (int k : mids) for (int l : midR) keepR[k][l] = true;
-      OP_TRY(build_lxr(op, op->gen, GL, A.masked(keepL), Dl, Dl, -1, GR, B.masked(keepR), Dr, Dr, -1, mids));
-      fl += op->gen.flops();
+      const Wh Am = A.masked(keepL), Bm = B.masked(keepR);
+      // the channels that reach a connected one
+      std::vector<int> gs, ls;
+      for (int g : midL)
+        if (any_nz(Am, {g}, mids)) gs.push_back(g);
+      for (int l : midR)
+        if (any_nz(Bm, mids, {l})) ls.push_back(l);
+      const double lf = lxr_flops(M, N, (int64_t)mids.size(), N, M);
+      bool channel_form = false;
+      OP_TRY(build_xrl(op, lf, (int64_t)mids.size(), GL, Am, Dl, Dl, gs, GR, &Bm, Dr, Dr, ls, &channel_form));
+      if (!channel_form) OP_TRY(build_lxr(op, op->gen, GL, Am, Dl, Dl, -1, GR, Bm, Dr, Dr, -1, mids));
+      fl += lf;
     }
   }
   op->x_elems = M * N;
@@ -1328,19 +1491,35 @@ extern "C" mk_status mk_prepare_ac_jordan(mk_ctx h, const double* GL, const doub
     auto keep = mask_none((int)wl, (int)wr);
     for (int g : midL) for (int l : midR) keep[g][l] = true;
     Wh Wa = Wm.masked(keep);
-    LxR& gb = op->gen;
-    DevBuf wad, kd;
-    OP_TRY(upload(Wa.v.data(), Wa.v.size() * 8, wad, st));
-    OP_TRY(upload(midR.data(), midR.size() * sizeof(int), kd, st));
-    const int nA = (int)midR.size();
-    OP_TRY(gb.L.alloc('A', Dl * d, Dl * d * nA));
-    OP_TRY(k_prep_L(GL, static_cast<double*>(wad.ptr), static_cast<int*>(kd.ptr), nA, Dl, Dl, (int)wl, (int)d,
-                    (int)wr, -1, gb.L.f64(), st));
-    OP_TRY(gb.R.alloc('B', Dr, nA * Dr));
-    OP_TRY(k_env_channels(GR, Dr, (int)wr, Dr, static_cast<int*>(kd.ptr), nA, gb.R.f64(), st));
-    OP_TRY(hipStreamSynchronize(st) == hipSuccess ? MK_OK : MK_HIP_ERROR);
-    gb.Mx = Dl * d; gb.Ki = Dr; gb.nk = nA; gb.Ny = Dr; gb.Mo = Dl * d;
-    fl += gb.flops();
+    std::vector<int> gs, ls;
+    for (int g : midL) {
+      bool any = false;
+      for (int l : midR) any = any || Wa.block_nz(g, l);
+      if (any) gs.push_back(g);
+    }
+    for (int l : midR) {
+      bool any = false;
+      for (int g : midL) any = any || Wa.block_nz(g, l);
+      if (any) ls.push_back(l);
+    }
+    const double lf = lxr_flops(Dl * d, Dr, (int64_t)midR.size(), Dr, Dl * d);
+    bool channel_form = false;
+    OP_TRY(build_xrl(op, lf, (int64_t)midR.size(), GL, Wa, Dl, Dl, gs, GR, nullptr, Dr, Dr, ls, &channel_form));
+    fl += lf;
+    if (!channel_form) {
+      LxR& gb = op->gen;
+      DevBuf wad, kd;
+      OP_TRY(upload(Wa.v.data(), Wa.v.size() * 8, wad, st));
+      OP_TRY(upload(midR.data(), midR.size() * sizeof(int), kd, st));
+      const int nA = (int)midR.size();
+      OP_TRY(gb.L.alloc('A', Dl * d, Dl * d * nA));
+      OP_TRY(k_prep_L(GL, static_cast<double*>(wad.ptr), static_cast<int*>(kd.ptr), nA, Dl, Dl, (int)wl, (int)d,
+                      (int)wr, -1, gb.L.f64(), st));
+      OP_TRY(gb.R.alloc('B', Dr, nA * Dr));
+      OP_TRY(k_env_channels(GR, Dr, (int)wr, Dr, static_cast<int*>(kd.ptr), nA, gb.R.f64(), st));
+      OP_TRY(hipStreamSynchronize(st) == hipSuccess ? MK_OK : MK_HIP_ERROR);
+      gb.Mx = Dl * d; gb.Ki = Dr; gb.nk = nA; gb.Ny = Dr; gb.Mo = Dl * d;
+    }
   }
   op->x_elems = Dl * d * Dr;
   op->y_elems = Dl * d * Dr;

@@ -79,6 +79,10 @@ struct FixedScratchGuard {
 mk_status noalloc_setup(int device);
 inline int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 int64_t pad8(int64_t k);
+int64_t up8(int64_t k);   // rounded up to a multiple of 8
+// K length of a mixed operand whose K comes in nrun equal runs, each padded to
+// a multiple of 8 (one run: K itself, padded with the row)
+int64_t runs_k(int64_t K, int nrun);
 
 // An operator matrix used as GEMM operand: role 'A' (rows = M, cols = K) or
 // 'B' (rows = K, cols = N).  float64 column-major, plus optional mixed copies.
@@ -89,6 +93,7 @@ struct OpMat {
   double* fp = nullptr;
   DevBuf hi, lo, f32;
   int64_t kpad = 0;
+  int nrun = 1;   // K runs of the mixed copies (runs_k)
   double* f64() const { return fp; }
   bool present() const { return fp != nullptr; }
   mk_status alloc(char r, int64_t nr, int64_t nc) {
@@ -113,10 +118,10 @@ struct MixedView {
 };
 
 mk_status convert_view(Ctx* ctx, const double* M, int64_t rows, int64_t cols, int64_t ld, char role,
-                       int prec, MixedView* out, void* mem);
+                       int prec, MixedView* out, void* mem, int nrun = 1);
 // Where convert_view puts the converted (rows x cols) view in `mem`, without converting.
-MixedView view_layout(int64_t rows, int64_t cols, char role, int prec, void* mem);
-size_t view_bytes(int64_t rows, int64_t cols, char role, int prec);
+MixedView view_layout(int64_t rows, int64_t cols, char role, int prec, void* mem, int nrun = 1);
+size_t view_bytes(int64_t rows, int64_t cols, char role, int prec, int nrun = 1);
 // A GEMM in arithmetic `prec` on the context's stream, with its K-split workspace.
 mk_status run_gemm(Ctx* ctx, const ProbSpec* p, int np, int prec, GemmShape sh);
 
@@ -130,6 +135,22 @@ struct LxR {
   double flops() const { return 2.0 * Mx * Ki * nk * Ny + 2.0 * Mo * Mx * nk * Ny; }
 };
 
+// The same sum over MPO channels without the fused L and R:
+//   t1[f,h,l,c,j] = x[f,h,i,j] GR[i,l,c]
+//   t2[f,g,b,c,e] = Wc[(g,b,e)][(h,l,j)] t1[f,h,l,c,j]
+//   y[a,b,c,e]    = GL[a,g,f] t2[f,g,b,c,e]
+// (d2 = 1 for one site).  Two products of 2 d1 d2 wr Df Di Dc and 2 d1 d2 wl
+// Da Df Dc flops against the fused form's d1 times (and, two-site, d2 times)
+// larger L and R, for one more pass over memory in between.
+struct Xrl {
+  OpMat R, L;   // GR (Di x wr Dc), GL (Da x Df wl, channels slow), the channels the MPO block connects
+  DevBuf Wc;
+  int64_t Da = 0, Df = 0, Di = 0, Dc = 0;
+  int wl = 0, d1 = 0, wr = 0, d2 = 1;
+  int64_t nk = 0;   // channels of the fused form
+  bool present() const { return L.present(); }
+};
+
 struct Op {
   Ctx* ctx = nullptr;
   OpKind kind = OP_C;
@@ -138,8 +159,10 @@ struct Op {
   int64_t x_elems = 0, y_elems = 0;
   double flops = 0.0;
 
-  // generic operators and the A/AA parts of Jordan operators
+  // generic operators and the A/AA parts of Jordan operators, in one of two forms
   LxR gen;
+  Xrl xrl;
+  bool has_gen() const { return gen.present() || xrl.present(); }
 
   // Jordan two-site terms
   OpMat IC, BE, CA;
