@@ -108,8 +108,8 @@ namespace {
 
 bool nn_jordan(const Op* op) {
   // charge-blocked operators leave y outside their blocks to the physical pass
-  return op->kind == OP_AC2_JOR && !op->CA.present() && op->AB.empty() && !op->has_gen() &&
-         (op->IC.present() || op->BE.present()) && (op->blocks.empty() || op->hasP) && !op->compact;
+  return op->kind == OP_AC2_JOR && !op->long_range() && (op->IC.present() || op->BE.present() || op->hasP) &&
+         (op->blocks.empty() || op->hasP) && !op->compact;
 }
 
 }  // namespace
@@ -146,35 +146,66 @@ mk_status Batch::ensure_plan(int prec) {
         block_probs(op, prec, xoff(i), 0, 0, 1.0, block_specs);
         continue;
       }
+      if (op->by_block()) {
+        JordanViews jv;
+        jv.x = x;
+        jordan_probs(op, prec, jv, p.C, 1.0, p.beta, block_specs);
+        continue;
+      }
       if (op->IC.present()) p.add(x, M, op->IC.f64(), N, N);
       if (op->BE.present()) p.add(op->BE.f64(), M, x, M, M);
       continue;
     }
-    // x as left factor (K = N contiguous rows) and as right factor (K = M)
+    // x as left factor (K = N contiguous rows) and as right factor (K = M),
+    // K in one run per physical state for d = 2 (the fused pass's layout)
     const bool bf = prec == MK_BF16X3;
-    const int64_t lda = pad8(N), ldb = pad8(M);
+    const int nrun = nn_runs(op);
+    const int64_t KA = runs_k(N, nrun), KB = runs_k(M, nrun);
+    const int64_t lda = pad8(KA), ldb = pad8(KB);
     const int64_t eb = bf ? 2 : 4;
     const int64_t a_hi = sbytes, a_lo = a_hi + align256(M * lda * eb);
     const int64_t b_hi = a_lo + (bf ? align256(M * lda * eb) : 0), b_lo = b_hi + align256(N * ldb * eb);
     sbytes = b_lo + (bf ? align256(N * ldb * eb) : 0);
-    if (op->IC.present()) {
-      SplitItem s{static_cast<const double*>(x), M, N, M, lda, 0, split_blocks(M, N, 0, lda),
-                  const_cast<void*>(rel_ptr(3, a_hi)), bf ? const_cast<void*>(rel_ptr(3, a_lo)) : nullptr};
-      items.push_back(s);
-      const OpMat& m = op->IC;
-      p.add(rel_ptr(3, a_hi), lda, bf ? m.hi.ptr : m.f32.ptr, m.kpad, N, bf ? rel_ptr(3, a_lo) : nullptr,
-            bf ? m.lo.ptr : nullptr);
+    const bool fused = op->hasP && op->blocks.empty() && op->d1 == 2 && op->d2 == 2;
+    if (op->by_block()) {
+      JordanViews jv;
+      jv.xa = rel_ptr(3, a_hi); jv.ka = lda; jv.alo = a_lo - a_hi;
+      jv.xb = rel_ptr(3, b_hi); jv.kb = ldb; jv.blo = b_lo - b_hi;
+      if (op->blocks.empty()) jordan_probs(op, prec, jv, p.C, 1.0, p.beta, block_specs);
+    } else {
+      if (op->IC.present()) {
+        const OpMat& m = op->IC;
+        p.add(rel_ptr(3, a_hi), lda, bf ? m.hi.ptr : m.f32.ptr, m.kpad, KA, bf ? rel_ptr(3, a_lo) : nullptr,
+              bf ? m.lo.ptr : nullptr);
+      }
+      if (op->BE.present()) {
+        const OpMat& m = op->BE;
+        p.add(bf ? m.hi.ptr : m.f32.ptr, m.kpad, rel_ptr(3, b_hi), ldb, KB, bf ? m.lo.ptr : nullptr,
+              bf ? rel_ptr(3, b_lo) : nullptr);
+      }
     }
-    if (op->BE.present()) {
-      SplitItem s{static_cast<const double*>(x), M, N, M, ldb, 1, split_blocks(M, N, 1, ldb),
-                  const_cast<void*>(rel_ptr(3, b_hi)), bf ? const_cast<void*>(rel_ptr(3, b_lo)) : nullptr};
-      items.push_back(s);
-      const OpMat& m = op->BE;
-      p.add(bf ? m.hi.ptr : m.f32.ptr, m.kpad, rel_ptr(3, b_hi), ldb, M, bf ? m.lo.ptr : nullptr,
-            bf ? rel_ptr(3, b_lo) : nullptr);
+    for (int role = 0; role < 2; ++role) {
+      if (!(role == 0 ? op->IC.present() : op->BE.present())) continue;
+      const int64_t hi = role == 0 ? a_hi : b_hi, lo = role == 0 ? a_lo : b_lo;
+      const int64_t run = (role == 0 ? N : M) / nrun, ld = role == 0 ? lda : ldb;
+      // one item per run; the last one also zeroes what the row has left
+      for (int q = 0; q < nrun; ++q) {
+        const int64_t width = q + 1 < nrun ? up8(run) : ld - q * up8(run);
+        SplitItem s{};
+        s.src = reinterpret_cast<const double*>(static_cast<const char*>(x) + (role == 0 ? M * run * q : run * q) * 8);
+        s.rows = role == 0 ? M : run;
+        s.cols = role == 0 ? run : N;
+        s.ld = M;
+        s.ldo = ld;
+        s.width = width;
+        s.trans = role;
+        s.nblocks = split_blocks(s.rows, s.cols, s.trans, width);
+        s.hi = const_cast<void*>(rel_ptr(3, hi + q * up8(run) * eb));
+        s.lo = bf ? const_cast<void*>(rel_ptr(3, lo + q * up8(run) * eb)) : nullptr;
+        items.push_back(s);
+      }
     }
-    if (op->hasP && op->IC.present() && op->BE.present() && op->blocks.empty() && op->d1 == 2 && op->d2 == 2 &&
-        M % 8 == 0 && N % 8 == 0) {
+    if (fused) {
       NNItem it{};
       it.P = static_cast<const double*>(op->P.ptr);
       it.x = static_cast<const double*>(x);
@@ -196,11 +227,11 @@ mk_status Batch::ensure_plan(int prec) {
     }
     if (!op->blocks.empty()) block_probs(op, prec, xoff(i), a_hi, b_hi, 1.0, block_specs);
   }
-  // operators with charge blocks contribute their block problems instead of the dense one
+  // operators with charge blocks, and by-block operators, contribute their block problems instead of the dense one
   {
     std::vector<ProbSpec> kept;
     for (int i = 0; i < n; ++i)
-      if (ops[i]->blocks.empty()) kept.push_back(probs[i]);
+      if (ops[i]->blocks.empty() && !ops[i]->by_block()) kept.push_back(probs[i]);
     kept.insert(kept.end(), block_specs.begin(), block_specs.end());
     probs.swap(kept);
   }

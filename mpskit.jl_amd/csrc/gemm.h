@@ -15,7 +15,7 @@
 
 namespace mk {
 
-constexpr int MAX_SEG = 4;
+constexpr int MAX_SEG = 8;
 constexpr int MAX_PROB = 4;
 
 struct GemmSeg {

@@ -122,16 +122,22 @@ int gen_mid_nin(int nin);
 mk_status k_gen_mid(const double* t1, const double* Wc, int64_t Df, int wl, int d1, int wr, int d2, int64_t nc,
                     int prec, double* t2, int64_t ldo, void* hi, void* lo, hipStream_t st);
 
-// One pass over x (d1 = d2 = 2, M = 2 Dl and N = 2 Dr multiples of 8) for the
-// mixed-precision nearest-neighbour apply: y = alpha CB(x) + beta y and the
-// K-contiguous conversions of x as left factor (xa, rows of length ka >= N) and
-// as right factor (xb, rows of length kb >= M); split = 1: bf16 hi/lo, 0: fp32
-// (xa_hi / xb_hi only).  Row padding is not written.  packed = 1: both views
-// in the packed panel layout of the 256 x 256 mixed kernel (ka = N, kb = M;
-// 2 Dl and 2 Dr multiples of 256).
-mk_status k_nn_prologue(const double* P, const double* x, int64_t Dl, int64_t Dr, double alpha, double beta,
+// One pass over x (d1 = 2, d2 = 1 or 2; x is Dl x 2 x Dr x d2) for the mixed
+// Jordan applies: y = alpha P(x) + beta y (P null: y untouched) and the
+// K-contiguous conversions of x as left factor (xa, rows (a, h) of length ka, K
+// in d2 runs) and as right factor (xb, rows (c, j) of length kb, K in 2 runs);
+// split = 1: bf16 hi/lo, 0: fp32 (xa_hi / xb_hi only).  Runs are padded with
+// zeros to a multiple of 8; the rest of a row is not written.  packed = 1 (bf16,
+// d2 = 2): both views in the packed panel layout of the 256 x 256 mixed kernel
+// (ka = N, kb = M; 2 Dl and 2 Dr multiples of 256).
+mk_status k_nn_prologue(const double* P, const double* x, int64_t Dl, int64_t Dr, int d2, double alpha, double beta,
                         double* y, int split, void* xa_hi, void* xa_lo, int64_t ka, void* xb_hi, void* xb_lo,
                         int64_t kb, int packed, hipStream_t st);
+// nq D x D blocks, block q the combination coef[q w ..] of the w levels of an
+// environment E (D x w x D): left = 0: block q at out + q D D; 1: rows
+// [q D, (q + 1) D) of an nq D x D matrix.
+mk_status k_env_blocks(const double* E, const double* coef, int64_t D, int w, int nq, int left, double* out,
+                       hipStream_t st);
 // Packed panel layout (packed_offset) of an operand held as MN K-contiguous
 // rows of length kpad >= K, element size eb (2 or 4 bytes).
 mk_status k_repack(const void* in, int64_t MN, int64_t K, int64_t kpad, int eb, void* out, hipStream_t st);

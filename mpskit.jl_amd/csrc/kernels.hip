@@ -731,7 +731,7 @@ __global__ __launch_bounds__(256) void gen_mid_kernel(const double* t1, const do
   }
 }
 
-template <bool SPLIT, bool PACK>
+template <bool SPLIT, bool PACK, int D2>
 __global__ __launch_bounds__(256) void nn_prologue_kernel(const double* __restrict__ P,
                                                           const double* __restrict__ x, int64_t Dl, int64_t Dr,
                                                           double alpha, double beta, double* __restrict__ y,
@@ -739,8 +739,37 @@ __global__ __launch_bounds__(256) void nn_prologue_kernel(const double* __restri
                                                           int64_t ka, void* __restrict__ xb_hi,
                                                           void* __restrict__ xb_lo, int64_t kb) {
   __shared__ ProTile t;
-  nn_prologue_tile<SPLIT, PACK>(P, x, Dl, Dr, alpha, beta, y, xa_hi, xa_lo, ka, xb_hi, xb_lo, kb,
-                                (int64_t)blockIdx.x * PRO_A, (int64_t)blockIdx.y * PRO_C, t);
+  nn_prologue_tile<SPLIT, PACK, D2>(P, x, Dl, Dr, alpha, beta, y, xa_hi, xa_lo, ka, xb_hi, xb_lo, kb,
+                                    (int64_t)blockIdx.x * PRO_A, (int64_t)blockIdx.y * PRO_C, t);
+}
+
+// D x D operator blocks as combinations of environment levels:
+//   right (LEFT = false): out[i + D (c + D q)]      = sum_l coef[q w + l] E[i + D (l + w c)]
+//   left  (LEFT = true):  out[a + D q + D nq f]     = sum_g coef[q w + g] E[a + D (g + w f)]
+// One thread per (row, column) writes all nq blocks and reads every level once:
+// memory-bound in its w reads and nq writes per element.
+template <bool LEFT>
+__global__ __launch_bounds__(256) void env_blocks_kernel(const double* __restrict__ E, const double* __restrict__ coef,
+                                                         int64_t D, int w, int nq, double* __restrict__ out) {
+  typedef __attribute__((address_space(1))) double gd;
+  GRID_STRIDE(idx, D * D) {
+    const int64_t c = idx / D, r = idx - c * D;
+    const gd* e = (const gd*)E + r + D * (int64_t)w * c;
+    for (int q0 = 0; q0 < nq; q0 += 4) {
+      double s[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int l = 0; l < w; ++l) {
+        const double v = e[D * l];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const double k = q0 + q < nq ? coef[(int64_t)(q0 + q) * w + l] : 0.0;
+          if (k != 0.0) s[q] += k * v;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q0 + q < nq) ((gd*)out)[LEFT ? r + D * (q0 + q) + D * nq * c : r + D * (c + D * (int64_t)(q0 + q))] = s[q];
+    }
+  }
 }
 
 // Packed panel layout from K-contiguous rows (row length kpad >= K, element
@@ -925,6 +954,8 @@ mk_status k_tr_mid_mixed(const double* t1, const double* O, int64_t Da, int wl, 
 mk_status k_phys2(const double* P, const double* x, int64_t Dl, int d1, int64_t Dr, int d2,
                   double alpha, double beta, double* y, hipStream_t st) {
   switch (d1 * d2) {
+    case 2: LAUNCH_1D(phys2_reg_kernel<2>, Dl * Dr, st, P, x, Dl, d1, Dr, d2, alpha, beta, y);
+    case 3: LAUNCH_1D(phys2_reg_kernel<3>, Dl * Dr, st, P, x, Dl, d1, Dr, d2, alpha, beta, y);
     case 4: LAUNCH_1D(phys2_reg_kernel<4>, Dl * Dr, st, P, x, Dl, d1, Dr, d2, alpha, beta, y);
     case 9: LAUNCH_1D(phys2_reg_kernel<9>, Dl * Dr, st, P, x, Dl, d1, Dr, d2, alpha, beta, y);
     case 16: LAUNCH_1D(phys2_reg_kernel<16>, Dl * Dr, st, P, x, Dl, d1, Dr, d2, alpha, beta, y);
@@ -1087,26 +1118,34 @@ mk_status k_gen_mid(const double* t1, const double* Wc, int64_t Df, int wl, int 
   return launch_gen_mid<2>(nin, g, st, t1, Wc, Df, wl, d1, wr, d2, nc, t2, ldo, hi, lo);
 }
 
-mk_status k_nn_prologue(const double* P, const double* x, int64_t Dl, int64_t Dr, double alpha, double beta,
+mk_status k_nn_prologue(const double* P, const double* x, int64_t Dl, int64_t Dr, int d2, double alpha, double beta,
                         double* y, int split, void* xa_hi, void* xa_lo, int64_t ka, void* xb_hi, void* xb_lo,
                         int64_t kb, int packed, hipStream_t st) {
   if (Dl * Dr == 0) return MK_OK;
   dim3 g((unsigned)cdiv(Dl, (int64_t)PRO_A), (unsigned)cdiv(Dr, (int64_t)PRO_C));
+  MK_REQUIRE(d2 == 1 || d2 == 2, MK_BAD_ARG, "nn_prologue: d2 = %d", d2);
   if (packed)
-    MK_REQUIRE((2 * Dl) % 256 == 0 && (2 * Dr) % 256 == 0 && ka == 2 * Dr && kb == 2 * Dl, MK_BAD_ARG,
-               "nn_prologue: packed views need 2 Dl, 2 Dr multiples of 256 and unpadded rows");
-  if (split && packed)
-    hipLaunchKernelGGL((nn_prologue_kernel<true, true>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi,
-                       xa_lo, ka, xb_hi, xb_lo, kb);
-  else if (split)
-    hipLaunchKernelGGL((nn_prologue_kernel<true, false>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi,
-                       xa_lo, ka, xb_hi, xb_lo, kb);
-  else if (packed)
-    hipLaunchKernelGGL((nn_prologue_kernel<false, true>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi,
-                       nullptr, ka, xb_hi, nullptr, kb);
-  else
-    hipLaunchKernelGGL((nn_prologue_kernel<false, false>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi,
-                       nullptr, ka, xb_hi, nullptr, kb);
+    MK_REQUIRE(split && d2 == 2 && (2 * Dl) % 256 == 0 && (2 * Dr) % 256 == 0 && ka == 2 * Dr && kb == 2 * Dl,
+               MK_BAD_ARG, "nn_prologue: packed views are bf16, with 2 Dl, 2 Dr multiples of 256 and unpadded rows");
+#define NN_PROLOGUE(S, K, N) \
+  hipLaunchKernelGGL((nn_prologue_kernel<S, K, N>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi, \
+                     S ? xa_lo : nullptr, ka, xb_hi, S ? xb_lo : nullptr, kb)
+  if (packed) NN_PROLOGUE(true, true, 2);
+  else if (split && d2 == 2) NN_PROLOGUE(true, false, 2);
+  else if (split) NN_PROLOGUE(true, false, 1);
+  else if (d2 == 2) NN_PROLOGUE(false, false, 2);
+  else NN_PROLOGUE(false, false, 1);
+#undef NN_PROLOGUE
+  MK_CHECK_HIP(hipGetLastError());
+  return MK_OK;
+}
+
+mk_status k_env_blocks(const double* E, const double* coef, int64_t D, int w, int nq, int left, double* out,
+                       hipStream_t st) {
+  if (nq == 0) return MK_OK;
+  const dim3 g = grid1d(D * D, 1);
+  if (left) hipLaunchKernelGGL((env_blocks_kernel<true>), g, dim3(256), 0, st, E, coef, D, w, nq, out);
+  else hipLaunchKernelGGL((env_blocks_kernel<false>), g, dim3(256), 0, st, E, coef, D, w, nq, out);
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
 }

@@ -110,20 +110,21 @@ bool packing_enabled() {
 }
 
 bool nn_fused(const Op* op) {
-  const int64_t M = op->Dl * op->d1, N = op->Dr * op->d2;
-  return op->hasP && op->IC.present() && op->BE.present() && !op->CA.present() && op->AB.empty() &&
-         op->d1 == 2 && op->d2 == 2 && M % 8 == 0 && N % 8 == 0;
+  return op->hasP && op->IC.present() && op->BE.present() && !op->long_range() && op->d1 == 2 && op->d2 == 2;
 }
 
 mk_status make_all_mixed(Op* op) {
   hipStream_t st = op->ctx->stream;
   const int pm = op->precisions & (MK_PREC_BF16X3 | MK_PREC_FP32);
   if (!pm) return MK_OK;
-  OpMat* mats[] = {&op->gen.L, &op->gen.R, &op->xrl.L, &op->xrl.R, &op->IC, &op->BE, &op->CA, &op->Cp, &op->Bp, &op->TA, &op->TB};
+  OpMat* mats[] = {&op->gen.L, &op->gen.R, &op->xrl.L, &op->xrl.R, &op->RB, &op->LB, &op->IC, &op->BE, &op->CA, &op->Cp, &op->Bp, &op->TA, &op->TB};
   for (OpMat* m : mats)
-    if (m->present()) MK_TRY(m->make_mixed(pm, st));
+    if (m->present()) {
+      if (op->kind == OP_AC2_JOR && (m == &op->IC || m == &op->BE)) m->nrun = nn_runs(op);
+      MK_TRY(m->make_mixed(pm, st));
+    }
   for (OpMat& m : op->AB) MK_TRY(m.make_mixed(pm, st));
-  if (op->kind == OP_AC2_JOR && nn_fused(op) && packing_enabled()) {
+  if (op->kind == OP_AC2_JOR && nn_fused(op) && !op->by_block() && packing_enabled()) {
     const int64_t M = op->Dl * op->d1, N = op->Dr * op->d2;
     const int64_t Ks[2] = {N, M};
     // BF16x3 only: the FP32 kernel measured 2% slower on packed operands
@@ -383,6 +384,169 @@ Side packed_side(const OpMat& m, int prec) {
 
 }  // namespace
 
+int nn_runs(const Op* op) { return op->d1 == 2 && op->d2 == 2 ? 2 : 1; }
+
+void jordan_probs(const Op* op, int prec, const JordanViews& v, const void* y, double alpha, double beta,
+                  std::vector<ProbSpec>& out) {
+  const int64_t Dl = op->Dl, Dr = op->Dr, M = Dl * op->d1, N = Dr * op->d2;
+  const int64_t eb = prec == MK_FP64 ? 8 : prec == MK_BF16X3 ? 2 : 4;
+  const bool bf = prec == MK_BF16X3;
+  auto at = [&](const void* p, int64_t elems) -> const void* { return static_cast<const char*>(p) + elems * eb; };
+  auto lo_of = [&](const void* p, int64_t bytes) -> const void* {
+    return bf ? static_cast<const char*>(p) + bytes : nullptr;
+  };
+  // an operator matrix's element offset as (hi, lo)
+  auto mat = [&](const OpMat& m, int64_t elems, const void** lo) -> const void* {
+    *lo = bf ? at(m.lo.ptr, elems) : nullptr;
+    return prec == MK_FP64 ? at(m.f64(), elems) : at(bf ? m.hi.ptr : m.f32.ptr, elems);
+  };
+  for (const Op::JProb& jp : op->jprobs) {
+    ProbSpec p;
+    p.M = Dl;
+    p.N = Dr;
+    p.C = const_cast<double*>(static_cast<const double*>(y)) + jp.b * Dl + jp.e * M * Dr;
+    p.ldc = M;
+    p.alpha = alpha;
+    p.beta = beta;
+    for (size_t q = 0; q < jp.seg.size(); ++q) {
+      const Op::JSeg& sg = jp.seg[q];
+      // both runs of an I or E row of blocks are one segment
+      const bool two = q + 1 < jp.seg.size() && jp.seg[q + 1].kind == sg.kind &&
+                       ((sg.kind == 'I' && sg.j == 0) || (sg.kind == 'E' && sg.h == 0));
+      const void *lo_m = nullptr, *m = nullptr;
+      if (prec == MK_FP64) {
+        const void* xs = at(v.x, sg.h * Dl + sg.j * M * Dr);
+        switch (sg.kind) {
+          case 'I':
+            p.add(xs, M, mat(op->IC, sg.j * Dr + jp.e * Dr * N, &lo_m), N, two ? 2 * Dr : Dr);
+            break;
+          case 'E':
+            p.add(mat(op->BE, jp.b * Dl + sg.h * Dl * M, &lo_m), M, xs, M, two ? 2 * Dl : Dl);
+            break;
+          case 'R':
+            p.add(xs, M, mat(op->RB, sg.blk * Dr * Dr, &lo_m), Dr, Dr);
+            break;
+          default:
+            p.add(mat(op->LB, sg.blk * Dl, &lo_m), Dl * op->nL, xs, M, Dl);
+        }
+      } else {
+        const int64_t rr = up8(Dr), rl = up8(Dl);
+        const void* a = at(v.xa, sg.h * Dl * v.ka + sg.j * rr);
+        const void* b = at(v.xb, sg.j * Dr * v.kb + sg.h * rl);
+        switch (sg.kind) {
+          case 'I':
+            m = mat(op->IC, jp.e * Dr * op->IC.kpad + sg.j * rr, &lo_m);
+            p.add(a, v.ka, m, op->IC.kpad, two ? 2 * rr : Dr, lo_of(a, v.alo), lo_m);
+            break;
+          case 'E':
+            m = mat(op->BE, jp.b * Dl * op->BE.kpad + sg.h * rl, &lo_m);
+            p.add(m, op->BE.kpad, b, v.kb, two ? 2 * rl : Dl, lo_m, lo_of(b, v.blo));
+            break;
+          case 'R':
+            m = mat(op->RB, sg.blk * Dr * op->RB.kpad, &lo_m);
+            p.add(a, v.ka, m, op->RB.kpad, Dr, lo_of(a, v.alo), lo_m);
+            break;
+          default:
+            m = mat(op->LB, sg.blk * Dl * op->LB.kpad, &lo_m);
+            p.add(m, op->LB.kpad, b, v.kb, Dl, lo_m, lo_of(b, v.blo));
+        }
+      }
+      if (two) ++q;
+    }
+    out.push_back(p);
+  }
+}
+
+namespace {
+
+// By-block Jordan apply: the physical term (and the mixed views of x) in one
+// pass over x, then one launch over the output blocks, which also takes in the
+// channel form's last product (its first product and MPO step run before).
+mk_status apply_by_block(Op* op, const double* x, double* y, double alpha, double beta, int prec) {
+  Ctx* ctx = op->ctx;
+  hipStream_t st = ctx->stream;
+  const int64_t Dl = op->Dl, Dr = op->Dr;
+  const int d1 = (int)op->d1, d2 = (int)op->d2;
+  const int64_t M = Dl * d1, N = Dr * d2;
+  const bool f64 = prec == MK_FP64, bf = prec == MK_BF16X3;
+  const Xrl& k = op->xrl;
+  const bool in_place = f64 && k.wl == k.wr;
+  // the left-factor view has one row per (a, h) and a K run per j
+  const size_t va = f64 ? 0 : view_bytes(M, N, 'A', prec, d2), vb = f64 ? 0 : view_bytes(M, N, 'B', prec, d1);
+  size_t s1 = 0, s2 = 0;
+  if (k.present()) {
+    s1 = (size_t)M * k.wr * N * 8;
+    s2 = in_place ? 0 : f64 ? (size_t)Dl * k.wl * d1 * N * 8 : view_bytes(Dl * k.wl, d1 * N, 'B', prec);
+  }
+  // too much for a caller that cannot allocate: the channel form by itself, in chunks
+  const FixedScratch& fx = fixed_scratch();
+  const bool with_xrl = k.present() && (!fx.base || align256(va) + align256(vb) + align256(s1) + align256(s2) <=
+                                                        (int64_t)fx.bytes);
+  if (!with_xrl) s1 = s2 = 0;
+  void *ma = nullptr, *mb = nullptr;
+  double *t1 = nullptr, *t2 = nullptr;
+  MK_TRY(carve(ctx, {{va, &ma}, {vb, &mb}, {s1, (void**)&t1}, {s2, (void**)&t2}}));
+  if (in_place) t2 = t1;
+  BetaSeq bs{beta};
+  JordanViews v;
+  v.x = x;
+  const double* P = op->hasP ? static_cast<const double*>(op->P.ptr) : nullptr;
+  if (f64) {
+    if (P) MK_TRY(k_phys2(P, x, Dl, d1, Dr, d2, alpha, bs.next(), y, st));
+  } else {
+    const MixedView a = view_layout(M, N, 'A', prec, ma, d2), b = view_layout(M, N, 'B', prec, mb, d1);
+    if (d1 == 2 && d2 <= 2) {
+      MK_TRY(k_nn_prologue(P, x, Dl, Dr, d2, alpha, P ? bs.next() : 0.0, y, bf ? 1 : 0, a.hi, a.lo, a.kpad, b.hi, b.lo,
+                           b.kpad, 0, st));
+    } else {
+      MixedView t;
+      if (P) MK_TRY(k_phys2(P, x, Dl, d1, Dr, d2, alpha, bs.next(), y, st));
+      MK_TRY(convert_view(ctx, x, M, N, M, 'A', prec, &t, ma, d2));
+      MK_TRY(convert_view(ctx, x, M, N, M, 'B', prec, &t, mb, d1));
+    }
+    v.xa = a.hi; v.ka = a.kpad; v.alo = bf ? static_cast<char*>(a.lo) - static_cast<char*>(a.hi) : 0;
+    v.xb = b.hi; v.kb = b.kpad; v.blo = bf ? static_cast<char*>(b.lo) - static_cast<char*>(b.hi) : 0;
+  }
+  std::vector<ProbSpec> probs;
+  jordan_probs(op, prec, v, y, alpha, bs.next(), probs);
+  if (with_xrl) {
+    ProbSpec p1[MAX_PROB];
+    for (int j = 0; j < d2; ++j) {
+      p1[j].M = M; p1[j].N = k.wr * Dr; p1[j].C = t1 + j * M * k.wr * Dr; p1[j].ldc = M;
+      if (f64) {
+        p1[j].add(x + j * M * Dr, M, k.R.f64(), Dr, Dr);
+      } else {
+        const int64_t o = j * up8(Dr) * (bf ? 2 : 4);
+        const char* a = static_cast<const char*>(v.xa) + o;
+        p1[j].add(a, v.ka, bf ? k.R.hi.ptr : k.R.f32.ptr, k.R.kpad, Dr, bf ? a + v.alo : nullptr, k.R.lo.ptr);
+      }
+    }
+    MK_TRY(run_gemm(ctx, p1, d2, prec, GemmShape{}));
+    MixedView w;
+    const int64_t K2 = Dl * k.wl;
+    if (!f64) w = view_layout(K2, d1 * N, 'B', prec, t2);
+    MK_TRY(k_gen_mid(t1, static_cast<const double*>(k.Wc.ptr), Dl, k.wl, d1, k.wr, d2, Dr, prec, t2, w.kpad, w.hi, w.lo,
+                     st));
+    // rows (b, c, e) of t2: block (b, e) is every d1-th
+    for (size_t q = 0; q < probs.size(); ++q) {
+      const int64_t row = op->jprobs[q].b + d1 * Dr * op->jprobs[q].e;
+      if (f64) {
+        probs[q].add(k.L.f64(), Dl, t2 + row * K2, d1 * K2, K2);
+      } else {
+        const int64_t o = row * w.kpad * (bf ? 2 : 4);
+        probs[q].add(bf ? k.L.hi.ptr : k.L.f32.ptr, k.L.kpad, static_cast<const char*>(w.hi) + o, d1 * w.kpad, K2,
+                     k.L.lo.ptr, bf ? static_cast<const char*>(w.lo) + o : nullptr);
+      }
+    }
+  }
+  for (size_t q0 = 0; q0 < probs.size(); q0 += MAX_PROB)
+    MK_TRY(run_gemm(ctx, probs.data() + q0, (int)std::min<size_t>(MAX_PROB, probs.size() - q0), prec, GemmShape{}));
+  if (op->has_gen() && !with_xrl) MK_TRY(apply_gen(op, x, y, alpha, 1.0, prec));
+  return MK_OK;
+}
+
+}  // namespace
+
 void block_probs(const Op* op, int prec, int64_t xoff, int64_t sa, int64_t sb, double beta,
                  std::vector<ProbSpec>& out) {
   const int64_t M = op->Dl * op->d1, N = op->Dr * op->d2;
@@ -446,7 +610,7 @@ mk_status apply_blocks(Op* op, const double* x, double* y, double alpha, double 
   if (fused) {
     const MixedView xa = view_layout(M, N, 'A', prec, mv);
     const MixedView xb = view_layout(M, N, 'B', prec, static_cast<char*>(mv) + va);
-    MK_TRY(k_nn_prologue(static_cast<const double*>(op->P.ptr), x, Dl, Dr, 1.0, b0, out, prec == MK_BF16X3, xa.hi,
+    MK_TRY(k_nn_prologue(static_cast<const double*>(op->P.ptr), x, Dl, Dr, 2, 1.0, b0, out, prec == MK_BF16X3, xa.hi,
                          xa.lo, xa.kpad, xb.hi, xb.lo, xb.kpad, 0, st));
   } else if (op->hasP) {
     MK_TRY(k_phys2(static_cast<const double*>(op->P.ptr), x, Dl, (int)d1, Dr, (int)d2, 1.0, b0, out, st));
@@ -568,7 +732,7 @@ mk_status apply_compact(Op* op, const double* x, double* y, double alpha, double
         it.cols = bp.n;
         it.ld = bp.m;
         it.trans = role;   // 0: left-factor view (K = columns), 1: right-factor view (K = rows)
-        it.ldo = role == 0 ? pad8(bp.n) : pad8(bp.m);
+        it.ldo = it.width = role == 0 ? pad8(bp.n) : pad8(bp.m);
         it.nblocks = split_blocks(it.rows, it.cols, it.trans, it.ldo);
         it.hi = const_cast<void*>(rel_ptr(3, role == 0 ? cv.a[b] : cv.b[b]));
         it.lo = prec == MK_BF16X3 ? const_cast<void*>(rel_ptr(3, role == 0 ? cv.alo[b] : cv.blo[b])) : nullptr;
@@ -619,8 +783,12 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
   const int64_t Dl = op->Dl, Dr = op->Dr, d1 = op->d1, d2 = op->d2;
   const int64_t M = Dl * d1, N = Dr * d2;
   BetaSeq bs{beta};
+  if (op->by_block()) return apply_by_block(op, x, y, alpha, beta, prec);
   // mixed-precision views of x: as left factor (M x N) and as right factor (K = M rows)
   MixedView xa, xb, xca;
+  // K runs of the IC and BE copies (AB's, which take the same view of x as BE, have one)
+  const int ra = op->IC.present() ? op->IC.nrun : 1, rb = op->BE.present() ? op->BE.nrun : 1;
+  const int64_t KA = prec == MK_FP64 ? N : runs_k(N, ra), KB = prec == MK_FP64 ? M : runs_k(M, rb);
   // nearest-neighbour chains with d = 2: the CB term and both conversions of x
   // come from one pass over x
   const bool fused = prec != MK_FP64 && nn_fused(op);
@@ -630,12 +798,12 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
     void *ma = nullptr, *mb = nullptr, *mc = nullptr;
     const bool need_a = op->IC.present(), need_b = op->BE.present() || !op->AB.empty();
     const bool need_ca = op->CA.present();
-    MK_TRY(carve(ctx, {{need_a ? view_bytes(M, N, 'A', prec) : 0, &ma},
-                       {need_b ? view_bytes(M, N, 'B', prec) : 0, &mb},
+    MK_TRY(carve(ctx, {{need_a ? view_bytes(M, N, 'A', prec, ra) : 0, &ma},
+                       {need_b ? view_bytes(M, N, 'B', prec, rb) : 0, &mb},
                        {need_ca ? view_bytes(Dl, d1 * N, 'A', prec) : 0, &mc}}));
     if (fused) {
-      xa = view_layout(M, N, 'A', prec, ma);
-      xb = view_layout(M, N, 'B', prec, mb);
+      xa = view_layout(M, N, 'A', prec, ma, ra);
+      xb = view_layout(M, N, 'B', prec, mb, rb);
       if (packed) {
         // the same memory, packed: no row padding, so kpad is the K length
         // (N for xa, M for xb); the lo parts stay where the row layout puts them
@@ -643,15 +811,15 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
         xb.kpad = M;
       }
     } else {
-      if (need_a) MK_TRY(convert_view(ctx, x, M, N, M, 'A', prec, &xa, ma));
-      if (need_b) MK_TRY(convert_view(ctx, x, M, N, M, 'B', prec, &xb, mb));
+      if (need_a) MK_TRY(convert_view(ctx, x, M, N, M, 'A', prec, &xa, ma, ra));
+      if (need_b) MK_TRY(convert_view(ctx, x, M, N, M, 'B', prec, &xb, mb, rb));
       if (need_ca) MK_TRY(convert_view(ctx, x, Dl, d1 * N, Dl, 'A', prec, &xca, mc));
     }
   }
   const GemmShape nn{};
   // two-site CB term first: a memory-bound pass that reads x once
   if (fused)
-    MK_TRY(k_nn_prologue(static_cast<const double*>(op->P.ptr), x, Dl, Dr, alpha, bs.next(), y,
+    MK_TRY(k_nn_prologue(static_cast<const double*>(op->P.ptr), x, Dl, Dr, 2, alpha, bs.next(), y,
                          prec == MK_BF16X3, xa.hi, xa.lo, xa.kpad, xb.hi, xb.lo, xb.kpad, packed ? 1 : 0,
                          ctx->stream));
   else if (op->hasP)
@@ -663,13 +831,13 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
     if (op->IC.present()) {
       Side a = prec == MK_FP64 ? Side{x, nullptr, M} : view_side(xa);
       Side b = packed ? packed_side(op->IC, prec) : mat_side(op->IC, prec);
-      p.add(a.p, a.ld, b.p, b.ld, N, a.lo, b.lo);
+      p.add(a.p, a.ld, b.p, b.ld, KA, a.lo, b.lo);
       p.seg[p.nseg - 1].packA = p.seg[p.nseg - 1].packB = packed;
     }
     if (op->BE.present()) {
       Side a = packed ? packed_side(op->BE, prec) : mat_side(op->BE, prec);
       Side b = prec == MK_FP64 ? Side{x, nullptr, M} : view_side(xb);
-      p.add(a.p, a.ld, b.p, b.ld, M, a.lo, b.lo);
+      p.add(a.p, a.ld, b.p, b.ld, KB, a.lo, b.lo);
       p.seg[p.nseg - 1].packA = p.seg[p.nseg - 1].packB = packed;
     }
     MK_TRY(run_gemm(ctx, &p, 1, prec, nn));
@@ -707,6 +875,7 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
 }
 
 mk_status apply_ac_jordan(Op* op, const double* x, double* y, double alpha, double beta, int prec) {
+  if (op->by_block()) return apply_by_block(op, x, y, alpha, beta, prec);
   Ctx* ctx = op->ctx;
   const int64_t Dl = op->Dl, Dr = op->Dr, d = op->d1;
   BetaSeq bs{beta};
@@ -896,7 +1065,7 @@ extern "C" mk_status mk_op_set_charge_blocks(mk_op h, int nl, const int64_t* lof
                                              const int64_t* roff, const int* rq, const int* pq) {
   MK_REQUIRE(h != nullptr && loff && lq && roff && rq && pq, MK_BAD_ARG, "charge blocks: null argument");
   Op* op = reinterpret_cast<Op*>(h);
-  MK_REQUIRE(op->kind == OP_AC2_JOR && !op->CA.present() && op->AB.empty() && !op->has_gen(),
+  MK_REQUIRE(op->kind == OP_AC2_JOR && !op->long_range(),
              MK_NOT_SUPPORTED, "charge blocks: only nearest-neighbour two-site Jordan operators");
   MK_REQUIRE(op->d1 == op->d2 && op->d1 + op->d2 <= MAX_SEG, MK_NOT_SUPPORTED,
              "charge blocks: equal physical spaces with d1 + d2 <= %d", MAX_SEG);
@@ -1171,6 +1340,229 @@ extern "C" mk_status mk_prepare_ac2_generic(mk_ctx h, const double* GL, const do
   return finish(op, out);
 }
 
+namespace {
+
+bool any_block(const Wh& W, const std::vector<int>& gs, const std::vector<int>& ks) {
+  for (int g : gs)
+    for (int k : ks)
+      if (W.block_nz(g, k)) return true;
+  return false;
+}
+
+// The coefficient rows of D x D blocks over the w levels of an environment,
+// each different row kept once.
+struct BlockSet {
+  int w;
+  std::vector<double> coef;
+  int n = 0;
+  // the index of a row, or -1 for a zero one
+  int add(const std::vector<double>& row) {
+    bool nz = false;
+    for (double c : row) nz = nz || c != 0.0;
+    if (!nz) return -1;
+    for (int q = 0; q < n; ++q)
+      if (std::equal(row.begin(), row.end(), coef.begin() + (size_t)q * w)) return q;
+    coef.insert(coef.end(), row.begin(), row.end());
+    return n++;
+  }
+};
+
+mk_status build_blocks(Op* op, const BlockSet& bs, const double* E, int64_t D, bool left) {
+  if (bs.n == 0) return MK_OK;
+  hipStream_t st = op->ctx->stream;
+  OpMat& m = left ? op->LB : op->RB;
+  if (left) MK_TRY(m.alloc('A', D * bs.n, D));
+  else MK_TRY(m.alloc('B', D, D * bs.n));
+  DevBuf cd;
+  MK_TRY(upload(bs.coef.data(), bs.coef.size() * 8, cd, st));
+  MK_TRY(k_env_blocks(E, static_cast<double*>(cd.ptr), D, bs.w, bs.n, left ? 1 : 0, m.f64(), st));
+  MK_CHECK_HIP(hipStreamSynchronize(st));
+  (left ? op->nL : op->nR) = bs.n;
+  return MK_OK;
+}
+
+// Jordan two-site operator for d1 = d2 = 2 (hamiltonian_derivatives.jl:272-468
+// with its terms kept by output block).  With GL's "not started" and GR's
+// "finished" level the identity, the terms that are the identity on both
+// environments (ID, DE, CB) form the physical term P; what is left of
+//   sum_{g,k,l} GL_g W1[g,b,h,k] W2[k,e,j,l] GR_l
+// acts from the right alone (g = not started, l below finished), from the left
+// alone, or from both (AA).  The reference folds ID into IC, DE into BE and, on
+// longer-ranged chains, IC, BE and CB into CA and AB, which fills blocks that are
+// zero: apart, half of the blocks of an Ising chain and a quarter of those of
+// J1-J2 need no product.
+mk_status prepare_ac2_by_block(Op* op, const double* GL, const Wh& A, const Wh& B, const double* GR,
+                               const std::vector<int>& midL, const std::vector<int>& midM,
+                               const std::vector<int>& midR) {
+  hipStream_t st = op->ctx->stream;
+  const int64_t Dl = op->Dl, Dr = op->Dr, M = 2 * Dl, N = 2 * Dr;
+  const int wl = A.wl, wm = A.wr, wr = B.wr, kEnd = wm - 1, lEnd = wr - 1;
+  const bool hasCA = any_block(A, {0}, midM) && any_block(B, midM, midR);
+  const bool hasAB = any_block(A, midL, midM) && any_block(B, midM, {lEnd});
+  // the flops of the reference's prepared form
+  double fl = hasCA ? 2.0 * Dl * (2.0 * N) * (2.0 * N) : 2.0 * M * (double)N * N;
+  if (hasAB) fl += 8.0 * (double)M * M * Dr;
+  else if (wl > 1 || A.block_nz(0, kEnd)) fl += 2.0 * M * (double)M * N;
+
+  std::vector<double> P(16, 0.0);
+  bool pnz = false, cbnz = false;
+  for (int b = 0; b < 2; ++b)
+    for (int e = 0; e < 2; ++e)
+      for (int h = 0; h < 2; ++h)
+        for (int j = 0; j < 2; ++j) {
+          double s = 0.0, cb = 0.0;
+          for (int k = 0; k < wm; ++k) {
+            const double t = A.at(0, b, h, k) * B.at(k, e, j, lEnd);
+            s += t;
+            if (k != 0 && k != kEnd) cb += t;
+          }
+          P[b + 2 * (e + 2 * (h + 2 * j))] = s;
+          pnz = pnz || s != 0.0;
+          cbnz = cbnz || cb != 0.0;
+        }
+  if (!hasCA && !hasAB && cbnz) fl += 32.0 * Dl * Dr;
+  if (pnz) {
+    MK_TRY(upload(P.data(), P.size() * 8, op->P, st));
+    op->hasP = true;
+  }
+
+  if (!hasCA && !hasAB) {
+    // nearest neighbours: right blocks are the identity in (b, h), left ones in (e, j)
+    bool nzI[2][2], nzE[2][2], anyI = false, anyE = false, full = true;
+    for (int q = 0; q < 2; ++q)
+      for (int o = 0; o < 2; ++o) {
+        nzI[q][o] = nzE[q][o] = false;   // [in][out]
+        for (int l = 0; l < lEnd; ++l) nzI[q][o] = nzI[q][o] || B.at(0, o, q, l) != 0.0;
+        for (int g = 1; g < wl; ++g) nzE[q][o] = nzE[q][o] || A.at(g, o, q, kEnd) != 0.0;
+        anyI = anyI || nzI[q][o];
+        anyE = anyE || nzE[q][o];
+        full = full && nzI[q][o] && nzE[q][o];
+      }
+    std::vector<int> kl = {0, kEnd};
+    DevBuf wd, kd;
+    Wh Bm = B, Am = A;
+    for (int e = 0; e < 2; ++e)
+      for (int j = 0; j < 2; ++j) {
+        Bm.at(0, e, j, lEnd) = 0.0;
+        Am.at(0, e, j, kEnd) = 0.0;
+      }
+    std::vector<double> both(Bm.v);
+    both.insert(both.end(), Am.v.begin(), Am.v.end());
+    MK_TRY(upload(both.data(), both.size() * 8, wd, st));
+    MK_TRY(upload(kl.data(), kl.size() * sizeof(int), kd, st));
+    const double* w2 = static_cast<double*>(wd.ptr);
+    const int* kp = static_cast<int*>(kd.ptr);
+    if (anyI) {
+      MK_TRY(op->IC.alloc('B', N, N));
+      MK_TRY(k_prep_R(GR, w2, kp, 1, Dr, Dr, wm, 2, wr, lEnd, op->IC.f64(), st));
+    }
+    if (anyE) {
+      MK_TRY(op->BE.alloc('A', M, M));
+      MK_TRY(k_prep_L(GL, w2 + Bm.v.size(), kp + 1, 1, Dl, Dl, wl, 2, wm, 0, op->BE.f64(), st));
+    }
+    MK_CHECK_HIP(hipStreamSynchronize(st));
+    // with every block filled the two products of the whole matrices are the
+    // larger, better filled launch
+    if (!full)
+      for (int e = 0; e < 2; ++e)
+        for (int b = 0; b < 2; ++b) {
+          Op::JProb jp{b, e, {}};
+          for (int j = 0; j < 2; ++j)
+            if (nzI[j][e]) jp.seg.push_back({'I', b, j, 0});
+          for (int h = 0; h < 2; ++h)
+            if (nzE[h][b]) jp.seg.push_back({'E', h, e, 0});
+          op->jprobs.push_back(jp);
+        }
+  } else {
+    BlockSet R{wr, {}, 0}, L{wl, {}, 0};
+    for (int e = 0; e < 2; ++e)
+      for (int b = 0; b < 2; ++b) {
+        Op::JProb jp{b, e, {}};
+        for (int j = 0; j < 2; ++j)
+          for (int h = 0; h < 2; ++h) {
+            std::vector<double> rc((size_t)wr, 0.0);
+            for (int l = 0; l < lEnd; ++l)
+              for (int k = 0; k < kEnd; ++k) rc[l] += A.at(0, b, h, k) * B.at(k, e, j, l);
+            const int q = R.add(rc);
+            if (q >= 0) jp.seg.push_back({'R', h, j, q});
+          }
+        for (int j = 0; j < 2; ++j)
+          for (int h = 0; h < 2; ++h) {
+            std::vector<double> lc((size_t)wl, 0.0);
+            for (int g = 1; g < wl; ++g)
+              for (int k = 1; k <= kEnd; ++k) lc[g] += A.at(g, b, h, k) * B.at(k, e, j, lEnd);
+            const int q = L.add(lc);
+            if (q >= 0) jp.seg.push_back({'L', h, j, q});
+          }
+        op->jprobs.push_back(jp);
+      }
+    MK_TRY(build_blocks(op, R, GR, Dr, false));
+    MK_TRY(build_blocks(op, L, GL, Dl, true));
+  }
+  // AA over the connected channels (hamiltonian_derivatives.jl:243-270)
+  std::vector<int> mids, gs, ls;
+  for (int k : midM)
+    if (any_block(A, midL, {k}) && any_block(B, {k}, midR)) mids.push_back(k);
+  for (int g : midL)
+    if (any_block(A, {g}, mids)) gs.push_back(g);
+  for (int l : midR)
+    if (any_block(B, mids, {l})) ls.push_back(l);
+  if (!mids.empty()) {
+    auto keepL = mask_none(wl, wm), keepR = mask_none(wm, wr);
+    for (int g : midL) for (int k : mids) keepL[g][k] = true;
+    for (int k : mids) for (int l : midR) keepR[k][l] = true;
+    const Wh Am = A.masked(keepL), Bm = B.masked(keepR);
+    const double lf = lxr_flops(M, N, (int64_t)mids.size(), N, M);
+    bool channel_form = false;
+    MK_TRY(build_xrl(op, lf, (int64_t)mids.size(), GL, Am, Dl, Dl, gs, GR, &Bm, Dr, Dr, ls, &channel_form));
+    if (!channel_form) MK_TRY(build_lxr(op, op->gen, GL, Am, Dl, Dl, -1, GR, Bm, Dr, Dr, -1, mids));
+    fl += lf;
+  }
+  op->x_elems = op->y_elems = M * N;
+  op->flops = fl;
+  return MK_OK;
+}
+
+// Jordan one-site operator for d <= 3 (hamiltonian_derivatives.jl:57-157), by
+// output block as above: C and I act from the right, B and E from the left, D is
+// the physical term, A the channel form's (its last product joins the launch).
+mk_status prepare_ac_by_block(Op* op, const double* GL, const Wh& W, const double* GR) {
+  hipStream_t st = op->ctx->stream;
+  const int d = W.d, wl = W.wl, wr = W.wr, lEnd = wr - 1;
+  std::vector<double> P((size_t)d * d);
+  bool pnz = false;
+  for (int b = 0; b < d; ++b)
+    for (int h = 0; h < d; ++h) {
+      P[b + d * h] = W.at(0, b, h, lEnd);
+      pnz = pnz || P[b + d * h] != 0.0;
+    }
+  if (pnz) {
+    MK_TRY(upload(P.data(), P.size() * 8, op->P, st));
+    op->hasP = true;
+  }
+  BlockSet R{wr, {}, 0}, L{wl, {}, 0};
+  for (int b = 0; b < d; ++b) {
+    Op::JProb jp{b, 0, {}};
+    for (int h = 0; h < d; ++h) {
+      std::vector<double> rc((size_t)wr, 0.0);
+      for (int l = 0; l < lEnd; ++l) rc[l] = W.at(0, b, h, l);
+      const int q = R.add(rc);
+      if (q >= 0) jp.seg.push_back({'R', h, 0, q});
+    }
+    for (int h = 0; h < d; ++h) {
+      std::vector<double> lc((size_t)wl, 0.0);
+      for (int g = 1; g < wl; ++g) lc[g] = W.at(g, b, h, lEnd);
+      const int q = L.add(lc);
+      if (q >= 0) jp.seg.push_back({'L', h, 0, q});
+    }
+    op->jprobs.push_back(jp);
+  }
+  MK_TRY(build_blocks(op, R, GR, op->Dr, false));
+  return build_blocks(op, L, GL, op->Dl, true);
+}
+
+}  // namespace
+
 extern "C" mk_status mk_prepare_ac2_jordan(mk_ctx h, const double* GL, const double* W1, const double* W2,
                                            const double* GR, int64_t Dl, int64_t wl, int64_t d1, int64_t wm,
                                            int64_t d2, int64_t wr, int64_t Dr, int precisions, mk_op* out) {
@@ -1197,6 +1589,10 @@ extern "C" mk_status mk_prepare_ac2_jordan(mk_ctx h, const double* GL, const dou
   for (int k = 1; k + 1 < wm; ++k) midM.push_back(k);
   if (wr > 1) for (int l = 1; l + 1 < wr; ++l) midR.push_back(l);
   const int kEnd = (int)wm - 1, lEnd = (int)wr - 1;
+  if (d1 == 2 && d2 == 2) {
+    OP_TRY(prepare_ac2_by_block(op, GL, A, B, GR, midL, midM, midR));
+    return finish(op, out);
+  }
 
   auto any_nz = [](const Wh& W, const std::vector<int>& gs, const std::vector<int>& ks) {
     for (int g : gs) for (int k : ks) if (W.block_nz(g, k)) return true;
@@ -1465,24 +1861,28 @@ extern "C" mk_status mk_prepare_ac_jordan(mk_ctx h, const double* GL, const doub
   double fl = 0.0;
   DevBuf wd;
   OP_TRY(upload(Wm.v.data(), Wm.v.size() * 8, wd, st));
-  // C'[(h,i),(b,c)] = sum_l W[0,b,h,l] GR~(i,l,c): row 0 (I, C and D)
-  OP_TRY(op->Cp.alloc('B', d * Dr, d * Dr));
-  OP_TRY(k_prep_Cp(GR, static_cast<double*>(wd.ptr), Dr, Dr, (int)wl, (int)d, (int)wr, lEnd, op->Cp.f64(), st));
   fl += 2.0 * Dl * (double)(d * Dr) * (d * Dr);
-  if (wl > 1) {
-    // B'[(a,b),(f,h)] = sum_{g>0} GL(a,g,f) W[g,b,h,end]: B and E
-    auto keep = mask_none((int)wl, (int)wr);
-    for (int g = 1; g < wl; ++g) keep[g][lEnd] = true;
-    Wh Wb = Wm.masked(keep);
-    DevBuf wbd, kd;
-    std::vector<int> kl = {lEnd};
-    OP_TRY(upload(Wb.v.data(), Wb.v.size() * 8, wbd, st));
-    OP_TRY(upload(kl.data(), sizeof(int), kd, st));
-    OP_TRY(op->Bp.alloc('A', Dl * d, Dl * d));
-    OP_TRY(k_prep_L(GL, static_cast<double*>(wbd.ptr), static_cast<int*>(kd.ptr), 1, Dl, Dl, (int)wl, (int)d,
-                    (int)wr, 0, op->Bp.f64(), st));
-    OP_TRY(hipStreamSynchronize(st) == hipSuccess ? MK_OK : MK_HIP_ERROR);
-    fl += 2.0 * (double)(Dl * d) * (Dl * d) * Dr;
+  if (wl > 1) fl += 2.0 * (double)(Dl * d) * (Dl * d) * Dr;
+  if (2 * d + 1 <= MAX_SEG && d <= MAX_PROB) {
+    OP_TRY(prepare_ac_by_block(op, GL, Wm, GR));
+  } else {
+    // C'[(h,i),(b,c)] = sum_l W[0,b,h,l] GR~(i,l,c): row 0 (I, C and D)
+    OP_TRY(op->Cp.alloc('B', d * Dr, d * Dr));
+    OP_TRY(k_prep_Cp(GR, static_cast<double*>(wd.ptr), Dr, Dr, (int)wl, (int)d, (int)wr, lEnd, op->Cp.f64(), st));
+    if (wl > 1) {
+      // B'[(a,b),(f,h)] = sum_{g>0} GL(a,g,f) W[g,b,h,end]: B and E
+      auto keep = mask_none((int)wl, (int)wr);
+      for (int g = 1; g < wl; ++g) keep[g][lEnd] = true;
+      Wh Wb = Wm.masked(keep);
+      DevBuf wbd, kd;
+      std::vector<int> kl = {lEnd};
+      OP_TRY(upload(Wb.v.data(), Wb.v.size() * 8, wbd, st));
+      OP_TRY(upload(kl.data(), sizeof(int), kd, st));
+      OP_TRY(op->Bp.alloc('A', Dl * d, Dl * d));
+      OP_TRY(k_prep_L(GL, static_cast<double*>(wbd.ptr), static_cast<int*>(kd.ptr), 1, Dl, Dl, (int)wl, (int)d,
+                      (int)wr, 0, op->Bp.f64(), st));
+      OP_TRY(hipStreamSynchronize(st) == hipSuccess ? MK_OK : MK_HIP_ERROR);
+    }
   }
   bool anyA = false;
   for (int g : midL) for (int l : midR) anyA = anyA || Wm.block_nz(g, l);

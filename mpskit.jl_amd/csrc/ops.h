@@ -177,6 +177,27 @@ struct Op {
   // Jordan one-site terms
   OpMat Cp, Bp;
 
+  // Jordan operators by output block (b, e) of the physical legs:
+  //   y_(b,e) = sum over segments of x_(h,j) RB_blk ('R') and LB_blk x_(h,j) ('L'),
+  // only the D x D blocks that are not zero, all in one launch (jordan_probs).
+  // Nearest-neighbour two-site operators take theirs out of IC ('I': h = b) and
+  // BE ('E': j = e); the others hold each different block once, right blocks
+  // side by side in RB (Dr x Dr nR), left blocks stacked in LB (Dl nL x Dl).
+  struct JSeg {
+    char kind;
+    int h, j, blk;
+  };
+  struct JProb {
+    int b, e;
+    std::vector<JSeg> seg;
+  };
+  std::vector<JProb> jprobs;
+  OpMat RB, LB;
+  int nR = 0, nL = 0;
+  bool by_block() const { return !jprobs.empty(); }
+  // a two-site operator with terms beyond nearest neighbours
+  bool long_range() const { return CA.present() || !AB.empty() || RB.present() || LB.present() || has_gen(); }
+
   // transfer matrices (OP_TL, OP_TR): the ket tensor TA and the bra tensor TB
   // as GEMM operands, the MPO tensor (none for an MPS transfer) and the sizes
   //   left:  x (Dm, wl, Dn) -> y (Da, wr, Dc), A (Dn, d, Dc), Abar (Dm, d, Da)
@@ -220,6 +241,20 @@ struct Op {
 // pitch pad8(N)) and slot 3 + sb (right-factor view, pitch pad8(M)).
 void block_probs(const Op* op, int prec, int64_t xoff, int64_t sa, int64_t sb, double beta,
                  std::vector<ProbSpec>& out);
+
+// GEMM problems of a by-block Jordan operator: x (float64 at `x`, or its views
+// xa, xb in the layout of k_nn_prologue, rows of length ka / kb, lo parts behind
+// by alo / blo bytes for bf16) into y, y = alpha ... + beta y.  Pointers may be
+// relative (rel_ptr).
+struct JordanViews {
+  const void* x = nullptr;
+  const void *xa = nullptr, *xb = nullptr;
+  int64_t ka = 0, kb = 0, alo = 0, blo = 0;
+};
+// K runs of a two-site operator's mixed copies and views: one per physical state for d = 2.
+int nn_runs(const Op* op);
+void jordan_probs(const Op* op, int prec, const JordanViews& v, const void* y, double alpha, double beta,
+                  std::vector<ProbSpec>& out);
 
 mk_status op_apply(Op* op, const double* x, double* y, double alpha, double beta, int prec);
 

@@ -17,11 +17,12 @@ struct Segs {
   const int* count = nullptr;      // chunks of every segment
 };
 
-// One conversion of a float64 column-major matrix into a K-contiguous mixed
-// operand (see k_split_bf16 / k_to_f32); pointers may be relative.
+// One conversion of a float64 column-major matrix into `width` elements (zero
+// past the matrix) of each row of a K-contiguous mixed operand (see k_convert);
+// pointers may be relative.
 struct SplitItem {
   const double* src;
-  int64_t rows, cols, ld, ldo;
+  int64_t rows, cols, ld, ldo, width;
   int32_t trans, nblocks;
   void* hi;
   void* lo;
@@ -67,7 +68,7 @@ mk_status seg_normalize(const Segs& sg, const double* x, const double* d, int ds
 
 mk_status split_group(const SplitItem* items, int n, int max_blocks, bool bf16, const void* const base[NBASE],
                       hipStream_t st);
-int split_blocks(int64_t rows, int64_t cols, int trans, int64_t ldo);
+int split_blocks(int64_t rows, int64_t cols, int trans, int64_t width);
 mk_status phys2_group(const PhysItem* items, int n, int max_blocks, int d12, const void* const base[NBASE],
                       hipStream_t st);
 int phys2_blocks(int64_t Dl, int64_t Dr);

@@ -159,13 +159,13 @@ __global__ void split_group_kernel(const SplitItem* __restrict__ items, BaseArgs
   void* hi = rslv(ba, d.hi);
   void* lo = BF ? rslv(ba, d.lo) : nullptr;
   if (d.trans) {
-    const int64_t n = d.ldo * d.cols;
+    const int64_t n = d.width * d.cols;
     const int64_t b0 = (int64_t)blockIdx.x * 1024;
     for (int t = threadIdx.x; t < 1024; t += TPB) {
       const int64_t idx = b0 + t;
       if (idx >= n) break;
-      const int64_t r = idx % d.ldo, c = idx / d.ldo;
-      put<BF>(d, hi, lo, idx, r < d.rows ? M[r + c * d.ld] : 0.0);
+      const int64_t r = idx % d.width, c = idx / d.width;
+      put<BF>(d, hi, lo, c * d.ldo + r, r < d.rows ? M[r + c * d.ld] : 0.0);
     }
   } else {
     __shared__ double tile[64][65];
@@ -179,7 +179,7 @@ __global__ void split_group_kernel(const SplitItem* __restrict__ items, BaseArgs
     __syncthreads();
     for (int rr = ty; rr < 64; rr += 4) {
       const int64_t r = r0 + rr, c = c0 + tx;
-      if (r < d.rows && c < d.ldo) put<BF>(d, hi, lo, r * d.ldo + c, tile[tx][rr]);
+      if (r < d.rows && c < d.width) put<BF>(d, hi, lo, r * d.ldo + c, tile[tx][rr]);
     }
   }
 }
@@ -313,9 +313,9 @@ mk_status split_group(const SplitItem* items, int n, int max_blocks, bool bf16, 
   return MK_OK;
 }
 
-int split_blocks(int64_t rows, int64_t cols, int trans, int64_t ldo) {
-  if (trans) return (int)cdiv(ldo * cols, (int64_t)1024);
-  return (int)(cdiv(rows, (int64_t)64) * cdiv(ldo, (int64_t)64));
+int split_blocks(int64_t rows, int64_t cols, int trans, int64_t width) {
+  if (trans) return (int)cdiv(width * cols, (int64_t)1024);
+  return (int)(cdiv(rows, (int64_t)64) * cdiv(width, (int64_t)64));
 }
 
 mk_status phys2_group(const PhysItem* items, int n, int max_blocks, int d12, const void* const base[NBASE],
