@@ -239,9 +239,13 @@ void gemm_f64_kernel(Src src) {
 // once per segment, and a chunk outside the operand (row past M / N, k past K)
 // gets an offset past num_records, for which the hardware returns zeros.  A K
 // step then issues its eight 16-byte loads with two VALU ops each and no
-// exec-mask branches.  Needs (checked on the host, buf_ok): 16-byte aligned
-// operands, even leading dimensions, even K, an even row count for operands
-// stored along their rows, and every in-tile offset below 2 GiB.
+// exec-mask branches.  Needs (checked on the host, buf_ok): every in-tile
+// offset below 2 GiB, and for ODD = false 16-byte aligned operands, even leading
+// dimensions, even K and an even row count for operands stored along their rows.
+// ODD = true takes any of them (a 16-byte load needs its address aligned to 4
+// only): the pair that would straddle the end of an odd row range or of an odd K
+// is read one element lower and shifted when it is stored, so no load leaves
+// the operand.  It needs two elements in each odd range.
 // ---------------------------------------------------------------------------
 constexpr unsigned OOB = 0x80000000u;
 typedef unsigned int ux4 __attribute__((ext_vector_type(4)));
@@ -250,7 +254,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, 0x7fffffff, 0x00020000);
 }
 
-template <int BM, int BN, bool TA, bool TB, class Src, bool ROT>
+template <int BM, int BN, bool TA, bool TB, class Src, bool ROT, bool ODD>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f64_buf_kernel(Src src) {
   constexpr int BK = 16;
@@ -310,6 +314,7 @@ void gemm_f64_buf_kernel(Src src) {
   unsigned cA = 0, cB = 0;         // bytes from chunk c to chunk c + 1
   unsigned stepA = 0, stepB = 0;   // bytes per unit of k0
   int K = 0;
+  bool shA = false, shB = false;   // the loaded pairs hold (element before the last, last)
   auto set_seg = [&](int s) {
     const GemmSeg& S = P.seg[s];
     const char* pa = static_cast<const char*>(resolve(src, S.A));
@@ -324,6 +329,16 @@ void gemm_f64_buf_kernel(Src src) {
     } else {
       cA = (unsigned)((NT / RA2) * S.lda * 8);
       oA = m0 + 2 * (tid % RA2) < M ? (unsigned)((2 * (tid % RA2) + (int64_t)(tid / RA2) * S.lda) * 8) : OOB;
+      // the tile's first row is no pair's second, so m0 = M - 1 steps below the base
+      if (ODD) {
+        shA = m0 + 2 * (tid % RA2) == M - 1;
+        if (m0 == M - 1) {
+          rA = raw_rsrc(pa + ((int64_t)m0 - 1) * 8);
+          oA = shA ? oA : OOB;
+        } else if (shA) {
+          oA -= 8;
+        }
+      }
     }
     if (BKD) {
       cB = (unsigned)((NT / 8) * S.ldb * 8);
@@ -331,18 +346,32 @@ void gemm_f64_buf_kernel(Src src) {
     } else {
       cB = (unsigned)((NT / RB2) * S.ldb * 8);
       oB = n0 + 2 * (tid % RB2) < N ? (unsigned)((2 * (tid % RB2) + (int64_t)(tid / RB2) * S.ldb) * 8) : OOB;
+      if (ODD) {
+        shB = n0 + 2 * (tid % RB2) == N - 1;
+        if (n0 == N - 1) {
+          rB = raw_rsrc(pb + ((int64_t)n0 - 1) * 8);
+          oB = shB ? oB : OOB;
+        } else if (shB) {
+          oB -= 8;
+        }
+      }
     }
     K = S.K;
   };
 
   dx2 ra[CHA], rb[CHB];
   auto load = [&](int k0) {
+    // the pair at the end of an odd K (for operands stored along k)
+    const bool last = ODD && k0 + 2 * (tid % 8) == K - 1;
+    if (ODD && AK) shA = last;
+    if (ODD && BKD) shB = last;
+    const unsigned back = last ? 8u : 0u;
 #pragma unroll
     for (int c = 0; c < CHA; ++c) {
       bool ok;
       if (AK) ok = (m0 + tid / 8 + c * (NT / 8) < M) & (k0 + 2 * (tid % 8) < K);
       else    ok = (oA != OOB) & (k0 + tid / RA2 + c * (NT / RA2) < K);
-      const unsigned o = ok ? oA + (unsigned)c * cA + (unsigned)k0 * stepA : OOB;
+      const unsigned o = ok ? oA + (unsigned)c * cA + (unsigned)k0 * stepA - (ODD && AK ? back : 0u) : OOB;
       ra[c] = __builtin_bit_cast(dx2, __builtin_amdgcn_raw_buffer_load_b128(rA, (int)o, 0, 0));
     }
 #pragma unroll
@@ -350,11 +379,17 @@ void gemm_f64_buf_kernel(Src src) {
       bool ok;
       if (BKD) ok = (n0 + tid / 8 + c * (NT / 8) < N) & (k0 + 2 * (tid % 8) < K);
       else     ok = (oB != OOB) & (k0 + tid / RB2 + c * (NT / RB2) < K);
-      const unsigned o = ok ? oB + (unsigned)c * cB + (unsigned)k0 * stepB : OOB;
+      const unsigned o = ok ? oB + (unsigned)c * cB + (unsigned)k0 * stepB - (ODD && BKD ? back : 0u) : OOB;
       rb[c] = __builtin_bit_cast(dx2, __builtin_amdgcn_raw_buffer_load_b128(rB, (int)o, 0, 0));
     }
   };
   auto store = [&](int buf) {
+    if constexpr (ODD) {
+#pragma unroll
+      for (int c = 0; c < CHA; ++c) ra[c] = shA ? dx2{ra[c].y, 0.0} : ra[c];
+#pragma unroll
+      for (int c = 0; c < CHB; ++c) rb[c] = shB ? dx2{rb[c].y, 0.0} : rb[c];
+    }
     if (!TA) store_fastdir<BM, LDA_S, BK>(As[buf], ra);
     else     store_kdir<BM, LDA_S, BK>(As[buf], ra);
     if (!TB) store_kdir<BN, LDB_S, BK>(Bs[buf], rb);
@@ -440,20 +475,26 @@ void gemm_f64_buf_kernel(Src src) {
 }
 
 // Host check of the branch-free kernel's conditions for one problem.
+enum BufFit { BUF_NO = 0, BUF_ODD = 1, BUF_EVEN = 2 };
 template <int BM, int BN>
-bool buf_ok_prob(const ProbSpec& ps, GemmShape sh) {
+BufFit buf_ok_prob(const ProbSpec& ps, GemmShape sh) {
+  BufFit fit = BUF_EVEN;
   for (int s = 0; s < ps.nseg; ++s) {
     const SegSpec& g = ps.seg[s];
     if (g.K <= 0) continue;
-    if ((uintptr_t)g.A % 16 || (uintptr_t)g.B % 16 || g.lda % 2 || g.ldb % 2 || g.K % 2) return false;
-    if (!sh.ta && ps.M % 2) return false;
-    if (sh.tb && ps.N % 2) return false;
     // largest in-tile byte offset (plus the 16-byte chunk) below 2^31
     const int64_t offA = sh.ta ? (g.K + (int64_t)(BM - 1) * g.lda) * 8 : (BM + (int64_t)(g.K - 1) * g.lda) * 8;
     const int64_t offB = !sh.tb ? (g.K + (int64_t)(BN - 1) * g.ldb) * 8 : (BN + (int64_t)(g.K - 1) * g.ldb) * 8;
-    if (offA + 16 >= (1ll << 31) || offB + 16 >= (1ll << 31)) return false;
+    if (offA + 16 >= (1ll << 31) || offB + 16 >= (1ll << 31)) return BUF_NO;
+    if ((uintptr_t)g.A % 16 || (uintptr_t)g.B % 16 || g.lda % 2 || g.ldb % 2 || g.K % 2 || (!sh.ta && ps.M % 2) ||
+        (sh.tb && ps.N % 2)) {
+      fit = BUF_ODD;
+      if ((uintptr_t)g.A % 8 || (uintptr_t)g.B % 8 || ((sh.ta || !sh.tb) && g.K < 2) || (!sh.ta && ps.M < 2) ||
+          (sh.tb && ps.N < 2))
+        return BUF_NO;
+    }
   }
-  return true;
+  return fit;
 }
 
 // Load path of the FP64 kernels, read once from MK_F64_VARIANT ("rot", "buf"
@@ -469,12 +510,12 @@ int f64_variant() {
   return v;
 }
 
-template <int BM, int BN, class Src, bool ROT>
+template <int BM, int BN, class Src, bool ROT, bool ODD>
 void launch4_buf(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
-  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, false, Src, ROT>), grid, block, 0, stream, b);
-  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, false, Src, ROT>), grid, block, 0, stream, b);
-  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, true, Src, ROT>), grid, block, 0, stream, b);
-  else hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, true, Src, ROT>), grid, block, 0, stream, b);
+  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, false, Src, ROT, ODD>), grid, block, 0, stream, b);
+  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, false, Src, ROT, ODD>), grid, block, 0, stream, b);
+  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, true, Src, ROT, ODD>), grid, block, 0, stream, b);
+  else hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, true, Src, ROT, ODD>), grid, block, 0, stream, b);
 }
 
 // K depth of a stage, read once from MK_F64_BK (16 or 32; default 16).  BK = 16
@@ -539,14 +580,16 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
   MK_REQUIRE(tail == 0 || (ws != nullptr && (size_t)tail * sp.ksplit * BM * BN * 8 <= GEMM_WS_BYTES), MK_BAD_ARG,
              "gemm_f64: %d tiles split %d ways exceed the workspace", tail, sp.ksplit);
   const int var = f64_variant();
-  bool buf = var != F64_BRANCH && f64_bk() == 16;
-  for (int i = 0; i < nprob && buf; ++i) buf = buf_ok_prob<BM, BN>(probs[i], sh);
+  int fit = var != F64_BRANCH && f64_bk() == 16 ? BUF_EVEN : BUF_NO;
+  for (int i = 0; i < nprob && fit != BUF_NO; ++i) fit = std::min<int>(fit, buf_ok_prob<BM, BN>(probs[i], sh));
+  const bool rot = var == F64_ROT && !sh.ta;
   dim3 grid(b.full_tiles + tail * b.ksplit), block(NT);
   ProfScope prof("gemm_f64", stream);
   // the rotated schedule holds two fragment sets; with a K-contiguous A the
   // extra registers would spill, so those launches keep the plain schedule
-  if (buf && var == F64_ROT && !sh.ta) launch4_buf<BM, BN, GemmBatch, true>(sh, grid, block, stream, b);
-  else if (buf) launch4_buf<BM, BN, GemmBatch, false>(sh, grid, block, stream, b);
+  if (fit == BUF_EVEN && rot) launch4_buf<BM, BN, GemmBatch, true, false>(sh, grid, block, stream, b);
+  else if (fit == BUF_EVEN) launch4_buf<BM, BN, GemmBatch, false, false>(sh, grid, block, stream, b);
+  else if (fit == BUF_ODD) launch4_buf<BM, BN, GemmBatch, false, true>(sh, grid, block, stream, b);
   else if (f64_bk() == 16) launch4<BM, BN, GemmBatch, 16>(sh, grid, block, stream, b);
   else launch4<BM, BN, GemmBatch, BK32>(sh, grid, block, stream, b);
   MK_CHECK_HIP(hipGetLastError());
@@ -565,9 +608,10 @@ mk_status launch_group(const GemmGroup& g, GemmShape sh, int grid, hipStream_t s
   dim3 gr(grid), block(NT);
   ProfScope prof("gemm_f64", stream);
   const int var = f64_variant();
-  const bool buf = g.f64_buf && var != F64_BRANCH && f64_bk() == 16;
-  if (buf && var == F64_ROT && !sh.ta) launch4_buf<BM, BN, GemmGroup, true>(sh, gr, block, stream, g);
-  else if (buf) launch4_buf<BM, BN, GemmGroup, false>(sh, gr, block, stream, g);
+  const int fit = var != F64_BRANCH && f64_bk() == 16 ? g.f64_buf : BUF_NO;
+  if (fit == BUF_EVEN && var == F64_ROT && !sh.ta) launch4_buf<BM, BN, GemmGroup, true, false>(sh, gr, block, stream, g);
+  else if (fit == BUF_EVEN) launch4_buf<BM, BN, GemmGroup, false, false>(sh, gr, block, stream, g);
+  else if (fit == BUF_ODD) launch4_buf<BM, BN, GemmGroup, false, true>(sh, gr, block, stream, g);
   else if (f64_bk() == 16) launch4<BM, BN, GemmGroup, 16>(sh, gr, block, stream, g);
   else launch4<BM, BN, GemmGroup, BK32>(sh, gr, block, stream, g);
   MK_CHECK_HIP(hipGetLastError());
@@ -596,10 +640,11 @@ int f64_group_grid(int kind, int total_tiles, int cus) {
   return (int)std::min<int64_t>(total_tiles, (int64_t)occ * cus);
 }
 
-bool f64_buf_ok(const ProbSpec* probs, int n, GemmShape sh, int kind) {
-  for (int i = 0; i < n; ++i)
-    if (!(kind == TK_128 ? buf_ok_prob<128, 128>(probs[i], sh) : buf_ok_prob<64, 64>(probs[i], sh))) return false;
-  return true;
+int f64_buf_ok(const ProbSpec* probs, int n, GemmShape sh, int kind) {
+  int fit = BUF_EVEN;
+  for (int i = 0; i < n && fit != BUF_NO; ++i)
+    fit = std::min<int>(fit, kind == TK_128 ? buf_ok_prob<128, 128>(probs[i], sh) : buf_ok_prob<64, 64>(probs[i], sh));
+  return fit;
 }
 
 mk_status gemm_f64_group(const GemmGroup& g, int kind, GemmShape sh, int grid, hipStream_t st) {
