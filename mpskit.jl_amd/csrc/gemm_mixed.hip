@@ -31,7 +31,15 @@ typedef unsigned int ux4 __attribute__((ext_vector_type(4)));
 
 constexpr int NT = 256;
 constexpr int ROWB = 64;          // bytes of K per LDS row per step
-constexpr int ROWP = ROWB + 16;   // padded LDS row (80 B: conflict-free 16-B reads)
+
+// Place of 16-byte chunk q of tile row r in an LDS slab of 64-byte rows.  A
+// 64-lane ds_read_b128 goes through the 256 B / cycle LDS in four groups of 16
+// lanes, {0-3, 12-15, 20-27} and its like, so a fragment read (row lane % 16,
+// chunk lane / 16) mixes rows of two chunks: with the chunks of rows 4 t .. 4 t + 3
+// XORed by -t (mod 4) the 16 lanes of every group hit distinct banks.  (XORed by
+// t, or in rows padded to 80 bytes, every read took two passes.)  The stores of
+// 16 consecutive lanes fill 256 contiguous bytes in any order.
+__device__ __forceinline__ int swz(int r, int q) { return r * ROWB + ((q ^ (-(r >> 2) & 3)) << 4); }
 
 enum Mode { M_BF16X3 = 0, M_F32 = 1 };
 
@@ -87,7 +95,7 @@ __device__ __forceinline__ void store_slab(char* S, const ux4 (&reg)[R * ROWB / 
     const int id = threadIdx.x + c * NT;
     const int r = id / (ROWB / 16);
     const int q = id % (ROWB / 16);
-    *reinterpret_cast<ux4*>(S + r * ROWP + q * 16) = reg[c];
+    *reinterpret_cast<ux4*>(S + swz(r, q)) = reg[c];
   }
 }
 
@@ -100,8 +108,8 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
   constexpr int CHA = BM * ROWB / 16 / NT;
   constexpr int CHB = BN * ROWB / 16 / NT;
 
-  __shared__ __attribute__((aligned(16))) char As[2][NPART][BM * ROWP];
-  __shared__ __attribute__((aligned(16))) char Bs[2][NPART][BN * ROWP];
+  __shared__ __attribute__((aligned(16))) char As[2][NPART][BM * ROWB];
+  __shared__ __attribute__((aligned(16))) char Bs[2][NPART][BN * ROWB];
 
   for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
   int t, slice, nslice;
@@ -167,10 +175,10 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
     for (int p = 0; p < NPART; ++p) {
 #pragma unroll
       for (int i = 0; i < FM; ++i)
-        fa[p][i] = *reinterpret_cast<const ux4*>(As[buf][p] + (wm0 + i * 16 + li) * ROWP + lg * 16);
+        fa[p][i] = *reinterpret_cast<const ux4*>(As[buf][p] + swz(wm0 + li, lg) + i * 16 * ROWB);
 #pragma unroll
       for (int j = 0; j < FN; ++j)
-        fb[p][j] = *reinterpret_cast<const ux4*>(Bs[buf][p] + (wn0 + j * 16 + li) * ROWP + lg * 16);
+        fb[p][j] = *reinterpret_cast<const ux4*>(Bs[buf][p] + swz(wn0 + li, lg) + j * 16 * ROWB);
     }
     if constexpr (MODE == M_BF16X3) {
 #pragma unroll
@@ -218,14 +226,11 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
 // Large-tile variant: 256 x 256 output tile, 512 threads = 8 waves (2 x 4), each
 // wave 128 x 64.  Halves the operand re-reads of the 128 x 128 kernel and
 // doubles the MFMA work per LDS fragment.  LDS rows hold 64 B of K without
-// padding; 16-B chunks are XOR-swizzled by (row >> 2) & 3 so that the 16 rows
-// read by one 16-lane group hit distinct banks.  Double-buffered: 128 KB (bf16).
+// padding, swizzled (swz).  Double-buffered: 128 KB (bf16).
 // ---------------------------------------------------------------------------
 
 constexpr int BIG = 256;
 constexpr int BNT = 512;
-
-__device__ __forceinline__ int swz(int r, int q) { return r * ROWB + ((q ^ ((r >> 2) & 3)) << 4); }
 
 template <int R>
 __device__ __forceinline__ void load_slab_big(const char* __restrict__ base, int64_t ld_bytes, int r0,
@@ -563,7 +568,7 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big2_kernel(Src src) {
 // covers less than one L2-miss latency at this MFMA rate.  Lane l of a wave's
 // 16-byte LDS load writes LDS bytes [16 l, 16 l + 16) after the wave base, so
 // the swizzle is applied on the global side: LDS chunk qp of row r receives
-// logical chunk qp ^ ((r >> 2) & 3).  Out-of-range rows and K chunks get a
+// logical chunk qp ^ (-(r >> 2) & 3).  Out-of-range rows and K chunks get a
 // buffer offset past num_records, which the hardware turns into zeros.
 // Three stages of hi + lo bf16 slabs: 3 x (32 + 16) KB = 144 KB of LDS.
 // ---------------------------------------------------------------------------
@@ -601,7 +606,7 @@ __device__ __forceinline__ void dma_slab(__amdgpu_buffer_rsrc_t rs, char* S, int
   for (int c = 0; c < CH; ++c) {
     const int idx = c * PNT + t;
     const int r = idx >> 2, qp = idx & 3;
-    const int q = qp ^ ((r >> 2) & 3);
+    const int q = qp ^ (-(r >> 2) & 3);
     const int gr = r0 + r, kb = kb0 + q * 16;
     const unsigned vo = (gr < Rlim && kb < Kbytes) ? (unsigned)(gr * ld_bytes + kb) : OOB;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(S + (c * PNT + wave * 64) * 16), 16, vo, 0, 0, 0);
