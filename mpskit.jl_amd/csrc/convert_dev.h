@@ -25,24 +25,25 @@ __device__ __forceinline__ void split2(double v, __hip_bfloat16& hi, __hip_bfloa
 // with conv the bf16 hi/lo split (SPLIT) or the fp32 rounding.  Each run of K
 // (one h, one j) is padded with zeros to a multiple of 8, so any Dl and Dr do,
 // and a GEMM segment may cover one run or several.  A 256-thread
-// block owns the (a, c) tile [a0, a0 + 32) x [c0, c0 + 64) and all (h, j)
+// block owns the (a, c) tile [a0, a0 + 32) x [c0, c0 + PC) and all (h, j)
 // sub-tiles of it, so x is read once: the thread holding x[a, :, c, :] produces
 // the P outputs of that pair, and the converted values pass through the LDS
-// array t (33 KB) for the transposed xa stores.  What follows the last run of a
+// array t (33 KB for PC = 64) for the transposed xa stores.  What follows the last run of a
 // row is not written (no K chunk the GEMMs read reaches into it).
 constexpr int PRO_A = 32, PRO_C = 64;
-typedef unsigned int ProTile[4][PRO_C][PRO_A + 1];
+template <int PC>
+using ProTile = unsigned int[4][PC][PRO_A + 1];
 
 // PACK: the two views are written in the packed panel layout of the 256 x 256
 // mixed kernel (packed_offset, with ka = N and kb = M their K lengths; Dl and Dr
 // are multiples of 128 then) instead of K-contiguous rows of length ka / kb.
-template <bool SPLIT, bool PACK = false, int D2 = 2>
+template <bool SPLIT, bool PACK = false, int D2 = 2, int PC = PRO_C>
 __device__ __forceinline__ void nn_prologue_tile(const double* __restrict__ P, const double* __restrict__ x,
                                                  int64_t Dl, int64_t Dr, double alpha, double beta,
                                                  double* __restrict__ y, void* __restrict__ xa_hi,
                                                  void* __restrict__ xa_lo, int64_t ka, void* __restrict__ xb_hi,
                                                  void* __restrict__ xb_lo, int64_t kb, int64_t a0, int64_t c0,
-                                                 ProTile& t) {
+                                                 ProTile<PC>& t) {
   // all arrays are in device memory: access them through global-typed pointers
   typedef __attribute__((address_space(1))) double gdouble;
   const gdouble* __restrict__ gx = (const gdouble*)x;
@@ -61,7 +62,7 @@ __device__ __forceinline__ void nn_prologue_tile(const double* __restrict__ P, c
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // a offset, c phase (8)
     const int64_t a = a0 + tx;
 #pragma unroll
-    for (int k = 0; k < PRO_C / 8; ++k) {
+    for (int k = 0; k < PC / 8; ++k) {
       const int cc = ty + 8 * k;
       const int64_t c = c0 + cc;
       if (a < runl && c < Dr) {
@@ -105,13 +106,14 @@ __device__ __forceinline__ void nn_prologue_tile(const double* __restrict__ P, c
   }
   __syncthreads();
   {
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;   // c offset, a phase (4)
+    constexpr int NA = 256 / PC;                              // a phases
+    const int tx = threadIdx.x % PC, ty = threadIdx.x / PC;   // c offset, a phase
     const int64_t c = c0 + tx;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
 #pragma unroll
-      for (int k = 0; k < PRO_A / 4; ++k) {
-        const int aa = ty + 4 * k;
+      for (int k = 0; k < PRO_A / NA; ++k) {
+        const int aa = ty + NA * k;
         const int64_t ar = a0 + aa;
         if (ar >= Dl || c >= runr) continue;
         const unsigned int v = c < Dr ? t[q][tx][aa] : 0u;

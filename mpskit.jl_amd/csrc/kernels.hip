@@ -178,40 +178,59 @@ __global__ void env_channels_last_kernel(const double* __restrict__ src, int64_t
   }
 }
 
-__global__ void tl_mid_kernel(const double* __restrict__ t1, const double* __restrict__ O,
-                              int64_t Dm, int wl, int d, int wr, int64_t Dc, double* __restrict__ t2) {
-  const int64_t n = Dm * d * wr * Dc;
-  GRID_STRIDE(idx, n) {
-    int64_t t = idx;
-    const int64_t m = t % Dm; t /= Dm;
-    const int k = (int)(t % d); t /= d;
-    const int b = (int)(t % wr); t /= wr;
-    const int64_t c = t;
-    double s = 0.0;
-    for (int h = 0; h < d; ++h)
-      for (int g = 0; g < wl; ++g) {
-        const double ov = O[g + wl * (k + d * (h + d * b))];
-        if (ov != 0.0) s += t1[m + Dm * (g + (int64_t)wl * (h + d * c))] * ov;
+// The MPO step of the float64 transfers.  One thread per environment row and
+// column (m, c) holds the NIN >= d wl inputs that meet the MPO tensor there in
+// registers, so t1 is read and t2 written once (memory-bound: a thread per
+// output, which re-read its inputs through the caches and divided the index
+// four times, ran at 2.1 TB/s of such traffic at D = 1024, w = 5).
+//   left:  t2[m,k,b,c] = sum_{g,h} t1[m,g,h,c] O[g,k,h,b]
+//   right: t2[a,b,k,o] = sum_{h,l} t1[a,h,l,o] O[b,k,h,l]
+template <int NIN, bool RIGHT>
+__global__ __launch_bounds__(256) void mpo_mid_kernel(const double* __restrict__ t1, const double* __restrict__ O,
+                                                      int64_t D1, int wl, int d, int wr, int64_t D2,
+                                                      double* __restrict__ t2) {
+  typedef __attribute__((address_space(1))) double gd;
+  const int nin = RIGHT ? d * wr : wl * d, nout = RIGHT ? wl * d : d * wr;
+  GRID_STRIDE(idx, D1 * D2) {
+    const int64_t c = idx / D1, m = idx - c * D1;
+    const gd* in = (const gd*)t1 + m + D1 * (int64_t)nin * c;
+    gd* out = (gd*)t2 + m + D1 * (int64_t)nout * c;
+    double v[NIN];
+#pragma unroll
+    for (int i = 0; i < NIN; ++i) v[i] = i < nin ? in[D1 * i] : 0.0;
+    for (int q = 0; q < nout; ++q) {
+      // output q: left (k, b) = (q % d, q / d), right (b, k) = (q % wl, q / wl)
+      const double* w = RIGHT ? O + q % wl + wl * (q / wl) : O + wl * (q % d + d * d * (int64_t)(q / d));
+      double s = 0.0;
+#pragma unroll
+      for (int i = 0; i < NIN; ++i) {
+        if (i < nin) {
+          // input i: left (g, h), O step wl d per h; right (h, l), O step wl d per h, wl d d per l
+          const double ov = RIGHT ? w[(int64_t)wl * d * i] : w[i % wl + (int64_t)wl * d * (i / wl)];
+          if (ov != 0.0) s += v[i] * ov;
+        }
       }
-    t2[idx] = s;
+      out[D1 * q] = s;
+    }
   }
 }
 
-__global__ void tr_mid_kernel(const double* __restrict__ t1, const double* __restrict__ O,
-                              int64_t Da, int wl, int d, int wr, int64_t Do, double* __restrict__ t2) {
-  const int64_t n = Da * wl * d * Do;
-  GRID_STRIDE(idx, n) {
+// The same with any number of inputs (a thread per output).
+template <bool RIGHT>
+__global__ void mpo_mid_wide_kernel(const double* __restrict__ t1, const double* __restrict__ O, int64_t D1, int wl,
+                                    int d, int wr, int64_t D2, double* __restrict__ t2) {
+  const int nin = RIGHT ? d * wr : wl * d, nout = RIGHT ? wl * d : d * wr;
+  GRID_STRIDE(idx, D1 * nout * D2) {
     int64_t t = idx;
-    const int64_t a = t % Da; t /= Da;
-    const int b = (int)(t % wl); t /= wl;
-    const int k = (int)(t % d); t /= d;
-    const int64_t o = t;
+    const int64_t m = t % D1; t /= D1;
+    const int q = (int)(t % nout);
+    const int64_t c = t / nout;
+    const double* w = RIGHT ? O + q % wl + wl * (q / wl) : O + wl * (q % d + d * d * (int64_t)(q / d));
     double s = 0.0;
-    for (int l = 0; l < wr; ++l)
-      for (int h = 0; h < d; ++h) {
-        const double ov = O[b + wl * (k + d * (h + d * l))];
-        if (ov != 0.0) s += t1[a + Da * (h + d * (l + (int64_t)wr * o))] * ov;
-      }
+    for (int i = 0; i < nin; ++i) {
+      const double ov = RIGHT ? w[(int64_t)wl * d * i] : w[i % wl + (int64_t)wl * d * (i / wl)];
+      if (ov != 0.0) s += t1[m + D1 * (i + (int64_t)nin * c)] * ov;
+    }
     t2[idx] = s;
   }
 }
@@ -731,16 +750,16 @@ __global__ __launch_bounds__(256) void gen_mid_kernel(const double* t1, const do
   }
 }
 
-template <bool SPLIT, bool PACK, int D2>
+template <bool SPLIT, bool PACK, int D2, int PC>
 __global__ __launch_bounds__(256) void nn_prologue_kernel(const double* __restrict__ P,
                                                           const double* __restrict__ x, int64_t Dl, int64_t Dr,
                                                           double alpha, double beta, double* __restrict__ y,
                                                           void* __restrict__ xa_hi, void* __restrict__ xa_lo,
                                                           int64_t ka, void* __restrict__ xb_hi,
                                                           void* __restrict__ xb_lo, int64_t kb) {
-  __shared__ ProTile t;
-  nn_prologue_tile<SPLIT, PACK, D2>(P, x, Dl, Dr, alpha, beta, y, xa_hi, xa_lo, ka, xb_hi, xb_lo, kb,
-                                    (int64_t)blockIdx.x * PRO_A, (int64_t)blockIdx.y * PRO_C, t);
+  __shared__ ProTile<PC> t;
+  nn_prologue_tile<SPLIT, PACK, D2, PC>(P, x, Dl, Dr, alpha, beta, y, xa_hi, xa_lo, ka, xb_hi, xb_lo, kb,
+                                        (int64_t)blockIdx.x * PRO_A, (int64_t)blockIdx.y * PC, t);
 }
 
 // D x D operator blocks as combinations of environment levels:
@@ -920,13 +939,32 @@ mk_status k_env_channels_last(const double* src, int64_t Da, int w, int64_t Df, 
                               hipStream_t st) {
   LAUNCH_1D(env_channels_last_kernel, Da * Df * nk, st, src, Da, w, Df, klist, nk, dst);
 }
-mk_status k_tl_mid(const double* t1, const double* O, int64_t Dm, int wl, int d, int wr, int64_t Dc,
-                   double* t2, hipStream_t st) {
-  LAUNCH_1D(tl_mid_kernel, Dm * d * wr * Dc, st, t1, O, Dm, wl, d, wr, Dc, t2);
+template <bool RIGHT>
+static mk_status launch_mpo_mid(const double* t1, const double* O, int64_t D1, int wl, int d, int wr, int64_t D2,
+                                double* t2, hipStream_t st) {
+  const int nin = RIGHT ? d * wr : wl * d, nout = RIGHT ? wl * d : d * wr;
+  if (D1 * D2 * nout == 0) return MK_OK;
+  const dim3 g = grid1d(D1 * D2, 1);
+#define MPO_MID(N) hipLaunchKernelGGL((mpo_mid_kernel<N, RIGHT>), g, dim3(256), 0, st, t1, O, D1, wl, d, wr, D2, t2)
+  if (nin <= 4) MPO_MID(4);
+  else if (nin <= 6) MPO_MID(6);
+  else if (nin <= 10) MPO_MID(10);
+  else if (nin <= 16) MPO_MID(16);
+  else if (nin <= 32) MPO_MID(32);
+  else
+    hipLaunchKernelGGL((mpo_mid_wide_kernel<RIGHT>), grid1d(D1 * nout * D2, 4), dim3(TPB), 0, st, t1, O, D1, wl, d, wr,
+                       D2, t2);
+#undef MPO_MID
+  MK_CHECK_HIP(hipGetLastError());
+  return MK_OK;
 }
-mk_status k_tr_mid(const double* t1, const double* O, int64_t Da, int wl, int d, int wr, int64_t Do,
-                   double* t2, hipStream_t st) {
-  LAUNCH_1D(tr_mid_kernel, Da * wl * d * Do, st, t1, O, Da, wl, d, wr, Do, t2);
+mk_status k_tl_mid(const double* t1, const double* O, int64_t Dm, int wl, int d, int wr, int64_t Dc, double* t2,
+                   hipStream_t st) {
+  return launch_mpo_mid<false>(t1, O, Dm, wl, d, wr, Dc, t2, st);
+}
+mk_status k_tr_mid(const double* t1, const double* O, int64_t Da, int wl, int d, int wr, int64_t Do, double* t2,
+                   hipStream_t st) {
+  return launch_mpo_mid<true>(t1, O, Da, wl, d, wr, Do, t2, st);
 }
 mk_status k_swap_mid(const double* in, int64_t n0, int64_t n1, int64_t n2, int64_t n3, double* out,
                      hipStream_t st) {
@@ -1122,19 +1160,31 @@ mk_status k_nn_prologue(const double* P, const double* x, int64_t Dl, int64_t Dr
                         double* y, int split, void* xa_hi, void* xa_lo, int64_t ka, void* xb_hi, void* xb_lo,
                         int64_t kb, int packed, hipStream_t st) {
   if (Dl * Dr == 0) return MK_OK;
-  dim3 g((unsigned)cdiv(Dl, (int64_t)PRO_A), (unsigned)cdiv(Dr, (int64_t)PRO_C));
   MK_REQUIRE(d2 == 1 || d2 == 2, MK_BAD_ARG, "nn_prologue: d2 = %d", d2);
   if (packed)
     MK_REQUIRE(split && d2 == 2 && (2 * Dl) % 256 == 0 && (2 * Dr) % 256 == 0 && ka == 2 * Dr && kb == 2 * Dl,
                MK_BAD_ARG, "nn_prologue: packed views are bf16, with 2 Dl, 2 Dr multiples of 256 and unpadded rows");
-#define NN_PROLOGUE(S, K, N) \
-  hipLaunchKernelGGL((nn_prologue_kernel<S, K, N>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi, \
+  // 64 columns a block (128-byte runs of the bf16 left view) while that makes two
+  // blocks a CU, fewer below: at D = 512 the 128 blocks of 64 columns took 14.5 us
+  // and the 512 of 16 columns 7.6
+  const int64_t rows = cdiv(Dl, (int64_t)PRO_A);
+  const int pc = packed || rows * cdiv(Dr, (int64_t)64) >= 512 ? 64 : rows * cdiv(Dr, (int64_t)32) >= 512 ? 32 : 16;
+  const dim3 g((unsigned)rows, (unsigned)cdiv(Dr, (int64_t)pc));
+#define NN_PROLOGUE(S, K, N, C) \
+  hipLaunchKernelGGL((nn_prologue_kernel<S, K, N, C>), g, dim3(256), 0, st, P, x, Dl, Dr, alpha, beta, y, xa_hi, \
                      S ? xa_lo : nullptr, ka, xb_hi, S ? xb_lo : nullptr, kb)
-  if (packed) NN_PROLOGUE(true, true, 2);
-  else if (split && d2 == 2) NN_PROLOGUE(true, false, 2);
-  else if (split) NN_PROLOGUE(true, false, 1);
-  else if (d2 == 2) NN_PROLOGUE(false, false, 2);
-  else NN_PROLOGUE(false, false, 1);
+#define NN_PROLOGUE_C(S, N) \
+  do { \
+    if (pc == 64) NN_PROLOGUE(S, false, N, 64); \
+    else if (pc == 32) NN_PROLOGUE(S, false, N, 32); \
+    else NN_PROLOGUE(S, false, N, 16); \
+  } while (0)
+  if (packed) NN_PROLOGUE(true, true, 2, 64);
+  else if (split && d2 == 2) NN_PROLOGUE_C(true, 2);
+  else if (split) NN_PROLOGUE_C(true, 1);
+  else if (d2 == 2) NN_PROLOGUE_C(false, 2);
+  else NN_PROLOGUE_C(false, 1);
+#undef NN_PROLOGUE_C
 #undef NN_PROLOGUE
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;

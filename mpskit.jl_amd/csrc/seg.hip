@@ -244,7 +244,7 @@ __global__ void cphys_group_kernel(const CPhysItem* __restrict__ items, double a
 
 template <bool BF>
 __global__ __launch_bounds__(256) void nn_group_kernel(const NNItem* __restrict__ items, BaseArgs ba) {
-  __shared__ ProTile t;
+  __shared__ ProTile<PRO_C> t;
   const NNItem d = items[blockIdx.y];
   if ((int)blockIdx.x >= d.tiles) return;
   const int64_t a0 = (int64_t)(blockIdx.x % d.tiles_a) * PRO_A, c0 = (int64_t)(blockIdx.x / d.tiles_a) * PRO_C;

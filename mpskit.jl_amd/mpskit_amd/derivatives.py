@@ -24,6 +24,7 @@ MFMA with FP32 accumulation); inputs and outputs are float64 in every mode.
 from __future__ import annotations
 
 import ctypes as C
+import math
 import sys
 from typing import Iterable
 
@@ -153,6 +154,10 @@ class BatchedDerivative:
         self.offsets = [int(o) for o in offs]
         self.total = int(tot.value)
         self.grouped = bool(grp.value)
+        # positions between the segments, which the library does not write
+        ends = [o + math.prod(op.x_shape) for op, o in zip(self.ops, self.offsets)]
+        self._gaps = torch.cat([torch.arange(e, s) for e, s in zip(ends, self.offsets[1:] + [self.total])]
+                               ).to(torch.device("cuda", self.ctx.device))
 
     def pack(self, xs) -> torch.Tensor:
         flat = torch.zeros(self.total, dtype=torch.float64, device=xs[0].device)
@@ -176,7 +181,9 @@ class BatchedDerivative:
         """y = H x for every instance of a packed vector."""
         if flat.numel() != self.total or flat.dtype != torch.float64 or not flat.is_contiguous():
             raise SpaceMismatch(1, "BatchedDerivative.apply: wrong packed vector")
-        y = torch.zeros_like(flat)
+        y = torch.empty_like(flat)
+        if self._gaps.numel():
+            y.index_fill_(0, self._gaps, 0.0)
         self.ctx.sync_stream()
         check(load().mk_batch_apply(self.handle, T.ptr(flat), T.ptr(y), _prec(precision)))
         return y
