@@ -65,6 +65,22 @@ mk_status Ctx::small(size_t nbytes, void** out) {
 }
 
 
+mk_status Ctx::readback_init() {
+  if (readback) return MK_OK;
+  for (hipEvent_t& e : readback_ev)
+    if (!e) MK_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  void* p = nullptr;
+  MK_CHECK_HIP(hipHostMalloc(&p, READBACK_SLOTS * READBACK_LEN * sizeof(double), hipHostMallocDefault));
+  readback = static_cast<double*>(p);
+  return MK_OK;
+}
+
+Ctx::~Ctx() {
+  if (readback) (void)hipHostFree(readback);
+  for (hipEvent_t e : readback_ev)
+    if (e) (void)hipEventDestroy(e);
+}
+
 void* Ctx::gemm_ws() {
   const FixedScratch& fx = fixed_scratch();
   if (fx.base) return fx.gemm_ws;

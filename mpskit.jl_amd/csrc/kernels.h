@@ -85,9 +85,9 @@ mk_status k_multidot(const double* V, int64_t ldv, int k, const double* w, int64
 // Fused classical Gram-Schmidt passes over the k <= 32 columns of V (ldv):
 // u <- u - V cin, then out[0..k) = V^T u (update_dot) or out[0] = u^T u,
 // out[1] = w^T u (update_norm), all in one read of V.  partial holds
-// cgs_blocks(n) * k doubles.
+// cgs_blocks(n) * k doubles.  update_dot takes the entries of cin below lo as zero.
 int cgs_blocks(int64_t n);
-mk_status k_cgs_update_dot(const double* V, int64_t ldv, int k, const double* cin, double* u, int64_t n,
+mk_status k_cgs_update_dot(const double* V, int64_t ldv, int k, const double* cin, int lo, double* u, int64_t n,
                            double* out, double* partial, hipStream_t st);
 mk_status k_cgs_update_norm(const double* V, int64_t ldv, int k, const double* cin, double* u, const double* w,
                             int64_t n, double* out, double* partial, hipStream_t st);
@@ -96,6 +96,8 @@ mk_status k_multiaxpy(const double* V, int64_t ldv, int k, const double* c, doub
                       int64_t n, hipStream_t st);
 // y = a*x + b*y with a, b host scalars
 mk_status k_axpby(double a, const double* x, double b, double* y, int64_t n, hipStream_t st);
+// y = x / sqrt(*s2) (s2 on the device)
+mk_status k_normalize(const double* x, const double* s2, double* y, int64_t n, hipStream_t st);
 // y *= s where s = *sdev (device scalar) or 1/s if inv
 mk_status k_scale_dev(double* y, const double* sdev, int inv, int64_t n, hipStream_t st);
 // x = V s  (s on device, length k)

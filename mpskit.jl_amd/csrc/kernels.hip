@@ -532,14 +532,14 @@ __global__ void reduce_rows_kernel(const double* __restrict__ partial, int nb, d
 constexpr int CGS_KMAX = 32;
 template <int MODE, int KT, typename VT>
 __global__ __launch_bounds__(TPB) void cgs_update_kernel(const VT* __restrict__ V, int64_t ldv, int k,
-                                                         const double* __restrict__ cin, double* __restrict__ u,
+                                                         const double* __restrict__ cin, int lo, double* __restrict__ u,
                                                          const double* __restrict__ w, int64_t n,
                                                          double* __restrict__ partial) {
   __shared__ double sh[TPB / 64];
   constexpr int NO = MODE == 1 ? 2 : KT;
   double c[KT], acc[NO];
 #pragma unroll
-  for (int j = 0; j < KT; ++j) c[j] = (MODE != 2 && j < k) ? cin[j] : 0.0;
+  for (int j = 0; j < KT; ++j) c[j] = (MODE != 2 && j >= lo && j < k) ? cin[j] : 0.0;
 #pragma unroll
   for (int o = 0; o < NO; ++o) acc[o] = 0.0;
   GRID_STRIDE(r, n) {
@@ -594,6 +594,13 @@ __global__ void axpby_kernel(double a, const double* x, double b, double* y,
     if (b != 0.0) v += b * y[i];
     y[i] = v;
   }
+}
+
+// y = x / sqrt(*s2)
+__global__ void normalize_kernel(const double* __restrict__ x, const double* __restrict__ s2, double* __restrict__ y,
+                                 int64_t n) {
+  const double s = 1.0 / sqrt(*s2);
+  GRID_STRIDE(i, n) y[i] = s * x[i];
 }
 
 __global__ void scale_dev_kernel(double* __restrict__ y, const double* __restrict__ sdev, int inv,
@@ -1024,19 +1031,19 @@ int multidot_blocks(int64_t n) { return (int)std::max<int64_t>(1, cdiv(n, (int64
 int cgs_blocks(int64_t n);
 
 template <int MODE, typename VT>
-void launch_cgs(int k, int nb, hipStream_t st, const VT* V, int64_t ldv, const double* cin, double* u,
+void launch_cgs(int k, int nb, hipStream_t st, const VT* V, int64_t ldv, const double* cin, int lo, double* u,
                 const double* w, int64_t n, double* partial) {
   if (k <= 4)
-    hipLaunchKernelGGL((cgs_update_kernel<MODE, 4, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, u, w, n,
+    hipLaunchKernelGGL((cgs_update_kernel<MODE, 4, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, lo, u, w, n,
                        partial);
   else if (k <= 8)
-    hipLaunchKernelGGL((cgs_update_kernel<MODE, 8, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, u, w, n,
+    hipLaunchKernelGGL((cgs_update_kernel<MODE, 8, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, lo, u, w, n,
                        partial);
   else if (k <= 16)
-    hipLaunchKernelGGL((cgs_update_kernel<MODE, 16, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, u, w, n,
+    hipLaunchKernelGGL((cgs_update_kernel<MODE, 16, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, lo, u, w, n,
                        partial);
   else
-    hipLaunchKernelGGL((cgs_update_kernel<MODE, 32, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, u, w, n,
+    hipLaunchKernelGGL((cgs_update_kernel<MODE, 32, VT>), dim3(nb), dim3(TPB), 0, st, V, ldv, k, cin, lo, u, w, n,
                        partial);
 }
 
@@ -1047,7 +1054,7 @@ mk_status k_multidot(const double* V, int64_t ldv, int k, const double* w, int64
     // one read of V with register accumulators; at most multidot_blocks(n)
     // blocks, so callers' partial buffers sized for the wide kernel suffice
     const int nb = std::min(cgs_blocks(n), multidot_blocks(n));
-    launch_cgs<2, double>(k, nb, st, V, ldv, nullptr, const_cast<double*>(w), nullptr, n, partial);
+    launch_cgs<2, double>(k, nb, st, V, ldv, nullptr, 0, const_cast<double*>(w), nullptr, n, partial);
     MK_CHECK_HIP(hipGetLastError());
     hipLaunchKernelGGL(reduce_rows_kernel, dim3(k), dim3(TPB), 0, st, partial, nb, out);
     MK_CHECK_HIP(hipGetLastError());
@@ -1062,11 +1069,11 @@ mk_status k_multidot(const double* V, int64_t ldv, int k, const double* w, int64
 }
 int cgs_blocks(int64_t n) { return (int)std::min<int64_t>(1024, std::max<int64_t>(1, cdiv(n, (int64_t)TPB * 4))); }
 
-mk_status k_cgs_update_dot(const double* V, int64_t ldv, int k, const double* cin, double* u, int64_t n,
+mk_status k_cgs_update_dot(const double* V, int64_t ldv, int k, const double* cin, int lo, double* u, int64_t n,
                            double* out, double* partial, hipStream_t st) {
   MK_REQUIRE(k >= 1 && k <= CGS_KMAX, MK_BAD_ARG, "cgs_update_dot: k = %d not in [1, %d]", k, CGS_KMAX);
   const int nb = cgs_blocks(n);
-  launch_cgs<0, double>(k, nb, st, V, ldv, cin, u, nullptr, n, partial);
+  launch_cgs<0, double>(k, nb, st, V, ldv, cin, lo, u, nullptr, n, partial);
   MK_CHECK_HIP(hipGetLastError());
   hipLaunchKernelGGL(reduce_rows_kernel, dim3(k), dim3(TPB), 0, st, partial, nb, out);
   MK_CHECK_HIP(hipGetLastError());
@@ -1077,7 +1084,7 @@ mk_status k_cgs_update_norm(const double* V, int64_t ldv, int k, const double* c
                             int64_t n, double* out, double* partial, hipStream_t st) {
   MK_REQUIRE(k >= 1 && k <= CGS_KMAX, MK_BAD_ARG, "cgs_update_norm: k = %d not in [1, %d]", k, CGS_KMAX);
   const int nb = cgs_blocks(n);
-  launch_cgs<1, double>(k, nb, st, V, ldv, cin, u, w, n, partial);
+  launch_cgs<1, double>(k, nb, st, V, ldv, cin, 0, u, w, n, partial);
   MK_CHECK_HIP(hipGetLastError());
   hipLaunchKernelGGL(reduce_rows_kernel, dim3(2), dim3(TPB), 0, st, partial, nb, out);
   MK_CHECK_HIP(hipGetLastError());
@@ -1096,6 +1103,9 @@ mk_status k_gemv(const double* V, int64_t ldv, int k, const double* s, double* x
 
 mk_status k_axpby(double a, const double* x, double b, double* y, int64_t n, hipStream_t st) {
   LAUNCH_1D(axpby_kernel, n, st, a, x, b, y, n);
+}
+mk_status k_normalize(const double* x, const double* s2, double* y, int64_t n, hipStream_t st) {
+  LAUNCH_1D(normalize_kernel, n, st, x, s2, y, n);
 }
 mk_status k_scale_dev(double* y, const double* sdev, int inv, int64_t n, hipStream_t st) {
   LAUNCH_1D(scale_dev_kernel, n, st, y, sdev, inv, n);

@@ -153,7 +153,7 @@ extern "C" mk_status mk_krylov_orthogonalize(mk_ctx h, const double* V, int64_t 
   double* cd = static_cast<double*>(mem);
   double* part = cd + 3 * 32 + 2;
   MK_TRY(k_multidot(V, ldv, k, u, n, cd, part, st));
-  MK_TRY(k_cgs_update_dot(V, ldv, k, cd, u, n, cd + 32, part, st));
+  MK_TRY(k_cgs_update_dot(V, ldv, k, cd, 0, u, n, cd + 32, part, st));
   MK_TRY(k_cgs_update_norm(V, ldv, k, cd + 32, u, u, n, cd + 64, part, st));
   std::vector<double> hv(66);
   MK_CHECK_HIP(hipMemcpyAsync(hv.data(), cd, hv.size() * 8, hipMemcpyDeviceToHost, st));
@@ -182,23 +182,34 @@ extern "C" mk_status mk_eigsolve(mk_op h, double* x, int krylovdim, int maxiter,
   // (krylovdim / 4) and runs longer cycles.
   const int pmax = std::max(1, precision == MK_FP64 ? krylovdim / 2 : krylovdim / 4);
 
-  // basis Q = [x, y_2..y_p, v_0, ...] (column-major n x K), then pmax columns for
-  // the new Ritz vectors; w = H x, u = work
-  DevBuf Qb, wb, ub, cb, pb, sb;
-  MK_TRY(Qb.alloc((size_t)n * (K + pmax) * 8));
-  MK_TRY(wb.alloc((size_t)n * 8));
-  MK_TRY(ub.alloc((size_t)n * 8));
-  // coefficients: generic dots at [0, K + 4); fused passes at [FC, FC + 2 * 32 + 2)
-  constexpr int FC = 1024;
-  MK_TRY(cb.alloc((size_t)(FC + 2 * 32 + 2) * 8));
-  MK_TRY(sb.alloc((size_t)K * pmax * 8));
+  // One workspace, kept by the context while it is small: the basis
+  // Q = [x, y_2..y_p, v_0, ...] (column-major n x K) and after it pmax columns for
+  // the new Ritz vectors; w = H x, u = work; the coefficients (generic dots at
+  // [0, K + 4), the fused passes of step j at FC + FL (j mod 2)); the
+  // coefficients of the Ritz vectors; the partial sums of the reductions.
+  constexpr int FC = 1024, FL = Ctx::READBACK_LEN;
+  static_assert(FL >= 3 * 32 + 2, "a step's coefficients");
   const int64_t nb = std::max<int64_t>(1, cdiv(n, 256 * 16));
-  MK_TRY(pb.alloc((size_t)std::max<int64_t>(nb * (K + 4), (int64_t)cgs_blocks(n) * 34) * 8));
-  double* Q = static_cast<double*>(Qb.ptr);
-  double* w = static_cast<double*>(wb.ptr);
-  double* u = static_cast<double*>(ub.ptr);
+  const size_t nq = (size_t)n * (K + pmax), ncoef = FC + 2 * FL, ns = (size_t)K * pmax;
+  const size_t npart = (size_t)std::max<int64_t>(nb * (K + 4), (int64_t)cgs_blocks(n) * 34);
+  const size_t bytes = (nq + 2 * (size_t)n + ncoef + ns + npart) * 8;
+  if (ctx->krylovbuf.bytes < bytes) MK_TRY(ctx->krylovbuf.alloc(bytes));
+  struct Done {
+    Ctx* c;
+    ~Done() {
+      (void)hipStreamSynchronize(c->stream);   // also after an error, or with a step too many in flight
+      if (c->krylovbuf.bytes > Ctx::KRYLOV_KEEP) c->krylovbuf.release();
+    }
+  } done{ctx};
+  MK_TRY(ctx->readback_init());
+  double* Q = static_cast<double*>(ctx->krylovbuf.ptr);
+  double* w = Q + nq;
+  double* u = w + n;
+  double* coefs = u + n;
+  double* sb = coefs + ncoef;
+  double* part = sb + ns;
   auto col = [&](int j) { return Q + (int64_t)j * n; };
-  Dev dv{ctx, static_cast<double*>(cb.ptr), static_cast<double*>(pb.ptr)};
+  Dev dv{ctx, coefs, part};
 
   int ops = 0;
   MK_CHECK_HIP(hipMemcpyAsync(col(0), x, (size_t)n * 8, hipMemcpyDeviceToDevice, st));
@@ -270,41 +281,64 @@ extern "C" mk_status mk_eigsolve(mk_op h, double* x, int krylovdim, int maxiter,
     int k = 1;                                 // Krylov vectors v_0..v_{k-1} in the cycle
     const double thresh = std::max(tol, inner_eta(precision) * res);
     const int mmax = K - p;                    // room for Krylov vectors
+    // Device work of Krylov step j (basis columns 0 .. p + j <= 32): u = H_p v_j,
+    // two classical Gram-Schmidt passes against [x, y.., v_0..v_j], fused
+    // (c1 = Q^T u; u -= Q c1 with c2 = Q^T u in the same read of Q; u -= Q c2 with
+    // |u|^2 and <w, u>), v_{j+1} = u / |u|, and the readback of the coefficients
+    auto enqueue = [&](int j) -> mk_status {
+      const int cj = p + j, kq = cj + 1, slot = j & 1;
+      double* cd = coefs + FC + FL * slot;
+      MK_TRY(op_apply(op, col(cj), u, 1.0, 0.0, precision));
+      // first pass on the last three columns only.  For j >= 1, H v_j lies
+      // in span{v_{j-1}, v_j, v_{j+1}} in exact arithmetic (x and the kept
+      // Ritz vectors couple to v_0 alone), so the three-term recurrence
+      // removes the large components; the full pass below removes what is
+      // left, which is small, so the pair is as orthogonal as two full
+      // passes (twice is enough) for one read of the columns instead of two
+      const int lo = j >= 1 && local_first_pass() ? std::max(0, cj - 2) : 0;
+      MK_TRY(k_multidot(col(lo), n, kq - lo, u, n, cd + lo, dv.partial, st));
+      MK_TRY(k_cgs_update_dot(Q, n, kq, cd, lo, u, n, cd + 32, dv.partial, st));
+      MK_TRY(k_cgs_update_norm(Q, n, kq, cd + 32, u, w, n, cd + 64, dv.partial, st));
+      if (j + 1 < mmax) MK_TRY(k_normalize(u, cd + 64, col(cj + 1), n, st));
+      MK_CHECK_HIP(hipMemcpyAsync(ctx->readback + FL * slot, cd, (size_t)66 * 8, hipMemcpyDeviceToHost, st));
+      MK_CHECK_HIP(hipEventRecord(ctx->readback_ev[slot], st));
+      return MK_OK;
+    };
+    // While the host reads step j back and solves the projected problem, the
+    // device would wait (75 us a step against 130 us of work at D = 512), so step
+    // j + 1 is enqueued first, unless step j is expected to end the cycle.  A
+    // step too many is thrown away; that is worth it while a step is short.
+    const double rate = precision == MK_BF16X3 ? 2.5e8 : precision == MK_FP32 ? 1.0e8 : 6.0e7;   // flops / us
+    const bool ahead = op->flops / rate + 8.0 * (double)n * (2 * K + 6) / 4.5e6 < 400.0;
+    int queued = 0;                            // steps of this cycle enqueued
+    double est_prev = INFINITY;
+    est_last = INFINITY;
     for (int j = 0; j < mmax; ++j) {
       const int cj = p + j;                    // column of v_j
-      // u = H_p v_j
-      MK_TRY(op_apply(op, col(cj), u, 1.0, 0.0, precision));
-      ++ops;
-      // two classical Gram-Schmidt passes against [x, y.., v_0..v_j]
       double beta = 0.0, uw = 0.0;
       const int kq = cj + 1;
+      ++ops;
       if (kq <= 32) {
-        // fused: c1 = Q^T u; u -= Q c1 with c2 = Q^T u in the same read of Q;
-        // u -= Q c2 with |u|^2 and <w, u>; one readback for the step
-        double* cd = dv.coef + FC;
-        if (j >= 1 && local_first_pass()) {
-          // first pass on the last three columns only.  For j >= 1, H v_j lies
-          // in span{v_{j-1}, v_j, v_{j+1}} in exact arithmetic (x and the kept
-          // Ritz vectors couple to v_0 alone), so the three-term recurrence
-          // removes the large components; the full pass below removes what is
-          // left, which is small, so the pair is as orthogonal as two full
-          // passes (twice is enough) for one read of the columns instead of two
-          MK_CHECK_HIP(hipMemsetAsync(cd, 0, (size_t)kq * 8, st));
-          const int lo = std::max(0, cj - 2);
-          MK_TRY(k_multidot(col(lo), n, cj + 1 - lo, u, n, cd + lo, dv.partial, st));
-        } else {
-          MK_TRY(k_multidot(Q, n, kq, u, n, cd, dv.partial, st));
+        if (queued <= j) {
+          MK_TRY(enqueue(j));
+          queued = j + 1;
         }
-        MK_TRY(k_cgs_update_dot(Q, n, kq, cd, u, n, cd + 32, dv.partial, st));
-        MK_TRY(k_cgs_update_norm(Q, n, kq, cd + 32, u, w, n, cd + 64, dv.partial, st));
-        std::vector<double> hv(2 * 32 + 2);
-        MK_CHECK_HIP(hipMemcpyAsync(hv.data(), cd, hv.size() * 8, hipMemcpyDeviceToHost, st));
-        MK_CHECK_HIP(hipStreamSynchronize(st));
-        c.assign(hv.begin(), hv.begin() + kq);
-        c2.assign(hv.begin() + 32, hv.begin() + 32 + kq);
+        // the estimate falls by about the last step's factor
+        const double expect = j >= 2 ? est_last * (est_last / est_prev) : INFINITY;
+        if (ahead && j + 1 < mmax && kq + 1 <= 32 && !(expect <= thresh)) {
+          MK_TRY(enqueue(j + 1));
+          queued = j + 2;
+        }
+        MK_CHECK_HIP(hipEventSynchronize(ctx->readback_ev[j & 1]));
+        const double* hv = ctx->readback + FL * (j & 1);
+        const int lo = j >= 1 && local_first_pass() ? std::max(0, cj - 2) : 0;
+        c.assign(hv, hv + kq);
+        std::fill(c.begin(), c.begin() + lo, 0.0);
+        c2.assign(hv + 32, hv + 32 + kq);
         beta = std::sqrt(std::max(hv[64], 0.0));
         uw = hv[65];
       } else {
+        MK_TRY(op_apply(op, col(cj), u, 1.0, 0.0, precision));
         MK_TRY(dv.dots(Q, n, kq, u, c));
         MK_TRY(dv.subtract(Q, n, kq, u));
         MK_TRY(dv.dots(Q, n, kq, u, c2));
@@ -319,10 +353,11 @@ extern "C" mk_status mk_eigsolve(mk_op h, double* x, int krylovdim, int maxiter,
       MK_REQUIRE(std::isfinite(beta), MK_NONFINITE, "eigsolve: non-finite Krylov vector");
       double lam;
       lowest(G, ldg, kq, lam, s);
+      est_prev = est_last;
       est_last = beta * std::fabs(s[cj]);
       k = j + 1;
       if (est_last <= thresh || beta <= 1e-14 * std::fabs(theta) || j + 1 == mmax) break;
-      MK_TRY(k_axpby(1.0 / beta, u, 0.0, col(cj + 1), n, st));
+      if (kq > 32) MK_TRY(k_axpby(1.0 / beta, u, 0.0, col(cj + 1), n, st));
       G[(size_t)(cj + 1) * ldg + cj] = G[(size_t)cj * ldg + cj + 1] = beta;
       // <v_{j+1}, w> = <u, w> / beta
       G[(size_t)(cj + 1)] = G[(size_t)(cj + 1) * ldg] = uw / beta;
@@ -332,10 +367,10 @@ extern "C" mk_status mk_eigsolve(mk_op h, double* x, int krylovdim, int maxiter,
     const int kk = p + k;
     const int pn = std::min(pmax, kk);
     lowest_p(G, ldg, kk, pn, lamv, S);
-    MK_CHECK_HIP(hipMemcpyAsync(sb.ptr, S.data(), S.size() * 8, hipMemcpyHostToDevice, st));
+    MK_CHECK_HIP(hipMemcpyAsync(sb, S.data(), S.size() * 8, hipMemcpyHostToDevice, st));
     ProbSpec ps;
     ps.M = n; ps.N = pn; ps.C = col(K); ps.ldc = n;
-    ps.add(Q, n, sb.ptr, kk, kk);
+    ps.add(Q, n, sb, kk, kk);
     MK_TRY(gemm_f64(&ps, 1, GemmShape{}, st, ctx->gemm_ws()));
     MK_CHECK_HIP(hipMemcpyAsync(col(0), col(K), (size_t)n * pn * 8, hipMemcpyDeviceToDevice, st));
     MK_TRY(dv.norm(col(0), n, nrm));

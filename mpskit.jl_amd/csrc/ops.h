@@ -34,6 +34,17 @@ struct Ctx {
     if (refs.fetch_sub(1) == 1) delete this;
   }
   DevBuf arena;      // stream-ordered scratch for applies / transfers
+  // Krylov solver workspace, kept between solves while it is at most
+  // KRYLOV_KEEP bytes (a solve's six allocations and frees took 1 ms, 10% of a
+  // local solve at D = 512); the solver waits for its work before it returns
+  static constexpr size_t KRYLOV_KEEP = (size_t)1 << 30;
+  DevBuf krylovbuf;
+  // pinned readback area of the Krylov solver and the events that mark its copies
+  static constexpr int READBACK_SLOTS = 2, READBACK_LEN = 128;
+  double* readback = nullptr;
+  hipEvent_t readback_ev[READBACK_SLOTS] = {};
+  mk_status readback_init();
+  ~Ctx();
   DevBuf smallbuf;   // small stream-ordered scratch (reduction partials, scalars)
   // K-split workspaces (GEMM_WS_BYTES each) of the streams this context has
   // enqueued on, at most MAX_GEMM_WS; kept until the context goes
