@@ -1,7 +1,7 @@
 // FP64 MFMA GEMM for CDNA4 (gfx950): v_mfma_f64_16x16x4_f64, LDS-staged
-// BK = 16 (or 32) deep tiles, double-buffered through registers, 256 threads =
-// 4 waves of 64 lanes in a 2x2 arrangement.  One workgroup computes one BM x BN output tile
-// of one problem, summing every segment of that problem into the same
+// BK = 16 deep tiles, double-buffered (through registers, or straight to LDS in
+// gemm_f64_dma_kernel), 256 threads = 4 waves of 64 lanes in a 2x2
+// arrangement.  One workgroup computes one BM x BN output tile of one problem, summing every segment of that problem into the same
 // accumulators before a single fused epilogue (alpha/beta and optional CB term).
 #include "gemm_dev.h"
 #include "gemm_plan.h"
@@ -18,7 +18,6 @@ typedef double dx4 __attribute__((ext_vector_type(4)));
 typedef double dx2 __attribute__((ext_vector_type(2)));
 
 constexpr int NT = 256;
-constexpr int BK32 = 32;  // default K depth of a stage
 constexpr int PAD = 16;     // LDS row padding (doubles): alternates 128-B bank halves
 
 // Stage a tile whose contiguous memory direction is the LDS fast direction.
@@ -106,9 +105,10 @@ __device__ __forceinline__ void store_kdir(double (*S)[LDR], const dx2 (&reg)[R 
   }
 }
 
-template <int BM, int BN, bool TA, bool TB, class Src, int BK = BK32>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(BK == 16 ? 2 : 1)))
+template <int BM, int BN, bool TA, bool TB, class Src>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f64_kernel(Src src) {
+  constexpr int BK = 16;
   constexpr int LDA_S = BM + PAD;
   constexpr int LDB_S = BN + PAD;
   constexpr int WM = BM / 2, WN = BN / 2;
@@ -233,19 +233,18 @@ void gemm_f64_kernel(Src src) {
 }
 
 // ---------------------------------------------------------------------------
-// Same tile, waves, LDS layout and epilogue as gemm_f64_kernel (BK = 16), with
+// Same tile, waves, LDS layout and epilogue as gemm_f64_kernel, with
 // a branch-free load path: each operand is read through a buffer resource based
 // at the tile's first row, the per-lane byte offsets of a segment are computed
 // once per segment, and a chunk outside the operand (row past M / N, k past K)
 // gets an offset past num_records, for which the hardware returns zeros.  A K
 // step then issues its eight 16-byte loads with two VALU ops each and no
-// exec-mask branches.  Needs (checked on the host, buf_ok): every in-tile
-// offset below 2 GiB, and for ODD = false 16-byte aligned operands, even leading
-// dimensions, even K and an even row count for operands stored along their rows.
-// ODD = true takes any of them (a 16-byte load needs its address aligned to 4
-// only): the pair that would straddle the end of an odd row range or of an odd K
-// is read one element lower and shifted when it is stored, so no load leaves
-// the operand.  It needs two elements in each odd range.
+// exec-mask branches.  For odd sizes, odd leading dimensions and 8-byte aligned
+// operands (a 16-byte load needs its address aligned to 4 only): the pair that
+// would straddle the end of an odd row range or of an odd K is read one element
+// lower and shifted when it is stored, so no load leaves the operand.  Needs
+// (checked on the host, buf_ok_prob) two elements in each odd range and every
+// in-tile offset below 2 GiB.
 // ---------------------------------------------------------------------------
 constexpr unsigned OOB = 0x80000000u;
 typedef unsigned int ux4 __attribute__((ext_vector_type(4)));
@@ -254,7 +253,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, 0x7fffffff, 0x00020000);
 }
 
-template <int BM, int BN, bool TA, bool TB, class Src, bool ROT, bool ODD>
+template <int BM, int BN, bool TA, bool TB, class Src>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f64_buf_kernel(Src src) {
   constexpr int BK = 16;
@@ -303,10 +302,8 @@ void gemm_f64_buf_kernel(Src src) {
   //     all c, row steps uniform.
   // So a segment keeps one byte offset per operand (chunk 0 at k0 = 0, OOB
   // if its rows lie outside the operand) and uniform strides; the per-chunk
-  // offsets and the bounds tests are formed at each load.  (Per-chunk offset
-  // arrays held 16 more registers through the K loop, which at this kernel's
-  // 256-register budget made the allocator alias load destinations and wait
-  // on the global loads inside the step.)
+  // offsets and the bounds tests are formed at each load (per-chunk offset
+  // arrays would hold 16 more registers through the K loop).
   constexpr int RA2 = BM / 2, RB2 = BN / 2;
   const int tid = threadIdx.x;
   __amdgpu_buffer_rsrc_t rA, rB;
@@ -330,14 +327,12 @@ void gemm_f64_buf_kernel(Src src) {
       cA = (unsigned)((NT / RA2) * S.lda * 8);
       oA = m0 + 2 * (tid % RA2) < M ? (unsigned)((2 * (tid % RA2) + (int64_t)(tid / RA2) * S.lda) * 8) : OOB;
       // the tile's first row is no pair's second, so m0 = M - 1 steps below the base
-      if (ODD) {
-        shA = m0 + 2 * (tid % RA2) == M - 1;
-        if (m0 == M - 1) {
-          rA = raw_rsrc(pa + ((int64_t)m0 - 1) * 8);
-          oA = shA ? oA : OOB;
-        } else if (shA) {
-          oA -= 8;
-        }
+      shA = m0 + 2 * (tid % RA2) == M - 1;
+      if (m0 == M - 1) {
+        rA = raw_rsrc(pa + ((int64_t)m0 - 1) * 8);
+        oA = shA ? oA : OOB;
+      } else if (shA) {
+        oA -= 8;
       }
     }
     if (BKD) {
@@ -346,14 +341,12 @@ void gemm_f64_buf_kernel(Src src) {
     } else {
       cB = (unsigned)((NT / RB2) * S.ldb * 8);
       oB = n0 + 2 * (tid % RB2) < N ? (unsigned)((2 * (tid % RB2) + (int64_t)(tid / RB2) * S.ldb) * 8) : OOB;
-      if (ODD) {
-        shB = n0 + 2 * (tid % RB2) == N - 1;
-        if (n0 == N - 1) {
-          rB = raw_rsrc(pb + ((int64_t)n0 - 1) * 8);
-          oB = shB ? oB : OOB;
-        } else if (shB) {
-          oB -= 8;
-        }
+      shB = n0 + 2 * (tid % RB2) == N - 1;
+      if (n0 == N - 1) {
+        rB = raw_rsrc(pb + ((int64_t)n0 - 1) * 8);
+        oB = shB ? oB : OOB;
+      } else if (shB) {
+        oB -= 8;
       }
     }
     K = S.K;
@@ -362,16 +355,16 @@ void gemm_f64_buf_kernel(Src src) {
   dx2 ra[CHA], rb[CHB];
   auto load = [&](int k0) {
     // the pair at the end of an odd K (for operands stored along k)
-    const bool last = ODD && k0 + 2 * (tid % 8) == K - 1;
-    if (ODD && AK) shA = last;
-    if (ODD && BKD) shB = last;
+    const bool last = k0 + 2 * (tid % 8) == K - 1;
+    if (AK) shA = last;
+    if (BKD) shB = last;
     const unsigned back = last ? 8u : 0u;
 #pragma unroll
     for (int c = 0; c < CHA; ++c) {
       bool ok;
       if (AK) ok = (m0 + tid / 8 + c * (NT / 8) < M) & (k0 + 2 * (tid % 8) < K);
       else    ok = (oA != OOB) & (k0 + tid / RA2 + c * (NT / RA2) < K);
-      const unsigned o = ok ? oA + (unsigned)c * cA + (unsigned)k0 * stepA - (ODD && AK ? back : 0u) : OOB;
+      const unsigned o = ok ? oA + (unsigned)c * cA + (unsigned)k0 * stepA - (AK ? back : 0u) : OOB;
       ra[c] = __builtin_bit_cast(dx2, __builtin_amdgcn_raw_buffer_load_b128(rA, (int)o, 0, 0));
     }
 #pragma unroll
@@ -379,33 +372,20 @@ void gemm_f64_buf_kernel(Src src) {
       bool ok;
       if (BKD) ok = (n0 + tid / 8 + c * (NT / 8) < N) & (k0 + 2 * (tid % 8) < K);
       else     ok = (oB != OOB) & (k0 + tid / RB2 + c * (NT / RB2) < K);
-      const unsigned o = ok ? oB + (unsigned)c * cB + (unsigned)k0 * stepB - (ODD && BKD ? back : 0u) : OOB;
+      const unsigned o = ok ? oB + (unsigned)c * cB + (unsigned)k0 * stepB - (BKD ? back : 0u) : OOB;
       rb[c] = __builtin_bit_cast(dx2, __builtin_amdgcn_raw_buffer_load_b128(rB, (int)o, 0, 0));
     }
   };
   auto store = [&](int buf) {
-    if constexpr (ODD) {
 #pragma unroll
-      for (int c = 0; c < CHA; ++c) ra[c] = shA ? dx2{ra[c].y, 0.0} : ra[c];
+    for (int c = 0; c < CHA; ++c) ra[c] = shA ? dx2{ra[c].y, 0.0} : ra[c];
 #pragma unroll
-      for (int c = 0; c < CHB; ++c) rb[c] = shB ? dx2{rb[c].y, 0.0} : rb[c];
-    }
+    for (int c = 0; c < CHB; ++c) rb[c] = shB ? dx2{rb[c].y, 0.0} : rb[c];
     if (!TA) store_fastdir<BM, LDA_S, BK>(As[buf], ra);
     else     store_kdir<BM, LDA_S, BK>(As[buf], ra);
     if (!TB) store_kdir<BN, LDB_S, BK>(Bs[buf], rb);
     else     store_fastdir<BN, LDB_S, BK>(Bs[buf], rb);
   };
-
-  auto read_frag = [&](int bi, int kk, double (&a)[FM], double (&b)[FN]) {
-    const int kr = kk * 4 + lk;
-    const int sa = TA ? kswz(kr) : 0;   // K-contiguous operands were stored swizzled
-    const int sb = TB ? 0 : kswz(kr);
-#pragma unroll
-    for (int i = 0; i < FM; ++i) a[i] = As[bi][kr][(wm0 + i * 16 + li) ^ sa];
-#pragma unroll
-    for (int j = 0; j < FN; ++j) b[j] = Bs[bi][kr][(wn0 + j * 16 + li) ^ sb];
-  };
-  double fa[2][FM], fb[2][FN];
 
   int s, k0, step0, step1;
   slice_range<BK>(P, nsteps, slice, nslice, step0, step1, s, k0);
@@ -415,7 +395,6 @@ void gemm_f64_buf_kernel(Src src) {
     store(0);
   }
   __syncthreads();
-  if (ROT && step1 > step0) read_frag(0, 0, fa[0], fb[0]);
   int buf = 0;
   for (int step = step0; step < step1; ++step) {
     k0 += BK;
@@ -426,49 +405,225 @@ void gemm_f64_buf_kernel(Src src) {
     }
     const bool has_next = step + 1 < step1;
     if (has_next) load(k0);
-    if constexpr (!ROT) {
 #pragma unroll
-      for (int kk = 0; kk < BK / 4; ++kk) {
-        double a[FM], b[FN];
-        read_frag(buf, kk, a, b);
+    for (int kk = 0; kk < BK / 4; ++kk) {
+      double a[FM], b[FN];
+      const int kr = kk * 4 + lk;
+      const int sa = TA ? kswz(kr) : 0;   // K-contiguous operands were stored swizzled
+      const int sb = TB ? 0 : kswz(kr);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FM; ++i) a[i] = As[buf][kr][(wm0 + i * 16 + li) ^ sa];
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
-      }
-      if (has_next) store(buf ^ 1);
-      __syncthreads();
-    } else {
-      // fragments of k slice kk + 1 are read while slice kk multiplies; the
-      // step barrier sits before the last slice's MFMAs, which then cover the
-      // latency of the next step's first fragment reads
+      for (int j = 0; j < FN; ++j) b[j] = Bs[buf][kr][(wn0 + j * 16 + li) ^ sb];
 #pragma unroll
-      for (int kk = 0; kk < BK / 4; ++kk) {
-        if (kk + 1 < BK / 4) {
-          read_frag(buf, kk + 1, fa[(kk + 1) & 1], fb[(kk + 1) & 1]);
-        } else {
-          // (storing the next tile earlier in the step measured slower: its
-          // global loads, issued at the step start, are often still in flight)
-          if (has_next) store(buf ^ 1);
-          __builtin_amdgcn_sched_barrier(0);
-          __syncthreads();
-          __builtin_amdgcn_sched_barrier(0);
-          if (has_next) read_frag(buf ^ 1, 0, fa[0], fb[0]);
-        }
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[kk & 1][j], fa[kk & 1][i], acc[i][j], 0, 0, 0);
-      }
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
     }
+    if (has_next) store(buf ^ 1);
+    __syncthreads();
     buf ^= 1;
   }
 
   // epilogue: as in gemm_f64_kernel
   if (slice < 0)
     epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, M, N, m0 + wm0, n0 + wn0, li, lk, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<double>(src, t, slice, BM * BN), wave, lane);
+  }  // units
+}
+
+// ---------------------------------------------------------------------------
+// Operands straight to LDS (buffer_load ... lds, 16 bytes a lane): no staging
+// registers and no LDS stores, so a K step is 8 DMA loads, the fragment reads and
+// the MFMAs.  For 16-byte aligned operands with even leading dimensions, even K
+// and an even row count where rows are contiguous.
+//
+// A DMA load writes 1 KB of LDS in lane order, so every swizzle is in which
+// element a lane loads:
+//   rows contiguous in memory: S[k][R] (R = 128: one k a load; 64: two), the row
+//     XORed by 16 for k with bit 1 set;
+//   k contiguous: S[row][16] as eight 16-byte chunks, chunk XORed by row % 8
+//     (eight rows a load).
+// An MFMA takes four k, one per lane quarter lq; quarter lq of slice s (8 deep)
+// owns k = 8 s + 2 lq and the next, which a 16-byte read of a k-contiguous
+// operand returns together and which lie in rows 2 lq, 2 lq + 1 of the other
+// kind.  Both read patterns hit every bank once per pass.
+//
+// Two stages.  The loads of step s + 1 go out at the start of step s, its barrier
+// sits before the last quarter of the MFMAs, which cover the latency of the
+// next step's first fragment reads; two workgroups a CU fill the rest.
+// Against the kernel that stages through registers (same tiles; MFMA busy 0.86
+// there at 4096 x 4096 x 8192): 4094 -> 3924 us at that shape, 1024 x 8192 x 1024
+// with 64 x 64 tiles 289 -> 261, 1024 x 5120 x 2048 with A transposed 562 -> 507.
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void lds_void;
+
+template <int BM, int BN, bool TA, bool TB, class Src>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_f64_dma_kernel(Src src) {
+  constexpr int BK = 16;
+  constexpr int WM = BM / 2, WN = BN / 2;
+  constexpr int FM = WM / 16, FN = WN / 16;
+  constexpr int CHA = BM * BK * 8 / 1024 / 4, CHB = BN * BK * 8 / 1024 / 4;   // DMA loads a wave
+  constexpr bool AK = TA, BKD = !TB;
+
+  __shared__ __attribute__((aligned(1024))) double As0[BM * BK];
+  __shared__ __attribute__((aligned(1024))) double As1[BM * BK];
+  __shared__ __attribute__((aligned(1024))) double Bs0[BN * BK];
+  __shared__ __attribute__((aligned(1024))) double Bs1[BN * BK];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave & 1) * WM;
+  const int wn0 = (wave >> 1) * WN;
+  const int li = lane & 15;
+  const int lq = lane >> 4;
+
+  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
+  int t, slice, nslice;
+  src_unit(src, un, t, slice, nslice);
+  const GemmProb& P = src_prob(src, t);
+  int tm, tn;
+  tile_coords(P, t - P.tile_start, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int M = P.M, N = P.N;
+
+  dx4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = dx4{0.0, 0.0, 0.0, 0.0};
+
+  int nsteps = 0;
+  for (int s = 0; s < P.nseg; ++s) nsteps += (P.seg[s].K + BK - 1) / BK;
+
+  // Load c of this wave (c < CH): byte offset v[c] of the lane (OOB where its row
+  // is outside the operand) plus the uniform (c cs + k0 ks)
+  __amdgpu_buffer_rsrc_t rA, rB;
+  unsigned vA[AK ? CHA : 1], vB[BKD ? CHB : 1];
+  unsigned csA = 0, csB = 0, ksA = 0, ksB = 0, w0A = 0, w0B = 0;
+  int K = 0;
+  auto set_side = [&](bool kdir, int R, int CH, const char* p, int64_t ld, int r0, int lim, __amdgpu_buffer_rsrc_t& rs,
+                      unsigned* v, unsigned& cs, unsigned& ks, unsigned& w0) {
+    if (kdir) {
+      rs = raw_rsrc(p + (int64_t)r0 * ld * 8);
+      ks = 8u;
+      cs = (unsigned)(32 * ld * 8);          // loads wave + 4 c: 8 rows each
+      w0 = (unsigned)(8 * wave * ld * 8);
+      const unsigned o = (unsigned)((lane >> 3) * ld * 8 + (((lane & 7) ^ (lane >> 3)) << 4));
+#pragma unroll
+      for (int c = 0; c < CH; ++c) v[c] = r0 + 8 * (wave + 4 * c) + (lane >> 3) < lim ? o : OOB;
+    } else {
+      rs = raw_rsrc(p + (int64_t)r0 * 8);
+      ks = (unsigned)(ld * 8);
+      const int kpl = 128 / R;               // k rows a load
+      cs = (unsigned)(4 * kpl * ld * 8);
+      w0 = (unsigned)(kpl * wave * ld * 8);
+      const int pairs = R / 2, kl = lane / pairs;
+      const int kw = kpl * wave;             // (k >> 1) & 1 is that of the wave's first load
+      const int row = (2 * (lane % pairs)) ^ (16 * ((kw >> 1) & 1));
+      v[0] = r0 + row < lim ? (unsigned)(row * 8 + kl * ld * 8) : OOB;
+    }
+  };
+  auto set_seg = [&](int s) {
+    const GemmSeg& S = P.seg[s];
+    set_side(AK, BM, CHA, static_cast<const char*>(resolve(src, S.A)), S.lda, m0, M, rA, vA, csA, ksA, w0A);
+    set_side(BKD, BN, CHB, static_cast<const char*>(resolve(src, S.B)), S.ldb, n0, N, rB, vB, csB, ksB, w0B);
+    K = S.K;
+  };
+  auto fetch_side = [&](bool kdir, int R, int CH, __amdgpu_buffer_rsrc_t rs, const unsigned* v, unsigned cs, unsigned ks,
+                        unsigned w0, int k0, double* S) {
+    const bool tail = k0 + BK > K;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      unsigned o = v[kdir ? c : 0];
+      if (tail) {
+        // K is even, and so are the k of a chunk or of a load's first row
+        const int k = kdir ? 2 * ((lane & 7) ^ (lane >> 3)) : (128 / R) * (wave + 4 * c);
+        o = k0 + k < K ? o : OOB;
+      }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(S + (wave + 4 * c) * 128), 16, (int)o,
+                                               (int)(w0 + c * cs + (unsigned)k0 * ks), 0, 0);
+    }
+  };
+
+  // fragments of slice s (8 deep): items m = 0, 1
+  auto read_side = [&](bool kdir, int R, int F, const double* S, int w0, int s, double (*f)[2]) {
+    if (kdir) {
+      const double* p = S + (w0 + li) * BK + (((4 * s + lq) ^ (li & 7)) << 1);
+#pragma unroll
+      for (int i = 0; i < F; ++i) {
+        const dx2 v = *reinterpret_cast<const dx2*>(p + i * 16 * BK);
+        f[i][0] = v.x;
+        f[i][1] = v.y;
+      }
+    } else {
+      // rows XORed by 16 in the odd quarters: blocks i and i ^ 1 change places
+      const int x = lq & 1;
+      const double* pe = S + (8 * s + 2 * lq) * R + w0 + li + 16 * x;
+      const double* po = S + (8 * s + 2 * lq) * R + w0 + li + 16 - 16 * x;
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) f[i][m] = (i & 1 ? po : pe)[m * R + (i >> 1) * 32];
+    }
+  };
+  double fa[2][FM][2], fb[2][FN][2];
+
+  int s, k0, step0, step1;
+  slice_range<BK>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  auto fetch = [&](double* A, double* B) {
+    fetch_side(AK, BM, CHA, rA, vA, csA, ksA, w0A, k0, A);
+    fetch_side(BKD, BN, CHB, rB, vB, csB, ksB, w0B, k0, B);
+  };
+  auto mfma = [&](int f, int m) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[f][j][m], fa[f][i][m], acc[i][j], 0, 0, 0);
+  };
+  auto body = [&](const double* A, const double* B, double* An, double* Bn, bool has_next) {
+    if (has_next) {
+      k0 += BK;
+      while (k0 >= K && s + 1 < P.nseg) {
+        ++s;
+        k0 = 0;
+        set_seg(s);
+      }
+      fetch(An, Bn);
+    }
+    read_side(AK, BM, FM, A, wm0, 1, fa[1]);
+    read_side(BKD, BN, FN, B, wn0, 1, fb[1]);
+    mfma(0, 0);
+    mfma(0, 1);
+    mfma(1, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    if (has_next) {
+      read_side(AK, BM, FM, An, wm0, 0, fa[0]);
+      read_side(BKD, BN, FN, Bn, wn0, 0, fb[0]);
+    }
+    mfma(1, 1);
+  };
+  if (step1 > step0) {
+    set_seg(s);
+    fetch(As0, Bs0);
+    __syncthreads();
+    read_side(AK, BM, FM, As0, wm0, 0, fa[0]);
+    read_side(BKD, BN, FN, Bs0, wn0, 0, fb[0]);
+  }
+  for (int step = step0; step < step1; step += 2) {
+    body(As0, Bs0, As1, Bs1, step + 1 < step1);
+    if (step + 1 < step1) body(As1, Bs1, As0, Bs0, step + 2 < step1);
+  }
+
+  // epilogue: as in gemm_f64_kernel
+  if (slice < 0)
+    epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, M, N, m0 + wm0, n0 + wn0, li, lq, P.alpha, P.beta);
   else
     store_partial(acc, src_partial<double>(src, t, slice, BM * BN), wave, lane);
   }  // units
@@ -497,45 +652,56 @@ BufFit buf_ok_prob(const ProbSpec& ps, GemmShape sh) {
   return fit;
 }
 
-// Load path of the FP64 kernels, read once from MK_F64_VARIANT ("rot", "buf"
-// or "branch"; default "rot"): lets benchmarks and tests pin one of them.
-enum F64Variant { F64_BRANCH = 0, F64_BUF = 1, F64_ROT = 2 };
+// Load path of the FP64 kernels, read once from MK_F64_VARIANT ("dma", "buf" or
+// "branch"; default "dma"): lets benchmarks and tests pin one of them.
+enum F64Variant { F64_BRANCH = 0, F64_BUF = 1, F64_DMA = 2 };
 int f64_variant() {
   static const int v = [] {
     const char* e = getenv("MK_F64_VARIANT");
     if (e && !strcmp(e, "branch")) return (int)F64_BRANCH;
     if (e && !strcmp(e, "buf")) return (int)F64_BUF;
-    return (int)F64_ROT;
+    return (int)F64_DMA;
   }();
   return v;
 }
 
-template <int BM, int BN, class Src, bool ROT, bool ODD>
+// The kernel for a launch whose problems fit `fit`: straight to LDS where sizes
+// and alignment allow, else branch-free, else branching.
+BufFit f64_path(int fit) {
+  const int var = f64_variant();
+  if (var == F64_BRANCH || fit == BUF_NO) return BUF_NO;
+  return var == F64_BUF ? BUF_ODD : (BufFit)fit;
+}
+
+template <int BM, int BN, class Src>
+void launch4_dma(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
+  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, false, false, Src>), grid, block, 0, stream, b);
+  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, true, false, Src>), grid, block, 0, stream, b);
+  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, false, true, Src>), grid, block, 0, stream, b);
+  else hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, true, true, Src>), grid, block, 0, stream, b);
+}
+
+template <int BM, int BN, class Src>
 void launch4_buf(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
-  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, false, Src, ROT, ODD>), grid, block, 0, stream, b);
-  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, false, Src, ROT, ODD>), grid, block, 0, stream, b);
-  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, true, Src, ROT, ODD>), grid, block, 0, stream, b);
-  else hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, true, Src, ROT, ODD>), grid, block, 0, stream, b);
+  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, false, Src>), grid, block, 0, stream, b);
+  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, false, Src>), grid, block, 0, stream, b);
+  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, true, Src>), grid, block, 0, stream, b);
+  else hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, true, Src>), grid, block, 0, stream, b);
 }
 
-// K depth of a stage, read once from MK_F64_BK (16 or 32; default 16).  BK = 16
-// halves the LDS footprint of a 128 x 128 workgroup (74 KB instead of 147 KB),
-// so two workgroups (two waves per SIMD) share a CU: 24% faster at
-// M = N = 4096, K = 8192 than BK = 32 with one wave per SIMD.
-int f64_bk() {
-  static const int bk = [] {
-    const char* e = getenv("MK_F64_BK");
-    return (e && atoi(e) == 32) ? 32 : 16;
-  }();
-  return bk;
-}
-
-template <int BM, int BN, class Src, int BK>
+template <int BM, int BN, class Src>
 void launch4(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
-  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, false, false, Src, BK>), grid, block, 0, stream, b);
-  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, true, false, Src, BK>), grid, block, 0, stream, b);
-  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, false, true, Src, BK>), grid, block, 0, stream, b);
-  else hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, true, true, Src, BK>), grid, block, 0, stream, b);
+  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, false, false, Src>), grid, block, 0, stream, b);
+  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, true, false, Src>), grid, block, 0, stream, b);
+  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, false, true, Src>), grid, block, 0, stream, b);
+  else hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, true, true, Src>), grid, block, 0, stream, b);
+}
+
+template <int BM, int BN, class Src>
+void launch_path(BufFit path, GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
+  if (path == BUF_EVEN) launch4_dma<BM, BN, Src>(sh, grid, block, stream, b);
+  else if (path == BUF_ODD) launch4_buf<BM, BN, Src>(sh, grid, block, stream, b);
+  else launch4<BM, BN, Src>(sh, grid, block, stream, b);
 }
 
 template <int BM, int BN>
@@ -579,19 +745,11 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
   const int tail = total - b.full_tiles;
   MK_REQUIRE(tail == 0 || (ws != nullptr && (size_t)tail * sp.ksplit * BM * BN * 8 <= GEMM_WS_BYTES), MK_BAD_ARG,
              "gemm_f64: %d tiles split %d ways exceed the workspace", tail, sp.ksplit);
-  const int var = f64_variant();
-  int fit = var != F64_BRANCH && f64_bk() == 16 ? BUF_EVEN : BUF_NO;
+  int fit = BUF_EVEN;
   for (int i = 0; i < nprob && fit != BUF_NO; ++i) fit = std::min<int>(fit, buf_ok_prob<BM, BN>(probs[i], sh));
-  const bool rot = var == F64_ROT && !sh.ta;
   dim3 grid(b.full_tiles + tail * b.ksplit), block(NT);
   ProfScope prof("gemm_f64", stream);
-  // the rotated schedule holds two fragment sets; with a K-contiguous A the
-  // extra registers would spill, so those launches keep the plain schedule
-  if (fit == BUF_EVEN && rot) launch4_buf<BM, BN, GemmBatch, true, false>(sh, grid, block, stream, b);
-  else if (fit == BUF_EVEN) launch4_buf<BM, BN, GemmBatch, false, false>(sh, grid, block, stream, b);
-  else if (fit == BUF_ODD) launch4_buf<BM, BN, GemmBatch, false, true>(sh, grid, block, stream, b);
-  else if (f64_bk() == 16) launch4<BM, BN, GemmBatch, 16>(sh, grid, block, stream, b);
-  else launch4<BM, BN, GemmBatch, BK32>(sh, grid, block, stream, b);
+  launch_path<BM, BN>(f64_path(fit), sh, grid, block, stream, b);
   MK_CHECK_HIP(hipGetLastError());
   if (tail > 0) {
     constexpr int NBLK = BM * BN / 256;
@@ -607,13 +765,7 @@ mk_status launch_group(const GemmGroup& g, GemmShape sh, int grid, hipStream_t s
   if (g.total_tiles == 0) return MK_OK;
   dim3 gr(grid), block(NT);
   ProfScope prof("gemm_f64", stream);
-  const int var = f64_variant();
-  const int fit = var != F64_BRANCH && f64_bk() == 16 ? g.f64_buf : BUF_NO;
-  if (fit == BUF_EVEN && var == F64_ROT && !sh.ta) launch4_buf<BM, BN, GemmGroup, true, false>(sh, gr, block, stream, g);
-  else if (fit == BUF_EVEN) launch4_buf<BM, BN, GemmGroup, false, false>(sh, gr, block, stream, g);
-  else if (fit == BUF_ODD) launch4_buf<BM, BN, GemmGroup, false, true>(sh, gr, block, stream, g);
-  else if (f64_bk() == 16) launch4<BM, BN, GemmGroup, 16>(sh, gr, block, stream, g);
-  else launch4<BM, BN, GemmGroup, BK32>(sh, gr, block, stream, g);
+  launch_path<BM, BN>(f64_path(g.f64_buf), sh, gr, block, stream, g);
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
 }
@@ -623,10 +775,7 @@ int occupancy() {
   static const int occ = [] {
     int n = 0;
     const hipError_t e =
-        f64_bk() == 16
-            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemm_f64_kernel<BM, BN, false, false, GemmGroup, 16>, NT, 0)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemm_f64_kernel<BM, BN, false, false, GemmGroup, BK32>, NT,
-                                                           0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemm_f64_kernel<BM, BN, false, false, GemmGroup>, NT, 0);
     if (e != hipSuccess) n = 1;
     return n > 0 ? n : 1;
   }();
@@ -662,13 +811,22 @@ mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_
     for (int s = 0; s < probs[i].nseg; ++s)
       MK_REQUIRE(probs[i].seg[s].K >= 0 && probs[i].seg[s].K < (1ll << 31), MK_BAD_SHAPE, "gemm_f64: bad K");
   }
-  // Measured on 1024 x 1024 x 8192 (us, 64 x 64 tiles: 1, 2, 3, 4 workgroups a
-  // CU 419, 331, 305, 298; 128 x 128: 1, 2 a CU 309, 279); one step is 64 (16)
-  // v_mfma_f64_16x16x4 of 64 cycles per wave.
-  static const TileModel m128{128, 128, 16, 1.74, {0.76, 0.87, 0.87, 0.87}, 2, 128 * 128 * 8};
-  static const TileModel m64{64, 64, 16, 0.436, {0.53, 0.70, 0.77, 0.79}, 4, 64 * 64 * 8};
-  const bool split = ws != nullptr && f64_bk() == 16;
-  const TileChoice c128 = plan_launch(m128, probs, nprob, split), c64 = plan_launch(m64, probs, nprob, split);
+  // One step is 64 (128 tile) or 16 v_mfma_f64_16x16x4 of 64 cycles a wave.
+  // Straight to LDS, measured (us): 1024 x 1024 x 2048 with 64 x 64 tiles, 1 and 3
+  // workgroups a CU 83 and 83 (split 3 ways, reduction included), 1024 x 8192 x
+  // 1024 8 rounds of 64 tiles 261, 2 of 128 tiles 255; 1024 x 5120 x 2048 with A
+  // transposed 374 (64 tiles) and 331 (256 tiles of 128, 64 split 8 ways).  Through
+  // registers (odd sizes): 1024 x 1024 x 8192, 64 tiles 1, 2, 3, 4 a CU 419, 331,
+  // 305, 298, 128 tiles 1, 2 a CU 309, 279.
+  static const TileModel d128{128, 128, 16, 1.74, {0.88, 0.90, 0.90, 0.90}, 2, 128 * 128 * 8};
+  static const TileModel d64{64, 64, 16, 0.436, {0.70, 0.83, 0.87, 0.88}, 4, 64 * 64 * 8};
+  static const TileModel d64t{64, 64, 16, 0.436, {0.62, 0.73, 0.77, 0.78}, 4, 64 * 64 * 8};
+  static const TileModel b128{128, 128, 16, 1.74, {0.76, 0.87, 0.87, 0.87}, 2, 128 * 128 * 8};
+  static const TileModel b64{64, 64, 16, 0.436, {0.53, 0.70, 0.77, 0.79}, 4, 64 * 64 * 8};
+  const bool direct = f64_path(f64_buf_ok(probs, nprob, shape, TK_128)) == BUF_EVEN;
+  const TileModel& m64 = !direct ? b64 : shape.ta || shape.tb ? d64t : d64;
+  const TileChoice c128 = plan_launch(direct ? d128 : b128, probs, nprob, ws != nullptr);
+  const TileChoice c64 = plan_launch(m64, probs, nprob, ws != nullptr);
   if (c128.us <= c64.us) return launch_cfg<128, 128>(probs, nprob, shape, stream, c128.split, ws);
   return launch_cfg<64, 64>(probs, nprob, shape, stream, c64.split, ws);
 }
