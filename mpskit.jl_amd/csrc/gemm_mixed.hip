@@ -43,16 +43,13 @@ __device__ __forceinline__ int swz(int r, int q) { return r * ROWB + ((q ^ (-(r 
 
 enum Mode { M_BF16X3 = 0, M_F32 = 1 };
 
-// Kernel family for large problems, read once from MK_GEMM_VARIANT ("big2",
-// "big", "pipe", "tile"; default "big2"): lets benchmarks and tests pin one family.
-enum Variant { V_PIPE = 0, V_BIG = 1, V_TILE = 2, V_BIG2 = 3 };
+// Load path of the kernels, read once from MK_GEMM_VARIANT ("dma" or "tile";
+// default "dma"): lets benchmarks and tests pin the register-staged kernel.
+enum Variant { V_TILE = 0, V_DMA = 1 };
 int variant() {
   static const int v = [] {
     const char* e = getenv("MK_GEMM_VARIANT");
-    if (e && !strcmp(e, "pipe")) return (int)V_PIPE;
-    if (e && !strcmp(e, "tile")) return (int)V_TILE;
-    if (e && !strcmp(e, "big")) return (int)V_BIG;
-    return (int)V_BIG2;
+    return e && !strcmp(e, "tile") ? (int)V_TILE : (int)V_DMA;
   }();
   return v;
 }
@@ -222,164 +219,6 @@ __global__ __launch_bounds__(NT) void gemm_mixed_kernel(Src src) {
   }  // units
 }
 
-// ---------------------------------------------------------------------------
-// Large-tile variant: 256 x 256 output tile, 512 threads = 8 waves (2 x 4), each
-// wave 128 x 64.  Halves the operand re-reads of the 128 x 128 kernel and
-// doubles the MFMA work per LDS fragment.  LDS rows hold 64 B of K without
-// padding, swizzled (swz).  Double-buffered: 128 KB (bf16).
-// ---------------------------------------------------------------------------
-
-constexpr int BIG = 256;
-constexpr int BNT = 512;
-
-template <int R>
-__device__ __forceinline__ void load_slab_big(const char* __restrict__ base, int64_t ld_bytes, int r0,
-                                              int64_t kbyte0, int Rlim, int64_t Kbytes,
-                                              ux4 (&reg)[R * ROWB / 16 / BNT]) {
-  constexpr int CH = R * ROWB / 16 / BNT;
-#pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int id = threadIdx.x + c * BNT;
-    const int r = id >> 2, q = id & 3;
-    const int gr = r0 + r;
-    const int64_t kb = kbyte0 + q * 16;
-    ux4 v = {0u, 0u, 0u, 0u};
-    if (gr < Rlim && kb < Kbytes) v = *gptr(reinterpret_cast<const ux4*>(base + (int64_t)gr * ld_bytes + kb));
-    reg[c] = v;
-  }
-}
-
-template <int R>
-__device__ __forceinline__ void store_slab_big(char* S, const ux4 (&reg)[R * ROWB / 16 / BNT]) {
-  constexpr int CH = R * ROWB / 16 / BNT;
-#pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int id = threadIdx.x + c * BNT;
-    const int r = id >> 2, q = id & 3;
-    *reinterpret_cast<ux4*>(S + swz(r, q)) = reg[c];
-  }
-}
-
-template <int MODE, class Src>
-__global__ __launch_bounds__(BNT) void gemm_mixed_big_kernel(Src src) {
-  constexpr int NPART = MODE == M_BF16X3 ? 2 : 1;
-  constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
-  constexpr int WM = 128, WN = 64;
-  constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int CH = BIG * ROWB / 16 / BNT;   // 16-B chunks per thread per operand part
-
-  __shared__ __attribute__((aligned(16))) char As[2][NPART][BIG * ROWB];
-  __shared__ __attribute__((aligned(16))) char Bs[2][NPART][BIG * ROWB];
-
-  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
-  int t, slice, nslice;
-  src_unit(src, un, t, slice, nslice);
-  const GemmProb& P = src_prob(src, t);
-  int tm, tn;
-  tile_coords(P, t - P.tile_start, tm, tn);
-  const int m0 = tm * BIG, n0 = tn * BIG;
-
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm0 = (wave & 1) * WM;
-  const int wn0 = (wave >> 1) * WN;
-  const int li = lane & 15;
-  const int lg = lane >> 4;
-
-  fx4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = fx4{0.f, 0.f, 0.f, 0.f};
-
-  constexpr int KSTEP = ROWB / EB;
-  int nsteps = 0;
-  for (int s = 0; s < P.nseg; ++s) nsteps += (P.seg[s].K + KSTEP - 1) / KSTEP;
-
-  ux4 ra[NPART][CH], rb[NPART][CH];
-  auto load = [&](int s, int k0) {
-    const GemmSeg& S = P.seg[s];
-    const int64_t ldab = S.lda * EB, ldbb = S.ldb * EB;
-    const int64_t kb0 = (int64_t)k0 * EB, Kb = (int64_t)S.K * EB;
-    load_slab_big<BIG>(static_cast<const char*>(resolve(src, S.A)), ldab, m0, kb0, P.M, Kb, ra[0]);
-    load_slab_big<BIG>(static_cast<const char*>(resolve(src, S.B)), ldbb, n0, kb0, P.N, Kb, rb[0]);
-    if (NPART == 2) {
-      load_slab_big<BIG>(static_cast<const char*>(resolve(src, S.Alo)), ldab, m0, kb0, P.M, Kb, ra[NPART - 1]);
-      load_slab_big<BIG>(static_cast<const char*>(resolve(src, S.Blo)), ldbb, n0, kb0, P.N, Kb, rb[NPART - 1]);
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < NPART; ++p) {
-      store_slab_big<BIG>(As[buf][p], ra[p]);
-      store_slab_big<BIG>(Bs[buf][p], rb[p]);
-    }
-  };
-
-  int s, k0, step0, step1;
-  slice_range<KSTEP>(P, nsteps, slice, nslice, step0, step1, s, k0);
-  if (step1 > step0) {
-    load(s, k0);
-    store(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  const int aoff = swz(wm0 + li, lg);   // same swizzle for every 16-row block
-  const int boff = swz(wn0 + li, lg);
-  for (int step = step0; step < step1; ++step) {
-    int ns = s, nk0 = k0 + KSTEP;
-    if (nk0 >= P.seg[s].K) { ns = s + 1; nk0 = 0; }
-    const bool has_next = step + 1 < step1;
-    if (has_next) load(ns, nk0);
-
-    ux4 fb[NPART][FN];
-#pragma unroll
-    for (int p = 0; p < NPART; ++p)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) fb[p][j] = *reinterpret_cast<const ux4*>(Bs[buf][p] + boff + j * 16 * ROWB);
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      ux4 fa[NPART];
-#pragma unroll
-      for (int p = 0; p < NPART; ++p) fa[p] = *reinterpret_cast<const ux4*>(As[buf][p] + aoff + i * 16 * ROWB);
-      if constexpr (MODE == M_BF16X3) {
-        const bfx8 ah = __builtin_bit_cast(bfx8, fa[0]);
-        const bfx8 al = __builtin_bit_cast(bfx8, fa[1]);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const bfx8 bh = __builtin_bit_cast(bfx8, fb[0][j]);
-          const bfx8 bl = __builtin_bit_cast(bfx8, fb[1][j]);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, al, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl, ah, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, ah, acc[i][j], 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int sub = 0; sub < 4; ++sub) {
-          const unsigned int ua = fa[0][sub];
-          const float a = __uint_as_float(ua);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const unsigned int ub = fb[0][j][sub];
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ub), a, acc[i][j], 0, 0, 0);
-          }
-        }
-      }
-    }
-    if (has_next) store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-    s = ns;
-    k0 = nk0;
-  }
-
-  if (slice < 0)
-    store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
-  else
-    store_partial(acc, src_partial<float>(src, t, slice, BIG * BIG), wave, lane);
-  }  // units
-}
-
 // Raw (stride 0) buffer resource over p with num_records = 2^31 - 1 bytes and
 // the gfx9 data-format word; offsets at or past num_records load zeros.
 constexpr unsigned OOB = 0x80000000u;
@@ -387,37 +226,49 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, 0x7fffffff, 0x00020000);
 }
 
-// Same tile, waves and LDS layout as gemm_mixed_big_kernel, with a lighter
-// load path: the segment's operand descriptors are read once per segment (not
-// once per K step), each operand is addressed through a buffer resource based
-// at the tile's first row, and rows or K chunks outside the operand get a
-// buffer offset past num_records (the hardware returns zeros), so a K step
-// issues its loads without scalar loads or branches.  Needs 256 rows of every
-// operand within 2 GiB of the row base (checked on the host).
-template <int MODE, class Src>
-__global__ __launch_bounds__(BNT) void gemm_mixed_big2_kernel(Src src) {
+typedef __attribute__((address_space(3))) void lds_void;
+
+// ---------------------------------------------------------------------------
+// Operands straight to LDS (buffer_load ... lds, 16 bytes a lane).  A K step is
+// 64 bytes of every row; a load instruction fills 16 rows of the slab in lane
+// order, and lane l takes the chunk of row l / 4 that swz puts at slot l % 4.
+// Packed operands (256-row panels of contiguous 16 KB K steps) are read the same
+// way with rows of 64 bytes.  Two stages; the loads of step s + 1 go out at the
+// start of step s, and its barrier sits before the last MFMAs, which cover the
+// latency of the next step's first fragment reads.  Rows and K chunks outside an
+// operand get a buffer offset past num_records, which loads zeros.  Needs 256
+// rows of every operand within 2 GiB of the row base (checked on the host).
+//
+// 128 x 128 and 64 x 64 tiles: 4 waves (2 x 2), two or more workgroups a CU, both
+// fragment sets in registers.  256 x 256: 8 waves (2 x 4) of 128 x 64, one
+// workgroup a CU; the next step's B fragments and first A fragment are read
+// ahead, the other A fragments one block ahead of their MFMAs.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int WGM, int WGN, int MODE, class Src>
+__global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_mixed_dma_kernel(Src src) {
   constexpr int NPART = MODE == M_BF16X3 ? 2 : 1;
   constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
-  constexpr int WM = 128, WN = 64;
+  constexpr int NW = WGM * WGN;
+  constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int CH = BIG * ROWB / 16 / BNT;   // 16-B chunks per thread per operand part
+  constexpr int CHA = BM / 16 / NW, CHB = BN / 16 / NW;   // load instructions a wave and part
   constexpr int KSTEP = ROWB / EB;
+  constexpr bool BIGT = FM > 4;                           // A fragments streamed
 
-  __shared__ __attribute__((aligned(16))) char As[2][NPART][BIG * ROWB];
-  __shared__ __attribute__((aligned(16))) char Bs[2][NPART][BIG * ROWB];
+  __shared__ __attribute__((aligned(1024))) char As0[NPART * BM * ROWB];
+  __shared__ __attribute__((aligned(1024))) char As1[NPART * BM * ROWB];
+  __shared__ __attribute__((aligned(1024))) char Bs0[NPART * BN * ROWB];
+  __shared__ __attribute__((aligned(1024))) char Bs1[NPART * BN * ROWB];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm0 = (wave & 1) * WM;
-  const int wn0 = (wave >> 1) * WN;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave % WGM) * WM;
+  const int wn0 = (wave / WGM) * WN;
   const int li = lane & 15;
   const int lg = lane >> 4;
-  const int cq = threadIdx.x & 3;             // 16-B chunk of the 64-B row slab
-  int crow[CH];
-#pragma unroll
-  for (int c = 0; c < CH; ++c) crow[c] = (threadIdx.x + c * BNT) >> 2;
-  const int aoff = swz(wm0 + li, lg);
-  const int boff = swz(wn0 + li, lg);
+  const int cq = (lane & 3) ^ (-(lane >> 4) & 3);         // chunk this lane loads (row lane / 4)
+  const int aoff = swz(wm0 + li, lg), boff = swz(wn0 + li, lg);
 
   for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
   int t, slice, nslice;
@@ -425,220 +276,7 @@ __global__ __launch_bounds__(BNT) void gemm_mixed_big2_kernel(Src src) {
   const GemmProb& P = src_prob(src, t);
   int tm, tn;
   tile_coords(P, t - P.tile_start, tm, tn);
-  const int m0 = tm * BIG, n0 = tn * BIG;
-  const int nseg = P.nseg;
-
-  fx4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = fx4{0.f, 0.f, 0.f, 0.f};
-
-  // per-segment load state.  A row-layout operand is addressed by row; a
-  // packed one (256-row panels of contiguous 16 KB K steps, every row present)
-  // by its panel, with the K step at 16 KB per 64 bytes of K.
-  __amdgpu_buffer_rsrc_t rA[NPART], rB[NPART];
-  unsigned vA[CH], vB[CH];
-  unsigned kmulA = 1, kmulB = 1;   // bytes of offset per byte of K
-  int Kb = 0, kend = 0;
-  auto set_seg = [&](int s) {
-    const GemmSeg& S = P.seg[s];
-    const bool pa = (S.vec & 2) != 0, pb = (S.vec & 4) != 0;
-    const int64_t panel = (int64_t)S.K * EB * 256;
-    const int64_t ldab = S.lda * EB, ldbb = S.ldb * EB;
-    const int64_t offa = pa ? (int64_t)(m0 / 256) * panel : (int64_t)m0 * ldab;
-    const int64_t offb = pb ? (int64_t)(n0 / 256) * panel : (int64_t)n0 * ldbb;
-    rA[0] = raw_rsrc(static_cast<const char*>(resolve(src, S.A)) + offa);
-    rB[0] = raw_rsrc(static_cast<const char*>(resolve(src, S.B)) + offb);
-    if constexpr (NPART == 2) {
-      rA[1] = raw_rsrc(static_cast<const char*>(resolve(src, S.Alo)) + offa);
-      rB[1] = raw_rsrc(static_cast<const char*>(resolve(src, S.Blo)) + offb);
-    }
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      vA[c] = pa ? (unsigned)((threadIdx.x + c * BNT) * 16)
-                 : (m0 + crow[c] < P.M ? (unsigned)(crow[c] * ldab + cq * 16) : OOB);
-      vB[c] = pb ? (unsigned)((threadIdx.x + c * BNT) * 16)
-                 : (n0 + crow[c] < P.N ? (unsigned)(crow[c] * ldbb + cq * 16) : OOB);
-    }
-    kmulA = pa ? 256u : 1u;
-    kmulB = pb ? 256u : 1u;
-    Kb = S.K * EB;
-    kend = S.K;
-  };
-
-  int nsteps = 0;
-  for (int s = 0; s < nseg; ++s) nsteps += (P.seg[s].K + KSTEP - 1) / KSTEP;
-
-  ux4 ra[NPART][CH], rb[NPART][CH];
-  auto load = [&](int k0) {
-    const int kb0 = k0 * EB;
-    const bool kin = kb0 + cq * 16 < Kb;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const unsigned oa = kin ? vA[c] + (unsigned)kb0 * kmulA : OOB;
-      const unsigned ob = kin ? vB[c] + (unsigned)kb0 * kmulB : OOB;
-#pragma unroll
-      for (int p = 0; p < NPART; ++p) {
-        ra[p][c] = __builtin_amdgcn_raw_buffer_load_b128(rA[p], (int)oa, 0, 0);
-        rb[p][c] = __builtin_amdgcn_raw_buffer_load_b128(rB[p], (int)ob, 0, 0);
-      }
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < NPART; ++p)
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        *reinterpret_cast<ux4*>(As[buf][p] + swz(crow[c], cq)) = ra[p][c];
-        *reinterpret_cast<ux4*>(Bs[buf][p] + swz(crow[c], cq)) = rb[p][c];
-      }
-  };
-
-  int s, k0, step0, step1;
-  slice_range<KSTEP>(P, nsteps, slice, nslice, step0, step1, s, k0);
-  if (step1 > step0) {
-    set_seg(s);
-    load(k0);
-    store(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  for (int step = step0; step < step1; ++step) {
-    k0 += KSTEP;
-    while (k0 >= kend && s + 1 < nseg) {
-      ++s;
-      k0 = 0;
-      set_seg(s);
-    }
-    const bool has_next = step + 1 < step1;
-    if (has_next) load(k0);
-
-    ux4 fb[NPART][FN];
-#pragma unroll
-    for (int p = 0; p < NPART; ++p)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) fb[p][j] = *reinterpret_cast<const ux4*>(Bs[buf][p] + boff + j * 16 * ROWB);
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      ux4 fa[NPART];
-#pragma unroll
-      for (int p = 0; p < NPART; ++p) fa[p] = *reinterpret_cast<const ux4*>(As[buf][p] + aoff + i * 16 * ROWB);
-      if constexpr (MODE == M_BF16X3) {
-        const bfx8 ah = __builtin_bit_cast(bfx8, fa[0]);
-        const bfx8 al = __builtin_bit_cast(bfx8, fa[1]);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const bfx8 bh = __builtin_bit_cast(bfx8, fb[0][j]);
-          const bfx8 bl = __builtin_bit_cast(bfx8, fb[1][j]);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, al, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl, ah, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, ah, acc[i][j], 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int sub = 0; sub < 4; ++sub) {
-          const unsigned int ua = fa[0][sub];
-          const float a = __uint_as_float(ua);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const unsigned int ub = fb[0][j][sub];
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ub), a, acc[i][j], 0, 0, 0);
-          }
-        }
-      }
-    }
-    if (has_next) store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-
-  if (slice < 0)
-    store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
-  else
-    store_partial(acc, src_partial<float>(src, t, slice, BIG * BIG), wave, lane);
-  }  // units
-}
-
-// ---------------------------------------------------------------------------
-// Pipelined variant for large problems: 256 x 128 output tile, 256 threads =
-// 4 waves (2 x 2) of 128 x 64, three LDS stages.  Operand slabs go global ->
-// LDS through buffer_load ... lds (no staging registers), so the loads of step
-// s + 2 are in flight while step s computes; a single-stage register prefetch
-// covers less than one L2-miss latency at this MFMA rate.  Lane l of a wave's
-// 16-byte LDS load writes LDS bytes [16 l, 16 l + 16) after the wave base, so
-// the swizzle is applied on the global side: LDS chunk qp of row r receives
-// logical chunk qp ^ (-(r >> 2) & 3).  Out-of-range rows and K chunks get a
-// buffer offset past num_records, which the hardware turns into zeros.
-// Three stages of hi + lo bf16 slabs: 3 x (32 + 16) KB = 144 KB of LDS.
-// ---------------------------------------------------------------------------
-
-constexpr int PBM = 256, PBN = 128, PNT = 256, NSTAGE = 3;
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-// s_waitcnt on vmcnt only (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14])
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// Workgroup barrier without the release fence of __syncthreads(): that fence
-// would wait for every outstanding LDS-DMA load (vmcnt(0)) and serialise the
-// pipeline.  Each wave waits for its own loads of the stage it is about to read
-// (wait_vm) before the barrier, and every LDS read of the previous stage has
-// been consumed by an MFMA before it, so the barrier alone orders the stages.
-// The empty asm statements keep the compiler from moving LDS accesses across.
-__device__ __forceinline__ void stage_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// One R x 64 B slab of a K-contiguous operand into LDS stage memory S.
-template <int R>
-__device__ __forceinline__ void dma_slab(__amdgpu_buffer_rsrc_t rs, char* S, int ld_bytes, int r0, int Rlim,
-                                         int kb0, int Kbytes, int wave) {
-  constexpr int CH = R * (ROWB / 16) / PNT;
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int idx = c * PNT + t;
-    const int r = idx >> 2, qp = idx & 3;
-    const int q = qp ^ (-(r >> 2) & 3);
-    const int gr = r0 + r, kb = kb0 + q * 16;
-    const unsigned vo = (gr < Rlim && kb < Kbytes) ? (unsigned)(gr * ld_bytes + kb) : OOB;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(S + (c * PNT + wave * 64) * 16), 16, vo, 0, 0, 0);
-  }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(PNT) void gemm_mixed_pipe_kernel(GemmBatch batch) {
-  constexpr int NPART = MODE == M_BF16X3 ? 2 : 1;
-  constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
-  constexpr int WM = 128, WN = 64;
-  constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int KSTEP = ROWB / EB;
-  constexpr int ABYTES = PBM * ROWB, BBYTES = PBN * ROWB;
-  constexpr int SBYTES = NPART * (ABYTES + BBYTES);
-  // loads issued per thread per stage (each counts once in vmcnt)
-  constexpr int LPS = NPART * (PBM + PBN) * (ROWB / 16) / PNT;
-
-  __shared__ __attribute__((aligned(16))) char smem[NSTAGE * SBYTES];
-
-  const int t = src_first(batch);
-  const GemmProb& P = src_prob(batch, t);
-  int tm, tn;
-  tile_coords(P, t - P.tile_start, tm, tn);
-  const int m0 = tm * PBM, n0 = tn * PBN;
-
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm0 = (wave & 1) * WM;
-  const int wn0 = (wave >> 1) * WN;
-  const int li = lane & 15;
-  const int lg = lane >> 4;
+  const int m0 = tm * BM, n0 = tn * BN;
 
   fx4 acc[FM][FN];
 #pragma unroll
@@ -649,79 +287,165 @@ __global__ __launch_bounds__(PNT) void gemm_mixed_pipe_kernel(GemmBatch batch) {
   int nsteps = 0;
   for (int s = 0; s < P.nseg; ++s) nsteps += (P.seg[s].K + KSTEP - 1) / KSTEP;
 
-  // load cursor (segment, k) of the next stage to fetch
-  int ls = 0, lk = 0;
-  auto fetch = [&](int stage) {
-    const GemmSeg& S = P.seg[ls];
-    const int ldab = (int)S.lda * EB, ldbb = (int)S.ldb * EB;
-    const int kb0 = lk * EB, Kb = S.K * EB;
-    char* base = smem + stage * SBYTES;
-    dma_slab<PBM>(raw_rsrc(S.A), base, ldab, m0, P.M, kb0, Kb, wave);
-    dma_slab<PBN>(raw_rsrc(S.B), base + NPART * ABYTES, ldbb, n0, P.N, kb0, Kb, wave);
-    if constexpr (NPART == 2) {
-      dma_slab<PBM>(raw_rsrc(S.Alo), base + ABYTES, ldab, m0, P.M, kb0, Kb, wave);
-      dma_slab<PBN>(raw_rsrc(S.Blo), base + 2 * ABYTES + BBYTES, ldbb, n0, P.N, kb0, Kb, wave);
-    }
-    lk += KSTEP;
-    if (lk >= S.K) { ++ls; lk = 0; }
+  __amdgpu_buffer_rsrc_t rA[NPART], rB[NPART];
+  unsigned vA[CHA], vB[CHB];               // the lane's offset in load c (OOB: row outside)
+  unsigned csA = 0, csB = 0, w0A = 0, w0B = 0, kmA = 1, kmB = 1;
+  int Kb = 0, kend = 0;
+  auto set_side = [&](bool packed, const char* hi, const char* lo, int64_t ld, int64_t Kbytes, int r0, int lim, int CH,
+                      __amdgpu_buffer_rsrc_t* rs, unsigned* v, unsigned& cs, unsigned& w0, unsigned& km) {
+    const int64_t pitch = packed ? ROWB : ld * EB;
+    const int64_t off = packed ? (int64_t)(r0 / 256) * Kbytes * 256 : (int64_t)r0 * pitch;
+    rs[0] = raw_rsrc(hi + off);
+    if constexpr (NPART == 2) rs[1] = raw_rsrc(lo + off);
+    km = packed ? 256u : 1u;
+    cs = (unsigned)(16 * NW * pitch);
+    w0 = (unsigned)(16 * wave * pitch);
+    const unsigned o = (unsigned)((lane >> 2) * pitch + cq * 16);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) v[c] = r0 + 16 * (wave + NW * c) + (lane >> 2) < lim ? o : OOB;
   };
-
-  if (nsteps > 0) fetch(0);
-  if (nsteps > 1) fetch(1);
-  const int aoff = swz(wm0 + li, lg);   // same swizzle for every 16-row block
-  const int boff = swz(wn0 + li, lg);
-  int stage = 0;
-  for (int step = 0; step < nsteps; ++step) {
-    // this wave's loads of `step` are done once at most one newer stage is pending
-    if (step + 1 < nsteps) wait_vm<LPS>();
-    else wait_vm<0>();
-    stage_barrier();   // every wave's loads of `step` landed; stage (step + 2) % 3 is free
-    if (step + 2 < nsteps) fetch(stage == 0 ? 2 : stage - 1);
-
-    const char* As = smem + stage * SBYTES;
-    const char* Bs = As + NPART * ABYTES;
-    ux4 fb[NPART][FN];
+  auto set_seg = [&](int s) {
+    const GemmSeg& S = P.seg[s];
+    const int64_t kb = (int64_t)S.K * EB;
+    set_side((S.vec & 2) != 0, static_cast<const char*>(resolve(src, S.A)),
+             NPART == 2 ? static_cast<const char*>(resolve(src, S.Alo)) : nullptr, S.lda, kb, m0, P.M, CHA, rA, vA, csA,
+             w0A, kmA);
+    set_side((S.vec & 4) != 0, static_cast<const char*>(resolve(src, S.B)),
+             NPART == 2 ? static_cast<const char*>(resolve(src, S.Blo)) : nullptr, S.ldb, kb, n0, P.N, CHB, rB, vB, csB,
+             w0B, kmB);
+    Kb = (int)kb;
+    kend = S.K;
+  };
+  auto fetch_side = [&](int R, int CH, const __amdgpu_buffer_rsrc_t* rs, const unsigned* v, unsigned cs, unsigned w0,
+                        unsigned km, int kb0, char* S) {
+    const bool tail = kb0 + ROWB > Kb;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      unsigned o = v[c];
+      if (tail) o = kb0 + cq * 16 < Kb ? o : OOB;
+      const int so = (int)(w0 + c * cs + (unsigned)kb0 * km);
+#pragma unroll
+      for (int p = 0; p < NPART; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs[p], (lds_void*)(S + p * R * ROWB + (wave + NW * c) * 1024), 16,
+                                                 (int)o, so, 0, 0);
+    }
+  };
+  int s, k0, step0, step1;
+  slice_range<KSTEP>(P, nsteps, slice, nslice, step0, step1, s, k0);
+  auto fetch = [&](char* A, char* B) {
+    fetch_side(BM, CHA, rA, vA, csA, w0A, kmA, k0 * EB, A);
+    fetch_side(BN, CHB, rB, vB, csB, w0B, kmB, k0 * EB, B);
+  };
+  auto read_a = [&](const char* A, int i, ux4 (&f)[NPART]) {
+#pragma unroll
+    for (int p = 0; p < NPART; ++p) f[p] = *reinterpret_cast<const ux4*>(A + p * BM * ROWB + aoff + i * 16 * ROWB);
+  };
+  auto read_b = [&](const char* B, ux4 (&f)[NPART][FN]) {
 #pragma unroll
     for (int p = 0; p < NPART; ++p)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) fb[p][j] = *reinterpret_cast<const ux4*>(Bs + p * BBYTES + boff + j * 16 * ROWB);
+      for (int j = 0; j < FN; ++j) f[p][j] = *reinterpret_cast<const ux4*>(B + p * BN * ROWB + boff + j * 16 * ROWB);
+  };
+  // one product (MODE F32: one of the four k of a chunk) of row block i
+  auto mfma1 = [&](int i, const ux4 (&a)[NPART], const ux4 (&b)[NPART][FN], int part) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      ux4 fa[NPART];
-#pragma unroll
-      for (int p = 0; p < NPART; ++p) fa[p] = *reinterpret_cast<const ux4*>(As + p * ABYTES + aoff + i * 16 * ROWB);
+    for (int j = 0; j < FN; ++j) {
       if constexpr (MODE == M_BF16X3) {
-        const bfx8 ah = __builtin_bit_cast(bfx8, fa[0]);
-        const bfx8 al = __builtin_bit_cast(bfx8, fa[1]);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const bfx8 bh = __builtin_bit_cast(bfx8, fb[0][j]);
-          const bfx8 bl = __builtin_bit_cast(bfx8, fb[1][j]);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, al, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl, ah, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, ah, acc[i][j], 0, 0, 0);
-        }
+        // hi*lo, lo*hi, then hi*hi
+        const bfx8 av = __builtin_bit_cast(bfx8, part == 0 ? a[NPART - 1] : a[0]);
+        const bfx8 bv = __builtin_bit_cast(bfx8, part == 1 ? b[NPART - 1][j] : b[0][j]);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, av, acc[i][j], 0, 0, 0);
       } else {
-#pragma unroll
-        for (int sub = 0; sub < 4; ++sub) {
-          const unsigned int ua = fa[0][sub];
-          const float a = __uint_as_float(ua);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const unsigned int ub = fb[0][j][sub];
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ub), a, acc[i][j], 0, 0, 0);
-          }
-        }
+        const unsigned int ua = a[0][part], ub = b[0][j][part];
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ub), __uint_as_float(ua), acc[i][j], 0, 0, 0);
       }
     }
-    stage = stage == NSTAGE - 1 ? 0 : stage + 1;
+  };
+  constexpr int NPROD = MODE == M_BF16X3 ? 3 : 4;
+  ux4 fa[BIGT ? 2 : FM][NPART], fb[NPART][FN];
+  auto body = [&](const char* A, const char* B, char* An, char* Bn, bool has_next) {
+    if (has_next) {
+      k0 += KSTEP;
+      while (k0 >= kend && s + 1 < P.nseg) {
+        ++s;
+        k0 = 0;
+        set_seg(s);
+      }
+      fetch(An, Bn);
+    }
+    if constexpr (!BIGT) {
+      ux4 na[FM][NPART], nb[NPART][FN];
+#pragma unroll
+      for (int q = 0; q + 1 < NPROD; ++q)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) mfma1(i, fa[i], fb, q);
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+      if (has_next) {
+        read_b(Bn, nb);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) read_a(An, i, na[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i) mfma1(i, fa[i], fb, NPROD - 1);
+#pragma unroll
+      for (int p = 0; p < NPART; ++p) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) fb[p][j] = nb[p][j];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) fa[i][p] = na[i][p];
+      }
+    } else {
+      ux4 nb[NPART][FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        if (i + 1 < FM) {
+          read_a(A, i + 1, fa[(i + 1) & 1]);
+        } else {
+          __builtin_amdgcn_sched_barrier(0);
+          __syncthreads();
+          __builtin_amdgcn_sched_barrier(0);
+          if (has_next) {
+            read_b(Bn, nb);
+            read_a(An, 0, fa[0]);
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < NPROD; ++q) mfma1(i, fa[i & 1], fb, q);
+      }
+#pragma unroll
+      for (int p = 0; p < NPART; ++p)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) fb[p][j] = nb[p][j];
+    }
+  };
+  if (step1 > step0) {
+    set_seg(s);
+    fetch(As0, Bs0);
+    __syncthreads();
+    read_b(Bs0, fb);
+    if constexpr (BIGT) {
+      read_a(As0, 0, fa[0]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) read_a(As0, i, fa[i]);
+    }
+  }
+  for (int step = step0; step < step1; step += 2) {
+    body(As0, Bs0, As1, Bs1, step + 1 < step1);
+    if (step + 1 < step1) body(As1, Bs1, As0, Bs0, step + 2 < step1);
   }
 
-  store_tile<FM, FN>(acc, P.C, P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
+  if (slice < 0)
+    store_tile<FM, FN>(acc, resolve(src, P.C), P.ldc, P.M, P.N, m0 + wm0, n0 + wn0, li, lg, P.alpha, P.beta);
+  else
+    store_partial(acc, src_partial<float>(src, t, slice, BM * BN), wave, lane);
+  }  // units
 }
 
 template <int BM, int BN, int MODE, int VAR>
-mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream, SplitPlan sp = {}, void* ws = nullptr) {
+mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream, SplitPlan sp, void* ws) {
   constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
   GemmBatch b{};
   int total = 0;
@@ -749,7 +473,7 @@ mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream, Spl
       // bit 0: vector loads; bits 1, 2: A, B in the packed panel layout
       gs.vec = 1 | (q.packA ? 2 : 0) | (q.packB ? 4 : 0);
       if (q.packA || q.packB)
-        MK_REQUIRE(VAR == V_BIG2 && ps.M % 256 == 0 && ps.N % 256 == 0 && q.K % 32 == 0, MK_BAD_ARG,
+        MK_REQUIRE(VAR == V_DMA && BM == 256 && ps.M % 256 == 0 && ps.N % 256 == 0 && q.K % 32 == 0, MK_BAD_ARG,
                    "mixed gemm: packed operands need the 256 x 256 kernel, M, N multiples of 256 and K of 32");
     }
     P.tiles_m = (int32_t)cdiv(ps.M, BM);
@@ -762,25 +486,20 @@ mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream, Spl
   b.nprob = nprob;
   b.total_tiles = total;
   if (total == 0) return MK_OK;
-  b.full_tiles = sp.ksplit > 1 && VAR != V_PIPE ? sp.full : total;
+  b.full_tiles = sp.ksplit > 1 ? sp.full : total;
   b.ksplit = b.full_tiles < total ? sp.ksplit : 1;
   b.ws = ws;
   const int tail = total - b.full_tiles, units = b.full_tiles + tail * b.ksplit;
   MK_REQUIRE(tail == 0 || (ws != nullptr && (size_t)tail * b.ksplit * BM * BN * 4 <= GEMM_WS_BYTES), MK_BAD_ARG,
              "mixed gemm: %d tiles split %d ways exceed the workspace", tail, b.ksplit);
   ProfScope prof(MODE == M_BF16X3 ? "gemm_bf16x3" : "gemm_f32", stream);
-  if constexpr (VAR == V_PIPE)
-    hipLaunchKernelGGL((gemm_mixed_pipe_kernel<MODE>), dim3(total), dim3(PNT), 0, stream, b);
-  else if constexpr (VAR == V_BIG)
-    hipLaunchKernelGGL((gemm_mixed_big_kernel<MODE, GemmBatch>), dim3(units), dim3(BNT), 0, stream, b);
-  else if constexpr (VAR == V_BIG2)
-    hipLaunchKernelGGL((gemm_mixed_big2_kernel<MODE, GemmBatch>), dim3(units), dim3(BNT), 0, stream, b);
+  constexpr int WGN = BM == 256 ? 4 : 2;   // waves along N (two along M)
+  if constexpr (VAR == V_DMA)
+    hipLaunchKernelGGL((gemm_mixed_dma_kernel<BM, BN, 2, WGN, MODE, GemmBatch>), dim3(units), dim3(128 * WGN), 0, stream, b);
   else
     hipLaunchKernelGGL((gemm_mixed_kernel<BM, BN, MODE, GemmBatch>), dim3(units), dim3(NT), 0, stream, b);
   MK_CHECK_HIP(hipGetLastError());
   if (tail > 0) {
-    // waves of a tile: 2 x 2 of BM/2 x BN/2, or (256 x 256) 2 x 4 of 128 x 64
-    constexpr int WGN = VAR == V_TILE ? 2 : 4;
     constexpr int NBLK = BM * BN / 256;
     hipLaunchKernelGGL((splitk_reduce_kernel<true, 2, BM / 32, BN / 16 / WGN, WGN, fx4>),
                        dim3((unsigned)cdiv((int64_t)tail * NBLK, 4)), dim3(256), 0, stream, b);
@@ -789,7 +508,7 @@ mk_status launch_mixed(const ProbSpec* probs, int nprob, hipStream_t stream, Spl
   return MK_OK;
 }
 
-// 256 rows of every operand lie within the 32-bit buffer offsets of gemm_mixed_big2_kernel
+// 256 rows of every operand lie within the 32-bit buffer offsets of gemm_mixed_dma_kernel
 template <int MODE>
 bool rows256_fit(const ProbSpec* probs, int nprob) {
   constexpr int64_t EB = MODE == M_BF16X3 ? 2 : 4;
@@ -804,61 +523,54 @@ mk_status dispatch(const ProbSpec* probs, int nprob, hipStream_t stream, void* w
   MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "mixed gemm: too many problems");
   for (int i = 0; i < nprob; ++i)
     MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "mixed gemm: too many segments");
-  constexpr int64_t EB = MODE == M_BF16X3 ? 2 : 4;
-  int64_t tiles256 = 0, tilesp = 0;
-  bool off32 = true;   // buffer offsets of the pipelined kernel are 32-bit
-  for (int i = 0; i < nprob; ++i) {
-    tiles256 += cdiv(probs[i].M, 256) * cdiv(probs[i].N, 256);
-    tilesp += cdiv(probs[i].M, PBM) * cdiv(probs[i].N, PBN);
-    for (int s = 0; s < probs[i].nseg; ++s)
-      off32 = off32 && probs[i].M * probs[i].seg[s].lda * EB < (1ll << 31) &&
-              probs[i].N * probs[i].seg[s].ldb * EB < (1ll << 31);
-  }
-  const int var = variant();
+  constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
+  const bool dma = variant() == V_DMA && rows256_fit<MODE>(probs, nprob);
   bool packed = false;
   for (int i = 0; i < nprob; ++i)
     for (int s = 0; s < probs[i].nseg; ++s) packed = packed || probs[i].seg[s].packA || probs[i].seg[s].packB;
   if (packed) {
-    MK_REQUIRE(var == V_BIG2 && tiles256 >= 256 && rows256_fit<MODE>(probs, nprob), MK_BAD_ARG,
-               "mixed gemm: packed operands are read by the 256 x 256 kernel only");
-    return launch_mixed<256, 256, MODE, V_BIG2>(probs, nprob, stream);
+    MK_REQUIRE(dma, MK_BAD_ARG, "mixed gemm: packed operands are read by the 256 x 256 kernel only");
+    return launch_mixed<256, 256, MODE, V_DMA>(probs, nprob, stream, SplitPlan{}, ws);
   }
-  if (var == V_PIPE && tilesp >= 256 && off32) return launch_mixed<PBM, PBN, MODE, V_PIPE>(probs, nprob, stream);
-  // Measured on 2048 x 2048 x 4096 and 1024 x 2048 x 2048.  The bf16 steps are
-  // short (48 MFMAs of 16 cycles a wave on a 128 x 128 tile), so one step of
-  // prefetch covers little of the load latency and the operand traffic of a
-  // small tile (32 KB a step through the CU's 64 B / cycle) is near its limit:
-  // large tiles cut along K win.  The fp32 steps are 2.7 times longer.
-  static const TileModel m64{64, 64, 64 / (int)EB, MODE == M_BF16X3 ? 0.095 : 0.22,
-                             MODE == M_BF16X3 ? TileModel::Eff{0.18, 0.24, 0.28, 0.30} : TileModel::Eff{0.40, 0.55, 0.60, 0.62},
+  // Measured on 2048 x 2048 x 4096, 1024 x 2048 x 2048 and 1024 x 1024 x 2048.  The
+  // bf16 steps are short (48 MFMAs of 16 cycles a wave on a 128 x 128 tile), so
+  // one step of prefetch covers little of the load latency, and the operand
+  // traffic of a small tile (32 KB a step through the CU's 64 B / cycle) is near
+  // its limit: large tiles cut along K win.  The fp32 steps are 2.7 times longer.
+  static const TileModel m64{64, 64, ROWB / EB, MODE == M_BF16X3 ? 0.095 : 0.22,
+                             MODE == M_BF16X3 ? TileModel::Eff{0.18, 0.33, 0.38, 0.40} : TileModel::Eff{0.47, 0.70, 0.76, 0.78},
                              4, 64 * 64 * 4};
-  static const TileModel m128{128, 128, 64 / (int)EB, MODE == M_BF16X3 ? 0.38 : 0.87,
-                              MODE == M_BF16X3 ? TileModel::Eff{0.32, 0.45, 0.45, 0.45} : TileModel::Eff{0.63, 0.75, 0.75, 0.75},
+  static const TileModel m128{128, 128, ROWB / EB, MODE == M_BF16X3 ? 0.38 : 0.87,
+                              MODE == M_BF16X3 ? TileModel::Eff{0.39, 0.55, 0.55, 0.55} : TileModel::Eff{0.80, 0.84, 0.84, 0.84},
                               2, 128 * 128 * 4};
-  static const TileModel m256{256, 256, 64 / (int)EB, MODE == M_BF16X3 ? 1.5 : 3.5,
-                              MODE == M_BF16X3 ? TileModel::Eff{0.62, 0.62, 0.62, 0.62} : TileModel::Eff{0.82, 0.82, 0.82, 0.82},
+  static const TileModel m256{256, 256, ROWB / EB, MODE == M_BF16X3 ? 1.5 : 3.5,
+                              MODE == M_BF16X3 ? TileModel::Eff{0.60, 0.60, 0.60, 0.60} : TileModel::Eff{0.89, 0.89, 0.89, 0.89},
                               1, 256 * 256 * 4};
   const TileChoice c64 = plan_launch(m64, probs, nprob, ws != nullptr);
   const TileChoice c128 = plan_launch(m128, probs, nprob, ws != nullptr);
-  TileChoice c256 = plan_launch(m256, probs, nprob, ws != nullptr);
-  if (var == V_TILE) c256.us = 1e30;
-  if (c256.us <= c128.us && c256.us <= c64.us) {
-    if (var == V_BIG2 && rows256_fit<MODE>(probs, nprob))
-      return launch_mixed<256, 256, MODE, V_BIG2>(probs, nprob, stream, c256.split, ws);
-    return launch_mixed<256, 256, MODE, V_BIG>(probs, nprob, stream, c256.split, ws);
+  if (!dma) {
+    if (c128.us <= c64.us) return launch_mixed<128, 128, MODE, V_TILE>(probs, nprob, stream, c128.split, ws);
+    return launch_mixed<64, 64, MODE, V_TILE>(probs, nprob, stream, c64.split, ws);
   }
-  if (c128.us <= c64.us) return launch_mixed<128, 128, MODE, V_TILE>(probs, nprob, stream, c128.split, ws);
-  return launch_mixed<64, 64, MODE, V_TILE>(probs, nprob, stream, c64.split, ws);
+  const TileChoice c256 = plan_launch(m256, probs, nprob, ws != nullptr);
+  if (c256.us <= c128.us && c256.us <= c64.us)
+    return launch_mixed<256, 256, MODE, V_DMA>(probs, nprob, stream, c256.split, ws);
+  if (c128.us <= c64.us) return launch_mixed<128, 128, MODE, V_DMA>(probs, nprob, stream, c128.split, ws);
+  return launch_mixed<64, 64, MODE, V_DMA>(probs, nprob, stream, c64.split, ws);
 }
 
 template <int MODE>
 mk_status launch_group(const GemmGroup& g, int kind, int grid, hipStream_t stream) {
   if (g.total_tiles == 0) return MK_OK;
   ProfScope prof(MODE == M_BF16X3 ? "gemm_bf16x3" : "gemm_f32", stream);
-  if (kind == TK_256 && variant() == V_BIG2 && g.rows256_fit)
-    hipLaunchKernelGGL((gemm_mixed_big2_kernel<MODE, GemmGroup>), dim3(grid), dim3(BNT), 0, stream, g);
-  else if (kind == TK_256)
-    hipLaunchKernelGGL((gemm_mixed_big_kernel<MODE, GemmGroup>), dim3(grid), dim3(BNT), 0, stream, g);
+  const bool dma = variant() == V_DMA && g.rows256_fit;
+  MK_REQUIRE(kind != TK_256 || dma, MK_BAD_ARG, "grouped mixed gemm: 256 x 256 tiles need operand rows within 2 GiB");
+  if (kind == TK_256)
+    hipLaunchKernelGGL((gemm_mixed_dma_kernel<256, 256, 2, 4, MODE, GemmGroup>), dim3(grid), dim3(512), 0, stream, g);
+  else if (kind == TK_128 && dma)
+    hipLaunchKernelGGL((gemm_mixed_dma_kernel<128, 128, 2, 2, MODE, GemmGroup>), dim3(grid), dim3(NT), 0, stream, g);
+  else if (dma)
+    hipLaunchKernelGGL((gemm_mixed_dma_kernel<64, 64, 2, 2, MODE, GemmGroup>), dim3(grid), dim3(NT), 0, stream, g);
   else if (kind == TK_128)
     hipLaunchKernelGGL((gemm_mixed_kernel<128, 128, MODE, GemmGroup>), dim3(grid), dim3(NT), 0, stream, g);
   else
@@ -878,9 +590,9 @@ int occ_of(K kern, int threads) {
 
 int mixed_group_grid(int prec, int kind, int total_tiles, int cus) {
   // occupancy is a property of the kernel's resources; the BF16X3 instances are the larger
-  static const int occ[3] = {occ_of(gemm_mixed_kernel<64, 64, M_BF16X3, GemmGroup>, NT),
-                             occ_of(gemm_mixed_kernel<128, 128, M_BF16X3, GemmGroup>, NT),
-                             occ_of(gemm_mixed_big_kernel<M_BF16X3, GemmGroup>, BNT)};
+  static const int occ[3] = {occ_of(gemm_mixed_dma_kernel<64, 64, 2, 2, M_BF16X3, GemmGroup>, NT),
+                             occ_of(gemm_mixed_dma_kernel<128, 128, 2, 2, M_BF16X3, GemmGroup>, NT),
+                             occ_of(gemm_mixed_dma_kernel<256, 256, 2, 4, M_BF16X3, GemmGroup>, 512)};
   (void)prec;
   return (int)std::min<int64_t>(total_tiles, (int64_t)occ[kind] * cus);
 }
@@ -891,8 +603,10 @@ mk_status gemm_mixed_group(const GemmGroup& g, int prec, int kind, int grid, hip
   return launch_group<M_F32>(g, kind, grid, st);
 }
 
+bool mixed_256_ok() { return variant() == V_DMA; }
+
 bool mixed_packed_ok(int64_t M, int64_t N, const int64_t* Ks, int nk) {
-  if (variant() != V_BIG2 || M % 256 || N % 256 || (M / 256) * (N / 256) < 256) return false;
+  if (variant() != V_DMA || M % 256 || N % 256 || (M / 256) * (N / 256) < 256) return false;
   for (int i = 0; i < nk; ++i)
     // a panel (256 rows x K, fp32 the wider) must stay within 32-bit buffer offsets
     if (Ks[i] % 32 || Ks[i] * 4 * 256 >= (1ll << 31)) return false;

@@ -61,9 +61,9 @@ inline TileChoice plan_tile(const TileModel& m, int64_t tiles, int64_t nsteps, b
     for (int s = 2; s <= MAX_KSPLIT && nsteps / s >= MIN_SLICE_STEPS; ++s) {
       // past one round of workgroups a finer cut gains nothing
       if (tail * (s - 1) >= round || (size_t)tail * s * m.part_bytes > GEMM_WS_BYTES) break;
-      // partial tiles written and read back at about 4.5 TB/s
+      // partial tiles written and read back at about 6 TB/s (partly out of the Infinity Cache)
       const double us = base + tile_rounds_us(m, tail * s, (double)cdiv(nsteps, s)) + 4.0 +
-                        2.0 * (double)tail * s * m.part_bytes / 4.5e6;
+                        2.0 * (double)tail * s * m.part_bytes / 6.0e6;
       if (us < best.us) {
         best.us = us;
         best.split.full = (int)full;

@@ -173,6 +173,14 @@ bool large_fp64(const std::vector<ProbSpec>& specs) {
 
 }  // namespace
 
+bool GroupPlan::rows256_fit() const {
+  const int64_t eb = prec == MK_FP32 ? 4 : 2;
+  for (const ProbSpec& p : specs)
+    for (int s = 0; s < p.nseg; ++s)
+      if (256 * std::max(p.seg[s].lda, p.seg[s].ldb) * eb >= (1ll << 31)) return false;
+  return true;
+}
+
 mk_status GroupPlan::run(const void* const base[NBASE], hipStream_t st) const {
   if (total_tiles == 0) return MK_OK;
   if (prec == MK_FP64 && large_fp64(specs)) {
@@ -195,12 +203,8 @@ mk_status GroupPlan::run(const void* const base[NBASE], hipStream_t st) const {
   g.probs = static_cast<const GemmProb*>(dev.ptr);
   g.nprob = nprob;
   g.total_tiles = total_tiles;
-  const int64_t eb = prec == MK_FP32 ? 4 : 2;
   g.f64_buf = f64_buf;
-  g.rows256_fit = 1;
-  for (const ProbSpec& p : specs)
-    for (int s = 0; s < p.nseg; ++s)
-      if (256 * std::max(p.seg[s].lda, p.seg[s].ldb) * eb >= (1ll << 31)) g.rows256_fit = 0;
+  g.rows256_fit = rows256_fit() ? 1 : 0;
   for (int s = 0; s < NBASE; ++s) {
     g.base[s] = static_cast<const char*>(base ? base[s] : nullptr);
     MK_REQUIRE(reinterpret_cast<uintptr_t>(g.base[s]) % 16 == 0, MK_BAD_ARG,
@@ -227,14 +231,16 @@ mk_status group_plan(Ctx* ctx, const ProbSpec* probs, int n, int prec, GemmShape
     rel_out = rel_out && (reinterpret_cast<uint64_t>(p.C) >> 62) != 0;
   }
   if (kind >= 0) return out->build(kind);
-  const int heur = heuristic_kind(out->specs.data(), n, prec);
+  const bool big = prec == MK_FP64 || (mixed_256_ok() && out->rows256_fit());
+  int heur = heuristic_kind(out->specs.data(), n, prec);
+  if (!big && heur == TK_256) heur = TK_128;
   if (!autotune_enabled() || !rel_out || n == 0) return out->build(heur);
 
   const Key key = signature(out->specs, prec, sh, out->flops);
   {
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_cache.find(key);
-    if (it != g_cache.end()) {
+    if (it != g_cache.end() && (it->second != TK_256 || big)) {
       ++g_hits;
       return out->build(it->second);
     }
@@ -256,7 +262,7 @@ mk_status group_plan(Ctx* ctx, const ProbSpec* probs, int n, int prec, GemmShape
   int best = heur;
   float best_ms = 1e30f;
   for (int k = TK_64; k <= TK_256; ++k) {
-    if (!tile_valid(prec, k)) continue;
+    if (!tile_valid(prec, k) || (k == TK_256 && !big)) continue;
     mk_status s = out->build(k, st);
     if (s == MK_OK) s = out->run(base, st);  // warm-up
     if (s == MK_OK && hipEventRecord(e0, st) != hipSuccess) s = MK_HIP_ERROR;

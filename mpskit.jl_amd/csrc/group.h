@@ -20,6 +20,7 @@ namespace mk {
 
 int f64_group_grid(int kind, int total_tiles, int cus);
 int mixed_group_grid(int prec, int kind, int total_tiles, int cus);
+bool mixed_256_ok();   // whether the 256 x 256 mixed kernel may be chosen
 
 struct GroupPlan {
   int prec = MK_FP64;
@@ -30,6 +31,7 @@ struct GroupPlan {
   int grid = 0;
   double flops = 0.0;
   int f64_buf = 0;              // the branch-free FP64 kernel the problems fit (f64_buf_ok; set by build)
+  bool rows256_fit() const;     // 256 rows of every mixed operand span < 2 GiB
   std::vector<ProbSpec> specs;  // problems in launch order (largest per-tile work first)
   DevBuf dev;                   // GemmProb array
   // fill and upload the descriptors for one tile kind; a rebuild first waits for
