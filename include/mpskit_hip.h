@@ -54,7 +54,8 @@ typedef enum mk_status {
 /* Arithmetic used for the bulk contractions of an apply.  FP64 is the
  * reference arithmetic; FP32 runs the GEMMs on FP32 MFMA; BF16X3 splits each
  * float64 operand into bf16 hi+lo and accumulates hi*hi + hi*lo + lo*hi in
- * FP32 on BF16 MFMA.  Inputs and outputs stay float64 in every mode. */
+ * FP32 on BF16 MFMA.  Inputs and outputs stay float64 in every mode.  The
+ * smallest applies, which are all latency, run in FP64 whatever is asked for. */
 typedef enum mk_precision { MK_FP64 = 0, MK_FP32 = 1, MK_BF16X3 = 2 } mk_precision;
 /* bit masks for mk_prepare_* "precisions" arguments */
 #define MK_PREC_FP64 (1 << MK_FP64)

@@ -28,6 +28,16 @@ struct GemmSeg {
   int32_t vec;       // 1 if 16-byte vector loads are legal for A and B
 };
 
+// A physical term added by the epilogue of the small FP64 kernel:
+//   C[r, c] += alpha sum_{h,j} P[b + d1 (e + d2 (h + d1 j))] x[r + sh h + ldx c + sj j]
+// (x at the output block's rows and columns, h = j = 0; P null: none).
+struct GemmPhys {
+  const double* P = nullptr;
+  const double* x = nullptr;
+  int64_t sh = 0, sj = 0, ldx = 0;
+  int32_t b = 0, e = 0, d1 = 0, d2 = 0;
+};
+
 struct GemmProb {
   GemmSeg seg[MAX_SEG];
   int32_t nseg;
@@ -36,6 +46,7 @@ struct GemmProb {
   double* C;
   int64_t ldc;
   double alpha, beta;
+  GemmPhys phys;
 };
 
 // Up to MAX_PROB problems passed by value as the kernel argument.
@@ -107,6 +118,7 @@ struct ProbSpec {
   double* C = nullptr;
   int64_t ldc = 0;
   double alpha = 1.0, beta = 0.0;
+  GemmPhys phys;   // only for launches that gemm_f64_small says yes to
   void add(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t K,
            const void* Alo = nullptr, const void* Blo = nullptr) {
     seg[nseg].A = A; seg[nseg].lda = lda; seg[nseg].B = B; seg[nseg].ldb = ldb;
@@ -132,6 +144,9 @@ constexpr size_t GEMM_WS_BYTES = (size_t)64 << 20;
 // FP64 MFMA path (gemm_f64.hip).  Enqueues on `stream`; `ws` (GEMM_WS_BYTES, or
 // null: no K split) must not be in use by other work than the stream's own.
 mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream, void* ws);
+// Whether the launch is so small that it runs on the kernel that splits K over
+// the wavefronts of a workgroup (the one that takes GemmPhys).
+bool gemm_f64_small(const ProbSpec* probs, int nprob, GemmShape shape, bool ws);
 
 // Mixed paths (gemm_mixed.hip).  Operands are pre-converted and K-contiguous:
 //   A(i,k) = A[i*lda + k], B(k,j) = B[j*ldb + k]  (bf16 hi/lo or fp32),

@@ -629,6 +629,123 @@ void gemm_f64_dma_kernel(Src src) {
   }  // units
 }
 
+// ---------------------------------------------------------------------------
+// Small launches.  With a handful of 64 x 64 tiles the K loop is one serial chain
+// of load latencies.  Here a workgroup takes a 32 x 32 tile and its eight waves an
+// eighth of K each, straight from memory to the MFMA operands (no LDS stage, no
+// barrier until the sums are added), eight slices of four k in flight at a time.
+// Loads are single elements from clamped addresses, zeroed outside the operand,
+// so any size, stride and alignment will do.  The epilogue may add the physical
+// term (GemmPhys), which saves a launch.
+// ---------------------------------------------------------------------------
+constexpr int ST = 32, SW = 8, SG = 4;   // tile, waves, slices loaded together
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(64 * SW) void gemm_f64_small_kernel(GemmBatch src) {
+  __shared__ double red[SW][ST * (ST + 1)];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int t = blockIdx.x;
+  const GemmProb& P = src_prob(src, t);
+  const int u = t - P.tile_start;
+  const int m0 = (u % P.tiles_m) * ST, n0 = (u / P.tiles_m) * ST;
+  const int M = P.M, N = P.N;
+  dx4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = dx4{0.0, 0.0, 0.0, 0.0};
+
+  int total = 0;
+  for (int s = 0; s < P.nseg; ++s) total += (P.seg[s].K + 3) / 4;
+  int g0 = (int)((int64_t)wave * total / SW);
+  const int g1 = (int)((int64_t)(wave + 1) * total / SW);
+  typedef const __attribute__((address_space(1))) double gd;
+  int first = 0;   // slice the segment starts at
+  for (int s = 0; s < P.nseg && g0 < g1; ++s) {
+    const GemmSeg& S = P.seg[s];
+    const int K = S.K, ns = (K + 3) / 4;
+    const int e = min(g1, first + ns) - first;
+    const int64_t sak = TA ? 1 : S.lda, sbk = TB ? S.ldb : 1;
+    gd *pa[2], *pb[2];
+    bool oka[2], okb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = m0 + 16 * i + li, c = n0 + 16 * i + li;
+      oka[i] = r < M;
+      okb[i] = c < N;
+      pa[i] = (gd*)static_cast<const double*>(S.A) + (int64_t)min(r, M - 1) * (TA ? S.lda : 1);
+      pb[i] = (gd*)static_cast<const double*>(S.B) + (int64_t)min(c, N - 1) * (TB ? 1 : S.ldb);
+    }
+    auto load = [&](int g, double (&a)[SG][2], double (&b)[SG][2]) {
+#pragma unroll
+      for (int q = 0; q < SG; ++q) {
+        const int k = 4 * (g + q) + lk, kc = min(k, K - 1);
+        const bool ok = g + q < e && k < K;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const double av = pa[i][kc * sak], bv = pb[i][kc * sbk];
+          a[q][i] = ok && oka[i] ? av : 0.0;
+          b[q][i] = ok && okb[i] ? bv : 0.0;
+        }
+      }
+    };
+    int g = g0 - first;
+    if (g < e) {
+      double a[2][SG][2], b[2][SG][2];
+      load(g, a[0], b[0]);
+      for (int it = 0; g < e; ++it) {
+        auto step = [&](double (&ac)[SG][2], double (&bc)[SG][2], double (&an)[SG][2], double (&bn)[SG][2]) {
+          if (g + SG < e) load(g + SG, an, bn);
+#pragma unroll
+          for (int q = 0; q < SG; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bc[q][j], ac[q][i], acc[i][j], 0, 0, 0);
+          g += SG;
+        };
+        step(a[0], b[0], a[1], b[1]);
+        if (g < e) step(a[1], b[1], a[0], b[0]);
+      }
+      g0 = first + e;
+    }
+    first += ns;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][(16 * j + lk + 4 * r) * (ST + 1) + 16 * i + li] = acc[i][j][r];
+  __syncthreads();
+  gptr_t<double> C = gptr(P.C);
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int r = threadIdx.x % ST, c = threadIdx.x / ST + 16 * q;
+    const int row = m0 + r, col = n0 + c;
+    if (row >= M || col >= N) continue;
+    double v = 0.0;
+#pragma unroll
+    for (int w = 0; w < SW; ++w) v += red[w][c * (ST + 1) + r];
+    if (P.phys.P) {
+      gd* x = (gd*)P.phys.x + row + (int64_t)col * P.phys.ldx;
+      gd* pp = (gd*)P.phys.P + P.phys.b + P.phys.d1 * P.phys.e;
+      double pv = 0.0;
+      for (int j = 0; j < P.phys.d2; ++j)
+        for (int h = 0; h < P.phys.d1; ++h)
+          pv += pp[P.phys.d1 * P.phys.d2 * (h + P.phys.d1 * j)] * x[P.phys.sh * h + P.phys.sj * j];
+      v += pv;
+    }
+    v *= P.alpha;
+    const int64_t o = row + (int64_t)col * P.ldc;
+    if (P.beta != 0.0) v += P.beta * C[o];
+    C[o] = v;
+  }
+}
+
 // Host check of the branch-free kernel's conditions for one problem.
 enum BufFit { BUF_NO = 0, BUF_ODD = 1, BUF_EVEN = 2 };
 template <int BM, int BN>
@@ -704,9 +821,9 @@ void launch_path(BufFit path, GemmShape sh, dim3 grid, dim3 block, hipStream_t s
   else launch4<BM, BN, Src>(sh, grid, block, stream, b);
 }
 
+// One output-tile grid of `BM` x `BN` tiles over the problems.
 template <int BM, int BN>
-mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t stream, SplitPlan sp, void* ws) {
-  GemmBatch b{};
+int fill_batch(const ProbSpec* probs, int nprob, GemmBatch& b) {
   int total = 0;
   for (int i = 0; i < nprob; ++i) {
     const ProbSpec& ps = probs[i];
@@ -735,9 +852,33 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
     P.ldc = ps.ldc;
     P.alpha = ps.alpha;
     P.beta = ps.beta;
+    P.phys = ps.phys;
   }
   b.nprob = nprob;
   b.total_tiles = total;
+  return total;
+}
+
+mk_status launch_small(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t stream) {
+  GemmBatch b{};
+  const int total = fill_batch<ST, ST>(probs, nprob, b);
+  if (total == 0) return MK_OK;
+  b.full_tiles = total;
+  b.ksplit = 1;
+  ProfScope prof("gemm_f64", stream);
+  const dim3 grid(total), block(64 * SW);
+  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_small_kernel<false, false>), grid, block, 0, stream, b);
+  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_small_kernel<true, false>), grid, block, 0, stream, b);
+  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_small_kernel<false, true>), grid, block, 0, stream, b);
+  else hipLaunchKernelGGL((gemm_f64_small_kernel<true, true>), grid, block, 0, stream, b);
+  MK_CHECK_HIP(hipGetLastError());
+  return MK_OK;
+}
+
+template <int BM, int BN>
+mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t stream, SplitPlan sp, void* ws) {
+  GemmBatch b{};
+  const int total = fill_batch<BM, BN>(probs, nprob, b);
   if (total == 0) return MK_OK;
   b.full_tiles = sp.ksplit > 1 ? sp.full : total;
   b.ksplit = sp.ksplit;
@@ -802,15 +943,14 @@ mk_status gemm_f64_group(const GemmGroup& g, int kind, GemmShape sh, int grid, h
   return launch_group<64, 64>(g, sh, grid, st);
 }
 
-mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream, void* ws) {
-  MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "gemm_f64: %d problems (max %d)", nprob, MAX_PROB);
-  for (int i = 0; i < nprob; ++i) {
-    MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "gemm_f64: too many segments");
-    MK_REQUIRE(probs[i].M >= 0 && probs[i].N >= 0 && probs[i].M < (1ll << 31) && probs[i].N < (1ll << 31),
-               MK_BAD_SHAPE, "gemm_f64: bad M/N");
-    for (int s = 0; s < probs[i].nseg; ++s)
-      MK_REQUIRE(probs[i].seg[s].K >= 0 && probs[i].seg[s].K < (1ll << 31), MK_BAD_SHAPE, "gemm_f64: bad K");
-  }
+namespace {
+
+struct F64Plan {
+  bool small = false;
+  TileChoice c128, c64;
+};
+
+F64Plan plan_f64(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
   // One step is 64 (128 tile) or 16 v_mfma_f64_16x16x4 of 64 cycles a wave.
   // Straight to LDS, measured (us): 1024 x 1024 x 2048 with 64 x 64 tiles, 1 and 3
   // workgroups a CU 83 and 83 (split 3 ways, reduction included), 1024 x 8192 x
@@ -825,8 +965,49 @@ mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_
   static const TileModel b64{64, 64, 16, 0.436, {0.53, 0.70, 0.77, 0.79}, 4, 64 * 64 * 8};
   const bool direct = f64_path(f64_buf_ok(probs, nprob, shape, TK_128)) == BUF_EVEN;
   const TileModel& m64 = !direct ? b64 : shape.ta || shape.tb ? d64t : d64;
-  const TileChoice c128 = plan_launch(direct ? d128 : b128, probs, nprob, ws != nullptr);
-  const TileChoice c64 = plan_launch(m64, probs, nprob, ws != nullptr);
+  F64Plan pl;
+  pl.c128 = plan_launch(direct ? d128 : b128, probs, nprob, ws);
+  pl.c64 = plan_launch(m64, probs, nprob, ws);
+  // The small kernel, up to 12 slices a wave (K = 384) on at most one 32 x 32 tile
+  // per CU, where it saves a launch: the reduction of a split one, or that of a
+  // physical term.  Measured with launches (us, the tile kernels beside it, which
+  // split): 128 x 128 x 256 10.8 and 14.3, 192 x 192 x 384 12.4 and 13.6, past the
+  // line 256 x 256 x 512 15.2 and 13.6, 512 x 512 x 1024 31 and 22.
+  int64_t tiles = 0, slices = 0;
+  bool phys = false;
+  for (int i = 0; i < nprob; ++i) {
+    int64_t n = 0;
+    for (int s = 0; s < probs[i].nseg; ++s) n += cdiv(std::max<int64_t>(probs[i].seg[s].K, 0), 4);
+    const int64_t t = cdiv(probs[i].M, ST) * cdiv(probs[i].N, ST);
+    tiles += t;
+    if (t > 0) slices = std::max(slices, n);
+    phys = phys || probs[i].phys.P != nullptr;
+  }
+  const bool split = (pl.c128.us <= pl.c64.us ? pl.c128 : pl.c64).split.ksplit > 1;
+  pl.small = f64_variant() == F64_DMA && tiles <= PLAN_CUS && slices <= 96 && (split || phys);
+  return pl;
+}
+
+}  // namespace
+
+bool gemm_f64_small(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
+  return plan_f64(probs, nprob, shape, ws).small;
+}
+
+mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream, void* ws) {
+  MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "gemm_f64: %d problems (max %d)", nprob, MAX_PROB);
+  for (int i = 0; i < nprob; ++i) {
+    MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "gemm_f64: too many segments");
+    MK_REQUIRE(probs[i].M >= 0 && probs[i].N >= 0 && probs[i].M < (1ll << 31) && probs[i].N < (1ll << 31),
+               MK_BAD_SHAPE, "gemm_f64: bad M/N");
+    for (int s = 0; s < probs[i].nseg; ++s)
+      MK_REQUIRE(probs[i].seg[s].K >= 0 && probs[i].seg[s].K < (1ll << 31), MK_BAD_SHAPE, "gemm_f64: bad K");
+  }
+  const F64Plan pl = plan_f64(probs, nprob, shape, ws != nullptr);
+  if (pl.small) return launch_small(probs, nprob, shape, stream);
+  for (int i = 0; i < nprob; ++i)
+    MK_REQUIRE(probs[i].phys.P == nullptr, MK_BAD_ARG, "gemm_f64: a physical term in a launch that is not small");
+  const TileChoice &c128 = pl.c128, &c64 = pl.c64;
   if (c128.us <= c64.us) return launch_cfg<128, 128>(probs, nprob, shape, stream, c128.split, ws);
   return launch_cfg<64, 64>(probs, nprob, shape, stream, c64.split, ws);
 }

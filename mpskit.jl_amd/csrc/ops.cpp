@@ -290,7 +290,7 @@ mk_status apply_xrl(Op* op, const Xrl& k, const double* x, double* y, double alp
   const int64_t M1 = k.Df * k.d1, K2 = k.Df * k.wl;
   const int d2 = k.d2;
   const bool in_place = f64 && k.wl == k.wr;
-  const size_t vx = f64 ? 0 : align256(view_bytes(M1, k.Di, 'A', prec));
+  const size_t vx = f64 ? 0 : view_bytes(M1, k.Di * d2, 'A', prec, d2);
   auto t1_bytes = [&](int64_t nc) { return (size_t)M1 * k.wr * nc * d2 * 8; };
   auto t2_bytes = [&](int64_t nc) {
     if (in_place) return (size_t)0;
@@ -307,16 +307,15 @@ mk_status apply_xrl(Op* op, const Xrl& k, const double* x, double* y, double alp
                fx.bytes);
   }
   if (fx.base)
-    while (nc > 1 && align256(t1_bytes(nc)) + align256(t2_bytes(nc)) + (int64_t)vx * d2 > (int64_t)fx.bytes)
+    while (nc > 1 && align256(t1_bytes(nc)) + align256(t2_bytes(nc)) + align256(vx) > (int64_t)fx.bytes)
       nc = cdiv(nc, 2);
   double *t1 = nullptr, *t2 = nullptr;
-  char* mx = nullptr;
-  MK_TRY(carve(ctx, {{t1_bytes(nc), (void**)&t1}, {t2_bytes(nc), (void**)&t2}, {vx * d2, (void**)&mx}}));
+  void* mx = nullptr;
+  MK_TRY(carve(ctx, {{t1_bytes(nc), (void**)&t1}, {t2_bytes(nc), (void**)&t2}, {vx, &mx}}));
   if (in_place) t2 = t1;
-  std::vector<MixedView> v((size_t)d2);
-  if (!f64)
-    for (int j = 0; j < d2; ++j)
-      MK_TRY(convert_view(ctx, x + j * M1 * k.Di, M1, k.Di, M1, 'A', prec, &v[j], mx + j * vx));
+  // the views of x_j, rows (f, h), side by side in one conversion: a K run per j
+  MixedView v;
+  if (!f64) MK_TRY(convert_view(ctx, x, M1, k.Di * d2, M1, 'A', prec, &v, mx, d2));
   for (int64_t c0 = 0; c0 < k.Dc; c0 += nc) {
     const int64_t n = std::min(nc, k.Dc - c0);
     for (int j0 = 0; j0 < d2; j0 += MAX_PROB) {
@@ -330,7 +329,10 @@ mk_status apply_xrl(Op* op, const Xrl& k, const double* x, double* y, double alp
         } else {
           const size_t o = (size_t)k.wr * c0 * k.R.kpad * (bf ? 2 : 4);
           const char* r = static_cast<const char*>(bf ? k.R.hi.ptr : k.R.f32.ptr) + o;
-          p[q].add(v[j].hi, v[j].kpad, r, k.R.kpad, k.Di, v[j].lo, bf ? static_cast<const char*>(k.R.lo.ptr) + o : nullptr);
+          const int64_t xo = j * up8(k.Di) * (bf ? 2 : 4);
+          p[q].add(static_cast<const char*>(v.hi) + xo, v.kpad, r, k.R.kpad, k.Di,
+                   bf ? static_cast<const char*>(v.lo) + xo : nullptr,
+                   bf ? static_cast<const char*>(k.R.lo.ptr) + o : nullptr);
         }
       }
       MK_TRY(run_gemm(ctx, p, np, prec, GemmShape{}));
@@ -458,6 +460,36 @@ void jordan_probs(const Op* op, int prec, const JordanViews& v, const void* y, d
 }
 
 namespace {
+
+// The smallest Jordan applies: every output block, its physical term included,
+// in one FP64 launch (gemm_f64_small).  Such an apply is all latency, so the
+// mixed arithmetics, which would convert x in a launch of their own, take the
+// same one: at D = 64 two launches take 14.5 us, mostly on the host, and one 11.
+mk_status apply_small(Op* op, const double* x, double* y, double alpha, double beta, int prec, bool* done) {
+  *done = false;
+  if (op->jprobs.empty() || op->jprobs.size() > MAX_PROB || op->xrl.present() || op->Dl * op->Dr > (1 << 18)) return MK_OK;
+  Ctx* ctx = op->ctx;
+  const int64_t Dl = op->Dl, Dr = op->Dr, M = Dl * op->d1;
+  JordanViews v;
+  v.x = x;
+  std::vector<ProbSpec> probs;
+  jordan_probs(op, MK_FP64, v, y, alpha, beta, probs);
+  if (op->hasP)
+    for (size_t q = 0; q < probs.size(); ++q) {
+      GemmPhys& ph = probs[q].phys;
+      ph.P = static_cast<const double*>(op->P.ptr);
+      ph.x = x;
+      ph.sh = Dl; ph.sj = M * Dr; ph.ldx = M;
+      ph.b = op->jprobs[q].b; ph.e = op->jprobs[q].e;
+      ph.d1 = (int)op->d1; ph.d2 = (int)op->d2;
+    }
+  void* ws = ctx->gemm_ws();
+  if (!gemm_f64_small(probs.data(), (int)probs.size(), GemmShape{}, ws != nullptr)) return MK_OK;
+  MK_TRY(gemm_f64(probs.data(), (int)probs.size(), GemmShape{}, ctx->stream, ws));
+  if (op->has_gen()) MK_TRY(apply_gen(op, x, y, alpha, 1.0, prec));
+  *done = true;
+  return MK_OK;
+}
 
 // By-block Jordan apply: the physical term (and the mixed views of x) in one
 // pass over x, then one launch over the output blocks, which also takes in the
@@ -783,6 +815,9 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
   const int64_t Dl = op->Dl, Dr = op->Dr, d1 = op->d1, d2 = op->d2;
   const int64_t M = Dl * d1, N = Dr * d2;
   BetaSeq bs{beta};
+  bool done = false;
+  MK_TRY(apply_small(op, x, y, alpha, beta, prec, &done));
+  if (done) return MK_OK;
   if (op->by_block()) return apply_by_block(op, x, y, alpha, beta, prec);
   // mixed-precision views of x: as left factor (M x N) and as right factor (K = M rows)
   MixedView xa, xb, xca;
@@ -875,6 +910,9 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
 }
 
 mk_status apply_ac_jordan(Op* op, const double* x, double* y, double alpha, double beta, int prec) {
+  bool done = false;
+  MK_TRY(apply_small(op, x, y, alpha, beta, prec, &done));
+  if (done) return MK_OK;
   if (op->by_block()) return apply_by_block(op, x, y, alpha, beta, prec);
   Ctx* ctx = op->ctx;
   const int64_t Dl = op->Dl, Dr = op->Dr, d = op->d1;
@@ -1463,16 +1501,16 @@ mk_status prepare_ac2_by_block(Op* op, const double* GL, const Wh& A, const Wh& 
     MK_CHECK_HIP(hipStreamSynchronize(st));
     // with every block filled the two products of the whole matrices are the
     // larger, better filled launch
-    if (!full)
-      for (int e = 0; e < 2; ++e)
-        for (int b = 0; b < 2; ++b) {
-          Op::JProb jp{b, e, {}};
-          for (int j = 0; j < 2; ++j)
-            if (nzI[j][e]) jp.seg.push_back({'I', b, j, 0});
-          for (int h = 0; h < 2; ++h)
-            if (nzE[h][b]) jp.seg.push_back({'E', h, e, 0});
-          op->jprobs.push_back(jp);
-        }
+    op->blocks_full = full;
+    for (int e = 0; e < 2; ++e)
+      for (int b = 0; b < 2; ++b) {
+        Op::JProb jp{b, e, {}};
+        for (int j = 0; j < 2; ++j)
+          if (nzI[j][e]) jp.seg.push_back({'I', b, j, 0});
+        for (int h = 0; h < 2; ++h)
+          if (nzE[h][b]) jp.seg.push_back({'E', h, e, 0});
+        op->jprobs.push_back(jp);
+      }
   } else {
     BlockSet R{wr, {}, 0}, L{wl, {}, 0};
     for (int e = 0; e < 2; ++e)

@@ -205,7 +205,10 @@ struct Op {
   std::vector<JProb> jprobs;
   OpMat RB, LB;
   int nR = 0, nL = 0;
-  bool by_block() const { return !jprobs.empty(); }
+  // every block of a nearest-neighbour operator is filled: all but the smallest
+  // applies take IC and BE whole
+  bool blocks_full = false;
+  bool by_block() const { return !jprobs.empty() && !blocks_full; }
   // a two-site operator with terms beyond nearest neighbours
   bool long_range() const { return CA.present() || !AB.empty() || RB.present() || LB.present() || has_gen(); }
 
