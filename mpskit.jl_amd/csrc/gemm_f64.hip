@@ -633,7 +633,7 @@ void gemm_f64_dma_kernel(Src src) {
 // Small launches.  With a handful of 64 x 64 tiles the K loop is one serial chain
 // of load latencies.  Here a workgroup takes a 32 x 32 tile and its eight waves an
 // eighth of K each, straight from memory to the MFMA operands (no LDS stage, no
-// barrier until the sums are added), eight slices of four k in flight at a time.
+// barrier until the sums are added), two groups of four slices of four k in flight.
 // Loads are single elements from clamped addresses, zeroed outside the operand,
 // so any size, stride and alignment will do.  The epilogue may add the physical
 // term (GemmPhys), which saves a launch.
@@ -968,11 +968,14 @@ F64Plan plan_f64(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
   F64Plan pl;
   pl.c128 = plan_launch(direct ? d128 : b128, probs, nprob, ws);
   pl.c64 = plan_launch(m64, probs, nprob, ws);
-  // The small kernel, up to 12 slices a wave (K = 384) on at most one 32 x 32 tile
-  // per CU, where it saves a launch: the reduction of a split one, or that of a
-  // physical term.  Measured with launches (us, the tile kernels beside it, which
-  // split): 128 x 128 x 256 10.8 and 14.3, 192 x 192 x 384 12.4 and 13.6, past the
-  // line 256 x 256 x 512 15.2 and 13.6, 512 x 512 x 1024 31 and 22.
+  // The small kernel, on at most one 32 x 32 tile per CU.  Where it saves the launch
+  // of a physical term, up to 12 slices a wave (K = 384): measured with launches (us,
+  // the tile kernels beside it, which split) 128 x 128 x 256 10.8 and 14.3, 192 x 192
+  // x 384 12.4 and 13.6, past the line 256 x 256 x 512 15.2 and 13.6.  Without one it
+  // gains where the tile kernel goes through registers (odd sizes; up to 8 slices a
+  // wave: one-site apply w = 5 D = 33 9.4 and 12.6, bond apply D = 33 15.4 and 19.2);
+  // elsewhere the two are even up to 4 and it falls behind after (transfer w = 5 D =
+  // 150 36 and 33, bond apply D = 64 20 and 17), so 4 is the line.
   int64_t tiles = 0, slices = 0;
   bool phys = false;
   for (int i = 0; i < nprob; ++i) {
@@ -984,7 +987,8 @@ F64Plan plan_f64(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
     phys = phys || probs[i].phys.P != nullptr;
   }
   const bool split = (pl.c128.us <= pl.c64.us ? pl.c128 : pl.c64).split.ksplit > 1;
-  pl.small = f64_variant() == F64_DMA && tiles <= PLAN_CUS && slices <= 96 && (split || phys);
+  pl.small = f64_variant() == F64_DMA && tiles <= PLAN_CUS &&
+             slices <= (phys ? 96 : direct ? 32 : 64) && (split || phys);
   return pl;
 }
 
