@@ -77,7 +77,7 @@ struct GemmGroup {
   int32_t total_tiles;
   const char* base[NBASE];
   int32_t rows256_fit;   // 256 rows of every mixed operand span < 2 GiB (32-bit buffer offsets)
-  int32_t f64_buf;       // the branch-free FP64 kernel that every problem fits (f64_buf_ok)
+  int32_t f64_buf;       // the FP64 LDS-DMA kernel that every problem fits (f64_buf_ok)
 };
 
 constexpr uint64_t REL_MASK = (1ull << 62) - 1;
@@ -175,7 +175,7 @@ bool tile_valid(int prec, int kind);
 // Workgroups of one persistent launch: resident workgroups per CU x CUs, capped by the tiles.
 int group_grid(int prec, int kind, GemmShape sh, int total_tiles);
 mk_status gemm_f64_group(const GemmGroup& g, int kind, GemmShape sh, int grid, hipStream_t st);
-// Whether the FP64 problems may run on the branch-free (buffer-load) kernel
+// Whether the FP64 problems may run on the LDS-DMA kernel
 // with tile kind `kind` (in-tile offsets below 2 GiB): 0 no, 1 on its form for
 // odd sizes and 8-byte alignment, 2 on the 16-byte aligned one (relative
 // pointers: their offsets; even leading dimensions and K, even row counts for

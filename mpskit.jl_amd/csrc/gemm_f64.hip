@@ -1,6 +1,6 @@
 // FP64 MFMA GEMM for CDNA4 (gfx950): v_mfma_f64_16x16x4_f64, LDS-staged
-// BK = 16 deep tiles, double-buffered (through registers, or straight to LDS in
-// gemm_f64_dma_kernel), 256 threads = 4 waves of 64 lanes in a 2x2
+// BK = 16 deep tiles, double-buffered (straight to LDS in gemm_f64_dma_kernel, the
+// usual one, or through registers), 256 threads = 4 waves of 64 lanes in a 2x2
 // arrangement.  One workgroup computes one BM x BN output tile of one problem, summing every segment of that problem into the same
 // accumulators before a single fused epilogue (alpha/beta and optional CB term).
 #include "gemm_dev.h"
@@ -233,212 +233,14 @@ void gemm_f64_kernel(Src src) {
 }
 
 // ---------------------------------------------------------------------------
-// Same tile, waves, LDS layout and epilogue as gemm_f64_kernel, with
-// a branch-free load path: each operand is read through a buffer resource based
-// at the tile's first row, the per-lane byte offsets of a segment are computed
-// once per segment, and a chunk outside the operand (row past M / N, k past K)
-// gets an offset past num_records, for which the hardware returns zeros.  A K
-// step then issues its eight 16-byte loads with two VALU ops each and no
-// exec-mask branches.  For odd sizes, odd leading dimensions and 8-byte aligned
-// operands (a 16-byte load needs its address aligned to 4 only): the pair that
-// would straddle the end of an odd row range or of an odd K is read one element
-// lower and shifted when it is stored, so no load leaves the operand.  Needs
-// (checked on the host, buf_ok_prob) two elements in each odd range and every
-// in-tile offset below 2 GiB.
-// ---------------------------------------------------------------------------
-constexpr unsigned OOB = 0x80000000u;
-typedef unsigned int ux4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, 0x7fffffff, 0x00020000);
-}
-
-template <int BM, int BN, bool TA, bool TB, class Src>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_f64_buf_kernel(Src src) {
-  constexpr int BK = 16;
-  constexpr int LDA_S = BM + PAD;
-  constexpr int LDB_S = BN + PAD;
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int CHA = BM * BK / 2 / NT;
-  constexpr int CHB = BN * BK / 2 / NT;
-  static_assert(CHA >= 1 && CHB >= 1, "tile too small for 256 threads");
-  // A is K-contiguous when transposed, B when not
-  constexpr bool AK = TA, BKD = !TB;
-
-  __shared__ double As[2][BK][LDA_S];
-  __shared__ double Bs[2][BK][LDB_S];
-
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm0 = (wave & 1) * WM;
-  const int wn0 = (wave >> 1) * WN;
-  const int li = lane & 15;
-  const int lk = lane >> 4;
-
-  for (int un = src_first(src); un < src_units(src); un += src_stride(src)) {
-  int t, slice, nslice;
-  src_unit(src, un, t, slice, nslice);
-  const GemmProb& P = src_prob(src, t);
-  int tm, tn;
-  tile_coords(P, t - P.tile_start, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int M = P.M, N = P.N;
-
-  dx4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = dx4{0.0, 0.0, 0.0, 0.0};
-
-  int nsteps = 0;
-  for (int s = 0; s < P.nseg; ++s) nsteps += (P.seg[s].K + BK - 1) / BK;
-
-  // Chunk c of a thread (the mapping of load_fastdir / load_kdir):
-  //   along rows (R rows): rows r0, r0 + 1 with r0 = 2 (t % (R/2)), depth
-  //     t / (R/2) + c NT / (R/2): one row pair for all c, depth steps uniform;
-  //   along k: row t / 8 + 32 c, depths 2 (t % 8), + 1: one depth pair for
-  //     all c, row steps uniform.
-  // So a segment keeps one byte offset per operand (chunk 0 at k0 = 0, OOB
-  // if its rows lie outside the operand) and uniform strides; the per-chunk
-  // offsets and the bounds tests are formed at each load (per-chunk offset
-  // arrays would hold 16 more registers through the K loop).
-  constexpr int RA2 = BM / 2, RB2 = BN / 2;
-  const int tid = threadIdx.x;
-  __amdgpu_buffer_rsrc_t rA, rB;
-  unsigned oA = 0, oB = 0;         // chunk 0, k0 = 0
-  unsigned cA = 0, cB = 0;         // bytes from chunk c to chunk c + 1
-  unsigned stepA = 0, stepB = 0;   // bytes per unit of k0
-  int K = 0;
-  bool shA = false, shB = false;   // the loaded pairs hold (element before the last, last)
-  auto set_seg = [&](int s) {
-    const GemmSeg& S = P.seg[s];
-    const char* pa = static_cast<const char*>(resolve(src, S.A));
-    const char* pb = static_cast<const char*>(resolve(src, S.B));
-    rA = raw_rsrc(pa + (AK ? (int64_t)m0 * S.lda : (int64_t)m0) * 8);
-    rB = raw_rsrc(pb + (BKD ? (int64_t)n0 * S.ldb : (int64_t)n0) * 8);
-    stepA = AK ? 8u : (unsigned)(S.lda * 8);
-    stepB = BKD ? 8u : (unsigned)(S.ldb * 8);
-    if (AK) {
-      cA = (unsigned)((NT / 8) * S.lda * 8);
-      oA = (unsigned)((2 * (tid % 8) + (int64_t)(tid / 8) * S.lda) * 8);
-    } else {
-      cA = (unsigned)((NT / RA2) * S.lda * 8);
-      oA = m0 + 2 * (tid % RA2) < M ? (unsigned)((2 * (tid % RA2) + (int64_t)(tid / RA2) * S.lda) * 8) : OOB;
-      // the tile's first row is no pair's second, so m0 = M - 1 steps below the base
-      shA = m0 + 2 * (tid % RA2) == M - 1;
-      if (m0 == M - 1) {
-        rA = raw_rsrc(pa + ((int64_t)m0 - 1) * 8);
-        oA = shA ? oA : OOB;
-      } else if (shA) {
-        oA -= 8;
-      }
-    }
-    if (BKD) {
-      cB = (unsigned)((NT / 8) * S.ldb * 8);
-      oB = (unsigned)((2 * (tid % 8) + (int64_t)(tid / 8) * S.ldb) * 8);
-    } else {
-      cB = (unsigned)((NT / RB2) * S.ldb * 8);
-      oB = n0 + 2 * (tid % RB2) < N ? (unsigned)((2 * (tid % RB2) + (int64_t)(tid / RB2) * S.ldb) * 8) : OOB;
-      shB = n0 + 2 * (tid % RB2) == N - 1;
-      if (n0 == N - 1) {
-        rB = raw_rsrc(pb + ((int64_t)n0 - 1) * 8);
-        oB = shB ? oB : OOB;
-      } else if (shB) {
-        oB -= 8;
-      }
-    }
-    K = S.K;
-  };
-
-  dx2 ra[CHA], rb[CHB];
-  auto load = [&](int k0) {
-    // the pair at the end of an odd K (for operands stored along k)
-    const bool last = k0 + 2 * (tid % 8) == K - 1;
-    if (AK) shA = last;
-    if (BKD) shB = last;
-    const unsigned back = last ? 8u : 0u;
-#pragma unroll
-    for (int c = 0; c < CHA; ++c) {
-      bool ok;
-      if (AK) ok = (m0 + tid / 8 + c * (NT / 8) < M) & (k0 + 2 * (tid % 8) < K);
-      else    ok = (oA != OOB) & (k0 + tid / RA2 + c * (NT / RA2) < K);
-      const unsigned o = ok ? oA + (unsigned)c * cA + (unsigned)k0 * stepA - (AK ? back : 0u) : OOB;
-      ra[c] = __builtin_bit_cast(dx2, __builtin_amdgcn_raw_buffer_load_b128(rA, (int)o, 0, 0));
-    }
-#pragma unroll
-    for (int c = 0; c < CHB; ++c) {
-      bool ok;
-      if (BKD) ok = (n0 + tid / 8 + c * (NT / 8) < N) & (k0 + 2 * (tid % 8) < K);
-      else     ok = (oB != OOB) & (k0 + tid / RB2 + c * (NT / RB2) < K);
-      const unsigned o = ok ? oB + (unsigned)c * cB + (unsigned)k0 * stepB - (BKD ? back : 0u) : OOB;
-      rb[c] = __builtin_bit_cast(dx2, __builtin_amdgcn_raw_buffer_load_b128(rB, (int)o, 0, 0));
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int c = 0; c < CHA; ++c) ra[c] = shA ? dx2{ra[c].y, 0.0} : ra[c];
-#pragma unroll
-    for (int c = 0; c < CHB; ++c) rb[c] = shB ? dx2{rb[c].y, 0.0} : rb[c];
-    if (!TA) store_fastdir<BM, LDA_S, BK>(As[buf], ra);
-    else     store_kdir<BM, LDA_S, BK>(As[buf], ra);
-    if (!TB) store_kdir<BN, LDB_S, BK>(Bs[buf], rb);
-    else     store_fastdir<BN, LDB_S, BK>(Bs[buf], rb);
-  };
-
-  int s, k0, step0, step1;
-  slice_range<BK>(P, nsteps, slice, nslice, step0, step1, s, k0);
-  if (step1 > step0) {
-    set_seg(s);
-    load(k0);
-    store(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  for (int step = step0; step < step1; ++step) {
-    k0 += BK;
-    while (k0 >= K && s + 1 < P.nseg) {
-      ++s;
-      k0 = 0;
-      set_seg(s);
-    }
-    const bool has_next = step + 1 < step1;
-    if (has_next) load(k0);
-#pragma unroll
-    for (int kk = 0; kk < BK / 4; ++kk) {
-      double a[FM], b[FN];
-      const int kr = kk * 4 + lk;
-      const int sa = TA ? kswz(kr) : 0;   // K-contiguous operands were stored swizzled
-      const int sb = TB ? 0 : kswz(kr);
-#pragma unroll
-      for (int i = 0; i < FM; ++i) a[i] = As[buf][kr][(wm0 + i * 16 + li) ^ sa];
-#pragma unroll
-      for (int j = 0; j < FN; ++j) b[j] = Bs[buf][kr][(wn0 + j * 16 + li) ^ sb];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
-    }
-    if (has_next) store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-
-  // epilogue: as in gemm_f64_kernel
-  if (slice < 0)
-    epilogue_c<false, FM, FN, dx4, 1>(acc, resolve(src, P.C), P.ldc, M, N, m0 + wm0, n0 + wn0, li, lk, P.alpha, P.beta);
-  else
-    store_partial(acc, src_partial<double>(src, t, slice, BM * BN), wave, lane);
-  }  // units
-}
-
-// ---------------------------------------------------------------------------
 // Operands straight to LDS (buffer_load ... lds, 16 bytes a lane): no staging
 // registers and no LDS stores, so a K step is 8 DMA loads, the fragment reads and
-// the MFMAs.  For 16-byte aligned operands with even leading dimensions, even K
-// and an even row count where rows are contiguous.
+// the MFMAs.  A load needs its address aligned to 4 bytes only, so odd leading
+// dimensions and 8-byte aligned operands will do.  ODD is for those and for odd
+// sizes: the pair that straddles the end of an odd row range or of an odd K is left
+// out of the DMA (the hardware writes zeros) and its one element goes through a
+// register of the same lane, before the step's barrier; no load leaves the operand,
+// and only the workgroups at the edge or in the last step do this.
 //
 // A DMA load writes 1 KB of LDS in lane order, so every swizzle is in which
 // element a lane loads:
@@ -457,10 +259,17 @@ void gemm_f64_buf_kernel(Src src) {
 // Against the kernel that stages through registers (same tiles; MFMA busy 0.86
 // there at 4096 x 4096 x 8192): 4094 -> 3924 us at that shape, 1024 x 8192 x 1024
 // with 64 x 64 tiles 289 -> 261, 1024 x 5120 x 2048 with A transposed 562 -> 507.
+// ODD (us, through registers before): 777 x 4000 x 3885 492 -> 437, with A transposed
+// 496 -> 419; 1023 x 8184 x 1023 292 -> 276; 2047 x 2047 x 4095 592 -> 557.
 // ---------------------------------------------------------------------------
+constexpr unsigned OOB = 0x80000000u;   // past every num_records: the hardware returns zeros
 typedef __attribute__((address_space(3))) void lds_void;
 
-template <int BM, int BN, bool TA, bool TB, class Src>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, 0x7fffffff, 0x00020000);
+}
+
+template <int BM, int BN, bool TA, bool TB, bool ODD, class Src>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f64_dma_kernel(Src src) {
   constexpr int BK = 16;
@@ -505,8 +314,13 @@ void gemm_f64_dma_kernel(Src src) {
   unsigned vA[AK ? CHA : 1], vB[BKD ? CHB : 1];
   unsigned csA = 0, csB = 0, ksA = 0, ksB = 0, w0A = 0, w0B = 0;
   int K = 0;
+  // ODD: element offset of the pair cut by the end of an odd row range, the elements
+  // themselves, and whether this step has any on either side
+  unsigned eA = OOB, eB = OOB;
+  double xA[CHA], xB[CHB];
+  bool fixA = false, fixB = false;
   auto set_side = [&](bool kdir, int R, int CH, const char* p, int64_t ld, int r0, int lim, __amdgpu_buffer_rsrc_t& rs,
-                      unsigned* v, unsigned& cs, unsigned& ks, unsigned& w0) {
+                      unsigned* v, unsigned& cs, unsigned& ks, unsigned& w0, unsigned& e) {
     if (kdir) {
       rs = raw_rsrc(p + (int64_t)r0 * ld * 8);
       ks = 8u;
@@ -525,27 +339,42 @@ void gemm_f64_dma_kernel(Src src) {
       const int kw = kpl * wave;             // (k >> 1) & 1 is that of the wave's first load
       const int row = (2 * (lane % pairs)) ^ (16 * ((kw >> 1) & 1));
       v[0] = r0 + row < lim ? (unsigned)(row * 8 + kl * ld * 8) : OOB;
+      if (ODD) {
+        e = r0 + row == lim - 1 ? v[0] : OOB;
+        v[0] = r0 + row == lim - 1 ? OOB : v[0];
+      }
     }
   };
   auto set_seg = [&](int s) {
     const GemmSeg& S = P.seg[s];
-    set_side(AK, BM, CHA, static_cast<const char*>(resolve(src, S.A)), S.lda, m0, M, rA, vA, csA, ksA, w0A);
-    set_side(BKD, BN, CHB, static_cast<const char*>(resolve(src, S.B)), S.ldb, n0, N, rB, vB, csB, ksB, w0B);
+    set_side(AK, BM, CHA, static_cast<const char*>(resolve(src, S.A)), S.lda, m0, M, rA, vA, csA, ksA, w0A, eA);
+    set_side(BKD, BN, CHB, static_cast<const char*>(resolve(src, S.B)), S.ldb, n0, N, rB, vB, csB, ksB, w0B, eB);
     K = S.K;
   };
   auto fetch_side = [&](bool kdir, int R, int CH, __amdgpu_buffer_rsrc_t rs, const unsigned* v, unsigned cs, unsigned ks,
-                        unsigned w0, int k0, double* S) {
+                        unsigned w0, int k0, double* S, int r0, int lim, unsigned e, double* x, bool& fix) {
     const bool tail = k0 + BK > K;
+    if (ODD) fix = kdir ? tail && (K & 1) : r0 + R > lim && (lim & 1);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      unsigned o = v[kdir ? c : 0];
+      unsigned o = v[kdir ? c : 0], oe = ODD ? kdir ? o : e : OOB;
+      const unsigned so = w0 + c * cs + (unsigned)k0 * ks;
       if (tail) {
-        // K is even, and so are the k of a chunk or of a load's first row
-        const int k = kdir ? 2 * ((lane & 7) ^ (lane >> 3)) : (128 / R) * (wave + 4 * c);
-        o = k0 + k < K ? o : OOB;
+        // with an even K, so are the k of a chunk or of a load's first row
+        const int k = kdir ? 2 * ((lane & 7) ^ (lane >> 3)) : (128 / R) * (wave + 4 * c) + (ODD ? lane / (R / 2) : 0);
+        if (ODD) oe = (kdir ? k0 + k == K - 1 : k0 + k < K) ? oe : OOB;
+        o = k0 + k + (ODD && kdir ? 1 : 0) < K ? o : OOB;
       }
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(S + (wave + 4 * c) * 128), 16, (int)o,
-                                               (int)(w0 + c * cs + (unsigned)k0 * ks), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(S + (wave + 4 * c) * 128), 16, (int)o, (int)so, 0, 0);
+      if (ODD && fix) x[c] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, (int)oe, (int)so, 0));
+    }
+  };
+  // ODD: the elements into the places that their own lane's DMA loads left zero
+  auto mend_side = [&](bool kdir, int CH, double* S, unsigned e, const double* x, int k0) {
+    const bool mine = kdir ? k0 + 2 * ((lane & 7) ^ (lane >> 3)) == K - 1 : e != OOB;
+    if (mine) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) S[(wave + 4 * c) * 128 + 2 * lane] = x[c];
     }
   };
 
@@ -575,8 +404,14 @@ void gemm_f64_dma_kernel(Src src) {
   int s, k0, step0, step1;
   slice_range<BK>(P, nsteps, slice, nslice, step0, step1, s, k0);
   auto fetch = [&](double* A, double* B) {
-    fetch_side(AK, BM, CHA, rA, vA, csA, ksA, w0A, k0, A);
-    fetch_side(BKD, BN, CHB, rB, vB, csB, ksB, w0B, k0, B);
+    fetch_side(AK, BM, CHA, rA, vA, csA, ksA, w0A, k0, A, m0, M, eA, xA, fixA);
+    fetch_side(BKD, BN, CHB, rB, vB, csB, ksB, w0B, k0, B, n0, N, eB, xB, fixB);
+  };
+  auto mend = [&](double* A, double* B) {
+    if (!ODD || !(fixA | fixB)) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (fixA) mend_side(AK, CHA, A, eA, xA, k0);
+    if (fixB) mend_side(BKD, CHB, B, eB, xB, k0);
   };
   auto mfma = [&](int f, int m) {
 #pragma unroll
@@ -601,6 +436,7 @@ void gemm_f64_dma_kernel(Src src) {
     mfma(0, 1);
     mfma(1, 0);
     __builtin_amdgcn_sched_barrier(0);
+    if (has_next) mend(An, Bn);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     if (has_next) {
@@ -612,6 +448,7 @@ void gemm_f64_dma_kernel(Src src) {
   if (step1 > step0) {
     set_seg(s);
     fetch(As0, Bs0);
+    mend(As0, Bs0);
     __syncthreads();
     read_side(AK, BM, FM, As0, wm0, 0, fa[0]);
     read_side(BKD, BN, FN, Bs0, wn0, 0, fb[0]);
@@ -746,7 +583,9 @@ __global__ __launch_bounds__(64 * SW) void gemm_f64_small_kernel(GemmBatch src) 
   }
 }
 
-// Host check of the branch-free kernel's conditions for one problem.
+// Host check of the LDS-DMA kernel's conditions for one problem: every in-tile
+// offset below 2 GiB, 8-byte aligned operands; BUF_ODD unless sizes, leading
+// dimensions and addresses are whole pairs.
 enum BufFit { BUF_NO = 0, BUF_ODD = 1, BUF_EVEN = 2 };
 template <int BM, int BN>
 BufFit buf_ok_prob(const ProbSpec& ps, GemmShape sh) {
@@ -758,52 +597,30 @@ BufFit buf_ok_prob(const ProbSpec& ps, GemmShape sh) {
     const int64_t offA = sh.ta ? (g.K + (int64_t)(BM - 1) * g.lda) * 8 : (BM + (int64_t)(g.K - 1) * g.lda) * 8;
     const int64_t offB = !sh.tb ? (g.K + (int64_t)(BN - 1) * g.ldb) * 8 : (BN + (int64_t)(g.K - 1) * g.ldb) * 8;
     if (offA + 16 >= (1ll << 31) || offB + 16 >= (1ll << 31)) return BUF_NO;
+    if ((uintptr_t)g.A % 8 || (uintptr_t)g.B % 8) return BUF_NO;
     if ((uintptr_t)g.A % 16 || (uintptr_t)g.B % 16 || g.lda % 2 || g.ldb % 2 || g.K % 2 || (!sh.ta && ps.M % 2) ||
-        (sh.tb && ps.N % 2)) {
+        (sh.tb && ps.N % 2))
       fit = BUF_ODD;
-      if ((uintptr_t)g.A % 8 || (uintptr_t)g.B % 8 || ((sh.ta || !sh.tb) && g.K < 2) || (!sh.ta && ps.M < 2) ||
-          (sh.tb && ps.N < 2))
-        return BUF_NO;
-    }
   }
   return fit;
 }
 
-// Load path of the FP64 kernels, read once from MK_F64_VARIANT ("dma", "buf" or
-// "branch"; default "dma"): lets benchmarks and tests pin one of them.
-enum F64Variant { F64_BRANCH = 0, F64_BUF = 1, F64_DMA = 2 };
-int f64_variant() {
-  static const int v = [] {
+// Load path of the FP64 kernels, read once from MK_F64_VARIANT ("dma" or "branch";
+// default "dma"): lets benchmarks and tests pin one of them.
+bool f64_direct() {
+  static const bool v = [] {
     const char* e = getenv("MK_F64_VARIANT");
-    if (e && !strcmp(e, "branch")) return (int)F64_BRANCH;
-    if (e && !strcmp(e, "buf")) return (int)F64_BUF;
-    return (int)F64_DMA;
+    return !(e && !strcmp(e, "branch"));
   }();
   return v;
 }
 
-// The kernel for a launch whose problems fit `fit`: straight to LDS where sizes
-// and alignment allow, else branch-free, else branching.
-BufFit f64_path(int fit) {
-  const int var = f64_variant();
-  if (var == F64_BRANCH || fit == BUF_NO) return BUF_NO;
-  return var == F64_BUF ? BUF_ODD : (BufFit)fit;
-}
-
-template <int BM, int BN, class Src>
+template <int BM, int BN, bool ODD, class Src>
 void launch4_dma(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
-  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, false, false, Src>), grid, block, 0, stream, b);
-  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, true, false, Src>), grid, block, 0, stream, b);
-  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, false, true, Src>), grid, block, 0, stream, b);
-  else hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, true, true, Src>), grid, block, 0, stream, b);
-}
-
-template <int BM, int BN, class Src>
-void launch4_buf(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
-  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, false, Src>), grid, block, 0, stream, b);
-  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, false, Src>), grid, block, 0, stream, b);
-  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, false, true, Src>), grid, block, 0, stream, b);
-  else hipLaunchKernelGGL((gemm_f64_buf_kernel<BM, BN, true, true, Src>), grid, block, 0, stream, b);
+  if (!sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, false, false, ODD, Src>), grid, block, 0, stream, b);
+  else if (sh.ta && !sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, true, false, ODD, Src>), grid, block, 0, stream, b);
+  else if (!sh.ta && sh.tb) hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, false, true, ODD, Src>), grid, block, 0, stream, b);
+  else hipLaunchKernelGGL((gemm_f64_dma_kernel<BM, BN, true, true, ODD, Src>), grid, block, 0, stream, b);
 }
 
 template <int BM, int BN, class Src>
@@ -815,9 +632,9 @@ void launch4(GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src&
 }
 
 template <int BM, int BN, class Src>
-void launch_path(BufFit path, GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
-  if (path == BUF_EVEN) launch4_dma<BM, BN, Src>(sh, grid, block, stream, b);
-  else if (path == BUF_ODD) launch4_buf<BM, BN, Src>(sh, grid, block, stream, b);
+void launch_path(int fit, GemmShape sh, dim3 grid, dim3 block, hipStream_t stream, const Src& b) {
+  if (f64_direct() && fit == BUF_EVEN) launch4_dma<BM, BN, false, Src>(sh, grid, block, stream, b);
+  else if (f64_direct() && fit == BUF_ODD) launch4_dma<BM, BN, true, Src>(sh, grid, block, stream, b);
   else launch4<BM, BN, Src>(sh, grid, block, stream, b);
 }
 
@@ -890,7 +707,7 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
   for (int i = 0; i < nprob && fit != BUF_NO; ++i) fit = std::min<int>(fit, buf_ok_prob<BM, BN>(probs[i], sh));
   dim3 grid(b.full_tiles + tail * b.ksplit), block(NT);
   ProfScope prof("gemm_f64", stream);
-  launch_path<BM, BN>(f64_path(fit), sh, grid, block, stream, b);
+  launch_path<BM, BN>(fit, sh, grid, block, stream, b);
   MK_CHECK_HIP(hipGetLastError());
   if (tail > 0) {
     constexpr int NBLK = BM * BN / 256;
@@ -906,7 +723,7 @@ mk_status launch_group(const GemmGroup& g, GemmShape sh, int grid, hipStream_t s
   if (g.total_tiles == 0) return MK_OK;
   dim3 gr(grid), block(NT);
   ProfScope prof("gemm_f64", stream);
-  launch_path<BM, BN>(f64_path(g.f64_buf), sh, gr, block, stream, g);
+  launch_path<BM, BN>(g.f64_buf, sh, gr, block, stream, g);
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
 }
@@ -955,15 +772,15 @@ F64Plan plan_f64(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
   // Straight to LDS, measured (us): 1024 x 1024 x 2048 with 64 x 64 tiles, 1 and 3
   // workgroups a CU 83 and 83 (split 3 ways, reduction included), 1024 x 8192 x
   // 1024 8 rounds of 64 tiles 261, 2 of 128 tiles 255; 1024 x 5120 x 2048 with A
-  // transposed 374 (64 tiles) and 331 (256 tiles of 128, 64 split 8 ways).  Through
-  // registers (odd sizes): 1024 x 1024 x 8192, 64 tiles 1, 2, 3, 4 a CU 419, 331,
-  // 305, 298, 128 tiles 1, 2 a CU 309, 279.
+  // transposed 374 (64 tiles) and 331 (256 tiles of 128, 64 split 8 ways).  Odd
+  // sizes: 1023 x 1023 x 8191, 64 tiles 1, 2, 3, 4 a CU 431, 337, 306, 295, 128 tiles
+  // 1, 2 a CU 312, 291; 2047 x 2047 x 4095, 64 tiles 562, 128 tiles 600 (split 561).
   static const TileModel d128{128, 128, 16, 1.74, {0.88, 0.90, 0.90, 0.90}, 2, 128 * 128 * 8};
   static const TileModel d64{64, 64, 16, 0.436, {0.70, 0.83, 0.87, 0.88}, 4, 64 * 64 * 8};
   static const TileModel d64t{64, 64, 16, 0.436, {0.62, 0.73, 0.77, 0.78}, 4, 64 * 64 * 8};
-  static const TileModel b128{128, 128, 16, 1.74, {0.76, 0.87, 0.87, 0.87}, 2, 128 * 128 * 8};
-  static const TileModel b64{64, 64, 16, 0.436, {0.53, 0.70, 0.77, 0.79}, 4, 64 * 64 * 8};
-  const bool direct = f64_path(f64_buf_ok(probs, nprob, shape, TK_128)) == BUF_EVEN;
+  static const TileModel b128{128, 128, 16, 1.74, {0.74, 0.82, 0.82, 0.82}, 2, 128 * 128 * 8};
+  static const TileModel b64{64, 64, 16, 0.436, {0.52, 0.68, 0.75, 0.79}, 4, 64 * 64 * 8};
+  const bool direct = f64_direct() && f64_buf_ok(probs, nprob, shape, TK_128) == BUF_EVEN;
   const TileModel& m64 = !direct ? b64 : shape.ta || shape.tb ? d64t : d64;
   F64Plan pl;
   pl.c128 = plan_launch(direct ? d128 : b128, probs, nprob, ws);
@@ -972,10 +789,10 @@ F64Plan plan_f64(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
   // of a physical term, up to 12 slices a wave (K = 384): measured with launches (us,
   // the tile kernels beside it, which split) 128 x 128 x 256 10.8 and 14.3, 192 x 192
   // x 384 12.4 and 13.6, past the line 256 x 256 x 512 15.2 and 13.6.  Without one it
-  // gains where the tile kernel goes through registers (odd sizes; up to 8 slices a
-  // wave: one-site apply w = 5 D = 33 9.4 and 12.6, bond apply D = 33 15.4 and 19.2);
-  // elsewhere the two are even up to 4 and it falls behind after (transfer w = 5 D =
-  // 150 36 and 33, bond apply D = 64 20 and 17), so 4 is the line.
+  // gains at odd sizes, whose tile kernel is the slower (up to 8 slices a wave: one-
+  // site apply w = 5 D = 33 9.4 and 12.6, bond apply D = 33 15.4 and 19.2); elsewhere
+  // the two are even up to 4 and it falls behind after (transfer w = 5 D = 150 36 and
+  // 33, bond apply D = 64 20 and 17), so 4 is the line.
   int64_t tiles = 0, slices = 0;
   bool phys = false;
   for (int i = 0; i < nprob; ++i) {
@@ -987,7 +804,7 @@ F64Plan plan_f64(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) {
     phys = phys || probs[i].phys.P != nullptr;
   }
   const bool split = (pl.c128.us <= pl.c64.us ? pl.c128 : pl.c64).split.ksplit > 1;
-  pl.small = f64_variant() == F64_DMA && tiles <= PLAN_CUS &&
+  pl.small = f64_direct() && tiles <= PLAN_CUS &&
              slices <= (phys ? 96 : direct ? 32 : 64) && (split || phys);
   return pl;
 }

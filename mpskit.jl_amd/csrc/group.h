@@ -30,7 +30,7 @@ struct GroupPlan {
   int total_tiles = 0;
   int grid = 0;
   double flops = 0.0;
-  int f64_buf = 0;              // the branch-free FP64 kernel the problems fit (f64_buf_ok; set by build)
+  int f64_buf = 0;              // the FP64 LDS-DMA kernel the problems fit (f64_buf_ok; set by build)
   bool rows256_fit() const;     // 256 rows of every mixed operand span < 2 GiB
   std::vector<ProbSpec> specs;  // problems in launch order (largest per-tile work first)
   DevBuf dev;                   // GemmProb array

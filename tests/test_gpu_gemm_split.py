@@ -35,7 +35,7 @@ def bound(prec, K):
 @pytest.mark.parametrize("M,N,K", [(64, 64, 4096), (1, 1, 5000), (130, 70, 4100), (129, 1, 1031), (777, 1001, 3001),
                                    (1024, 1024, 2048), (640, 512, 8190), (2176, 2048, 1026), (5120, 2048, 520),
                                    # odd row counts and K: pairs that straddle the end of a tile, a tile of one row
-                                   (2, 3, 5), (65, 63, 3),
+                                   (2, 3, 5), (65, 63, 3), (1, 1, 1), (127, 129, 17), (129, 65, 1025),
                                    # K split over the waves of a workgroup, and just past its line
                                    (31, 33, 253), (31, 33, 257), (98, 162, 128), (130, 70, 130), (129, 257, 33), (193, 129, 129), (1153, 1025, 257)])
 @pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
