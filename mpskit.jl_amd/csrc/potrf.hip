@@ -1,14 +1,12 @@
 // Blocked Cholesky factorisation A = L L^T of a symmetric positive definite
 // float64 matrix (column-major, lower triangle used), for the Cholesky QR of
-// the gauge steps.  A 64-column step is two small kernels and an MFMA GEMM:
-// the diagonal block is factored and inverted (L11^-1) by one workgroup; the
-// panel below it is then the product L21 = A21 L11^-T, in place, and the
-// trailing update A22 -= L21 L21^T the GEMM (the inverted diagonal block turns
-// the row-serial triangular solve into a parallel product, as GPU Cholesky
-// codes commonly do).
+// the gauge steps.  A 64-column step is one launch: the panel below the factored
+// diagonal block is L21 = A21 L11^-T, the trailing update A22 -= L21 L21^T, and the
+// first block of what is left is factored and inverted beside the rest of the update
+// (the inverted diagonal block turns the row-serial triangular solve into a parallel
+// product, as GPU Cholesky codes commonly do).
 #include <algorithm>
 
-#include "gemm.h"
 #include "kernels.h"
 #include "ops.h"
 
@@ -46,7 +44,8 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Factor the nb x nb diagonal block at (k0, k0) and invert the factor.  What
+// Factor the nb x nb diagonal block at (k0, k0), which the workgroup holds in S
+// (lower triangle, identity outside nb), and invert the factor.  What
 // bounds it is the serial chain of the 64 pivots.  The block goes through in 16
 // columns at a time: wave 0 keeps a row of them per lane and factors them
 // without a barrier (pivots and column entries pass between lanes by
@@ -58,23 +57,12 @@ __device__ __forceinline__ void wave_lds_fence() {
 // A non-positive or non-finite pivot sets *info = k0 + j + 1 (LAPACK's
 // convention) and nothing more is written.  Writes L11 (zeros above the
 // diagonal) into A and L11^-1 into Linv (ld NB, zeros above the diagonal);
-// columns nb and on are those of the identity.
-__global__ __launch_bounds__(PT) void potrf_diag_kernel(double* __restrict__ A, int64_t lda, int k0, int nb,
-                                                        double* __restrict__ Linv, int* __restrict__ info) {
-  __shared__ double S[NB * LD];    // the block, then its factor: S[r LD + c]
-  __shared__ double X[NB * LD];    // the inverse
-  __shared__ double T[3][SB * (SB + 1)];
-  __shared__ int bad;
+// columns nb and on are those of the identity.  S and X: S[r LD + c], X zero;
+// the caller's writes to them are its own threads' (the barrier is here).
+__device__ void factor_block(double* S, double* X, double (*T)[SB * (SB + 1)], int* bad, gdouble* gA, int64_t lda, int k0,
+                             int nb, double* __restrict__ Linv, int* __restrict__ info) {
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, li = lane & 15, lq = lane >> 4;
-  gdouble* gA = (gdouble*)A;
-  if (*(volatile int*)info != 0) return;   // an earlier block failed
-  if (t == 0) bad = 0;
-#pragma unroll
-  for (int q = 0; q < NB * NB / PT; ++q) {
-    const int c = wave + 4 * q, r = lane;
-    S[r * LD + c] = (r < nb && c <= r) ? gA[(int64_t)(k0 + r) + (int64_t)(k0 + c) * lda] : (r == c ? 1.0 : 0.0);
-    X[r * LD + c] = 0.0;
-  }
+  if (t == 0) *bad = 0;
   __syncthreads();
   for (int p = 0; p < NB / SB; ++p) {
     if (wave == 0) {
@@ -94,11 +82,11 @@ __global__ __launch_bounds__(PT) void potrf_diag_kernel(double* __restrict__ A, 
       }
 #pragma unroll
       for (int c = 0; c < SB; ++c) S[lane * LD + p * SB + c] = a[c];
-      if (lane == 0 && b != 0) bad = b;
+      if (lane == 0 && b != 0) *bad = b;
     }
     __syncthreads();
-    if (bad != 0) {
-      if (t == 0) *info = k0 + bad;
+    if (*bad != 0) {
+      if (t == 0) *info = k0 + *bad;
       return;
     }
     // blocks (rb, cb), p < cb <= rb, of the rest: S -= L_rb L_cb^T
@@ -163,47 +151,141 @@ __global__ __launch_bounds__(PT) void potrf_diag_kernel(double* __restrict__ A, 
   }
 }
 
-// L21 = A21 L11^-T in place for the m rows below a full (64-column) diagonal
-// block: a workgroup takes 64 rows, a wave 16 of them, so every row is read by
-// the workgroup that writes it.  Bounded by launch and one round trip to memory
-// (10 MFMAs a 16 x 16 block at most: the zero blocks of L11^-1 are left out).
-__global__ __launch_bounds__(PT) void potrf_panel_kernel(double* __restrict__ A21, int64_t lda, int64_t m,
-                                                         const double* __restrict__ Linv,
-                                                         const int* __restrict__ info) {
-  __shared__ double Rs[NB * LD];   // Rs[k LD + r] = A21(r, k)
-  __shared__ double Ls[NB * LD];   // Ls[j LD + k] = L11^-1(j, k)
+// One step of the factorisation in one launch, for the trailing matrix below and
+// right of the full diagonal block at (k0, k0), whose inverted factor is Linv: a
+// workgroup per 64 x 64 tile (i, j) of its lower triangle forms the panel blocks
+// L_ik = A_ik Linv^T and L_jk itself (the same products in every workgroup of a row,
+// on CUs that would idle) and subtracts L_ik L_jk^T; the first tile's workgroup
+// goes on to factor it, so the next step's pivot chain runs beside the rest of the
+// update.  As others still read A_ik, the workgroups of the first column leave L_ik
+// transposed above the diagonal, whence potrf_finish_kernel takes it.  k0 < 0: only
+// the first block is factored.  Bounded by the pivot chain of one workgroup, 16 of
+// them at n = 1024.  Against a launch each for block, panel and update (the GEMM;
+// us, with the copy of info): n = 512 340 -> 297, 1024 651 -> 557, 2048 1404 -> 1110,
+// 4096 3883 -> 3822.
+__global__ __launch_bounds__(PT) void potrf_step_kernel(double* __restrict__ A, int64_t lda, int64_t n, int k0,
+                                                        const double* __restrict__ Linv, double* __restrict__ Lnext,
+                                                        int* __restrict__ info) {
+  __shared__ double Ri[NB * LD];   // Ri[k LD + r] = A_ik(r, k), then L_ik; the factor of the first tile
+  __shared__ double Rj[NB * LD];
+  __shared__ double Ls[NB * LD];   // Ls[j LD + k] = Linv(j, k); the inverse
+  __shared__ double T[3][SB * (SB + 1)];
+  __shared__ int bad;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, li = lane & 15, lq = lane >> 4;
-  if (*(volatile const int*)info != 0) return;
-  const int64_t r0 = (int64_t)blockIdx.x * NB;
-  gdouble* gA = (gdouble*)A21;
-  const gdouble* gL = (const gdouble*)Linv;
-#pragma unroll
-  for (int q = 0; q < NB * NB / PT; ++q) {
-    const int k = wave + 4 * q;
-    Rs[k * LD + lane] = r0 + lane < m ? gA[r0 + lane + (int64_t)k * lda] : 0.0;
-    Ls[lane * LD + k] = gL[lane + k * NB];
+  if (__syncthreads_or(*(volatile const int*)info != 0)) return;   // an earlier block failed
+  gdouble* gA = (gdouble*)A;
+  const int64_t b0 = k0 < 0 ? 0 : k0 + NB, m = n - b0;   // the trailing matrix
+  int i = 0, j = 0;
+  if (k0 >= 0) {
+    // tiles by columns of the triangle: (0, 0), (1, 0), ..., (1, 1), ...
+    int u = blockIdx.x;
+    for (int h = (int)((m + NB - 1) / NB); u >= h; --h, ++j) u -= h;
+    i = j + u;
   }
-  __syncthreads();
-  const int64_t row = r0 + wave * SB + li;
+  const int64_t ri = (int64_t)i * NB, rj = (int64_t)j * NB;
+  gdouble* gC = gA + (b0 + ri) + (b0 + rj) * lda;
+  dx4 acc[NB / SB];
 #pragma unroll
-  for (int jb = 0; jb < NB / SB; ++jb) {
-    dx4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int jb = 0; jb < NB / SB; ++jb) acc[jb] = dx4{0.0, 0.0, 0.0, 0.0};
+  double c[NB / SB][4];   // lane's entries: row 16 wave + li, columns 16 jb + lq + 4 r
+  const int row = wave * SB + li;
 #pragma unroll
-    for (int kb = 0; kb <= jb; ++kb)
-      mm16(acc, Ls + jb * SB * LD + kb * SB, LD, 1, Rs + kb * SB * LD + wave * SB, LD, 1, li, lq);
-    if (row < m) {
+  for (int jb = 0; jb < NB / SB; ++jb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) gA[row + (int64_t)(jb * SB + lq + 4 * r) * lda] = acc[r];
+    for (int r = 0; r < 4; ++r) {
+      const int col = jb * SB + lq + 4 * r;
+      c[jb][r] = ri + row < m && rj + col < m ? gC[row + (int64_t)col * lda] : 0.0;
     }
+  if (k0 >= 0) {
+    const gdouble* gL = (const gdouble*)Linv;
+    gdouble* gP = gA + b0 + (int64_t)k0 * lda;   // the raw panel
+#pragma unroll
+    for (int q = 0; q < NB * NB / PT; ++q) {
+      const int k = wave + 4 * q;
+      Ri[k * LD + lane] = ri + lane < m ? gP[ri + lane + (int64_t)k * lda] : 0.0;
+      if (i != j) Rj[k * LD + lane] = rj + lane < m ? gP[rj + lane + (int64_t)k * lda] : 0.0;
+      Ls[lane * LD + k] = gL[lane + k * NB];
+    }
+    __syncthreads();
+    // a wave's 16 rows of the panel block, in place
+    auto panel = [&](double* R) {
+      dx4 p[NB / SB];
+#pragma unroll
+      for (int jb = 0; jb < NB / SB; ++jb) {
+        p[jb] = dx4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int kb = 0; kb <= jb; ++kb)
+          mm16(p[jb], Ls + jb * SB * LD + kb * SB, LD, 1, R + kb * SB * LD + wave * SB, LD, 1, li, lq);
+      }
+      wave_lds_fence();
+#pragma unroll
+      for (int jb = 0; jb < NB / SB; ++jb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) R[(jb * SB + lq + 4 * r) * LD + row] = p[jb][r];
+    };
+    panel(Ri);
+    if (i != j) panel(Rj);
+    __syncthreads();
+    if (j == 0) {
+#pragma unroll
+      for (int q = 0; q < NB * NB / PT; ++q) {
+        const int r = wave + 4 * q;
+        if (ri + r < m) gA[k0 + lane + (b0 + ri + r) * lda] = Ri[lane * LD + r];
+      }
+    }
+    const double* L = i == j ? Ri : Rj;
+#pragma unroll
+    for (int kb = 0; kb < NB / SB; ++kb)
+#pragma unroll
+      for (int jb = 0; jb < NB / SB; ++jb)
+        mm16(acc[jb], L + kb * SB * LD + jb * SB, 1, LD, Ri + kb * SB * LD + wave * SB, LD, 1, li, lq);
   }
+  if (i + j > 0) {
+#pragma unroll
+    for (int jb = 0; jb < NB / SB; ++jb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = jb * SB + lq + 4 * r;
+        if (ri + row < m && rj + col < m) gC[row + (int64_t)col * lda] = c[jb][r] - acc[jb][r];
+      }
+    return;
+  }
+  const int nb = (int)min((int64_t)NB, m);
+  __syncthreads();   // Ri and Ls have been read
+#pragma unroll
+  for (int jb = 0; jb < NB / SB; ++jb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int col = jb * SB + lq + 4 * r;
+      Ri[row * LD + col] = row < nb && col <= row ? c[jb][r] - acc[jb][r] : (row == col ? 1.0 : 0.0);
+      Ls[row * LD + col] = 0.0;
+    }
+  factor_block(Ri, Ls, T, &bad, gA, lda, (int)b0, nb, Lnext, info);
 }
 
-// Zero the strict upper triangle of the first n columns (the factor is L).
-__global__ void zero_upper_kernel(double* __restrict__ A, int64_t lda, int64_t n) {
+// The block row of L^T that the steps left above each diagonal block, to its place
+// below it, and zeros above (a workgroup per 64 x 64 block below the diagonal;
+// grid: first, second block index).
+__global__ __launch_bounds__(PT) void potrf_finish_kernel(double* __restrict__ A, int64_t lda, int64_t n) {
+  __shared__ double S[NB * LD];
+  if (blockIdx.x <= blockIdx.y) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t r0 = (int64_t)blockIdx.x * NB, c0 = (int64_t)blockIdx.y * NB;   // c0 + NB <= r0 < n
   gdouble* gA = (gdouble*)A;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n * n; e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = e % n, c = e / n;
-    if (r < c) gA[r + c * lda] = 0.0;
+#pragma unroll
+  for (int q = 0; q < NB * NB / PT; ++q) {
+    const int r = wave + 4 * q;
+    if (r0 + r < n) {
+      gdouble* p = gA + c0 + lane + (r0 + r) * lda;
+      S[r * LD + lane] = *p;
+      *p = 0.0;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NB * NB / PT; ++q) {
+    const int c = wave + 4 * q;
+    if (r0 + lane < n) gA[r0 + lane + (c0 + c) * lda] = S[lane * LD + c];
   }
 }
 
@@ -214,30 +296,14 @@ mk_status potrf_lower(double* A, int64_t n, int64_t lda, int* info_dev, double* 
              (long long)lda);
   MK_REQUIRE(n < (1 << 30), MK_BAD_SHAPE, "potrf: n %lld too large", (long long)n);
   if (n == 0) return MK_OK;
-  for (int64_t k0 = 0; k0 < n; k0 += NB) {
-    const int nb = (int)std::min<int64_t>(NB, n - k0);
-    hipLaunchKernelGGL(potrf_diag_kernel, dim3(1), dim3(PT), 0, st, A, lda, (int)k0, nb, Linv, info_dev);
+  for (int64_t k0 = -NB; k0 + NB < n; k0 += NB) {
+    const int64_t nt = k0 < 0 ? 1 : cdiv(n - k0 - NB, (int64_t)NB), odd = (k0 / NB) & 1;
+    hipLaunchKernelGGL(potrf_step_kernel, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(PT), 0, st, A, lda, n, (int)k0,
+                       Linv + odd * NB * NB, Linv + (1 - odd) * NB * NB, info_dev);
     MK_CHECK_HIP(hipGetLastError());
-    const int64_t m = n - k0 - nb;
-    if (m <= 0) break;
-    double* A21 = A + (k0 + nb) + k0 * lda;
-    hipLaunchKernelGGL(potrf_panel_kernel, dim3((unsigned)cdiv(m, (int64_t)NB)), dim3(PT), 0, st, A21, lda, m, Linv,
-                       info_dev);
-    MK_CHECK_HIP(hipGetLastError());
-    // A22 -= L21 L21^T (full square; the strict upper part is zeroed at the end)
-    ProbSpec p;
-    p.M = m; p.N = m;
-    p.C = A + (k0 + nb) + (k0 + nb) * lda;
-    p.ldc = lda;
-    p.alpha = -1.0;
-    p.beta = 1.0;
-    p.add(A21, lda, A21, lda, nb);
-    GemmShape tb;
-    tb.tb = true;   // B(k, j) = A21[j + k lda] = L21(j, k)
-    MK_TRY(gemm_f64(&p, 1, tb, st, nullptr));
   }
-  hipLaunchKernelGGL(zero_upper_kernel, dim3((unsigned)std::min<int64_t>(cdiv(n * n, (int64_t)256), 4096)), dim3(256),
-                     0, st, A, lda, n);
+  const unsigned nblk = (unsigned)cdiv(n, (int64_t)NB);
+  if (nblk > 1) hipLaunchKernelGGL(potrf_finish_kernel, dim3(nblk, nblk), dim3(PT), 0, st, A, lda, n);
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
 }
@@ -254,8 +320,8 @@ extern "C" mk_status mk_potrf(mk_ctx h, double* A, int64_t n, int64_t lda, int* 
   void* mem = nullptr;
   MK_TRY(ctx->small(256, &mem));
   int* dinfo = static_cast<int*>(mem);
-  double* Linv = nullptr;   // inverted diagonal block
-  MK_TRY(carve(ctx, {{(size_t)NB * NB * 8, (void**)&Linv}}));
+  double* Linv = nullptr;   // inverted diagonal blocks, this step's and the next's
+  MK_TRY(carve(ctx, {{(size_t)2 * NB * NB * 8, (void**)&Linv}}));
   MK_CHECK_HIP(hipMemsetAsync(dinfo, 0, sizeof(int), st));
   MK_TRY(potrf_lower(A, n, lda, dinfo, Linv, st));
   MK_CHECK_HIP(hipMemcpyAsync(info, dinfo, sizeof(int), hipMemcpyDeviceToHost, st));
