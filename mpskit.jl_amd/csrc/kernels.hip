@@ -182,7 +182,10 @@ __global__ void env_channels_last_kernel(const double* __restrict__ src, int64_t
 // column (m, c) holds the NIN >= d wl inputs that meet the MPO tensor there in
 // registers, so t1 is read and t2 written once (memory-bound: a thread per
 // output, which re-read its inputs through the caches and divided the index
-// four times, ran at 2.1 TB/s of such traffic at D = 1024, w = 5).
+// four times, ran at 2.1 TB/s of such traffic at D = 1024, w = 5).  Where the
+// threads are few the outputs are dealt out over blockIdx.y: there it is latency
+// that bounds it, of an output's MPO entries, which are fetched eight at a time, and
+// of the inputs (w = 8, 160 x 171: 22.5 -> 9.0 us).
 //   left:  t2[m,k,b,c] = sum_{g,h} t1[m,g,h,c] O[g,k,h,b]
 //   right: t2[a,b,k,o] = sum_{h,l} t1[a,h,l,o] O[b,k,h,l]
 template <int NIN, bool RIGHT>
@@ -190,7 +193,15 @@ __global__ __launch_bounds__(256) void mpo_mid_kernel(const double* __restrict__
                                                       int64_t D1, int wl, int d, int wr, int64_t D2,
                                                       double* __restrict__ t2) {
   typedef __attribute__((address_space(1))) double gd;
+  constexpr int OC = 8;
   const int nin = RIGHT ? d * wr : wl * d, nout = RIGHT ? wl * d : d * wr;
+  // input i: left (g, h), O step wl d per h; right (h, l), O step wl d per h, wl d d per l
+  int off[(NIN + OC - 1) / OC * OC];
+#pragma unroll
+  for (int i = 0; i < (NIN + OC - 1) / OC * OC; ++i) {
+    const int e = min(i, nin - 1);
+    off[i] = RIGHT ? wl * d * e : e % wl + wl * d * (e / wl);
+  }
   GRID_STRIDE(idx, D1 * D2) {
     const int64_t c = idx / D1, m = idx - c * D1;
     const gd* in = (const gd*)t1 + m + D1 * (int64_t)nin * c;
@@ -198,17 +209,18 @@ __global__ __launch_bounds__(256) void mpo_mid_kernel(const double* __restrict__
     double v[NIN];
 #pragma unroll
     for (int i = 0; i < NIN; ++i) v[i] = i < nin ? in[D1 * i] : 0.0;
-    for (int q = 0; q < nout; ++q) {
+    for (int q = blockIdx.y; q < nout; q += gridDim.y) {
       // output q: left (k, b) = (q % d, q / d), right (b, k) = (q % wl, q / wl)
       const double* w = RIGHT ? O + q % wl + wl * (q / wl) : O + wl * (q % d + d * d * (int64_t)(q / d));
       double s = 0.0;
 #pragma unroll
-      for (int i = 0; i < NIN; ++i) {
-        if (i < nin) {
-          // input i: left (g, h), O step wl d per h; right (h, l), O step wl d per h, wl d d per l
-          const double ov = RIGHT ? w[(int64_t)wl * d * i] : w[i % wl + (int64_t)wl * d * (i / wl)];
-          if (ov != 0.0) s += v[i] * ov;
-        }
+      for (int i0 = 0; i0 < NIN; i0 += OC) {
+        double ov[OC];
+#pragma unroll
+        for (int i = 0; i < OC; ++i) ov[i] = i0 + i < NIN ? w[off[i0 + i]] : 0.0;
+#pragma unroll
+        for (int i = 0; i < OC; ++i)
+          if (i0 + i < NIN && i0 + i < nin && ov[i] != 0.0) s += v[i0 + i] * ov[i];
       }
       out[D1 * q] = s;
     }
@@ -951,7 +963,9 @@ static mk_status launch_mpo_mid(const double* t1, const double* O, int64_t D1, i
                                 double* t2, hipStream_t st) {
   const int nin = RIGHT ? d * wr : wl * d, nout = RIGHT ? wl * d : d * wr;
   if (D1 * D2 * nout == 0) return MK_OK;
-  const dim3 g = grid1d(D1 * D2, 1);
+  // four workgroups a CU, as far as the outputs go
+  dim3 g = grid1d(D1 * D2, 1);
+  g.y = (unsigned)std::max<int64_t>(1, std::min<int64_t>(nout, 1024 / g.x));
 #define MPO_MID(N) hipLaunchKernelGGL((mpo_mid_kernel<N, RIGHT>), g, dim3(256), 0, st, t1, O, D1, wl, d, wr, D2, t2)
   if (nin <= 4) MPO_MID(4);
   else if (nin <= 6) MPO_MID(6);
