@@ -51,10 +51,25 @@ def _householder_pos_qr(M):
     return Q * s, s[:, None] * R
 
 
+def _gram(Q):
+    """Q^T Q.  On the library's GEMM, which cuts its tiles along K, for 384 to 1536
+    columns (us, the vendor library's beside it: 1024 x 512 22 and 35, 2048 x 1024 85
+    and 114, 3000 x 1500 224 and 261); with fewer the host's share of the call decides
+    (512 x 256 20 and 11), with more the vendor's is the faster (4096 x 2048 511 and
+    483)."""
+    if Q.is_cuda and Q.dtype == T.DTYPE and 384 <= Q.shape[1] <= 1536:
+        from .derivatives import gemm
+        if T.is_colmajor(Q):
+            return gemm(Q, Q, transa=True).t()
+        if T.is_colmajor(Q.t()):
+            return gemm(Q.t(), Q.t(), transb=True).t()
+    return Q.t() @ Q
+
+
 def _chol_step(Q, shift=0.0):
     """One Cholesky QR pass: G = Q^T Q (+ shift I) = R^T R, Q <- Q R^-1.  The
     factorisation is the library's blocked Cholesky (``mk_potrf``)."""
-    G = (Q.t() @ Q).contiguous()
+    G = _gram(Q).contiguous()
     if shift:
         G.diagonal().add_(shift)
     if not G.is_cuda:
@@ -89,7 +104,7 @@ def pos_qr(M):
         Rk = L.t()
         Q = torch.linalg.solve_triangular(Rk, Q, upper=True, left=False)
         R = Rk if R is None else Rk @ R
-    E = Q.t() @ Q
+    E = _gram(Q)
     E.diagonal().sub_(1.0)
     if float(torch.linalg.matrix_norm(E)) > 1e-13 * max(n, 1) ** 0.5:
         return _householder_pos_qr(M)

@@ -61,3 +61,17 @@ def test_cholesky_qr_matches_householder(env, m, n):
     assert float(torch.linalg.matrix_norm(E)) < 1e-13 * n ** 0.5
     assert float(torch.linalg.matrix_norm(R - Rh) / torch.linalg.matrix_norm(Rh)) < 1e-12
     assert float(torch.linalg.matrix_norm(Q @ R - A) / torch.linalg.matrix_norm(A)) < 1e-13
+
+
+@pytest.mark.parametrize("m,n", [(383, 383), (385, 384), (1000, 385), (1601, 1536), (1600, 1537)])
+@pytest.mark.parametrize("colmajor", [True, False])
+def test_gram_both_orders(env, m, n, colmajor):
+    """Each entry is a sum of m products, off by at most m u sum |q_ki q_kj|."""
+    mk, torch = env
+    from mpskit_amd.states import _gram
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + 2 * n)
+    Q = torch.randn(m, n, dtype=torch.float64, device="cuda", generator=g)
+    Q = Q.t().contiguous().t() if colmajor else Q
+    ref = torch.sum(Q[:, :7, None] * Q[:, None, :], 0)
+    assert bool(((_gram(Q)[:7] - ref).abs() <= 2 * m * 2.0 ** -53 * (Q[:, :7].abs().t() @ Q.abs())).all())
