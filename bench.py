@@ -846,14 +846,14 @@ def main():
         "tflops": {p: F / (r["ms"] * 1e-3) / 1e12 for p, r in res.items()},
         "roofline": {"bound": "mfma", "achieved": ach, "peak": PEAK_TF["bf16x3"], "unit": "TFLOP/s",
                      "frac": ach / PEAK_TF["bf16x3"],
-                     "traffic": traffic_from_profile("gemm_mixed_big2_kernel<BF16X3>", D),
-                     "kernel": "gemm_mixed_big2_kernel<BF16X3> (256x256 tiles, 8 waves)",
+                     "traffic": traffic_from_profile("gemm_mixed_dma_kernel<BF16X3>", D),
+                     "kernel": "gemm_mixed_dma_kernel<BF16X3> (256x256 tiles, 8 waves)",
                      "peak_note": "BF16 dense 2516.6 TF/s over 3 products per float64 product"},
         "roofline_fp64": {"bound": "mfma", "achieved": F / (res["fp64"]["gemm_ms"] * 1e-3) / 1e12,
                           "peak": PEAK_TF["fp64"], "unit": "TFLOP/s",
                           "frac": F / (res["fp64"]["gemm_ms"] * 1e-3) / 1e12 / PEAK_TF["fp64"],
-                          "traffic": traffic_from_profile("gemm_f64_buf_kernel<128,128>", D),
-                          "kernel": "gemm_f64_buf_kernel<128,128> (branch-free loads, rotated K step)"},
+                          "traffic": traffic_from_profile("gemm_f64_dma_kernel<128,128>", D),
+                          "kernel": "gemm_f64_dma_kernel<128,128> (operands straight to LDS)"},
     }
     print("# vendor GEMM reference ...", file=sys.stderr, flush=True)
     out["vendor_gemm_reference"] = vendor_gemm_reference(D)
