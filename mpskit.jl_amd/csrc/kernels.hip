@@ -967,14 +967,15 @@ static mk_status launch_mpo_mid(const double* t1, const double* O, int64_t D1, i
   dim3 g = grid1d(D1 * D2, 1);
   g.y = (unsigned)std::max<int64_t>(1, std::min<int64_t>(nout, 1024 / g.x));
 #define MPO_MID(N) hipLaunchKernelGGL((mpo_mid_kernel<N, RIGHT>), g, dim3(256), 0, st, t1, O, D1, wl, d, wr, D2, t2)
-  if (nin <= 4) MPO_MID(4);
+  // no input at all (an empty bond): a zero per output, without reading O
+  if (nin == 0 || nin > 32)
+    hipLaunchKernelGGL((mpo_mid_wide_kernel<RIGHT>), grid1d(D1 * nout * D2, 4), dim3(TPB), 0, st, t1, O, D1, wl, d, wr,
+                       D2, t2);
+  else if (nin <= 4) MPO_MID(4);
   else if (nin <= 6) MPO_MID(6);
   else if (nin <= 10) MPO_MID(10);
   else if (nin <= 16) MPO_MID(16);
-  else if (nin <= 32) MPO_MID(32);
-  else
-    hipLaunchKernelGGL((mpo_mid_wide_kernel<RIGHT>), grid1d(D1 * nout * D2, 4), dim3(TPB), 0, st, t1, O, D1, wl, d, wr,
-                       D2, t2);
+  else MPO_MID(32);
 #undef MPO_MID
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
