@@ -115,12 +115,17 @@ struct ProbSpec {
   int64_t M = 0, N = 0;
   SegSpec seg[MAX_SEG];
   int nseg = 0;
+  bool full = false;   // a segment found no place: every launch refuses the problem
   double* C = nullptr;
   int64_t ldc = 0;
   double alpha = 1.0, beta = 0.0;
   GemmPhys phys;   // only for launches that gemm_f64_small says yes to
   void add(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t K,
            const void* Alo = nullptr, const void* Blo = nullptr) {
+    if (nseg == MAX_SEG) {
+      full = true;
+      return;
+    }
     seg[nseg].A = A; seg[nseg].lda = lda; seg[nseg].B = B; seg[nseg].ldb = ldb;
     seg[nseg].K = K; seg[nseg].Alo = Alo; seg[nseg].Blo = Blo;
     ++nseg;

@@ -818,7 +818,7 @@ bool gemm_f64_small(const ProbSpec* probs, int nprob, GemmShape shape, bool ws) 
 mk_status gemm_f64(const ProbSpec* probs, int nprob, GemmShape shape, hipStream_t stream, void* ws) {
   MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "gemm_f64: %d problems (max %d)", nprob, MAX_PROB);
   for (int i = 0; i < nprob; ++i) {
-    MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "gemm_f64: too many segments");
+    MK_REQUIRE(!probs[i].full, MK_BAD_ARG, "gemm_f64: more than %d segments", MAX_SEG);
     MK_REQUIRE(probs[i].M >= 0 && probs[i].N >= 0 && probs[i].M < (1ll << 31) && probs[i].N < (1ll << 31),
                MK_BAD_SHAPE, "gemm_f64: bad M/N");
     for (int s = 0; s < probs[i].nseg; ++s)

@@ -522,7 +522,7 @@ template <int MODE>
 mk_status dispatch(const ProbSpec* probs, int nprob, hipStream_t stream, void* ws) {
   MK_REQUIRE(nprob >= 0 && nprob <= MAX_PROB, MK_BAD_ARG, "mixed gemm: too many problems");
   for (int i = 0; i < nprob; ++i)
-    MK_REQUIRE(probs[i].nseg <= MAX_SEG, MK_BAD_ARG, "mixed gemm: too many segments");
+    MK_REQUIRE(!probs[i].full, MK_BAD_ARG, "mixed gemm: more than %d segments", MAX_SEG);
   constexpr int EB = MODE == M_BF16X3 ? 2 : 4;
   const bool dma = variant() == V_DMA && rows256_fit<MODE>(probs, nprob);
   bool packed = false;

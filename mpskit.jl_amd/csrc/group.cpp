@@ -46,7 +46,7 @@ mk_status fill(const std::vector<ProbSpec>& specs, int prec, int kind, std::vect
     GemmProb& P = out[i];
     MK_REQUIRE(ps.M >= 0 && ps.N >= 0 && ps.M < (1ll << 31) && ps.N < (1ll << 31), MK_BAD_SHAPE,
                "grouped gemm: bad M/N");
-    MK_REQUIRE(ps.nseg <= MAX_SEG, MK_BAD_ARG, "grouped gemm: too many segments");
+    MK_REQUIRE(!ps.full, MK_BAD_ARG, "grouped gemm: more than %d segments", MAX_SEG);
     P.M = (int32_t)ps.M;
     P.N = (int32_t)ps.N;
     P.nseg = 0;

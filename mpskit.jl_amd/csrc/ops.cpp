@@ -493,7 +493,8 @@ mk_status apply_small(Op* op, const double* x, double* y, double alpha, double b
 
 // By-block Jordan apply: the physical term (and the mixed views of x) in one
 // pass over x, then one launch over the output blocks, which also takes in the
-// channel form's last product (its first product and MPO step run before).
+// channel form's last product where its segment lists have room (its first
+// product and MPO step run before).
 mk_status apply_by_block(Op* op, const double* x, double* y, double alpha, double beta, int prec) {
   Ctx* ctx = op->ctx;
   hipStream_t st = ctx->stream;
@@ -510,9 +511,10 @@ mk_status apply_by_block(Op* op, const double* x, double* y, double alpha, doubl
     s1 = (size_t)M * k.wr * N * 8;
     s2 = in_place ? 0 : f64 ? (size_t)Dl * k.wl * d1 * N * 8 : view_bytes(Dl * k.wl, d1 * N, 'B', prec);
   }
-  // too much for a caller that cannot allocate: the channel form by itself, in chunks
+  // no place left in a segment list, or too much for a caller that cannot
+  // allocate: the channel form by itself (there in chunks)
   const FixedScratch& fx = fixed_scratch();
-  const bool with_xrl = k.present() && (!fx.base || align256(va) + align256(vb) + align256(s1) + align256(s2) <=
+  const bool with_xrl = op->xrl_joins() && (!fx.base || align256(va) + align256(vb) + align256(s1) + align256(s2) <=
                                                         (int64_t)fx.bytes);
   if (!with_xrl) s1 = s2 = 0;
   void *ma = nullptr, *mb = nullptr;

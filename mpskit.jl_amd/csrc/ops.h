@@ -209,6 +209,14 @@ struct Op {
   // applies take IC and BE whole
   bool blocks_full = false;
   bool by_block() const { return !jprobs.empty() && !blocks_full; }
+  // every output block's segment list has a place left for the channel form's
+  // last product (a two-site operator with full 2 x 2 blocks has four right and
+  // four left ones: none left)
+  bool xrl_joins() const {
+    for (const JProb& p : jprobs)
+      if (p.seg.size() >= MAX_SEG) return false;
+    return xrl.present();
+  }
   // a two-site operator with terms beyond nearest neighbours
   bool long_range() const { return CA.present() || !AB.empty() || RB.present() || LB.present() || has_gen(); }
 

@@ -5,10 +5,11 @@ Edges: odd and unequal bonds (rows and K runs of the mixed operands end in
 padding), sizes below one tile, first and last sites of a chain (one MPO row or
 column), chains whose blocks are half empty (Ising), full (XXZ), longer-ranged
 (J1-J2, three neighbours, exponential decay), a chain of on-site terms only,
-spin 1 for one site, alpha / beta, and batches of uneven bonds.
+MPO tensors without a zero block (eight products an output block beside the channel
+form's), spin 1 for one site, alpha / beta, and batches of uneven bonds.
 
-Tolerances: sums of at most 8 products of length D and a short physical sum;
-2-norm error, relative to the size of a random sum of the same n = 4 D terms
+Tolerances: sums of at most 9 products of length D (of w D the channel form's) and
+a short physical sum; 2-norm error, relative to the size of a random sum of the same n = 4 D terms
 (the sum of their absolute values over sqrt(n); the result itself may cancel at
 the smallest sizes), below 8 sqrt(4 D) u of the accumulation (2^-53, 2^-24)
 plus twice the operand rounding (2^-24, 2^-16) in the mixed arithmetics.
@@ -143,6 +144,43 @@ def test_one_site(mk, name, Dl, Dr):
         print("blocks", name, Dl, Dr, site, flush=True)
         op = mk.prepare_operator(mk.JordanMPO_AC_Hamiltonian(GL, Wd, GR), precisions=PRECS)
         check(op, x, y0, lambda g: ac(g(GLi), g(Wd), g(GRi), g(x)), max(Dl, Dr))
+
+
+def dense(w, d=2):
+    """A Jordan tensor with every block of A, B, C and D full."""
+    W = np.random.default_rng(w).standard_normal((w, d, d, w))
+    W[1:, :, :, 0] = W[-1, :, :, :] = 0.0
+    W[0, :, :, 0] = W[-1, :, :, -1] = np.eye(d)
+    return W
+
+
+@pytest.mark.parametrize("w", [3, 5])
+@pytest.mark.parametrize("Dl,Dr", [(33, 20), (120, 131), (200, 215), (301, 264)])
+def test_full_blocks(mk, w, Dl, Dr):
+    """Below and past the sizes where the channel form takes over; the allocation-free apply too."""
+    import torch
+    from mpskit_amd._lib import PREC_NAMES, check as ok, load
+    T = mk.tensors
+    Wb = dense(w)
+    sites = {"bulk": (Wb, Wb), "first": (Wb[:1], Wb), "last": (Wb, Wb[..., -1:])}
+    for site, (W1, W2) in sites.items():
+        GL, GR, GLi, GRi = envs(mk, Dl, W1.shape[0], Dr, W2.shape[3])
+        W1d, W2d = T.from_numpy(W1), T.from_numpy(W2)
+        x, y0 = rnd(mk, (Dl, 2, Dr, 2), 3), rnd(mk, (Dl, 2, Dr, 2), 4)
+        print("full blocks", w, Dl, Dr, site, flush=True)
+        op = mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(GL, W1d, W2d, GR), precisions=PRECS)
+        f = lambda g: ac2(g(GLi), g(W1d), g(W2d), g(GRi), g(x))   # noqa: E731
+        check(op, x, y0, f, max(Dl, Dr))
+        ref, size = f(lambda t: t), float(torch.linalg.vector_norm(f(torch.abs))) / math.sqrt(4 * max(Dl, Dr))
+        for prec in PRECS:
+            y = y0.clone(memory_format=torch.preserve_format)
+            ok(load().mk_apply_noalloc(op.handle, T.ptr(x), T.ptr(y), 1.0, 0.0, PREC_NAMES[prec]))
+            torch.cuda.synchronize()
+            assert close(y, ref, bound(prec, max(Dl, Dr)), size), prec
+    GL, GR, GLi, GRi = envs(mk, Dl, w, Dr, w)
+    Wd, x, y0 = T.from_numpy(Wb), rnd(mk, (Dl, 2, Dr), 3), rnd(mk, (Dl, 2, Dr), 4)
+    op = mk.prepare_operator(mk.JordanMPO_AC_Hamiltonian(GL, Wd, GR), precisions=PRECS)
+    check(op, x, y0, lambda g: ac(g(GLi), g(Wd), g(GRi), g(x)), max(Dl, Dr))
 
 
 @pytest.mark.parametrize("name", ["tfim", "xxz", "onsite"])
