@@ -240,7 +240,10 @@ void gemm_f64_kernel(Src src) {
 // sizes: the pair that straddles the end of an odd row range or of an odd K is left
 // out of the DMA (the hardware writes zeros) and its one element goes through a
 // register of the same lane, before the step's barrier; no load leaves the operand,
-// and only the workgroups at the edge or in the last step do this.
+// and only the workgroups at the edge or in the last step do this.  Scalar offsets
+// run over whole K steps, past K in the last one, and stay below 2 GiB (f64_fit):
+// a masked lane's vector offset is then past num_records whichever way the
+// hardware counts the scalar one.
 //
 // A DMA load writes 1 KB of LDS in lane order, so every swizzle is in which
 // element a lane loads:
@@ -272,7 +275,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* p) {
 template <int BM, int BN, bool TA, bool TB, bool ODD, class Src>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f64_dma_kernel(Src src) {
-  constexpr int BK = 16;
+  constexpr int BK = (int)F64_BK;
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int FM = WM / 16, FN = WN / 16;
   constexpr int CHA = BM * BK * 8 / 1024 / 4, CHB = BN * BK * 8 / 1024 / 4;   // DMA loads a wave
@@ -583,28 +586,6 @@ __global__ __launch_bounds__(64 * SW) void gemm_f64_small_kernel(GemmBatch src) 
   }
 }
 
-// Host check of the LDS-DMA kernel's conditions for one problem: every in-tile
-// offset below 2 GiB, 8-byte aligned operands; BUF_ODD unless sizes, leading
-// dimensions and addresses are whole pairs.
-enum BufFit { BUF_NO = 0, BUF_ODD = 1, BUF_EVEN = 2 };
-template <int BM, int BN>
-BufFit buf_ok_prob(const ProbSpec& ps, GemmShape sh) {
-  BufFit fit = BUF_EVEN;
-  for (int s = 0; s < ps.nseg; ++s) {
-    const SegSpec& g = ps.seg[s];
-    if (g.K <= 0) continue;
-    // largest in-tile byte offset (plus the 16-byte chunk) below 2^31
-    const int64_t offA = sh.ta ? (g.K + (int64_t)(BM - 1) * g.lda) * 8 : (BM + (int64_t)(g.K - 1) * g.lda) * 8;
-    const int64_t offB = !sh.tb ? (g.K + (int64_t)(BN - 1) * g.ldb) * 8 : (BN + (int64_t)(g.K - 1) * g.ldb) * 8;
-    if (offA + 16 >= (1ll << 31) || offB + 16 >= (1ll << 31)) return BUF_NO;
-    if ((uintptr_t)g.A % 8 || (uintptr_t)g.B % 8) return BUF_NO;
-    if ((uintptr_t)g.A % 16 || (uintptr_t)g.B % 16 || g.lda % 2 || g.ldb % 2 || g.K % 2 || (!sh.ta && ps.M % 2) ||
-        (sh.tb && ps.N % 2))
-      fit = BUF_ODD;
-  }
-  return fit;
-}
-
 // Load path of the FP64 kernels, read once from MK_F64_VARIANT ("dma" or "branch";
 // default "dma"): lets benchmarks and tests pin one of them.
 bool f64_direct() {
@@ -704,7 +685,7 @@ mk_status launch_cfg(const ProbSpec* probs, int nprob, GemmShape sh, hipStream_t
   MK_REQUIRE(tail == 0 || (ws != nullptr && (size_t)tail * sp.ksplit * BM * BN * 8 <= GEMM_WS_BYTES), MK_BAD_ARG,
              "gemm_f64: %d tiles split %d ways exceed the workspace", tail, sp.ksplit);
   int fit = BUF_EVEN;
-  for (int i = 0; i < nprob && fit != BUF_NO; ++i) fit = std::min<int>(fit, buf_ok_prob<BM, BN>(probs[i], sh));
+  for (int i = 0; i < nprob && fit != BUF_NO; ++i) fit = std::min<int>(fit, f64_fit(probs[i], sh, BM, BN));
   dim3 grid(b.full_tiles + tail * b.ksplit), block(NT);
   ProfScope prof("gemm_f64", stream);
   launch_path<BM, BN>(fit, sh, grid, block, stream, b);
@@ -750,7 +731,7 @@ int f64_group_grid(int kind, int total_tiles, int cus) {
 int f64_buf_ok(const ProbSpec* probs, int n, GemmShape sh, int kind) {
   int fit = BUF_EVEN;
   for (int i = 0; i < n && fit != BUF_NO; ++i)
-    fit = std::min<int>(fit, kind == TK_128 ? buf_ok_prob<128, 128>(probs[i], sh) : buf_ok_prob<64, 64>(probs[i], sh));
+    fit = std::min<int>(fit, f64_fit(probs[i], sh, tile_m(kind), tile_n(kind)));
   return fit;
 }
 

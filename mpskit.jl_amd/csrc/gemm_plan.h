@@ -8,6 +8,8 @@
 // every CU the same number of workgroups therefore loses twice, in idle CUs and
 // in waiting; cutting the tiles of the last round along K (in the extreme all
 // of them) repairs both for one write and one read of the partial tiles.
+//
+// And the host's check of what the FP64 LDS-DMA kernel takes (f64_fit).
 #pragma once
 #include <algorithm>
 
@@ -93,6 +95,31 @@ inline TileChoice plan_launch(const TileModel& m, const ProbSpec* probs, int npr
   int64_t tiles, nsteps;
   tile_counts(m, probs, nprob, tiles, nsteps);
   return plan_tile(m, tiles, nsteps, ws);
+}
+
+// What gemm_f64_dma_kernel with bm x bn tiles makes of one problem: BUF_NO, or its
+// form for odd sizes and 8-byte alignment, or the one for whole pairs.  Its byte
+// offsets within a tile are 32 bits wide and a load's scalar part is not masked, so
+// the bound counts K up to the end of the last K step, not to the last element: an
+// operand stored along its rows has loads for those k too, whose lanes are masked.
+enum BufFit { BUF_NO = 0, BUF_ODD = 1, BUF_EVEN = 2 };
+constexpr int64_t F64_BK = 16;
+inline BufFit f64_fit(const ProbSpec& ps, GemmShape sh, int bm, int bn) {
+  BufFit fit = BUF_EVEN;
+  for (int s = 0; s < ps.nseg; ++s) {
+    const SegSpec& g = ps.seg[s];
+    if (g.K <= 0) continue;
+    const int64_t K = cdiv(g.K, F64_BK) * F64_BK;
+    // one past the largest offset, with the 16 bytes of a load
+    const int64_t endA = (sh.ta ? K + (bm - 1) * g.lda : bm + (K - 1) * g.lda) * 8 + 16;
+    const int64_t endB = (!sh.tb ? K + (bn - 1) * g.ldb : bn + (K - 1) * g.ldb) * 8 + 16;
+    if (endA >= (1ll << 31) || endB >= (1ll << 31)) return BUF_NO;
+    if ((uintptr_t)g.A % 8 || (uintptr_t)g.B % 8) return BUF_NO;
+    if ((uintptr_t)g.A % 16 || (uintptr_t)g.B % 16 || g.lda % 2 || g.ldb % 2 || g.K % 2 || (!sh.ta && ps.M % 2) ||
+        (sh.tb && ps.N % 2))
+      fit = BUF_ODD;
+  }
+  return fit;
 }
 
 }  // namespace mk

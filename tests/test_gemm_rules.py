@@ -10,7 +10,7 @@ ROOT = Path(__file__).resolve().parents[1]
 ROCM = Path("/opt/rocm/include")
 HEAD = r"""
 #include <cstdio>
-#include "gemm.h"
+#include "gemm_plan.h"
 #include "ops.h"
 using namespace mk;
 // device buffers stay empty here
@@ -69,4 +69,46 @@ def test_the_channel_form_joins_only_lists_with_room(tmp_path):
     Op none;
     none.jprobs.push_back({0, 0, {}});
     CHECK(!none.xrl_joins());
+    """)
+
+
+def test_f64_offsets_of_the_last_k_step_stay_below_2_gib(tmp_path):
+    """gemm_f64_dma_kernel adds an unmasked scalar offset to every load, the rows past K of the last
+    step among them: none of a problem that f64_fit takes reaches 2^31 - 1 (num_records)."""
+    run(tmp_path, r"""
+    // largest scalar offset of an operand with R rows (or columns) a tile, as the kernel forms them
+    auto largest = [](bool along_k, int64_t R, int64_t ld, int64_t K) {
+      int64_t m = 0;
+      const int64_t k0 = (K - 1) / 16 * 16;
+      for (int64_t wave = 0; wave < 4; ++wave)
+        for (int64_t c = 0; c < R * 16 * 8 / 1024 / 4; ++c)
+          m = std::max(m, along_k ? 8 * wave * ld * 8 + c * 32 * ld * 8 + k0 * 8
+                                  : 128 / R * wave * ld * 8 + c * 4 * (128 / R) * ld * 8 + k0 * ld * 8);
+      return m;
+    };
+    int taken = 0, left = 0;
+    for (int64_t ld : {64ll, 4097ll, 1ll << 17, 1000003ll, 2000000ll, 8000000ll, 9000000ll, 16000000ll, 16700000ll, 100000000ll})
+      for (int64_t K : {1, 2, 3, 8, 15, 16, 17, 18, 19, 29, 31, 32, 33, 100, 1031})
+        for (int bits = 0; bits < 4; ++bits)
+          for (int t : {64, 128}) {
+            const GemmShape sh{(bits & 1) != 0, (bits & 2) != 0};
+            ProbSpec p;
+            p.M = p.N = 4096;
+            p.add(reinterpret_cast<const void*>(1 << 20), ld, reinterpret_cast<const void*>(1 << 20), ld, K);
+            const bool fits = f64_fit(p, sh, t, t) != BUF_NO;
+            if (fits) CHECK(largest(sh.ta, t, ld, K) + 16 < (1ll << 31) && largest(!sh.tb, t, ld, K) + 16 < (1ll << 31));
+            (fits ? taken : left) += 1;
+          }
+    CHECK(taken > 200 && left > 200);
+    // the product of a Krylov basis with the coefficients of its Ritz vectors, at D = 1500 and 2048
+    auto ritz = [](int64_t n, int64_t K) {
+      ProbSpec p;
+      p.M = n; p.N = 5;
+      p.add(reinterpret_cast<const void*>(1 << 20), n, reinterpret_cast<const void*>(1 << 20), K, K);
+      return f64_fit(p, GemmShape{}, 64, 64);
+    };
+    CHECK(ritz(4 * 1500 * 1500, 16) == BUF_EVEN && ritz(4 * 1500 * 1500, 17) == BUF_NO);
+    CHECK(ritz(16000000, 17) == BUF_NO && ritz(4 * 2048 * 2048, 16) == BUF_EVEN);
+    CHECK(ritz(4 * 1024 * 1024, 30) == BUF_EVEN && ritz(4 * 1024 * 1024, 29) == BUF_ODD);
+    CHECK(ritz(20000000, 8) == BUF_NO);
     """)

@@ -56,6 +56,20 @@ def test_split_gemm_matches_torch(mk, M, N, K, prec):
         assert float(torch.linalg.vector_norm(out - ref)) <= bound(prec, K) * scale
 
 
+@pytest.mark.parametrize("M,K", [(9_000_001, 17), (9_000_000, 18), (8_000_000, 19), (16_000_000, 16)])
+def test_tall_operand(mk, M, K):
+    """A Krylov basis times the coefficients of its Ritz vectors: columns so long that the K step past the
+    last one would end beyond 2 GiB from the tile's first row (K = 16 has none)."""
+    import torch
+    T = mk.tensors
+    g = torch.Generator(device="cuda")
+    g.manual_seed(K)
+    A, B = T.randn((M, K), g), T.randn((K, 5), g)
+    print("tall gemm", M, K, flush=True)
+    out, ref = mk.gemm(A, B), A @ B
+    assert float(torch.linalg.vector_norm(out - ref)) <= bound("fp64", K) * float(torch.linalg.vector_norm(ref))
+
+
 def test_split_gemm_repeats_bitwise(mk):
     """The slices are added in a fixed order, and an unordered second stream has a workspace of its own."""
     import torch
