@@ -31,6 +31,9 @@ mk_status DevBuf::alloc(size_t nbytes) {
   hipError_t e = hipMalloc(&ptr, nbytes);
   if (e != hipSuccess) {
     ptr = nullptr;
+    // the status tells the caller; left pending, it would be taken for the error
+    // of the next kernel launch
+    (void)hipGetLastError();
     set_error("hipMalloc(%zu) failed: %s", nbytes, hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? MK_OOM : MK_HIP_ERROR;
   }

@@ -71,3 +71,21 @@ def test_mfma_output_lane_layout(env):
         C = mk.gemm(T.as_colmajor(A), T.as_colmajor(B), precision=prec)
         torch.cuda.synchronize()
         assert float((C - ref).abs().max()) == 0.0, prec
+
+
+def test_a_refused_allocation_leaves_no_error_behind(env):
+    """Operand views of 2^59 bytes each: the allocation is refused before anything is launched, and the next
+    launches (which read the runtime's pending error) succeed."""
+    mk, torch = env
+    from mpskit_amd._lib import BF16X3, MKError, check, load
+    T = mk.tensors
+    A = T.as_colmajor(torch.randn(64, 64, dtype=torch.float64, device="cuda"))
+    ctx = mk.derivatives.default_context()
+    M, K = 1 << 30, 1 << 27
+    with pytest.raises(MKError) as e:
+        check(load().mk_gemm(ctx.handle, 0, 0, M, 8, K, 1.0, T.ptr(A), M, T.ptr(A), K, 0.0, T.ptr(A), M, BF16X3))
+    print("refused with", e.value.status, flush=True)
+    assert e.value.status == "MK_OOM"
+    for prec in ("fp64", "fp32", "bf16x3"):
+        C = mk.gemm(A, A, precision=prec)
+        assert float(torch.linalg.vector_norm(C - A @ A) / torch.linalg.vector_norm(A @ A)) < TOL[prec]
