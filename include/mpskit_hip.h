@@ -70,7 +70,12 @@ int mk_version(void);
 const char* mk_last_error(void);
 mk_status mk_ctx_create(int device, mk_ctx* out);
 mk_status mk_ctx_destroy(mk_ctx ctx);
-/* stream is a hipStream_t (NULL = legacy default stream) */
+/* stream is a hipStream_t (NULL = legacy default stream).  A context keeps a
+ * workspace of 64 MiB for each stream that its GEMMs were enqueued on (16 at most;
+ * then those of streams no longer used are handed on), from which GEMMs too small
+ * to fill the GPU split their sums: destroy a stream only after its work is done.
+ * Under stream capture no workspace is used, so a captured call adds in another
+ * order and agrees with the eager one to rounding. */
 mk_status mk_ctx_set_stream(mk_ctx ctx, void* stream);
 mk_status mk_ctx_synchronize(mk_ctx ctx);
 

@@ -79,6 +79,7 @@ mk_status Ctx::readback_init() {
 }
 
 Ctx::~Ctx() {
+  gemmws.clear([](void* p) { (void)hipFree(p); });
   if (readback) (void)hipHostFree(readback);
   for (hipEvent_t e : readback_ev)
     if (e) (void)hipEventDestroy(e);
@@ -93,11 +94,16 @@ void* Ctx::gemm_ws() {
     return nullptr;
   }
   if (cap != hipStreamCaptureStatusNone) return nullptr;
-  for (int i = 0; i < ngemmws; ++i)
-    if (gemmws[i].stream == stream) return gemmws[i].buf.ptr;
-  if (ngemmws == MAX_GEMM_WS || gemmws[ngemmws].buf.alloc(GEMM_WS_BYTES) != MK_OK) return nullptr;
-  gemmws[ngemmws].stream = stream;
-  return gemmws[ngemmws++].buf.ptr;
+  return gemmws.get(
+      stream,
+      [] {
+        DevBuf b;
+        if (b.alloc(GEMM_WS_BYTES) != MK_OK) return (void*)nullptr;
+        void* p = b.ptr;
+        b.ptr = nullptr;   // the table's from here on
+        return p;
+      },
+      [] { return hipDeviceSynchronize() == hipSuccess; });
 }
 
 FixedScratch& fixed_scratch() {

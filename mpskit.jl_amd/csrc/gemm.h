@@ -139,9 +139,10 @@ struct GemmShape {
   bool ta = false, tb = false;
 };
 
-// Workspace of the K-split launches: a fixed GEMM_WS_BYTES region per context
-// (allocated with it, so a call under stream capture allocates nothing), or
-// per GPU for the allocation-free apply.  64 MiB hold the partial tiles of one
+// Workspace of the K-split launches: GEMM_WS_BYTES for each stream of a context,
+// allocated by the first launch that could use it (Ctx::gemm_ws; none under
+// stream capture, so that a captured launch neither allocates nor splits), or a
+// fixed region per GPU for the allocation-free apply.  64 MiB hold the partial tiles of one
 // full round of workgroups (512 FP64 tiles of 128 x 128, or 256 fp32 ones of
 // 256 x 256), and no split makes more.
 constexpr size_t GEMM_WS_BYTES = (size_t)64 << 20;

@@ -8,6 +8,7 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "ws_table.h"
 
 namespace mk {
 
@@ -47,21 +48,14 @@ struct Ctx {
   ~Ctx();
   DevBuf smallbuf;   // small stream-ordered scratch (reduction partials, scalars)
   // K-split workspaces (GEMM_WS_BYTES each) of the streams this context has
-  // enqueued on, at most MAX_GEMM_WS; kept until the context goes
-  static constexpr int MAX_GEMM_WS = 4;
-  struct GemmWs {
-    hipStream_t stream = nullptr;
-    DevBuf buf;
-  };
-  GemmWs gemmws[MAX_GEMM_WS];
-  int ngemmws = 0;
+  // enqueued on, kept until the context goes
+  WsTable gemmws;
   mk_status scratch(size_t nbytes, void** out);
   mk_status small(size_t nbytes, void** out);
   // The K-split workspace of a GEMM about to be enqueued on `stream`, or null
-  // (the launch then splits nothing): each stream has its own, so callers that
-  // move one context between streams need not order them; a stream past the
-  // first MAX_GEMM_WS gets none, and neither does one under capture, whose
-  // graph may later run beside the stream's eager work.
+  // (the launch then splits nothing): the stream's own (WsTable), and none for
+  // a stream under capture, whose graph may later run beside the stream's eager
+  // work.
   void* gemm_ws();
 };
 

@@ -12,6 +12,7 @@ HEAD = r"""
 #include <cstdio>
 #include "gemm_plan.h"
 #include "ops.h"
+#include "ws_table.h"
 using namespace mk;
 // device buffers stay empty here
 void mk::DevBuf::release() {}
@@ -111,4 +112,56 @@ def test_f64_offsets_of_the_last_k_step_stay_below_2_gib(tmp_path):
     CHECK(ritz(16000000, 17) == BUF_NO && ritz(4 * 2048 * 2048, 16) == BUF_EVEN);
     CHECK(ritz(4 * 1024 * 1024, 30) == BUF_EVEN && ritz(4 * 1024 * 1024, 29) == BUF_ODD);
     CHECK(ritz(20000000, 8) == BUF_NO);
+    """)
+
+
+def test_workspace_table_hands_idle_slots_on(tmp_path):
+    """Streams past the slots get a workspace once one of the others has been idle, after a wait for the
+    device; a rotation over too many streams swaps none; a refused allocation is tried again later."""
+    run(tmp_path, r"""
+    static char mem[64];
+    static int allocs = 0, waits = 0;
+    static bool refuse = false;
+    auto alloc = [] { return refuse ? (void*)nullptr : (void*)&mem[allocs++]; };
+    auto wait = [] { ++waits; return true; };
+    auto st = [](int i) { return reinterpret_cast<const void*>((uintptr_t)(1000 + i)); };
+    WsTable t;
+    void* own[WsTable::SLOTS];
+    for (int i = 0; i < WsTable::SLOTS; ++i) own[i] = t.get(st(i), alloc, wait);
+    for (int i = 0; i < WsTable::SLOTS; ++i) {
+      CHECK(own[i] && t.get(st(i), alloc, wait) == own[i]);
+      for (int j = 0; j < i; ++j) CHECK(own[i] != own[j]);
+    }
+    CHECK(allocs == WsTable::SLOTS);
+    // all in use: the streams past the slots go without, in any number of rounds
+    for (int r = 0; r < 1000; ++r)
+      for (int i = 0; i < WsTable::SLOTS + 2; ++i)
+        CHECK(t.get(st(i), alloc, wait) == (i < WsTable::SLOTS ? own[i] : nullptr));
+    CHECK(waits == 0);
+    // stream 3 is heard of no more: its slot goes to the next one past them, once
+    int got = -1;
+    for (uint64_t r = 0; r < 2 * WsTable::IDLE && got < 0; ++r)
+      for (int i = 0; i < WsTable::SLOTS + 1; ++i) {
+        if (i == 3) continue;
+        void* p = t.get(st(i), alloc, wait);
+        if (i == WsTable::SLOTS && p) { CHECK(p == own[3]); got = (int)r; }
+      }
+    CHECK(got > 0 && waits == 1 && allocs == WsTable::SLOTS);
+    CHECK(t.get(st(3), alloc, wait) == nullptr);
+    // a wait that fails hands nothing on
+    WsTable u;
+    for (int i = 0; i < WsTable::SLOTS; ++i) u.get(st(i), alloc, wait);
+    for (uint64_t r = 0; r < 3 * WsTable::IDLE; ++r) u.get(st(0), alloc, wait);
+    CHECK(u.get(st(99), alloc, [] { return false; }) == nullptr && u.slot[1].stream == st(1));
+    // refused allocations
+    WsTable v;
+    refuse = true;
+    for (uint64_t r = 0; r + 1 < WsTable::IDLE; ++r) CHECK(v.get(st(0), alloc, wait) == nullptr);
+    refuse = false;
+    CHECK(v.get(st(0), alloc, wait) == nullptr);
+    for (uint64_t r = 0; r < 3; ++r) v.get(st(0), alloc, wait);
+    CHECK(v.get(st(0), alloc, wait) != nullptr);
+    int freed = 0;
+    t.clear([&](void*) { ++freed; });
+    CHECK(freed == WsTable::SLOTS && t.n == 0);
     """)

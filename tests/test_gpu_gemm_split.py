@@ -88,6 +88,28 @@ def test_split_gemm_repeats_bitwise(mk):
         assert torch.equal(o, first)
 
 
+def test_split_gemm_on_many_streams(mk):
+    """A long-lived context splits on each of many streams, and for new ones once older ones are idle: the
+    result is that of the split launch, bit for bit."""
+    import torch
+    T = mk.tensors
+    A, B = T.randn((500, 3000)), T.randn((3000, 400))
+    first = mk.gemm(A, B).clone()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(24)]
+    for s in streams[:12]:
+        with torch.cuda.stream(s):
+            out = mk.gemm(A, B)
+        s.synchronize()
+        assert torch.equal(out, first)
+    for s in streams[12:]:
+        with torch.cuda.stream(s):
+            for _ in range(1100):
+                out = mk.gemm(A, B, out)
+        s.synchronize()
+        assert torch.equal(out, first)
+
+
 def test_split_gemm_not_split_under_capture(mk):
     """A captured call takes no shared workspace; replays agree with the eager result."""
     import torch
