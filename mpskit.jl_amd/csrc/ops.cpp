@@ -1107,8 +1107,8 @@ extern "C" mk_status mk_op_set_charge_blocks(mk_op h, int nl, const int64_t* lof
   Op* op = reinterpret_cast<Op*>(h);
   MK_REQUIRE(op->kind == OP_AC2_JOR && !op->long_range(),
              MK_NOT_SUPPORTED, "charge blocks: only nearest-neighbour two-site Jordan operators");
-  MK_REQUIRE(op->d1 == op->d2 && op->d1 + op->d2 <= MAX_SEG, MK_NOT_SUPPORTED,
-             "charge blocks: equal physical spaces with d1 + d2 <= %d", MAX_SEG);
+  // spin 1/2 only, whatever a problem's segment list could hold: no wider block layout is tested
+  MK_REQUIRE(op->d1 == op->d2 && op->d1 <= 2, MK_NOT_SUPPORTED, "charge blocks: equal physical spaces with d <= 2");
   const int64_t Dl = op->Dl, Dr = op->Dr, d = op->d1;
   MK_REQUIRE(nl >= 1 && nr >= 1 && loff[0] == 0 && loff[nl] == Dl && roff[0] == 0 && roff[nr] == Dr, MK_BAD_SHAPE,
              "charge blocks: sector offsets must cover [0, Dl) and [0, Dr)");
@@ -1609,7 +1609,7 @@ extern "C" mk_status mk_prepare_ac2_jordan(mk_ctx h, const double* GL, const dou
   MK_REQUIRE(okdim(Dl) && okdim(wl) && okdim(d1) && okdim(wm) && okdim(d2) && okdim(wr) && okdim(Dr),
              MK_BAD_SHAPE, "prepare_ac2_jordan: non-positive dimension");
   MK_REQUIRE(wm >= 2, MK_BAD_SHAPE, "prepare_ac2_jordan: the shared MPO bond needs >= 2 channels");
-  MK_REQUIRE(d2 <= MAX_PROB && d2 <= MAX_SEG, MK_NOT_SUPPORTED, "prepare_ac2_jordan: d2 > %d", MAX_SEG);
+  MK_REQUIRE(d2 <= MAX_PROB && d2 <= MAX_SEG, MK_NOT_SUPPORTED, "prepare_ac2_jordan: d2 > %d", std::min(MAX_PROB, MAX_SEG));
   MK_REQUIRE(GL && W1 && W2 && GR, MK_BAD_ARG, "prepare_ac2_jordan: null pointer");
   Op* op = nullptr;
   MK_TRY(new_op(h, OP_AC2_JOR, precisions, &op));
@@ -1759,7 +1759,8 @@ extern "C" mk_status mk_prepare_ac2_jordan_terms(mk_ctx h, const mk_jordan_ac2_t
   MK_REQUIRE(t != nullptr, MK_BAD_ARG, "prepare_ac2_jordan_terms: null terms");
   MK_REQUIRE(okdim(Dl) && okdim(d1) && okdim(Dr) && okdim(d2), MK_BAD_SHAPE,
              "prepare_ac2_jordan_terms: non-positive dimension");
-  MK_REQUIRE(d2 <= MAX_PROB && d2 <= MAX_SEG, MK_NOT_SUPPORTED, "prepare_ac2_jordan_terms: d2 > %d", MAX_SEG);
+  MK_REQUIRE(d2 <= MAX_PROB && d2 <= MAX_SEG, MK_NOT_SUPPORTED, "prepare_ac2_jordan_terms: d2 > %d",
+             std::min(MAX_PROB, MAX_SEG));
   const bool hasAA = t->AA_GL || t->AA_W1 || t->AA_W2 || t->AA_GR;
   MK_REQUIRE(!hasAA || (t->AA_GL && t->AA_W1 && t->AA_W2 && t->AA_GR && okdim(t->aa_wl) && okdim(t->aa_wm) &&
                         okdim(t->aa_wr)),

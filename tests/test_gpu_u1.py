@@ -87,6 +87,25 @@ def test_block_apply_matches_dense(mk):
     cmp.free()
 
 
+def test_charge_blocks_are_for_spin_one_half(mk):
+    """A spin-1 operator is refused, and applies as before."""
+    import torch
+    from mpskit_amd._lib import MKError
+    from mpskit_amd.u1 import U1Bond
+    T, D, d = mk.tensors, 8, 3
+    W = np.zeros((3, d, d, 3))
+    W[0, :, :, 0] = W[2, :, :, 2] = np.eye(d)
+    W[0, :, :, 1] = W[1, :, :, 2] = np.diag([1.0, 0.0, -1.0])
+    Wd, GL, GR, x = T.from_numpy(W), T.randn((D, 3, D)), T.randn((D, 3, D)), T.randn((D, d, D, d))
+    op = mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(GL, Wd, Wd, GR))
+    y = op(x)
+    bond = U1Bond([0], [D])
+    with pytest.raises(MKError) as e:
+        mk.set_charge_blocks(op, bond, bond, (1, 0, -1))
+    assert e.value.status == "MK_NOT_SUPPORTED"
+    assert torch.equal(op(x), y)
+
+
 def test_u1_dmrg_xxz_vs_exact(mk):
     L, nup, delta = 10, 5, 1.0
     e_ed = np.linalg.eigvalsh(B.dense_xxz(L, delta).toarray())[0]
