@@ -94,7 +94,7 @@ mk_status k_cgs_update_norm(const double* V, int64_t ldv, int k, const double* c
 // w -= V c (c on device, length k)
 mk_status k_multiaxpy(const double* V, int64_t ldv, int k, const double* c, double* w,
                       int64_t n, hipStream_t st);
-// y = a*x + b*y with a, b host scalars
+// y = a*x + b*y with a, b host scalars; an operand with factor 0 is not read
 mk_status k_axpby(double a, const double* x, double b, double* y, int64_t n, hipStream_t st);
 // y = x / sqrt(*s2) (s2 on the device)
 mk_status k_normalize(const double* x, const double* s2, double* y, int64_t n, hipStream_t st);

@@ -599,10 +599,11 @@ __global__ void gemv_kernel(const double* __restrict__ V, int64_t ldv, int k,
   }
 }
 
+// a = 0 or b = 0: that operand is not read (y may hold anything before its first write)
 __global__ void axpby_kernel(double a, const double* x, double b, double* y,
                              int64_t n) {
   GRID_STRIDE(i, n) {
-    double v = a * x[i];
+    double v = a != 0.0 ? a * x[i] : 0.0;
     if (b != 0.0) v += b * y[i];
     y[i] = v;
   }

@@ -106,6 +106,37 @@ def test_charge_blocks_are_for_spin_one_half(mk):
     assert torch.equal(op(x), y)
 
 
+def test_block_apply_without_a_physical_term(mk):
+    """An MPO of environments only: outside the blocks y is zero whatever its memory held, alone and in a batch."""
+    import torch
+    from mpskit_amd.u1 import U1Bond
+    T = mk.tensors
+    W = np.zeros((2, 2, 2, 2))
+    W[0, :, :, 0] = W[1, :, :, 1] = np.eye(2)
+    Wd, bond = T.from_numpy(W), U1Bond([-1, 1], [8, 16])
+    D = bond.D
+    q = bond.charge_of_index("cuda")
+    same = (q[:, None] == q[None, :]).double()
+    GL, GR = T.randn((D, 2, D)), T.randn((D, 2, D))
+    GL, GR = T.as_colmajor(GL * same[:, None, :]), T.as_colmajor(GR * same[:, None, :])
+    pq = torch.tensor([1, -1], device="cuda")
+    total = q[:, None, None, None] + pq[None, :, None, None] + pq[None, None, None, :] - q[None, None, :, None]
+    x = T.as_colmajor(T.randn((D, 2, D, 2)) * (total == 0).double())
+    dense = mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(GL, Wd, Wd, GR))
+    blk = mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(GL, Wd, Wd, GR))
+    mk.set_charge_blocks(blk, bond, bond, (1, -1))
+    ref = dense(x)
+    out = T.empty(blk.y_shape)
+    out.fill_(float("nan"))
+    assert rel(blk(x, out=out, alpha=1.0, beta=0.0), ref) < 1e-12
+    b = mk.BatchedDerivative([blk])
+    flat = b.pack([x])
+    torch.cuda.synchronize()
+    stale = torch.full_like(flat, float("nan"))   # the memory that the batch's result is put into
+    del stale
+    assert rel(b.unpack(b.apply(flat))[0], ref) < 1e-12
+
+
 def test_u1_dmrg_xxz_vs_exact(mk):
     L, nup, delta = 10, 5, 1.0
     e_ed = np.linalg.eigvalsh(B.dense_xxz(L, delta).toarray())[0]
