@@ -229,7 +229,8 @@ mk_status mk_krylov_orthogonalize(mk_ctx ctx, const double* V, int64_t ldv, int 
  * float64 matrix (column-major, leading dim lda, device pointer), in place:
  * the lower triangle becomes L and the strict upper triangle zero.  *info
  * (host) is 0 on success, else the 1-based column of the first non-positive
- * pivot (then A holds a partial result).  The factorisation inside the
+ * pivot (then the 64-column blocks before the failing one hold L, and what is
+ * below the diagonal from there on is a partial result).  The factorisation inside the
  * Cholesky QR of the gauge steps' positive QR / LQ (qr_compact / lq_compact
  * with positive = true in ortho.jl:215-340 and the finite-MPS gauge moves of
  * finitemps.jl; the reference factors by Householder QR in LAPACK, which this

@@ -55,7 +55,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // X_ij = -X_ii sum_k L_ik X_kj.  (One column per step over the whole block, with
 // a workgroup barrier each, took 94 us, all but 4 us of it waiting.)
 // A non-positive or non-finite pivot sets *info = k0 + j + 1 (LAPACK's
-// convention) and nothing more is written.  Writes L11 (zeros above the
+// convention); the block then stays as it was.  Writes L11 (zeros above the
 // diagonal) into A and L11^-1 into Linv (ld NB, zeros above the diagonal);
 // columns nb and on are those of the identity.  S and X: S[r LD + c], X zero;
 // the caller's writes to them are its own threads' (the barrier is here).
@@ -172,9 +172,12 @@ __global__ __launch_bounds__(PT) void potrf_step_kernel(double* __restrict__ A, 
   __shared__ double T[3][SB * (SB + 1)];
   __shared__ int bad;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, li = lane & 15, lq = lane >> 4;
-  if (__syncthreads_or(*(volatile const int*)info != 0)) return;   // an earlier block failed
   gdouble* gA = (gdouble*)A;
   const int64_t b0 = k0 < 0 ? 0 : k0 + NB, m = n - b0;   // the trailing matrix
+  // an earlier block failed (a failure of the block this launch factors comes with a
+  // larger *info: the other workgroups still owe their part of L)
+  const int failed = *(volatile const int*)info;
+  if (__syncthreads_or(failed != 0 && failed <= b0)) return;
   int i = 0, j = 0;
   if (k0 >= 0) {
     // tiles by columns of the triangle: (0, 0), (1, 0), ..., (1, 1), ...
@@ -264,14 +267,27 @@ __global__ __launch_bounds__(PT) void potrf_step_kernel(double* __restrict__ A, 
 }
 
 // The block row of L^T that the steps left above each diagonal block, to its place
-// below it, and zeros above (a workgroup per 64 x 64 block below the diagonal;
-// grid: first, second block index).
-__global__ __launch_bounds__(PT) void potrf_finish_kernel(double* __restrict__ A, int64_t lda, int64_t n) {
+// below it, and zeros above (a workgroup per 64 x 64 block on or below the diagonal;
+// grid: first, second block index).  After a failed pivot the blocks from the failing
+// one on have no such row: they are only cleared above the diagonal.
+__global__ __launch_bounds__(PT) void potrf_finish_kernel(double* __restrict__ A, int64_t lda, int64_t n,
+                                                          const int* __restrict__ info) {
   __shared__ double S[NB * LD];
-  if (blockIdx.x <= blockIdx.y) return;
+  if (blockIdx.x < blockIdx.y) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t r0 = (int64_t)blockIdx.x * NB, c0 = (int64_t)blockIdx.y * NB;   // c0 + NB <= r0 < n
+  const int64_t r0 = (int64_t)blockIdx.x * NB, c0 = (int64_t)blockIdx.y * NB;   // c0 <= r0 < n
+  const int failed = *info;
+  const bool done = failed == 0 || c0 + NB < failed;
   gdouble* gA = (gdouble*)A;
+  if (r0 == c0) {
+    if (done) return;
+#pragma unroll
+    for (int q = 0; q < NB * NB / PT; ++q) {
+      const int r = wave + 4 * q;
+      if (lane < r && r0 + r < n) gA[c0 + lane + (r0 + r) * lda] = 0.0;
+    }
+    return;
+  }
 #pragma unroll
   for (int q = 0; q < NB * NB / PT; ++q) {
     const int r = wave + 4 * q;
@@ -281,6 +297,7 @@ __global__ __launch_bounds__(PT) void potrf_finish_kernel(double* __restrict__ A
       *p = 0.0;
     }
   }
+  if (!done) return;
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NB * NB / PT; ++q) {
@@ -303,7 +320,7 @@ mk_status potrf_lower(double* A, int64_t n, int64_t lda, int* info_dev, double* 
     MK_CHECK_HIP(hipGetLastError());
   }
   const unsigned nblk = (unsigned)cdiv(n, (int64_t)NB);
-  if (nblk > 1) hipLaunchKernelGGL(potrf_finish_kernel, dim3(nblk, nblk), dim3(PT), 0, st, A, lda, n);
+  hipLaunchKernelGGL(potrf_finish_kernel, dim3(nblk, nblk), dim3(PT), 0, st, A, lda, n, info_dev);
   MK_CHECK_HIP(hipGetLastError());
   return MK_OK;
 }

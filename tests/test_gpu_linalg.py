@@ -47,6 +47,27 @@ def test_potrf_reports_the_failing_pivot(env):
     assert info == 4
 
 
+@pytest.mark.parametrize("n,col", [(50, 7), (300, 201), (300, 256), (300, 257), (2100, 200), (2100, 2099)])
+def test_potrf_before_a_failing_pivot(env, n, col):
+    """The blocks before the failing one hold L (1e-12 relative, as above), the strict upper triangle is zero."""
+    mk, torch = env
+    from mpskit_amd.krylov import potrf_
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + col)
+    X = torch.randn(n + 7, n, dtype=torch.float64, device="cuda", generator=g)
+    G = (X.t() @ X).contiguous()
+    ref = torch.linalg.cholesky(G)
+    G[col - 1, col - 1] = -1.0
+    print("potrf failing", n, col, flush=True)
+    L, info = potrf_(G)
+    torch.cuda.synchronize()
+    assert info == col
+    k = (col - 1) // 64 * 64
+    if k:
+        assert float(torch.linalg.matrix_norm(L[:, :k] - ref[:, :k]) / torch.linalg.matrix_norm(ref[:, :k])) < 1e-12
+    assert bool((torch.triu(L, 1) == 0).all())
+
+
 @pytest.mark.parametrize("m,n", [(2048, 1024), (4096, 2048), (300, 257), (96, 96)])
 def test_cholesky_qr_matches_householder(env, m, n):
     mk, torch = env
