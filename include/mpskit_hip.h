@@ -78,6 +78,11 @@ mk_status mk_ctx_destroy(mk_ctx ctx);
  * order and agrees with the eager one to rounding. */
 mk_status mk_ctx_set_stream(mk_ctx ctx, void* stream);
 mk_status mk_ctx_synchronize(mk_ctx ctx);
+/* Gives back what the context keeps between calls beside its scratch arena: the
+ * streams' workspaces above and the Krylov workspace of mk_eigsolve (kept while it
+ * is at most 1 GiB).  Waits for the GPU; the next call that needs them allocates
+ * again. */
+mk_status mk_ctx_release_workspaces(mk_ctx ctx);
 
 /* ---- derivative operators (prepare) -------------------------------------- */
 

@@ -281,6 +281,16 @@ extern "C" mk_status mk_ctx_synchronize(mk_ctx h) {
   return MK_OK;
 }
 
+extern "C" mk_status mk_ctx_release_workspaces(mk_ctx h) {
+  MK_REQUIRE(h != nullptr, MK_BAD_ARG, "null context");
+  auto* c = reinterpret_cast<Ctx*>(h);
+  MK_CHECK_HIP(hipSetDevice(c->device));
+  MK_CHECK_HIP(hipDeviceSynchronize());   // other streams than the current one may use theirs
+  c->krylovbuf.release();
+  c->gemmws.clear([](void* p) { (void)hipFree(p); });
+  return MK_OK;
+}
+
 // ---------------------------------------------------------------------------
 // C ABI: transfers
 // ---------------------------------------------------------------------------

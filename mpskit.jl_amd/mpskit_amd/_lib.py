@@ -75,6 +75,7 @@ _SIGS = {
     "mk_ctx_destroy": ([_P], _INT),
     "mk_ctx_set_stream": ([_P, _P], _INT),
     "mk_ctx_synchronize": ([_P], _INT),
+    "mk_ctx_release_workspaces": ([_P], _INT),
     "mk_prepare_c": ([_P, _P, _P] + [_I64] * 5 + [_INT, C.POINTER(_P)], _INT),
     "mk_prepare_ac_generic": ([_P, _P, _P, _P] + [_I64] * 7 + [_INT, C.POINTER(_P)], _INT),
     "mk_prepare_ac2_generic": ([_P, _P, _P, _P, _P] + [_I64] * 9 + [_INT, C.POINTER(_P)], _INT),

@@ -38,6 +38,11 @@ class Context:
     def synchronize(self) -> None:
         check(self._lib.mk_ctx_synchronize(self.handle))
 
+    def release_workspaces(self) -> None:
+        """Give back the device memory the context keeps between calls (up to 1 GiB of Krylov workspace
+        and 64 MiB a stream, outside torch's allocator); later calls allocate it again."""
+        check(self._lib.mk_ctx_release_workspaces(self.handle))
+
     def __del__(self):
         h = getattr(self, "handle", None)
         if sys.is_finalizing():      # the HIP runtime may already be torn down

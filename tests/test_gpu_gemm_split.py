@@ -110,6 +110,27 @@ def test_split_gemm_on_many_streams(mk):
         assert torch.equal(out, first)
 
 
+def test_workspaces_are_given_back(mk):
+    """The streams' workspaces and the Krylov workspace (26 columns of 2^20 doubles and more at D = 512)."""
+    import torch
+    T = mk.tensors
+    W, D = T.from_numpy(mk.models.tfim_bulk(1.0)), 512
+    GL, GR = T.randn((D, 3, D)) / D, T.randn((D, 3, D)) / D
+    GL, GR = (T.as_colmajor(0.5 * (E + E.permute(2, 1, 0))) for E in (GL, GR))
+    op = mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(GL, W, W, GR))
+    A, B, x = T.randn((500, 3000)), T.randn((3000, 400)), T.randn((D, 2, D, 2))
+    first, e = mk.gemm(A, B).clone(), op.eigsolve(x, krylovdim=20, maxiter=1, tol=1e-3)[0]
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    op.ctx.release_workspaces()
+    after = torch.cuda.mem_get_info()[0]
+    print("given back", (after - before) >> 20, "MiB", flush=True)
+    assert after - before >= (64 << 20) + 20 * 8 * 4 * D * D
+    op.ctx.release_workspaces()
+    assert torch.equal(mk.gemm(A, B), first)
+    assert op.eigsolve(x, krylovdim=20, maxiter=1, tol=1e-3)[0] == e
+
+
 def test_split_gemm_not_split_under_capture(mk):
     """A captured call takes no shared workspace; replays agree with the eager result."""
     import torch
