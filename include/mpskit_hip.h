@@ -290,7 +290,8 @@ mk_status mk_apply(mk_op op, const double* x, double* y, double alpha, double be
  * comes from a fixed device array of MK_NOALLOC_SCRATCH_MB MiB that the
  * library holds on every GPU it runs on until the process ends (its address
  * is resolved at mk_ctx_create), and the partial tiles of launches split along
- * K from a second one of 64 MiB; the call allocates nothing, creates no
+ * K from a second one of 64 MiB (row padding that the limit below does not count
+ * has 16 MiB more); the call allocates nothing, creates no
  * events and does not synchronise.  An apply whose scratch exceeds the array
  * returns MK_BAD_SHAPE (160 MiB hold the BF16X3 views of a two-site Jordan
  * operator up to d*D = 4096, i.e. D = 2048 at d = 2; FP64 applies of Jordan

@@ -113,14 +113,15 @@ FixedScratch& fixed_scratch() {
 
 // Carve several regions out of the context arena (or out of the calling
 // thread's fixed scratch region, if one is installed).
-mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regions) {
+mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regions, int64_t counted) {
   size_t total = 0;
   for (auto& r : regions) total += align256(r.first);
   void* base = nullptr;
   const FixedScratch& fx = fixed_scratch();
   if (fx.base) {
-    MK_REQUIRE(total <= fx.bytes, MK_BAD_SHAPE,
-               "this apply needs %zu bytes of scratch; the fixed scratch holds %zu", total, fx.bytes);
+    const size_t need = counted < 0 ? total : (size_t)counted;
+    MK_REQUIRE(need <= fx.bytes && total <= fx.bytes + fx.slack, MK_BAD_SHAPE,
+               "this apply needs %zu bytes of scratch; the fixed scratch holds %zu", std::max(need, total), fx.bytes);
     base = fx.base;
   } else {
     MK_TRY(ctx->scratch(total, &base));

@@ -7,6 +7,10 @@
 namespace {
 
 constexpr size_t kNoallocBytes = (size_t)MK_NOALLOC_SCRATCH_MB << 20;
+// The views of x in the layout of the by-block applies have a few more bytes a
+// row than what MK_NOALLOC_SCRATCH_MB counts (K runs and rows padded apart): at most
+// 9.3 MiB at the limit for bonds within a factor of 64.
+constexpr size_t kNoallocSlack = (size_t)16 << 20;
 constexpr int kMaxDevices = 64;
 
 }  // namespace
@@ -14,7 +18,7 @@ constexpr int kMaxDevices = 64;
 // The scratch array (one copy per GPU, held until the process ends).  In host
 // code `scratch` only names the array; its device address is resolved once per
 // device by noalloc_setup and only that address is handed to kernels.
-static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
+static __device__ __align__(256) unsigned char scratch[kNoallocBytes + kNoallocSlack];
 // The K-split workspace of the GEMMs, apart from it, so that an apply splits
 // (and rounds) as mk_apply does whatever its own scratch takes.
 static __device__ __align__(256) unsigned char gemm_scratch[mk::GEMM_WS_BYTES];
@@ -68,6 +72,6 @@ extern "C" mk_status mk_apply_noalloc(mk_op h, const double* x, double* y, doubl
     ws = ptr ? g_ws[dev] : nullptr;
   }
   MK_REQUIRE(ptr != nullptr, MK_HIP_ERROR, "apply_noalloc: scratch array not set up on device %d", dev);
-  FixedScratchGuard guard(ptr, kNoallocBytes, ws);
+  FixedScratchGuard guard(ptr, kNoallocBytes, kNoallocSlack, ws);
   return op_apply(op, x, y, alpha, beta, precision);
 }

@@ -491,6 +491,17 @@ mk_status apply_small(Op* op, const double* x, double* y, double alpha, double b
   return MK_OK;
 }
 
+// What the limit of a fixed scratch region counts the two views of x of a Jordan
+// apply as: rows whose K is one run (one-site: the left view's rows hold all physical
+// states).
+int64_t counted_views(const Op* op, int prec) {
+  if (prec == MK_FP64) return 0;
+  const int64_t M = op->Dl * op->d1, N = op->Dr * op->d2;
+  const bool one = op->kind == OP_AC_JOR;
+  return align256(one ? view_bytes(op->Dl, op->d1 * N, 'A', prec) : view_bytes(M, N, 'A', prec)) +
+         align256(view_bytes(M, N, 'B', prec));
+}
+
 // By-block Jordan apply: the physical term (and the mixed views of x) in one
 // pass over x, then one launch over the output blocks, which also takes in the
 // channel form's last product where its segment lists have room (its first
@@ -519,7 +530,8 @@ mk_status apply_by_block(Op* op, const double* x, double* y, double alpha, doubl
   if (!with_xrl) s1 = s2 = 0;
   void *ma = nullptr, *mb = nullptr;
   double *t1 = nullptr, *t2 = nullptr;
-  MK_TRY(carve(ctx, {{va, &ma}, {vb, &mb}, {s1, (void**)&t1}, {s2, (void**)&t2}}));
+  MK_TRY(carve(ctx, {{va, &ma}, {vb, &mb}, {s1, (void**)&t1}, {s2, (void**)&t2}},
+               with_xrl ? -1 : counted_views(op, prec)));
   if (in_place) t2 = t1;
   BetaSeq bs{beta};
   JordanViews v;
@@ -835,9 +847,12 @@ mk_status apply_ac2_jordan(Op* op, const double* x, double* y, double alpha, dou
     void *ma = nullptr, *mb = nullptr, *mc = nullptr;
     const bool need_a = op->IC.present(), need_b = op->BE.present() || !op->AB.empty();
     const bool need_ca = op->CA.present();
+    const size_t vc = need_ca ? view_bytes(Dl, d1 * N, 'A', prec) : 0;
+    const int64_t counted = (need_a ? align256(view_bytes(M, N, 'A', prec)) : 0) +
+                            (need_b ? align256(view_bytes(M, N, 'B', prec)) : 0) + align256(vc);
     MK_TRY(carve(ctx, {{need_a ? view_bytes(M, N, 'A', prec, ra) : 0, &ma},
                        {need_b ? view_bytes(M, N, 'B', prec, rb) : 0, &mb},
-                       {need_ca ? view_bytes(Dl, d1 * N, 'A', prec) : 0, &mc}}));
+                       {vc, &mc}}, counted));
     if (fused) {
       xa = view_layout(M, N, 'A', prec, ma, ra);
       xb = view_layout(M, N, 'B', prec, mb, rb);

@@ -59,7 +59,8 @@ struct Ctx {
   void* gemm_ws();
 };
 
-mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regions);
+// `counted`: the bytes a fixed scratch region's limit counts them as (-1: their sum).
+mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regions, int64_t counted = -1);
 
 // A fixed scratch region for the calling host thread.  While one is installed
 // (FixedScratchGuard), carve() takes its regions from it instead of the
@@ -67,13 +68,14 @@ mk_status carve(Ctx* ctx, std::initializer_list<std::pair<size_t, void**>> regio
 // with MK_BAD_SHAPE.  Ctx::small() refuses to run while one is installed.
 struct FixedScratch {
   char* base = nullptr;
-  size_t bytes = 0;
+  size_t bytes = 0;          // the limit on what carve() counts
+  size_t slack = 0;          // memory past it, for row padding that is not counted
   void* gemm_ws = nullptr;   // GEMM_WS_BYTES
 };
 FixedScratch& fixed_scratch();
 struct FixedScratchGuard {
-  FixedScratchGuard(void* base, size_t bytes, void* gemm_ws) {
-    fixed_scratch() = FixedScratch{static_cast<char*>(base), bytes, gemm_ws};
+  FixedScratchGuard(void* base, size_t bytes, size_t slack, void* gemm_ws) {
+    fixed_scratch() = FixedScratch{static_cast<char*>(base), bytes, slack, gemm_ws};
   }
   ~FixedScratchGuard() { fixed_scratch() = FixedScratch{}; }
   FixedScratchGuard(const FixedScratchGuard&) = delete;

@@ -135,3 +135,32 @@ def test_noalloc_rejects_oversized_scratch(mk):
     torch.cuda.synchronize()
     assert torch.equal(y1, y2)
     op.free()
+
+
+@pytest.mark.parametrize("model,Dl,Dr,sites,fits", [("tfim", 1617, 3233, 2, True), ("xxz", 1617, 3233, 2, True),
+                                                    ("xxz", 3042, 3441, 1, True), ("xxz", 2288, 2288, 2, True),
+                                                    ("xxz", 2289, 2289, 2, False), ("tfim", 2289, 2289, 2, False)])
+def test_noalloc_limit(mk, model, Dl, Dr, sites, fits):
+    """At the limit: 2 (4 M N + the padding of K to 8) bytes of views for an M x N matrix x, however the by-block
+    applies pad them."""
+    import torch
+    from mpskit_amd._lib import BF16X3, load
+    lib = load()
+    T = mk.tensors
+    W = T.from_numpy(mk.models.tfim_bulk(1.0) if model == "tfim" else mk.models.xxz_bulk(1.0))
+    w = W.shape[0]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(Dl + Dr)
+    GL, GR = T.randn((Dl, w, Dl), g), T.randn((Dr, w, Dr), g)
+    H = mk.JordanMPO_AC2_Hamiltonian(GL, W, W, GR) if sites == 2 else mk.JordanMPO_AC_Hamiltonian(GL, W, GR)
+    op = mk.prepare_operator(H, precisions=("bf16x3",))
+    x = T.randn(op.x_shape, g)
+    y = T.zeros(op.y_shape)
+    print("noalloc limit", model, Dl, Dr, sites, flush=True)
+    op.ctx.sync_stream()
+    s = lib.mk_apply_noalloc(op.handle, T.ptr(x), T.ptr(y), 1.0, 0.0, BF16X3)
+    torch.cuda.synchronize()
+    assert s == (0 if fits else 1), lib.mk_last_error()
+    if fits:
+        assert torch.equal(y, op(x, precision="bf16x3"))
+    op.free()
