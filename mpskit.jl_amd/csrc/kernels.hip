@@ -239,9 +239,20 @@ __global__ void mpo_mid_wide_kernel(const double* __restrict__ t1, const double*
     const int64_t c = t / nout;
     const double* w = RIGHT ? O + q % wl + wl * (q / wl) : O + wl * (q % d + d * d * (int64_t)(q / d));
     double s = 0.0;
-    for (int i = 0; i < nin; ++i) {
-      const double ov = RIGHT ? w[(int64_t)wl * d * i] : w[i % wl + (int64_t)wl * d * (i / wl)];
-      if (ov != 0.0) s += t1[m + D1 * (i + (int64_t)nin * c)] * ov;
+    if constexpr (RIGHT) {
+      for (int i = 0; i < nin; ++i) {
+        const double ov = w[(int64_t)wl * d * i];
+        if (ov != 0.0) s += t1[m + D1 * (i + (int64_t)nin * c)] * ov;
+      }
+    } else {
+      // by (h, g): with the index of an input divided by wl instead, the left transfer
+      // with w = 17 at D = 128 takes 106 us, so 86
+      const double* in = t1 + m + D1 * ((int64_t)nin * c);
+      for (int h = 0; h < d; ++h, w += (int64_t)wl * d)
+        for (int g = 0; g < wl; ++g, in += D1) {
+          const double ov = w[g];
+          if (ov != 0.0) s += *in * ov;
+        }
     }
     t2[idx] = s;
   }

@@ -106,3 +106,20 @@ def test_prepared_transfer_rejects_bad_shapes(mk):
     with pytest.raises(mk.SpaceMismatch):
         op(T.from_numpy(rng.standard_normal((6, 5))))
     op.free()
+
+
+@pytest.mark.parametrize("w,wr,d,D", [(17, 17, 2, 33), (16, 17, 2, 20), (17, 3, 2, 20), (3, 17, 2, 20), (12, 9, 3, 40)])
+def test_wide_mpo_transfers(mk, w, wr, d, D):
+    """MPO bonds past (and at) the 32 inputs that the MPO step holds in registers."""
+    T = mk.tensors
+    rng = np.random.default_rng(w + wr)
+    O4 = rng.standard_normal((w, d, d, wr)) * (rng.random((w, d, d, wr)) < 0.7)
+    A, Ab = rng.standard_normal((D + 1, d, D)), rng.standard_normal((D, d, D + 2))
+    x = rng.standard_normal((D, w, D + 1))
+    print("wide mpo transfers", w, wr, d, D, flush=True)
+    y = T.to_numpy(mk.transfer_left(*(T.from_numpy(t) for t in (x, O4, A, Ab))))
+    assert rel(y, O.transfer_left_mpo(x, O4, A, Ab)) < TOL["fp64"]
+    Ar, Abr = rng.standard_normal((D, d, D + 1)), rng.standard_normal((D + 2, d, D))
+    v = rng.standard_normal((D + 1, wr, D))
+    y = T.to_numpy(mk.transfer_right(*(T.from_numpy(t) for t in (v, O4, Ar, Abr))))
+    assert rel(y, O.transfer_right_mpo(v, O4, Ar, Abr)) < TOL["fp64"]
