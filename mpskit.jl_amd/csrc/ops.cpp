@@ -547,8 +547,12 @@ mk_status apply_by_block(Op* op, const double* x, double* y, double alpha, doubl
     } else {
       MixedView t;
       if (P) MK_TRY(k_phys2(P, x, Dl, d1, Dr, d2, alpha, bs.next(), y, st));
-      MK_TRY(convert_view(ctx, x, M, N, M, 'A', prec, &t, ma, d2));
-      MK_TRY(convert_view(ctx, x, M, N, M, 'B', prec, &t, mb, d1));
+      // (at the ends of a chain one of the two may have no reader)
+      bool need_a = with_xrl, need_b = false;
+      for (const Op::JProb& jp : op->jprobs)
+        for (const Op::JSeg& sg : jp.seg) (sg.kind == 'R' || sg.kind == 'I' ? need_a : need_b) = true;
+      if (need_a) MK_TRY(convert_view(ctx, x, M, N, M, 'A', prec, &t, ma, d2));
+      if (need_b) MK_TRY(convert_view(ctx, x, M, N, M, 'B', prec, &t, mb, d1));
     }
     v.xa = a.hi; v.ka = a.kpad; v.alo = bf ? static_cast<char*>(a.lo) - static_cast<char*>(a.hi) : 0;
     v.xb = b.hi; v.kb = b.kpad; v.blo = bf ? static_cast<char*>(b.lo) - static_cast<char*>(b.hi) : 0;
