@@ -178,8 +178,9 @@ enum TileKind { TK_64 = 0, TK_128 = 1, TK_256 = 2 };
 inline int tile_m(int kind) { return kind == TK_64 ? 64 : kind == TK_128 ? 128 : 256; }
 inline int tile_n(int kind) { return tile_m(kind); }
 bool tile_valid(int prec, int kind);
-// Workgroups of one persistent launch: resident workgroups per CU x CUs, capped by the tiles.
-int group_grid(int prec, int kind, GemmShape sh, int total_tiles);
+// Workgroups of one persistent launch: resident workgroups per CU x CUs, capped by the tiles
+// (f64_buf: the FP64 kernel, as in GemmGroup).
+int group_grid(int prec, int kind, int f64_buf, int total_tiles);
 mk_status gemm_f64_group(const GemmGroup& g, int kind, GemmShape sh, int grid, hipStream_t st);
 // Whether the FP64 problems may run on the LDS-DMA kernel
 // with tile kind `kind` (in-tile offsets below 2 GiB): 0 no, 1 on its form for

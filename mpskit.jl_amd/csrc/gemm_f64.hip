@@ -709,22 +709,25 @@ mk_status launch_group(const GemmGroup& g, GemmShape sh, int grid, hipStream_t s
   return MK_OK;
 }
 
+// Workgroups of the grouped kernel for `fit` (launch_path) that a CU holds, taken of
+// one storage order.
 template <int BM, int BN>
-int occupancy() {
-  static const int occ = [] {
+int occupancy(int fit) {
+  auto of = [](auto kern) {
     int n = 0;
-    const hipError_t e =
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemm_f64_kernel<BM, BN, false, false, GemmGroup>, NT, 0);
-    if (e != hipSuccess) n = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, NT, 0) != hipSuccess) n = 1;
     return n > 0 ? n : 1;
-  }();
-  return occ;
+  };
+  static const int occ[3] = {of(gemm_f64_kernel<BM, BN, false, false, GemmGroup>),
+                             of(gemm_f64_dma_kernel<BM, BN, false, false, true, GemmGroup>),
+                             of(gemm_f64_dma_kernel<BM, BN, false, false, false, GemmGroup>)};
+  return occ[f64_direct() ? fit : BUF_NO];
 }
 
 }  // namespace
 
-int f64_group_grid(int kind, int total_tiles, int cus) {
-  const int occ = kind == TK_128 ? occupancy<128, 128>() : occupancy<64, 64>();
+int f64_group_grid(int kind, int fit, int total_tiles, int cus) {
+  const int occ = kind == TK_128 ? occupancy<128, 128>(fit) : occupancy<64, 64>(fit);
   return (int)std::min<int64_t>(total_tiles, (int64_t)occ * cus);
 }
 

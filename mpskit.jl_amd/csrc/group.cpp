@@ -16,15 +16,14 @@ bool tile_valid(int prec, int kind) {
   return kind >= TK_64 && kind <= TK_256;
 }
 
-int group_grid(int prec, int kind, GemmShape sh, int total_tiles) {
-  (void)sh;
+int group_grid(int prec, int kind, int f64_buf, int total_tiles) {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) {
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) cus = v;
   }
   if (total_tiles <= 0) return 0;
-  return prec == MK_FP64 ? f64_group_grid(kind, total_tiles, cus) : mixed_group_grid(prec, kind, total_tiles, cus);
+  return prec == MK_FP64 ? f64_group_grid(kind, f64_buf, total_tiles, cus) : mixed_group_grid(prec, kind, total_tiles, cus);
 }
 
 namespace {
@@ -149,7 +148,7 @@ mk_status GroupPlan::build(int k, hipStream_t launched_on) {
   // relative pointers keep their offsets in the low bits and the base slots
   // are 16-byte aligned, so the alignment test reads the offsets
   f64_buf = prec == MK_FP64 && (k == TK_64 || k == TK_128) ? f64_buf_ok(specs.data(), (int)specs.size(), sh, k) : 0;
-  grid = group_grid(prec, k, sh, total);
+  grid = group_grid(prec, k, f64_buf, total);
   return MK_OK;
 }
 

@@ -18,7 +18,7 @@
 
 namespace mk {
 
-int f64_group_grid(int kind, int total_tiles, int cus);
+int f64_group_grid(int kind, int fit, int total_tiles, int cus);
 int mixed_group_grid(int prec, int kind, int total_tiles, int cus);
 bool mixed_256_ok();   // whether the 256 x 256 mixed kernel may be chosen
 
