@@ -4,6 +4,10 @@ Tolerances (relative Frobenius error of y):
   fp64   <= 1e-12   (the reference arithmetic)
   fp32   <= 1e-5    (FP32 MFMA products, fp32 accumulation)
   bf16x3 <= 3e-4    (hi*hi + hi*lo + lo*hi bf16 products, fp32 accumulation)
+
+The smallest Jordan applies run in FP64 whatever is asked for (the golden vectors of
+both Jordan kinds, D = 37 and 45 here): there the mixed loops check that the call is
+taken and right, and D >= 130 checks the arithmetics.
 """
 import numpy as np
 import pytest
@@ -258,3 +262,40 @@ def test_eigsolve_lowest_eigenpair(mk, prec):
     v = host(mk, vec).reshape(-1, order="F")
     r = Hd @ v - e_ref * v
     assert np.linalg.norm(r) < 1e-9
+
+
+@pytest.mark.parametrize("prec", PRECS)
+def test_eigsolve_past_the_smallest_applies(mk, prec):
+    """Krylov steps in the arithmetic asked for (D = 200, past the applies that are always FP64): the refined
+    eigenpair has the FP64 residual asked for, and the eigenvalue of the FP64 solve."""
+    import torch
+    T = mk.tensors
+    rng = np.random.default_rng(5)
+    D, part = 200, [0, 2, 1, 3, 4]
+    W = dev(mk, mk.models.xxz_bulk(0.5))
+
+    def env():
+        # blocks symmetric, or (S+ and S-) transposes of each other, with one low state
+        E = rng.standard_normal((D, 5, D)) / np.sqrt(D)
+        E = 0.5 * (E + E[:, part].transpose(2, 1, 0))
+        u = rng.standard_normal(D)
+        u /= np.linalg.norm(u)
+        E[:, 0] = E[:, 4] = 0.0
+        return E, u
+    (GLn, ul), (GRn, ur) = env(), env()
+    # GL's finished level and GR's not-started one are the blocks' own Hamiltonians; their first / last level is the identity
+    hl, hr = (0.5 * (h + h.T) for h in (rng.standard_normal((D, D)) / np.sqrt(D), rng.standard_normal((D, D)) / np.sqrt(D)))
+    GLn[:, 4], GRn[:, 0] = hl - 8.0 * np.outer(ul, ul), hr - 8.0 * np.outer(ur, ur)
+    op = mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(dev(mk, GLn), W, W, dev(mk, GRn)), precisions=PRECS)
+    x0 = dev(mk, rng.standard_normal((D, 2, D, 2)))
+    y, y64 = op(x0, precision=prec), op(x0)
+    assert torch.equal(y, y64) == (prec == "fp64")
+    print("eigsolve past the smallest", prec, flush=True)
+    val, vec, info = op.eigsolve(x0, krylovdim=30, maxiter=100, tol=1e-9, precision=prec)
+    print(f"  E={val:.12f} info={info}", flush=True)
+    assert info["converged"]
+    r = op(vec) - val * vec
+    assert float(torch.linalg.vector_norm(r)) < 2e-9 * float(torch.linalg.vector_norm(vec))
+    ref = op.eigsolve(x0, krylovdim=30, maxiter=100, tol=1e-9)[0]
+    # Hermitian: the error of a Ritz value is at most the residual's square over the gap, and the residual itself
+    assert abs(val - ref) < 4e-9

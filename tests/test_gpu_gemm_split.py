@@ -1,7 +1,8 @@
 """GEMM launches whose tiles are cut along K (mk_gemm, all three arithmetics).
 
 Sizes whose tiles do not fill the GPU are split: all of them, or those of the
-last round.  Edges: one tile with a long K, K that is not a multiple of a step
+last round.  Operands too large for 32-bit offsets within a tile take the kernels
+that the usual ones fall back to.  Edges: one tile with a long K, K that is not a multiple of a step
 or of the slices, odd sizes and leading dimensions, a last round of few tiles,
 beta != 0 (C is read by the reduction only).  Against float64 torch.
 
@@ -68,6 +69,52 @@ def test_tall_operand(mk, M, K):
     print("tall gemm", M, K, flush=True)
     out, ref = mk.gemm(A, B), A @ B
     assert float(torch.linalg.vector_norm(out - ref)) <= bound("fp64", K) * float(torch.linalg.vector_norm(ref))
+
+
+def mk_gemm(mk, A, lda, B, ldb, C, M, N, K, ta, tb, prec):
+    """C = -0.5 op(A) op(B) + 2 C through the C ABI, with leading dimensions of any length."""
+    import ctypes
+    from mpskit_amd._lib import PREC_NAMES, check, load
+    pa, pb, pc = (ctypes.c_void_p(t.data_ptr()) for t in (A, B, C))
+    check(load().mk_gemm(mk.derivatives.default_context().handle, int(ta), int(tb), M, N, K, -0.5, pa, lda, pb, ldb, 2.0,
+                         pc, M, PREC_NAMES[prec]))
+
+
+@pytest.mark.parametrize("ta,tb,K,lda,ldb", [(False, False, 1031, 1 << 18, 1031), (True, False, 1031, 2_200_000, 1040),
+                                             (False, True, 520, 131, 1 << 19), (True, True, 514, 520, 530_001)])
+def test_fp64_past_the_32_bit_offsets(mk, ta, tb, K, lda, ldb):
+    """Operands whose tiles span 2 GiB and more run on the branching kernel, whole and cut along K."""
+    import torch
+    M, N = 130, 70
+    g = torch.Generator(device="cuda")
+    g.manual_seed(K)
+    # column-major with leading dimensions lda, ldb: the columns are rows of the torch tensors
+    A = torch.full((M if ta else K, lda), float("nan"), dtype=torch.float64, device="cuda")
+    B = torch.full((K if tb else N, ldb), float("nan"), dtype=torch.float64, device="cuda")
+    a, b = A[:, :K if ta else M], B[:, :N if tb else K]
+    a.normal_(generator=g)
+    b.normal_(generator=g)
+    C = mk.tensors.randn((M, N), g)
+    ref = -0.5 * ((a if ta else a.t()) @ (b if tb else b.t())) + 2.0 * C
+    print("branching fp64 gemm", ta, tb, K, lda, ldb, flush=True)
+    mk_gemm(mk, A, lda, B, ldb, C, M, N, K, ta, tb, "fp64")
+    assert float(torch.linalg.vector_norm(C - ref)) <= bound("fp64", K) * float(torch.linalg.vector_norm(ref))
+
+
+@pytest.mark.parametrize("prec,K", [("bf16x3", 4_200_003), ("fp32", 2_100_005)])
+@pytest.mark.parametrize("M,N", [(70, 9), (129, 40)])
+def test_mixed_past_the_32_bit_offsets(mk, prec, K, M, N):
+    """Operands of which 256 rows span 2 GiB and more run on the register-staged kernel, cut along K."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(K)
+    # rows of K entries on both sides (transposed storage of A)
+    A, B = (torch.randn((n, K), dtype=torch.float64, device="cuda", generator=g) for n in (M, N))
+    C = mk.tensors.randn((M, N), g)
+    ref = -0.5 * (A @ B.t()) + 2.0 * C
+    print("register-staged mixed gemm", prec, M, N, K, flush=True)
+    mk_gemm(mk, A, K, B, K, C, M, N, K, True, False, prec)
+    assert float(torch.linalg.vector_norm(C - ref)) <= bound(prec, K) * float(torch.linalg.vector_norm(ref))
 
 
 def test_split_gemm_repeats_bitwise(mk):

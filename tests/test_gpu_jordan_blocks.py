@@ -183,6 +183,32 @@ def test_full_blocks(mk, w, Dl, Dr):
     check(op, x, y0, lambda g: ac(g(GLi), g(Wd), g(GRi), g(x)), max(Dl, Dr))
 
 
+@pytest.mark.parametrize("name", ["tfim", "xxz", "j1j2", "exp", "onsite"])
+@pytest.mark.parametrize("Dl,Dr", [(210, 203), (193, 260)])
+def test_mixed_arithmetic_is_used(mk, name, Dl, Dr):
+    """The smallest applies run in FP64 whatever is asked for (64 x 64 is one); past that line each arithmetic is
+    its own, on runs of K with every kind of padding."""
+    import torch
+    T = mk.tensors
+    W = T.from_numpy(chain(mk, name))
+    for D1, D2, small in ((Dl, Dr, False), (64, 64, True)):
+        GL, GR, GLi, GRi = envs(mk, D1, W.shape[0], D2, W.shape[3])
+        x2, x1 = rnd(mk, (D1, 2, D2, 2), 3), rnd(mk, (D1, 2, D2), 3)
+        for H, x, f in ((mk.JordanMPO_AC2_Hamiltonian(GL, W, W, GR), x2, lambda g: ac2(g(GLi), g(W), g(W), g(GRi), g(x2))),
+                        (mk.JordanMPO_AC_Hamiltonian(GL, W, GR), x1, lambda g: ac(g(GLi), g(W), g(GRi), g(x1)))):
+            op = mk.prepare_operator(H, precisions=PRECS)
+            print("mixed", name, D1, D2, x.dim(), flush=True)
+            check(op, x, torch.zeros_like(x), f, max(D1, D2))
+            y = {p: op(x, precision=p) for p in PRECS}
+            if small and name in ("tfim", "onsite"):
+                assert torch.equal(y["bf16x3"], y["fp64"]) and torch.equal(y["fp32"], y["fp64"])
+            if not small:
+                n64 = float(torch.linalg.vector_norm(y["fp64"]))
+                for p in ("fp32", "bf16x3"):   # off by a few roundings of the operands, not by those of FP64
+                    assert 1e-9 < float(torch.linalg.vector_norm(y[p] - y["fp64"])) / n64 < 1e-4, p
+                assert not torch.equal(y["fp32"], y["bf16x3"])
+
+
 @pytest.mark.parametrize("name", ["tfim", "xxz", "onsite"])
 def test_batch_of_uneven_bonds(mk, name):
     import torch
