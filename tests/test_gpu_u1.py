@@ -106,6 +106,36 @@ def test_charge_blocks_are_for_spin_one_half(mk):
     assert torch.equal(op(x), y)
 
 
+def test_block_apply_with_a_field(mk):
+    """On-site terms, which a two-site operator keeps in its physical term: dense and compact blocks, and a batch,
+    against the dense operator."""
+    from mpskit_amd.u1 import compact_charge_blocks, u1_gauge2
+    L, nup = 10, 5
+    psi = mk.U1FiniteMPS.random(L, nup, lambda k, q: 16, seed=5)
+    Ws = [W.copy() for W in mk.models.xxz(L, 0.8)]
+    for j, W in enumerate(Ws):
+        W[0, :, :, -1] += (0.3 + 0.1 * j) * np.diag([0.5, -0.5])
+    H = mk.FiniteMPOHamiltonian(Ws)
+    envs = mk.FiniteEnvironments(psi, H)
+    pos = L // 2 - 1
+    for p in range(pos):
+        u1_gauge2(psi, p, "right", psi.AC2(p), 10 ** 6)
+    GL, GR, x = envs.leftenv(pos, psi), envs.rightenv(pos + 1, psi), psi.AC2(pos)
+    ops = [mk.prepare_operator(mk.JordanMPO_AC2_Hamiltonian(GL, H[pos], H[pos + 1], GR),
+                               precisions=("fp64", "fp32", "bf16x3")) for _ in range(3)]
+    ref = ops[0](x)
+    for op in ops[1:]:
+        mk.set_charge_blocks(op, psi.bonds[pos], psi.bonds[pos + 2])
+    b = mk.BatchedDerivative([ops[1], ops[0]])
+    lay = compact_charge_blocks(ops[2], x.shape)
+    for prec in ("fp64", "fp32", "bf16x3"):
+        print("field", prec, flush=True)
+        assert rel(ops[1](x, precision=prec), ref) < TOL[prec]
+        assert rel(lay.scatter(ops[2](lay.gather(x), precision=prec)), ref) < TOL[prec]
+        for y in b.unpack(b.apply(b.pack([x, x]), prec)):
+            assert rel(y, ref) < TOL[prec]
+
+
 def test_block_apply_without_a_physical_term(mk):
     """An MPO of environments only: outside the blocks y is zero whatever its memory held, alone and in a batch."""
     import torch
