@@ -103,7 +103,11 @@ void* Ctx::gemm_ws() {
         b.ptr = nullptr;   // the table's from here on
         return p;
       },
-      [] { return hipDeviceSynchronize() == hipSuccess; });
+      [] {
+        if (hipDeviceSynchronize() == hipSuccess) return true;
+        (void)hipGetLastError();   // refused while another thread captures a graph
+        return false;
+      });
 }
 
 FixedScratch& fixed_scratch() {
